@@ -155,6 +155,35 @@ typedef struct chx_unit {
 /* Blocks per group of the grouped block layout. */
 #define CHX_BLOCK_GROUP 64
 
+/* Resident PCG (optional; chx_instance::res_plan).  The rows of an instance
+ * are put in a canonical order of compact mesh patches and cut into parts of
+ * `res_part_rows` consecutive positions (256, 512 or 1024); one workgroup
+ * holds a part's matrix blocks on chip for the whole solve.  Limits: rows
+ * per leaf (a wavefront's share of a part) and per largest part, upper and
+ * lower blocks of a row, halo rows (rows of other parts that a part reads)
+ * and ghost blocks (blocks of halo rows whose column is in the part).
+ *
+ * res_plan (32-bit words): 8 words per part {rows, halo rows, word offset of
+ * its halo list, ghost blocks, word offset of its ghost list, 0, 0, 0}; then
+ * over the n_rows positions: the row, (lower blocks | upper blocks << 4),
+ * the row's export index (CHX_RES_NONE: no other part reads it), and
+ * CHX_RES_HELD planes of (local index of the upper block's column) |
+ * (product slot << 16); then the halo lists {row, export index} and ghost
+ * lists {value slot, local index of the source row | product slot << 16}.
+ * Local indices: position in the part, or CHX_RES_PART_MAX + halo index.
+ * A product slot is (place among the target row's lower blocks) *
+ * CHX_RES_PART_MAX + (target's position in the part); 0xffff: none. */
+#define CHX_RES_LEAF 64
+#define CHX_RES_PART_MAX 1024
+#define CHX_RES_HELD 6
+#define CHX_RES_HALO_MAX 512
+#define CHX_RES_GHOST_MAX 512
+#define CHX_RES_NONE 0xffffffffu
+/* 64-bit words of `xbuf` before the instances' exchange areas, and of one
+ * instance's area with `parts` parts and `exports` exported rows. */
+#define CHX_RES_CONTROL_WORDS 4352
+#define CHX_RES_XWORDS(parts, exports) (2ull * (16ull * (parts) + 3ull * (exports)))
+
 /* One cloth instance: every array is the instance's own device memory, with
  * indices local to the instance, so the off-diagonal pattern is exactly the
  * reference's (ChysX/src/sparse/block_csr.h:59-135).  Slots of the gather
@@ -238,6 +267,11 @@ typedef struct chx_instance {
     float contact_friction;          /* Coulomb mu (0: off)                                  */
     float contact_friction_eps;      /* slip regularisation eps_u [m]                        */
     double tol;                      /* stop at ||r|| <= tol*||b||; <= 0: run max_iter       */
+    const unsigned* res_plan;        /* resident PCG plan, or NULL (no resident solve)       */
+    int res_part_rows;               /* rows per part                                        */
+    int res_parts;                   /* ceil(n_rows / res_part_rows)                         */
+    int res_exports;                 /* exported rows                                        */
+    unsigned res_xbase;              /* first word of the instance's exchange area in xbuf   */
 } chx_instance;
 
 /* A batch of instances advanced together.  Work lists are device int4
@@ -301,7 +335,19 @@ typedef struct chx_cloth_batch {
     int pcg_form;                    /* FP32 cloth instances: 0 one grid barrier per   */
                                      /* iteration (the two reductions merged), 1 two  */
                                      /* barriers per iteration                        */
-    int pad2;
+    int res_grid;                    /* resident PCG: workgroups of the launch (0: the      */
+                                     /* streaming kernels), dealt to res_groups groups    */
+    unsigned long long* xbuf;        /* control words and exchange areas of the resident  */
+                                     /* PCG; zero before the first launch that uses it    */
+    const int* res_items;            /* [res_n_items][4]: instance, parts, first rank, 0; */
+                                     /* instance-table batches, by falling parts          */
+    int res_n_items;
+    int res_n_big;                   /* leading items of more parts than a group has      */
+                                     /* workgroups: solved in list order by the ranks     */
+                                     /* from their first rank on                          */
+    int res_groups;
+    int res_pad;
+    unsigned long long res_xwords;   /* 64-bit words of xbuf                              */
 } chx_cloth_batch;
 
 /* ---- errors and runtime ------------------------------------------------- */
@@ -316,6 +362,8 @@ int chx_device_info(int* cu_count, int* max_pcg_blocks, int* occupancy_blocks_pe
 /* Co-resident workgroups of one form of the persistent PCG kernel on the
  * current device (the grid cap of a launch with those settings). */
 int chx_pcg_grid_limit(int lanes_per_row, int bf16_blocks, int no_lds_staging, int* max_blocks);
+/* The same for the resident PCG kernel (one workgroup per compute unit). */
+int chx_resident_grid_limit(int* max_blocks);
 
 /* Device memory: replaces CudaArray<T> (ChysX/src/memory/cuda_array.h:64-284,
  * cuda_array.cu:41-90). */

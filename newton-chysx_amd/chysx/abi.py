@@ -26,6 +26,7 @@ _SIGS = {
     "chx_device_count": (_I, [_P]),
     "chx_device_info": (_I, [_P, _P, _P]),
     "chx_pcg_grid_limit": (_I, [_I, _I, _I, _P]),
+    "chx_resident_grid_limit": (_I, [_P]),
     "chx_malloc": (_I, [_P, _S]),
     "chx_free": (_I, [_P]),
     "chx_get_device": (_I, [_P]),

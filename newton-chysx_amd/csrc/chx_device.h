@@ -298,6 +298,9 @@ struct Inst {
     float dt, damping, gx, gy, gz;
     int max_iter;
     double tol;
+    gp<const unsigned> res_plan;
+    int res_part_rows, res_parts, res_exports;
+    unsigned res_xbase;
 };
 
 template <class P>
@@ -362,6 +365,11 @@ __device__ __forceinline__ Inst make_inst(P d) {
     I.gz = d->gz;
     I.max_iter = d->max_iter;
     I.tol = d->tol;
+    I.res_plan = glb(d->res_plan);
+    I.res_part_rows = d->res_part_rows;
+    I.res_parts = d->res_parts;
+    I.res_exports = d->res_exports;
+    I.res_xbase = d->res_xbase;
     return I;
 }
 
@@ -572,8 +580,11 @@ __device__ __forceinline__ void backoff(unsigned& level) {
 // counter may already be changing in the next phase when a slow workgroup
 // leaves the barrier; the snapshot of this barrier is only rewritten two
 // barriers later, which needs that workgroup's arrival first.
+//
+// With `progress` (a word that working workgroups keep changing) a wait may
+// last as long as that word changes: its bound restarts at every change.
 __device__ __forceinline__ bool grid_sync(const Barrier& bar, unsigned nblocks, int snap = -1,
-                                          unsigned* active = nullptr) {
+                                          unsigned* active = nullptr, unsigned* progress = nullptr) {
     unsigned* sync = bar.sync;
     __shared__ int s_ok;
     __shared__ unsigned s_active;
@@ -619,14 +630,22 @@ __device__ __forceinline__ bool grid_sync(const Barrier& bar, unsigned nblocks, 
             // after lane 0's release fence in program order
             st_relaxed(&sync[SYNC_FLAGS + kFlagStride * lane], gen + 1u);
         } else if (lane == 0) {
-            const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
-            unsigned level = 0, polls = 0;
+            unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+            unsigned level = 0, polls = 0, seen = progress != nullptr ? ld_relaxed(progress) : 0u;
             while (ld_relaxed(flag) == gen) {
                 if ((++polls & 15u) == 0u && ld_relaxed(&sync[SYNC_ABORT]) != 0u) {
                     ok = 0;
                     break;
                 }
                 if (__builtin_amdgcn_s_memrealtime() - t0 > bar.ticks) {
+                    if (progress != nullptr) {
+                        const unsigned now = ld_relaxed(progress);
+                        if (now != seen) {
+                            seen = now;
+                            t0 = __builtin_amdgcn_s_memrealtime();
+                            continue;
+                        }
+                    }
                     unsigned waiting = 0;
                     for (unsigned q = 0; q < kSyncGroups; ++q) waiting += ld_relaxed(&sync[SYNC_XCOUNT + 64 * q]);
                     st_relaxed(&sync[SYNC_SEEN], ld_relaxed(&sync[SYNC_COUNT]));

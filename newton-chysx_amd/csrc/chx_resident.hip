@@ -1,0 +1,604 @@
+// Resident block-Jacobi PCG of the FP32 cloth instances: a workgroup keeps
+// its part of an instance's matrix in registers and its vectors in registers
+// and LDS from the first product to the last, so an iteration reads no
+// matrix from memory.  What crosses workgroups in an iteration is the halo
+// rows of q = A p and five partial sums, in one hop.
+//
+// Why: streaming the matrix every iteration cost 20.5 ms per solve of the
+// 512-cloth batch (2.08 M rows, 66 iterations on average), set by the
+// L1-L2 stream, and 19 us per iteration of one 256x256 cloth, set by the
+// grid barrier's cache write-backs.  A CU has 512 KB of registers: 1024 rows
+// of a sheet's matrix (six upper blocks a row) take 221 KB, so 256 CUs hold
+// 262,144 rows, and the instances of a batch are independent: they are
+// solved one after another by gangs of ceil(rows / 1024) workgroups.
+//
+// Arithmetic: the single-barrier recurrence of pcg1_kernel (chx_step.hip),
+// operation for operation; every row sums its diagonal product, its lower
+// blocks and its upper blocks in column order.  A row's upper blocks are in
+// its thread's registers: it forms A_ij p_j for itself and A_ij^T p_i for
+// row j, which it leaves in row j's product slot in LDS.  Blocks between
+// parts are held by both (the second copy is a "ghost block").  Halo rows'
+// r, z and p are kept by every part that reads them, updated from the
+// published q with the same operations as by their owner.
+//
+// Inner products: FP64, one sum per 64-row leaf (a wavefront), combined over
+// the leaves of the instance by a fixed binary tree that does not depend on
+// how many leaves a part has: the same bits for every part size and gang.
+//
+// Exchange: 64-bit words {value, tag}, the tag naming launch and phase, so a
+// reader needs no ordering between words and no cache maintenance: it reads
+// a word until its tag is the awaited one.  Words alternate between two
+// slots; slot t is rewritten in phase t + 2, which its writer enters only
+// after every part's sums of phase t + 1, sent after their reads of phase t.
+#include <algorithm>
+#include <mutex>
+
+#include "chx_pcg.h"
+#include "chx_resident.h"
+
+namespace chx {
+namespace {
+
+constexpr int kThreads = 512;  // two waves per SIMD with 256 VGPRs each
+constexpr int kWaves = kThreads / kWave;
+constexpr int kSlots = CHX_RES_PART_MAX / kThreads;  // own rows per thread
+constexpr int kHeld = CHX_RES_HELD;
+constexpr unsigned kPart = CHX_RES_PART_MAX;
+constexpr int kLeaves = CHX_RES_PART_MAX / CHX_RES_LEAF;
+constexpr int kSums = 5;  // rho, sigma, delta, gamma, ||r||^2 (set-up: ||b||^2 in place of sigma)
+constexpr int kMaxParts = 256;
+constexpr unsigned kNoSlot = 0xffffu;
+constexpr unsigned kExit = 0xffffffu;  // mailbox item: nothing left
+static_assert(CHX_RES_LEAF == kWave && kSlots == 2 && kLeaves == 16, "a leaf per wave and slot");
+static_assert(CHX_RES_HALO_MAX <= kThreads && CHX_RES_GHOST_MAX <= kThreads, "one halo row and ghost block a thread");
+
+typedef unsigned long long u64;
+
+__device__ __forceinline__ u64 ld64(const u64* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st64(u64* p, u64 v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ u64 tagged(unsigned v, unsigned tag) { return (u64(tag) << 32) | v; }
+
+struct ResLds {
+    f3 prod[kHeld * CHX_RES_PART_MAX];             // transposed products, by target row
+    f3 p[CHX_RES_PART_MAX + CHX_RES_HALO_MAX];     // source vector: own rows, halo rows
+    float diag[6][CHX_RES_PART_MAX];
+    f3 x[CHX_RES_PART_MAX];
+    double leaf[kLeaves][kSums];
+    double tot[8];
+    int bad_sums, bad_halo;  // a wait gave up (two words: each read before the other's next write)
+    unsigned mail;   // mailbox word of the workgroup
+};
+
+// Bounded wait of one lane: true while it may go on.  After the bound the
+// solve is aborted for every workgroup (the report of grid_sync).
+struct Watch {
+    const Barrier& bar;
+    u64 t0;
+    unsigned polls = 0;
+    __device__ explicit Watch(const Barrier& b) : bar(b), t0(__builtin_amdgcn_s_memrealtime()) {}
+    __device__ bool again(u64* progress, unsigned& seen) {
+        unsigned* sync = bar.sync;
+        if ((++polls & 15u) == 0u && ld_relaxed(&sync[SYNC_ABORT]) != 0u) return false;
+        if (__builtin_amdgcn_s_memrealtime() - t0 <= bar.ticks) return true;
+        if (progress != nullptr) {
+            const unsigned now = unsigned(ld64(progress));
+            if (now != seen) {
+                seen = now;
+                t0 = __builtin_amdgcn_s_memrealtime();
+                return true;
+            }
+        }
+        st_relaxed(&sync[SYNC_SEEN], 0u);
+        st_relaxed(&sync[SYNC_WAITING], 1u);
+        st_relaxed(&sync[SYNC_GRID], gridDim.x);
+        st_relaxed(&sync[SYNC_ABORT], 1u);
+        st_relaxed(&sync[SYNC_STATUS], 1u);
+        if (bar.status_host != nullptr)
+            __hip_atomic_store(bar.status_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        return false;
+    }
+};
+
+// N tagged words from p on; false: the wait was given up.
+template <int N>
+__device__ __forceinline__ bool await(const u64* p, unsigned tag, unsigned (&v)[N], const Barrier& bar) {
+    u64 w[N];
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < N; ++k) w[k] = ld64(p + k);
+#pragma unroll
+    for (int k = 0; k < N; ++k) ok = ok && unsigned(w[k] >> 32) == tag;
+    if (!ok) {
+        Watch watch(bar);
+        unsigned seen = 0;
+        do {
+            if (!watch.again(nullptr, seen)) return false;
+#pragma unroll
+            for (int k = 0; k < N; ++k) w[k] = ld64(p + k);
+            ok = true;
+#pragma unroll
+            for (int k = 0; k < N; ++k) ok = ok && unsigned(w[k] >> 32) == tag;
+        } while (!ok);
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = unsigned(w[k]);
+    return true;
+}
+
+__device__ __forceinline__ f3 mv9t(const float (&m)[9], f3 v) {
+    const float b[9] = {m[0], m[3], m[6], m[1], m[4], m[7], m[2], m[5], m[8]};
+    return mv9(b, v);
+}
+__device__ __forceinline__ f3 mv_sym(const float (&u)[6], f3 v) {
+    const float a[9] = {u[0], u[1], u[2], u[1], u[3], u[4], u[2], u[4], u[5]};
+    return mv9(a, v);
+}
+__device__ __forceinline__ void inverse_sym(const float (&u)[6], float (&mi)[6], float (&full)[9]) {
+    const float a[9] = {u[0], u[1], u[2], u[1], u[3], u[4], u[2], u[4], u[5]};
+    inverse9(a, full);
+#pragma unroll
+    for (unsigned q = 0; q < 6; ++q) mi[q] = full[sym6_pos(q)];
+}
+__device__ __forceinline__ void ld6u(gp<const float> m, unsigned i, float (&u)[6]) {
+#pragma unroll
+    for (unsigned q = 0; q < 6; q += 2) ld_pair(m, bp6(q, i), u[q], u[q + 1]);
+}
+__device__ __forceinline__ f3 axpy(float a, f3 x, f3 y) { return mk(fmaf(a, x.x, y.x), fmaf(a, x.y, y.y), fmaf(a, x.z, y.z)); }
+
+// Solves instance `inst` together with the workgroups that hold its other
+// parts; this one holds part `part`.  False: aborted.
+__device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst& I, int inst, int part, unsigned epoch, ResLds& S,
+                           const Barrier& bar, int& trace_e) {
+    const unsigned tid = threadIdx.x, lane = tid & (kWave - 1);
+    const unsigned wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const gp<const unsigned> plan = I.res_plan;
+    const unsigned n = unsigned(I.n_rows), parts = unsigned(I.res_parts);
+    const gp<const unsigned> hdr = plan + 8 * part;
+    const unsigned n_own = hdr[0], n_halo = hdr[1], halo_at = hdr[2], n_ghost = hdr[3], ghost_at = hdr[4];
+    const unsigned pos0 = unsigned(part) * unsigned(I.res_part_rows);
+    const unsigned rows_at = 8u * parts, meta_at = rows_at + n, exp_at = meta_at + n, held_at = exp_at + n;
+    // exchange areas: [2][parts] lines of 16 words, then [2][exports] rows of 3
+    u64* const xsum = B.xbuf + I.res_xbase;
+    u64* const xrow = xsum + 32ull * parts;
+    const unsigned exports = unsigned(I.res_exports);
+    auto tag_of = [&](int t) { return (epoch << 8) | (unsigned(t) & 255u); };
+    auto sum_line = [&](int t, unsigned q) { return xsum + 16ull * ((unsigned(t) & 1u) * parts + q); };
+    auto row_words = [&](int t, unsigned e) { return xrow + 3ull * ((unsigned(t) & 1u) * exports + e); };
+
+    auto send_row = [&](int t, unsigned e, f3 v) {
+        u64* const w = row_words(t, e);
+        st64(w, tagged(__float_as_uint(v.x), tag_of(t)));
+        st64(w + 1, tagged(__float_as_uint(v.y), tag_of(t)));
+        st64(w + 2, tagged(__float_as_uint(v.z), tag_of(t)));
+    };
+
+    // ---- load: own rows, ghost block, halo row ----
+    unsigned lp[kSlots], row[kSlots], ns[kSlots], nh[kSlots], ex[kSlots], word[kSlots][kHeld];
+    bool live[kSlots], on[kSlots];  // this lane's row exists; this wave has a row
+    float V[kSlots][kHeld][9], M[kSlots][6];
+    f3 r[kSlots], p[kSlots], q[kSlots];
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) {
+        lp[s] = (unsigned(s) * kWaves + wave) * kWave + lane;
+        on[s] = (unsigned(s) * kWaves + wave) * kWave < n_own;
+        live[s] = lp[s] < n_own;
+        const unsigned K = pos0 + (live[s] ? lp[s] : 0u);
+        row[s] = 0u;
+        ns[s] = nh[s] = 0u;
+        ex[s] = CHX_RES_NONE;
+        if (on[s]) {
+            row[s] = ldx(plan, rows_at + K);
+            const unsigned meta = ldx(plan, meta_at + K);
+            if (live[s]) {
+                ns[s] = meta & 15u;
+                nh[s] = meta >> 4;
+                ex[s] = ldx(plan, exp_at + K);
+            }
+            const unsigned vs = unsigned(ldx(I.upper_offsets, row[s] / CHX_SLICE_ROWS)) + row[s] % CHX_SLICE_ROWS;
+#pragma unroll
+            for (int u = 0; u < kHeld; ++u) {
+                const bool has = unsigned(u) < nh[s];
+                word[s][u] = has ? ldx(plan, held_at + unsigned(u) * n + K) : (kNoSlot << 16);
+#pragma unroll
+                for (int c = 0; c < 9; ++c) V[s][u][c] = 0.0f;
+                if (has) ld9p(gp<const float>(I.values), vs + unsigned(u) * CHX_SLICE_ROWS, V[s][u]);
+            }
+            float d[6], full[9];
+            ld6u(gp<const float>(I.diag), row[s], d);
+#pragma unroll
+            for (int c = 0; c < 6; ++c) S.diag[c][lp[s]] = d[c];
+            inverse_sym(d, M[s], full);
+            p[s] = ld3g(I.x, row[s]);
+            S.x[lp[s]] = p[s];
+            S.p[lp[s]] = p[s];
+        }
+    }
+    float Gv[9];
+    unsigned gword = 0;
+    if (tid < n_ghost) {
+        const unsigned vs = ldx(plan, ghost_at + 2u * tid);
+        gword = ldx(plan, ghost_at + 2u * tid + 1u);
+        ld9p(gp<const float>(I.values), vs, Gv);
+    }
+    float hM[6];
+    f3 hr = mk(0.f, 0.f, 0.f);
+    unsigned hex = 0;
+    if (tid < n_halo) {
+        const unsigned hrow = ldx(plan, halo_at + 2u * tid);
+        hex = ldx(plan, halo_at + 2u * tid + 1u);
+        float d[6], full[9];
+        ld6u(gp<const float>(I.diag), hrow, d);
+        inverse_sym(d, hM, full);
+        S.p[kPart + tid] = ld3g(I.x, hrow);
+    }
+    if (tid == 0) S.bad_sums = S.bad_halo = 0;
+    if (tid < kLeaves * kSums) S.leaf[tid / kSums][tid % kSums] = 0.0;
+
+    // A times the vector in S.p (own rows also in v); S.p and
+    // S.prod are read until the next workgroup barrier.
+    auto apply = [&](const f3 (&v)[kSlots], f3 (&out)[kSlots]) {
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s)
+            if (on[s]) {
+#pragma unroll
+                for (int u = 0; u < kHeld; ++u) {
+                    const unsigned t = word[s][u] >> 16;
+                    if (t != kNoSlot) S.prod[t] = mv9t(V[s][u], v[s]);
+                }
+            }
+        __syncthreads();
+        if (tid < n_ghost) S.prod[gword >> 16] = mv9t(Gv, S.p[gword & 0xffffu]);
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s)
+            if (on[s]) {
+                float d[6];
+#pragma unroll
+                for (int c = 0; c < 6; ++c) d[c] = S.diag[c][lp[s]];
+                f3 sum = mv_sym(d, v[s]);
+#pragma unroll
+                for (int l = 0; l < kHeld; ++l) {
+                    const f3 t = S.prod[unsigned(l) * kPart + lp[s]];
+                    if (unsigned(l) < ns[s]) sum = add(sum, t);
+                }
+#pragma unroll
+                for (int u = 0; u < kHeld; ++u) {
+                    const f3 t = mv9(V[s][u], S.p[word[s][u] & 0xffffu]);
+                    if (unsigned(u) < nh[s]) sum = add(sum, t);
+                }
+                out[s] = sum;
+            }
+    };
+    // Sums of phase t: per leaf, then over the part's leaves, sent to the gang.
+    auto send_sums = [&](int t, double (&acc)[kSlots][kSums]) {
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s)
+            if (on[s]) {
+#pragma unroll
+                for (int v = 0; v < kSums; ++v) {
+                    const double w = wave_sum(acc[s][v]);
+                    if (lane == 0) S.leaf[unsigned(s) * kWaves + wave][v] = w;
+                }
+            }
+        __syncthreads();
+        if (tid < 8 * kSums) {
+            const unsigned v = tid >> 3, i = tid & 7u;
+            double w = S.leaf[2 * i][v] + S.leaf[2 * i + 1][v];
+            w += __shfl_xor(w, 1);
+            w += __shfl_xor(w, 2);
+            w += __shfl_xor(w, 4);
+            if (i == 0) {
+                if (parts == 1) {
+                    S.tot[v] = w;
+                } else {
+                    const u64 b = u64(__double_as_longlong(w));
+                    u64* const line = sum_line(t, unsigned(part)) + 2 * v;
+                    st64(line, tagged(unsigned(b), tag_of(t)));
+                    st64(line + 1, tagged(unsigned(b >> 32), tag_of(t)));
+                }
+            }
+        }
+    };
+    // The instance's sums of phase t into S.tot (tree over the parts).
+    auto take_sums = [&](int t) -> bool {
+        if (parts > 1 && wave < kSums) {
+            double w = 0.0;
+            bool ok = true;
+            const unsigned per = parts > unsigned(kWave) ? 4u : 1u;
+            double part_sum[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (unsigned k = 0; k < 4; ++k) {
+                const unsigned j = per * lane + k;
+                if (k < per && j < parts) {
+                    unsigned b[2];
+                    ok = ok && await<2>(sum_line(t, j) + 2 * wave, tag_of(t), b, bar);
+                    if (ok) part_sum[k] = __longlong_as_double((long long)((u64(b[1]) << 32) | b[0]));
+                }
+            }
+            w = per == 4 ? (part_sum[0] + part_sum[1]) + (part_sum[2] + part_sum[3]) : part_sum[0];
+#pragma unroll
+            for (int m = 1; m < kWave; m <<= 1) w += __shfl_xor(w, m);
+            if (lane == 0) S.tot[wave] = w;
+            if (!ok) S.bad_sums = 1;
+        }
+        __syncthreads();
+        return S.bad_sums == 0;
+    };
+
+    // ---- set-up: r_0 = b - A x, z_0 = p_0 = M^-1 r_0 ----
+    apply(p, q);
+    {
+    double acc[kSlots][kSums];
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) {
+#pragma unroll
+        for (int v = 0; v < kSums; ++v) acc[s][v] = 0.0;
+        if (on[s] && live[s]) {
+            const f3 b = ld3g(I.rhs, row[s]);
+            r[s] = sub(b, q[s]);
+            p[s] = mv_sym(M[s], r[s]);
+            if (ex[s] != CHX_RES_NONE) send_row(0, ex[s], r[s]);
+            acc[s][0] = dot64(r[s], p[s]);
+            acc[s][1] = dot64(b, b);
+            acc[s][4] = dot64(r[s], r[s]);
+        }
+    }
+    send_sums(0, acc);
+    }
+    double bb = 0.0;
+    for (int k = 0;; ++k) {
+        if (!take_sums(k)) return false;
+        const double rho = S.tot[0], sig = S.tot[1], del = S.tot[2], gam = S.tot[3], rr = S.tot[4];
+        if (k == 0) bb = sig;
+        if (B.trace != nullptr) {
+            trace_point(B, trace_e, unsigned(B.n_instances) - unsigned(ld64(&B.xbuf[RES_DONE])));
+            ++trace_e;
+        }
+        const int its = k > 0 ? k - 1 : 0;  // updates of x so far
+        if (its >= I.max_iter || (I.tol > 0.0 && rr <= I.tol * I.tol * bb)) {
+            if (part == 0 && tid == 0) {
+                B.inst_iters[inst] = its;
+                B.inst_rr[inst] = rr;
+                B.inst_bb[inst] = bb;
+                if (B.inst_rho != nullptr) B.inst_rho[inst] = rho;
+                (void)__hip_atomic_fetch_add(&B.xbuf[RES_DONE], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            break;
+        }
+        if (part == 0 && tid == 0 && (k & 7) == 0)
+            (void)__hip_atomic_fetch_add(&B.xbuf[RES_PROGRESS], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        float alpha = 0.0f, beta = 0.0f;
+        if (k > 0) merged_scalars(rho, sig, del, gam, alpha, beta);
+        const bool last = k >= I.max_iter;  // at the cap: the last update only
+        // halo rows: r_k, z_k, p_k as their owners form them
+        if (tid < n_halo && !last) {
+            unsigned w[3];
+            if (await<3>(row_words(k, hex), tag_of(k), w, bar)) {
+                const f3 h = mk(__uint_as_float(w[0]), __uint_as_float(w[1]), __uint_as_float(w[2]));
+                if (k == 0) {
+                    hr = h;
+                    S.p[kPart + tid] = mv_sym(hM, hr);
+                } else {
+                    hr = axpy(-alpha, h, hr);
+                    S.p[kPart + tid] = axpy(beta, S.p[kPart + tid], mv_sym(hM, hr));
+                }
+            } else {
+                S.bad_halo = 1;
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s)
+            if (on[s]) {
+                if (k > 0) {
+                    r[s] = axpy(-alpha, q[s], r[s]);
+                    S.x[lp[s]] = axpy(alpha, p[s], S.x[lp[s]]);
+                    p[s] = axpy(beta, p[s], mv_sym(M[s], r[s]));
+                }
+                S.p[lp[s]] = p[s];
+            }
+        if (!last) {
+            apply(p, q);
+            if (S.bad_halo != 0) return false;
+        }
+        double acc[kSlots][kSums];
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) {
+#pragma unroll
+            for (int v = 0; v < kSums; ++v) acc[s][v] = 0.0;
+            if (on[s] && live[s]) {
+                if (!last && ex[s] != CHX_RES_NONE) send_row(k + 1, ex[s], q[s]);
+                const f3 z = mv_sym(M[s], r[s]);
+                acc[s][0] = dot64(r[s], z);
+                acc[s][4] = dot64(r[s], r[s]);
+                if (!last) {
+                    acc[s][1] = dot64(p[s], q[s]);
+                    acc[s][2] = dot64(q[s], z);
+                    acc[s][3] = dot64(q[s], mv_sym(M[s], q[s]));
+                }
+            }
+        }
+        send_sums(k + 1, acc);
+    }
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s)
+        if (on[s] && live[s]) st3g(I.x, row[s], S.x[lp[s]]);
+    return true;
+}
+
+// The workgroup's next (item, part), or kExit: it reports itself idle, hands
+// list items to the idle workgroups of its group while the next one fits,
+// and waits for its own.  Items come by falling number of parts, so what a
+// finished gang frees always holds the next one; with no gang left running
+// every workgroup of the group is idle and any item of the list fits.
+__device__ unsigned next_item(const chx_cloth_batch& B, unsigned group, unsigned first, unsigned stride, unsigned idx,
+                              unsigned epoch, unsigned had, ResLds& S, const Barrier& bar) {
+    __syncthreads();  // readers of S.mail are done
+    if (threadIdx.x == 0) {
+        u64* const idle = &B.xbuf[RES_IDLE + 16 * group];
+        u64* const next = &B.xbuf[RES_NEXT];
+        const gp<const int> items = glb(B.res_items);
+        const unsigned n_items = unsigned(B.res_n_items - B.res_n_big);
+        auto mail = [&](unsigned i) { return &B.xbuf[RES_MAIL + 16ull * (first + stride * i)]; };
+        auto add_idle = [&](unsigned m) {
+            return unsigned(__hip_atomic_fetch_or(idle, u64(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) | m;
+        };
+        auto send = [&](unsigned gang, unsigned item) {
+            unsigned part = 0;
+            for (unsigned m = gang; m != 0u; m &= m - 1u, ++part)
+                st64(mail(unsigned(__ffs(int(m))) - 1u), tagged((item << 8) | (item == kExit ? 0u : part), epoch));
+        };
+        unsigned have = add_idle(1u << idx);
+        unsigned i = unsigned(ld64(next));
+        for (;;) {
+            if (i >= n_items) {  // nothing left: everyone idle leaves
+                const unsigned m = unsigned(__hip_atomic_exchange(idle, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                send(m, kExit);
+                break;
+            }
+            const unsigned need = unsigned(items[4 * (unsigned(B.res_n_big) + i) + 1]);
+            if (unsigned(__popc(have)) < need) break;
+            unsigned gang = 0, m = have;
+            for (unsigned c = 0; c < need; ++c, m &= m - 1u) gang |= m & (0u - m);
+            u64 expect = have;
+            if (!__hip_atomic_compare_exchange_strong(idle, &expect, u64(have & ~gang), __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT)) {
+                have = unsigned(expect);
+                i = unsigned(ld64(next));
+                continue;
+            }
+            u64 at = i;
+            if (__hip_atomic_compare_exchange_strong(next, &at, u64(i + 1u), __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT)) {
+                send(gang, unsigned(B.res_n_big) + i);
+                have = unsigned(ld64(idle));
+                i = unsigned(ld64(next));
+            } else {
+                have = add_idle(gang);
+                i = unsigned(at);
+            }
+        }
+        // wait for this workgroup's own word
+        const u64* const mine = mail(idx);
+        Watch watch(bar);
+        unsigned seen = unsigned(ld64(&B.xbuf[RES_PROGRESS])), level = 0, got = kExit << 8;
+        for (;;) {
+            const u64 w = ld64(mine);
+            if (unsigned(w >> 32) == epoch && unsigned(w) != had) {
+                got = unsigned(w);
+                break;
+            }
+            if (!watch.again(&B.xbuf[RES_PROGRESS], seen)) {
+                got = kExit << 8 | 1u;  // aborted
+                break;
+            }
+            backoff(level);
+        }
+        S.mail = got;
+    }
+    __syncthreads();
+    return S.mail;
+}
+
+__global__ __launch_bounds__(kThreads, 2) void resident_kernel(chx_cloth_batch B, int finalize) {
+    __shared__ ResLds S;
+    const int G = int(gridDim.x);
+    const Barrier bar = make_barrier(B);
+    unsigned* const progress = reinterpret_cast<unsigned*>(&B.xbuf[RES_PROGRESS]);
+    const unsigned epoch = unsigned(ld64(&B.xbuf[RES_EPOCH]));
+    if (blockIdx.x == 0 && B.trace != nullptr)
+        for (int e = threadIdx.x; e < 2 * B.trace_entries; e += blockDim.x) glb(B.trace)[e] = 0ull;
+    if (ld64(&B.xbuf[RES_CLEAR]) != 0ull) {
+        // the launch numbers start over: no word may keep an old tag
+        for (u64 k = RES_MAIL + u64(blockIdx.x) * kThreads + threadIdx.x; k < B.res_xwords; k += u64(G) * kThreads)
+            st64(&B.xbuf[k], 0ull);
+        if (!grid_sync(bar, unsigned(G))) return;
+    }
+    __syncthreads();
+    // groups: workgroups b = x (mod 8), which the dispatcher places on one
+    // XCD, or all of them
+    const unsigned groups = unsigned(B.res_groups), group = blockIdx.x % groups, idx = blockIdx.x / groups;
+    const unsigned rank = group * (unsigned(G) / groups) + idx;
+    int trace_e = 0;
+    // the workgroup's work: the single instance's part, or the leading large
+    // items that use its rank, then items dealt to its group
+    const gp<const int> items = glb(B.res_items);
+    int big = 0;
+    unsigned had = 0xffffffffu;
+    bool ok = true;
+    for (;;) {
+        int inst = 0, part = -1;
+        if (B.inst == nullptr) {
+            if (big++ > 0 || rank >= unsigned(B.single.res_parts)) break;
+            part = int(rank);
+        } else if (big < B.res_n_big) {
+            const int base = items[4 * big + 2], parts = items[4 * big + 1];
+            inst = items[4 * big];
+            ++big;
+            if (int(rank) < base || int(rank) >= base + parts) continue;
+            part = int(rank) - base;
+            __syncthreads();  // the previous solve's readers of S are done
+        } else {
+            if (B.res_n_items == B.res_n_big) break;
+            had = next_item(B, group, group, groups, idx, epoch, had, S, bar);
+            if ((had >> 8) == kExit) {
+                ok = (had & 255u) == 0u;
+                break;
+            }
+            inst = __builtin_amdgcn_readfirstlane(items[4 * (had >> 8)]);
+            part = int(__builtin_amdgcn_readfirstlane(had & 255u));
+        }
+        const Inst I = inst_at(B, inst);
+        ok = solve_part(B, I, inst, part, epoch, S, bar, trace_e);
+        if (!ok) break;
+    }
+    // pos and vel change only when every instance was solved
+    if (!ok) return;
+    if (G > 1 && !grid_sync(bar, unsigned(G), -1, nullptr, progress)) return;
+    if (finalize) finalize_tiles(B, G);
+}
+
+std::mutex g_mu;
+int g_limit[16] = {0};
+
+}  // namespace
+
+int resident_grid_limit() {
+    int dev = 0;
+    hip_check(hipGetDevice(&dev), "hipGetDevice");
+    std::lock_guard<std::mutex> lk(g_mu);
+    int& l = g_limit[dev & 15];
+    if (l == 0) {
+        hipDeviceProp_t prop;
+        hip_check(hipGetDeviceProperties(&prop, dev), "hipGetDeviceProperties");
+        int per_cu = 0;
+        hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(resident_kernel),
+                                                               kThreads, 0),
+                  "hipOccupancyMaxActiveBlocksPerMultiprocessor");
+        l = per_cu < 1 ? -1 : std::min(kMaxParts, prop.multiProcessorCount);
+    }
+    return std::max(l, 0);
+}
+
+void launch_resident(const chx_cloth_batch& B, int finalize, hipStream_t stream) {
+    chx_cloth_batch arg = B;
+    int fin = finalize;
+    void* args[] = {&arg, &fin};
+    hip_check(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(resident_kernel), dim3(B.res_grid),
+                                         dim3(kThreads), args, 0, stream),
+              "hipLaunchCooperativeKernel(resident pcg)");
+}
+
+}  // namespace chx
+
+using namespace chx;
+
+extern "C" int chx_resident_grid_limit(int* max_blocks) {
+    return guarded([&] {
+        require(max_blocks != nullptr, "chx_resident_grid_limit: null output");
+        *max_blocks = resident_grid_limit();
+    });
+}

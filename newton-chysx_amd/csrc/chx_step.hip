@@ -31,6 +31,8 @@
 #include "chx_device.h"
 #include "chx_elements.h"
 #include "chx_internal.h"
+#include "chx_pcg.h"
+#include "chx_resident.h"
 
 namespace chx {
 namespace {
@@ -43,12 +45,6 @@ static_assert(CHX_ITEM_SIZE == kBlock, "one thread per work-item entry");
 // (refinements so far) + 1 if it is the true residual.  Every tile of an
 // instance holds the same state.
 enum { P_RHO0 = 0, P_RHO1 = 1, P_RR0 = 2, P_RR1 = 3, P_SIG = 4, P_BB = 5, P_TRUE0 = 6, P_TRUE1 = 7 };
-
-// Divide guard |den| > 1e-37 (ChysX/src/solver/pcg_solver.cu:122-127), with
-// the FP64 inner products rounded to FP32 once.
-__device__ __forceinline__ float guarded_div(double a, double b) {
-    return (b > 1e-37 || b < -1e-37) ? float(a / b) : 0.0f;
-}
 
 // Resets the persistent solver's barrier / control words before a PCG launch
 // on the same stream.  The status word and the abort report next to it are
@@ -252,7 +248,10 @@ struct AsmLds {
 };
 
 __global__ __launch_bounds__(kBlock) void assemble_kernel(chx_cloth_batch B) {
-    if (blockIdx.x == 0) reset_sync(B.sync, false);
+    if (blockIdx.x == 0) {
+        reset_sync(B.sync, false);
+        reset_resident(B.xbuf);
+    }
     __shared__ AsmLds L;
     int inst, u;
     get_unit_item(B, blockIdx.x, inst, u);
@@ -520,7 +519,10 @@ __global__ __launch_bounds__(kBlock) void compensate_kernel(chx_cloth_batch B) {
     }
 }
 
-__global__ void reset_sync_kernel(unsigned* sync, int all) { reset_sync(sync, all != 0); }
+__global__ void reset_sync_kernel(unsigned* sync, int all, unsigned long long* xbuf) {
+    reset_sync(sync, all != 0);
+    reset_resident(xbuf);
+}
 
 // ---------------------------------------------------------------------------
 // SpMV row loop: L lanes per block row, 64/L rows per wave and row group; R
@@ -1244,36 +1246,6 @@ struct PcgMats<3> : PcgMats<1> {};
 template <>
 struct PcgMats<4> : PcgMats<2> {};
 
-// Optional solver trace (workgroup 0, thread 0): real-time stamp and
-// active-instance count at barrier e.
-__device__ __forceinline__ void trace_point(const chx_cloth_batch& B, int e, unsigned active) {
-    if (B.trace != nullptr && blockIdx.x == 0 && threadIdx.x == 0 && e < B.trace_entries) {
-        const gp<unsigned long long> t = glb(B.trace);
-        t[2 * e] = __builtin_amdgcn_s_memrealtime();
-        t[2 * e + 1] = active;
-    }
-}
-
-// Finalize of every tile (cloth_simulator.cu:222-244): pos = x_n + dx,
-// vel = dx / dt, times exp(-damping dt) when damping > 0.
-__device__ __forceinline__ void finalize_tiles(const chx_cloth_batch& B, int G) {
-    for (int t = blockIdx.x; t < B.n_tiles; t += G) {
-        int inst, rb, re;
-        get_tile(B, t, inst, rb, re);
-        const Inst I = inst_at(B, inst);
-        const float inv_dt = 1.0f / I.dt;
-        const float decay = (I.damping > 0.0f) ? expf(-I.damping * I.dt) : 1.0f;
-        for (unsigned row = unsigned(rb) + threadIdx.x; row < unsigned(re); row += blockDim.x) {
-            const f3 d = ld3g(I.x, row);
-            const f3 p = ld3g(I.pos, row);
-            st3g(I.pos, row, add(p, d));
-            f3 v = mul(d, inv_dt);
-            if (I.damping > 0.0f) v = mul(v, decay);
-            st3g(I.vel, row, v);
-        }
-    }
-}
-
 template <int L, int V, bool ST>
 __global__ __launch_bounds__(kBlock) void pcg_kernel(chx_cloth_batch B, int finalize) {
     constexpr bool BF16 = V == 2 || V == 4;
@@ -1625,21 +1597,8 @@ __global__ __launch_bounds__(kBlock) void pcg1_kernel(chx_cloth_batch B, int fin
                         acc[4] += dot64(Ap, mv6p(minv, row, Ap));
                     });
                 } else {
-                    const float alpha = guarded_div(rho, sig);
-                    const double ad = double(alpha);
-                    // rho_k by the identity: its terms carry the FP32
-                    // rounding of the stored vectors, a few units of 2^-24
-                    // of their size.  Above 1e-5 of them (~100 such units)
-                    // rho_k, and so beta, is resolved to about 1%; below,
-                    // the direction restarts from z_k (beta = 0) instead of
-                    // taking a rounding-noise beta.  A tighter cut (1e-3)
-                    // restarts on ordinary fast-converging iterations and
-                    // costs the Krylov acceleration: 13 iterations instead
-                    // of 9 on a pin-driven substep of the 32x32 cloth.
-                    const double t1 = 2.0 * ad * del, t2 = ad * ad * gam;
-                    const double rho_k = rho - t1 + t2;
-                    const bool resolved = rho_k > 1.0e-5 * (fabs(rho) + fabs(t1) + fabs(t2));
-                    const float beta = resolved ? guarded_div(rho_k, rho) : 0.0f;
+                    float alpha, beta;
+                    merged_scalars(rho, sig, del, gam, alpha, beta);
                     // r_k and z_k of row j from the previous parity
                     auto rz = [&](unsigned j, f3& rn, f3& zn) {
                         const f3 r = ld3g(r_prev, j), q = ld3g(q_prev, j);
@@ -1841,8 +1800,18 @@ int pcg_variant(const chx_cloth_batch& B, bool row_major) {
     return (B.bf16_blocks != 0 ? 2 : 1) + (B.entries16 != 0 ? 2 : 0);
 }
 
+// Whether the resident kernel takes the launch: FP32 cloth instances that
+// all have a plan, in the default solver form.
+bool resident(const chx_cloth_batch& B, bool row_major) {
+    return !row_major && B.res_grid > 0 && B.bf16_blocks == 0 && B.pcg_form == 0 && B.no_lds_staging == 0;
+}
+
 void launch_pcg(const chx_cloth_batch& B, int finalize, hipStream_t stream, bool row_major = false) {
     if (B.n_tiles <= 0) return;
+    if (resident(B, row_major)) {
+        launch_resident(B, finalize, stream);
+        return;
+    }
     const int L = B.lanes_per_row;
     const int v = pcg_variant(B, row_major);
     const bool staged = B.no_lds_staging == 0;
@@ -1897,6 +1866,26 @@ void validate_batch(const chx_cloth_batch* b) {
         require(b->elem_items != nullptr || b->n_elem_items == 0, "chysx: batch without an element list");
         require(b->unit_items != nullptr || b->n_unit_items == 0, "chysx: batch without a unit list");
     }
+    if (b->res_grid > 0) {
+        require(b->xbuf != nullptr && b->res_grid <= resident_grid_limit() && b->res_groups > 0 &&
+                    b->res_grid % b->res_groups == 0 && b->res_groups <= kResGroups &&
+                    b->res_xwords >= CHX_RES_CONTROL_WORDS,
+                "chysx: resident solve without its exchange area, or a grid that does not fit the device");
+        if (b->inst == nullptr) {
+            const chx_instance& I = b->single;
+            require(I.n_rows == 0 ||
+                        (I.res_plan != nullptr &&
+                         (I.res_part_rows == 256 || I.res_part_rows == 512 || I.res_part_rows == CHX_RES_PART_MAX) &&
+                         I.res_parts == (I.n_rows + I.res_part_rows - 1) / I.res_part_rows &&
+                         I.res_parts <= b->res_grid && I.res_exports >= 0 &&
+                         I.res_xbase + CHX_RES_XWORDS(I.res_parts, I.res_exports) <= b->res_xwords),
+                    "chysx: resident plan does not match its instance");
+        } else {
+            require(b->res_items != nullptr && b->res_n_big >= 0 && b->res_n_items >= b->res_n_big &&
+                        b->res_grid / b->res_groups <= 32,
+                    "chysx: resident solve without its work list");
+        }
+    }
     if (b->n_tiles > 0) require(b->partials && b->inst_iters && b->inst_rr && b->inst_bb && b->inst_done,
                                 "chysx: batch without solver outputs");
 }
@@ -1926,7 +1915,7 @@ void assemble(const chx_cloth_batch& B, hipStream_t stream) {
             hip_check(hipGetLastError(), "compensate_kernel launch");
         }
     } else {
-        reset_sync_kernel<<<1, kBlock, 0, stream>>>(B.sync, 0);
+        reset_sync_kernel<<<1, kBlock, 0, stream>>>(B.sync, 0, B.xbuf);
         hip_check(hipGetLastError(), "reset_sync_kernel launch");
     }
 }
@@ -2043,7 +2032,7 @@ void read_workspace_stats(const chx_cloth_batch& B, int* iterations, double* rr,
               "hipMemcpyAsync(status)");
     hip_check(hipStreamSynchronize(s), "hipStreamSynchronize(pcg)");
     if (status != 0u) {
-        reset_sync_kernel<<<1, kBlock, 0, s>>>(B.sync, 1);
+        reset_sync_kernel<<<1, kBlock, 0, s>>>(B.sync, 1, nullptr);
         hip_check(hipStreamSynchronize(s), "hipStreamSynchronize(reset)");
         throw Error(CHX_ERR_DEVICE, "chysx::solver::PCGSolver: grid barrier timed out");
     }
@@ -2127,7 +2116,7 @@ void solve_bsr3(int n_rows, const float* diag, const int* row_offsets, const int
         // The workspace needs no initialisation: every control word is
         // cleared, status included (an earlier solve's abort is reported by
         // its own synchronous read or chx_pcg_last_stats before this call).
-        reset_sync_kernel<<<1, kBlock, 0, s>>>(B.sync, 1);
+        reset_sync_kernel<<<1, kBlock, 0, s>>>(B.sync, 1, nullptr);
         hip_check(hipGetLastError(), "reset_sync_kernel launch");
         launch_pcg(B, 0, s, true);
         if (iterations || rr || bb) read_workspace_stats(B, iterations, rr, bb, nullptr, s);
@@ -2208,7 +2197,7 @@ int chx_cloth_solve(const chx_cloth_batch* batch, int finalize, uintptr_t stream
     return guarded([&] {
         validate_batch(batch);
         const hipStream_t s = as_stream(stream);
-        reset_sync_kernel<<<1, kBlock, 0, s>>>(batch->sync, 0);
+        reset_sync_kernel<<<1, kBlock, 0, s>>>(batch->sync, 0, batch->xbuf);
         hip_check(hipGetLastError(), "reset_sync_kernel launch");
         launch_pcg(*batch, finalize, s);
     });
@@ -2281,7 +2270,7 @@ int chx_batch_check(const chx_cloth_batch* batch, uintptr_t stream) {
         hip_check(hipMemcpyAsync(words, batch->sync, sizeof(words), hipMemcpyDeviceToHost, s), "hipMemcpyAsync(sync)");
         hip_check(hipStreamSynchronize(s), "hipStreamSynchronize(check)");
         if (words[SYNC_STATUS] != 0u) {
-            reset_sync_kernel<<<1, kBlock, 0, s>>>(batch->sync, 1);
+            reset_sync_kernel<<<1, kBlock, 0, s>>>(batch->sync, 1, nullptr);
             hip_check(hipStreamSynchronize(s), "hipStreamSynchronize(reset)");
             if (batch->status_host != nullptr)
                 __atomic_store_n(batch->status_host, 0u, __ATOMIC_SEQ_CST);

@@ -11,6 +11,7 @@
 
 #include "cloth_batch.h"
 #include "mesh_io.h"
+#include "resident_plan.h"
 #include "cloth_simulator.h"
 #include "sparse_solver.h"
 #include "topology.h"
@@ -510,6 +511,29 @@ PYBIND11_MODULE(_chysx_native, m) {
             return py::make_tuple(to_array(p.row_offsets), to_array(p.col_indices));
         },
         py::arg("n"), py::arg("rows"), py::arg("cols"));
+    topo.def(
+        "resident_plan",
+        [](int n, IArr row_offsets, IArr col_indices, IArr block_slots, int part_rows) -> py::object {
+            // Canonical row order and part image of the resident solve, or
+            // None when the pattern does not fit it.
+            chysx::topology::Pattern p;
+            p.n = n;
+            p.row_offsets.assign(row_offsets.data(), row_offsets.data() + row_offsets.size());
+            p.col_indices.assign(col_indices.data(), col_indices.data() + col_indices.size());
+            const std::vector<int> bs(block_slots.data(), block_slots.data() + block_slots.size());
+            const std::vector<int> order = chysx::engine::resident_order(p);
+            const auto r = chysx::engine::resident_plan(p, bs, order, part_rows);
+            if (r.blob.empty()) return py::none();
+            py::dict d;
+            d["order"] = to_array(order);
+            d["parts"] = r.parts;
+            d["exports"] = r.exports;
+            py::array_t<std::uint32_t> b(static_cast<py::ssize_t>(r.blob.size()));
+            std::copy(r.blob.begin(), r.blob.end(), b.mutable_data());
+            d["blob"] = b;
+            return d;
+        },
+        py::arg("n"), py::arg("row_offsets"), py::arg("col_indices"), py::arg("block_slots"), py::arg("part_rows"));
     topo.def(
         "cloth_system",
         [](int n, IArr tris, IArr pins, bool stretch, bool shear, bool bending) {

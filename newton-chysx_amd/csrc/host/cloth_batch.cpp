@@ -29,10 +29,13 @@ void ClothBatch::clear() noexcept {
 }
 
 std::vector<chx_instance> ClothBatch::descriptors(float dt, std::uintptr_t cuda_stream) {
+    std::vector<int> rows;
+    for (ClothSimulator* s : sims_) rows.push_back(s->buffers().particle_count());
+    const int part_rows = engine::resident_part_rows(rows);
     std::vector<chx_instance> ds;
     ds.reserve(sims_.size());
     for (ClothSimulator* s : sims_) {
-        ds.push_back(s->prepare_instance(dt, cuda_stream));
+        ds.push_back(s->prepare_instance(dt, cuda_stream, part_rows));
         if (bf16_ && ds.back().n_rows > 0 && ds.back().diag_c == nullptr)
             throw std::invalid_argument(
                 "ClothBatch: BF16 mode needs every instance switched with set_bf16_blocks(true)");

@@ -233,7 +233,7 @@ void ClothSimulator::ensure_hessian_topology(std::uintptr_t stream) {
     inst_.build(source(), stream);
     runner_.set_lanes_per_row(lanes_per_row_);
     runner_.set_bf16(bf16_);
-    runner_.bind_single(inst_.descriptor(source()), stream);
+    runner_.bind_single(single_descriptor(source(), stream), stream);
     packed_k_[0] = pins_.stiffness();
     packed_k_[1] = fem_stretch_.stiffness();
     packed_k_[2] = fem_shear_.stiffness();
@@ -345,11 +345,18 @@ void ClothSimulator::step(float dt, std::uintptr_t cuda_stream) {
     }
     engine::InstanceSource s = source();
     s.dt = dt;
-    runner_.update_single(inst_.descriptor(s));
+    runner_.update_single(single_descriptor(s, cuda_stream));
     runner_.step(cuda_stream);
 }
 
-chx_instance ClothSimulator::prepare_instance(float dt, std::uintptr_t cuda_stream) {
+// The descriptor of the simulator's own (single-instance) launches.
+chx_instance ClothSimulator::single_descriptor(const engine::InstanceSource& s, std::uintptr_t stream) {
+    chx_instance d = inst_.descriptor(s);
+    if (!bf16_) inst_.attach_plan(d, pattern_, engine::resident_part_rows({s.n}), stream);
+    return d;
+}
+
+chx_instance ClothSimulator::prepare_instance(float dt, std::uintptr_t cuda_stream, int part_rows) {
     const int n = buffers_.particle_count();
     if (n <= 0) throw std::runtime_error("ClothSimulator::prepare_instance: no particles bound");
     if (buffers_.pos.data() == nullptr || buffers_.vel.data() == nullptr)
@@ -360,7 +367,9 @@ chx_instance ClothSimulator::prepare_instance(float dt, std::uintptr_t cuda_stre
     else check_elements_current(cuda_stream);
     engine::InstanceSource s = source();
     s.dt = dt;
-    return inst_.descriptor(s);
+    chx_instance d = inst_.descriptor(s);
+    if (!bf16_) inst_.attach_plan(d, pattern_, part_rows, cuda_stream);
+    return d;
 }
 
 int ClothSimulator::last_pcg_iterations(std::uintptr_t cuda_stream) {
@@ -504,7 +513,7 @@ double ClothSimulator::compute_energy(int kind_mask) {
     resize_work_buffers(n);
     if (topology_dirty_ || H_num_block_rows_ != n) ensure_hessian_topology();
     else check_elements_current();
-    runner_.update_single(inst_.descriptor(source()));
+    runner_.update_single(single_descriptor(source(), 0));
     return runner_.energy(kind_mask, 0);
 }
 

@@ -344,6 +344,8 @@ void InstanceData::build_units(const std::vector<unsigned>& goff, const std::vec
 void InstanceData::build(const InstanceSource& s, std::uintptr_t stream) {
     if (!s.pattern || s.pattern->n != s.n) throw std::invalid_argument("chysx::engine: pattern missing or sized wrong");
     bytes_ = 0;
+    for (Plan& pl : plans_) pl = Plan{};
+    order_.clear();
     n_ = s.n;
     nnz_ = s.pattern->nnz();
     row_offsets_.host() = s.pattern->row_offsets;
@@ -682,9 +684,146 @@ chx_instance InstanceData::descriptor(const InstanceSource& s) const {
     return I;
 }
 
+void InstanceData::attach_plan(chx_instance& d, const topology::Pattern& p, int part_rows, std::uintptr_t stream) {
+    if (part_rows == 0 || n_ == 0) return;
+    Plan& pl = plans_[part_rows == 256 ? 0 : (part_rows == 512 ? 1 : 2)];
+    if (!pl.tried) {
+        pl.tried = true;
+        if (order_.empty()) order_ = resident_order(p);
+        ResidentPlan r = resident_plan(p, block_slots_.host(), order_, part_rows);
+        if (!r.blob.empty()) {
+            pl.parts = r.parts;
+            pl.exports = r.exports;
+            pl.blob.host() = std::move(r.blob);
+            upload(pl.blob, bytes_, stream);
+            sync_stream(stream, "resident plan");
+            pl.blob.host() = {};
+        }
+    }
+    if (pl.parts == 0) return;
+    d.res_plan = pl.blob.gpu_data();
+    d.res_part_rows = part_rows;
+    d.res_parts = pl.parts;
+    d.res_exports = pl.exports;
+}
+
+int resident_part_rows(const std::vector<int>& rows) {
+    constexpr long kWorkgroups = 256;
+    for (int pr : {256, 512, CHX_RES_PART_MAX}) {
+        long parts = 0, most = 0;
+        for (int n : rows) {
+            const long q = (n + pr - 1) / pr;
+            parts += q;
+            most = std::max(most, q);
+        }
+        if (parts <= kWorkgroups) return pr;
+        if (pr == CHX_RES_PART_MAX && most <= kWorkgroups) return pr;
+    }
+    return 0;
+}
+
 // ---------------------------------------------------------------------------
 // BatchRunner
 // ---------------------------------------------------------------------------
+
+void BatchRunner::layout_resident(std::vector<chx_instance>& ds, std::uintptr_t stream) {
+    desc_.res_grid = 0;
+    desc_.res_n_items = desc_.res_n_big = 0;
+    int total = 0, most = 0;
+    for (const chx_instance& d : ds) {
+        if (d.n_rows == 0) continue;
+        if (d.res_plan == nullptr) return;
+        total += d.res_parts;
+        most = std::max(most, d.res_parts);
+    }
+    if (most == 0) return;
+    int limit = 0;
+    check(chx_resident_grid_limit(&limit), "engine", "resident grid limit");
+    const int cap = grid_ > 0 ? std::min(limit, grid_) : limit;
+    // Groups of workgroups b = x (mod 8) share an XCD (its L2): gangs of up
+    // to a group stay in one.
+    int grid = 0, groups = 1, per = 0;
+    if (ds.size() == 1) {
+        grid = most <= 32 ? most : (most + 7) / 8 * 8;
+        if (grid > cap) grid = most;
+        groups = grid > 32 && grid % 8 == 0 ? 8 : 1;
+    } else if (cap >= 8) {
+        per = std::min({cap / 8, 32, std::max((total + 7) / 8, std::min(most, 32))});
+        groups = 8;
+        grid = 8 * per;
+    } else {
+        grid = per = cap;
+    }
+    if (grid > cap || most > grid) return;
+    std::size_t words = CHX_RES_CONTROL_WORDS;
+    for (chx_instance& d : ds) {
+        if (d.n_rows == 0) continue;
+        if (words > 0xffffffffu) return;
+        d.res_xbase = static_cast<unsigned>(words);
+        words += CHX_RES_XWORDS(d.res_parts, d.res_exports);
+    }
+    if (xbuf_.gpu_size() < words) {
+        xbuf_.ensure_device(words);
+        xbuf_.zero_device(stream);
+    }
+    auto& it = res_items_.host();
+    it.clear();
+    if (ds.size() > 1) {
+        std::vector<int> by(ds.size());
+        for (std::size_t i = 0; i < by.size(); ++i) by[i] = static_cast<int>(i);
+        by.erase(std::remove_if(by.begin(), by.end(), [&](int i) { return ds[i].n_rows == 0; }), by.end());
+        std::stable_sort(by.begin(), by.end(), [&](int i, int j) {
+            return ds[i].res_parts != ds[j].res_parts ? ds[i].res_parts > ds[j].res_parts : ds[i].n_rows > ds[j].n_rows;
+        });
+        // large items: each on the run of ranks that is free first
+        std::vector<int> busy(static_cast<std::size_t>(grid), 0);
+        for (int i : by) {
+            const int parts = ds[i].res_parts;
+            int base = 0;
+            if (parts > per) {
+                int best = std::numeric_limits<int>::max();
+                for (int b = 0; b + parts <= grid; ++b) {
+                    const int t = *std::max_element(busy.begin() + b, busy.begin() + b + parts);
+                    if (t < best) {
+                        best = t;
+                        base = b;
+                    }
+                }
+                std::fill(busy.begin() + base, busy.begin() + base + parts, best + 1);
+                ++desc_.res_n_big;
+            }
+            it.insert(it.end(), {i, parts, base, 0});
+        }
+        res_items_.copy_to_device(stream);
+        desc_.res_items = res_items_.gpu_data();
+        desc_.res_n_items = static_cast<int>(by.size());
+    }
+    desc_.xbuf = xbuf_.gpu_data();
+    desc_.res_xwords = xbuf_.gpu_size();
+    desc_.res_groups = groups;
+    desc_.res_grid = grid;
+}
+
+void BatchRunner::set_grid_blocks(int g) {
+    g = g < 0 ? 0 : g;
+    if (g == grid_) return;
+    grid_ = g;
+    desc_.grid_blocks = g;
+    if (!bound()) return;
+    // Queued launches may still read the old lists.
+    check(chx_device_synchronize(), "engine", "work list rebuild");
+    if (desc_.inst == nullptr) {
+        std::vector<chx_instance> one{desc_.single};
+        layout_resident(one);
+        desc_.single = one[0];
+    } else {
+        layout_resident(table_host_);
+        table_.host() = table_host_;
+        table_.copy_to_device();
+        desc_.inst = table_.gpu_data();
+    }
+    check(chx_device_synchronize(), "engine", "work list rebuild");
+}
 
 void BatchRunner::set_lanes_per_row(int L) {
     if (L != 4 && L != 8 && L != 16) throw std::invalid_argument("chysx::engine: lanes_per_row must be 4, 8 or 16");
@@ -763,6 +902,8 @@ BatchRunner& BatchRunner::operator=(BatchRunner&& o) noexcept {
     inst_done_ = std::move(o.inst_done_);
     sync_ = std::move(o.sync_);
     trace_ = std::move(o.trace_);
+    xbuf_ = std::move(o.xbuf_);
+    res_items_ = std::move(o.res_items_);
     status_host_ = o.status_host_;
     o.graph_ = nullptr;
     o.status_host_ = nullptr;
@@ -843,6 +984,7 @@ static int entries16_all(const std::vector<chx_instance>& ds) {
 void BatchRunner::bind_single(const chx_instance& d, std::uintptr_t stream) {
     std::vector<chx_instance> one{d};
     build_tiles(one, stream);
+    layout_resident(one, stream);
     desc_.tiles = nullptr;  // implied by tile_rows: no tile record loads
     desc_.n_instances = 1;
     desc_.n_elem_items = 0;
@@ -870,6 +1012,7 @@ void BatchRunner::bind_many(const std::vector<chx_instance>& ds, std::uintptr_t 
     }
     table_host_ = ds;
     build_tiles(table_host_, stream);
+    layout_resident(table_host_, stream);
     auto& ei = elem_items_.host();
     auto& si = unit_items_.host();
     ei.clear();
@@ -915,6 +1058,7 @@ void BatchRunner::update_many(const std::vector<chx_instance>& ds, std::uintptr_
         chx_instance d = ds[i];
         d.tile_begin = table_host_[i].tile_begin;
         d.tile_end = table_host_[i].tile_end;
+        d.res_xbase = table_host_[i].res_xbase;
         if (std::memcmp(&d, &table_host_[i], sizeof(chx_instance)) != 0) {
             table_host_[i] = d;
             changed = true;

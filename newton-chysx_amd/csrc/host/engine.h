@@ -17,6 +17,7 @@
 
 #include "chysx_common.h"
 #include "constraints.h"
+#include "resident_plan.h"
 #include "topology.h"
 
 namespace chysx {
@@ -70,6 +71,10 @@ public:
     void update_shapes(const InstanceSource& s, std::uintptr_t stream = 0);
     // Descriptor for a launch: device arrays + the step scalars of `s`.
     chx_instance descriptor(const InstanceSource& s) const;
+    // Adds the resident-solve plan for parts of `part_rows` rows to a
+    // descriptor (none when the pattern does not fit it, or part_rows is 0).
+    // Plans are built on first use and kept until the next build().
+    void attach_plan(chx_instance& d, const topology::Pattern& p, int part_rows, std::uintptr_t stream);
     bool built() const noexcept { return built_; }
     int n_rows() const noexcept { return n_; }
     int nnz() const noexcept { return nnz_; }
@@ -116,9 +121,21 @@ private:
     DeviceArray<int> slice_offsets_, slice_entries_, upper_offsets_, block_slots_;  // sliced symmetric layout
     DeviceArray<uint16_t> slice_entries16_;  // the entries in 16 bits, when every one fits (else empty)
     bool entries16_ = false;
+    struct Plan {
+        bool tried = false;
+        int parts = 0, exports = 0;
+        DeviceArray<std::uint32_t> blob;
+    };
+    Plan plans_[3];           // parts of 256, 512 and 1024 rows
+    std::vector<int> order_;  // canonical row order of the plans
     DeviceArray<chx_plane> planes_;
     DeviceArray<chx_box> boxes_;
 };
+
+// Rows per part of the resident solve of cloths with `rows` vertices each:
+// the smallest part size whose parts all run at once on 256 workgroups, else
+// the largest; 0 when some cloth alone has more parts than that.
+int resident_part_rows(const std::vector<int>& rows);
 
 class BatchRunner {
 public:
@@ -136,10 +153,12 @@ public:
     // Per-step scalars / external pointers of the bound instances.
     void update_single(const chx_instance& d) {
         const int tb = desc_.single.tile_begin, te = desc_.single.tile_end;
+        const unsigned xb = desc_.single.res_xbase;
         desc_.entries16 = (d.n_rows > 0 && d.slice_entries16 == nullptr) ? 0 : 1;
         desc_.single = d;
         desc_.single.tile_begin = tb;
         desc_.single.tile_end = te;
+        desc_.single.res_xbase = xb;
     }
     void update_many(const std::vector<chx_instance>& ds, std::uintptr_t stream);
 
@@ -162,10 +181,7 @@ public:
     // list of a bound batch.
     void set_tile_rows(int rows);
     int tile_rows() const noexcept { return tile_rows_; }
-    void set_grid_blocks(int g) {
-        grid_ = g < 0 ? 0 : g;
-        desc_.grid_blocks = grid_;
-    }
+    void set_grid_blocks(int g);
     // SpMV form of the PCG launch: LDS-staged stages (default) or gathers
     // straight from global memory (smaller LDS, more workgroups per CU).
     void set_lds_staging(bool on) { desc_.no_lds_staging = on ? 0 : 1; }
@@ -215,6 +231,11 @@ private:
     // Tile list of the bound instances; sets their tile_begin / tile_end.
     void build_tiles(std::vector<chx_instance>& ds, std::uintptr_t stream = 0);
 
+    // Work lists and exchange area of the resident solve of the bound
+    // instances; leaves the launch to the streaming kernels when one of them
+    // has no plan or the grid does not hold its parts.
+    void layout_resident(std::vector<chx_instance>& ds, std::uintptr_t stream = 0);
+
     chx_cloth_batch desc_{};
     void* graph_ = nullptr;           // hipGraphExec_t of one substep
     chx_cloth_batch graph_desc_{};    // the descriptor it was captured with
@@ -231,6 +252,8 @@ private:
     DeviceArray<int> inst_iters_, inst_done_;
     DeviceArray<unsigned> sync_;
     DeviceArray<unsigned long long> trace_;
+    DeviceArray<unsigned long long> xbuf_;
+    DeviceArray<int> res_items_;
 };
 
 }  // namespace engine
