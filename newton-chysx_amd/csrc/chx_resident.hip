@@ -47,6 +47,9 @@ constexpr unsigned kPart = CHX_RES_PART_MAX;
 constexpr int kLeaves = CHX_RES_PART_MAX / CHX_RES_LEAF;
 constexpr int kSums = 5;  // rho, sigma, delta, gamma, ||r||^2 (set-up: ||b||^2 in place of sigma)
 constexpr int kMaxParts = 256;
+constexpr unsigned kFan = 16;    // parts per group and groups, above 64 parts
+constexpr unsigned kCopies = 16;  // copies of the groups' sums
+static_assert(kFan * kFan >= kMaxParts && 2 * kCopies <= 64, "two levels");
 constexpr unsigned kNoSlot = 0xffffu;
 constexpr unsigned kExit = 0xffffffu;  // mailbox item: nothing left
 static_assert(CHX_RES_LEAF == kWave && kSlots == 2 && kLeaves == 16, "a leaf per wave and slot");
@@ -62,14 +65,37 @@ __device__ __forceinline__ void st64(u64* p, u64 v) {
 }
 __device__ __forceinline__ u64 tagged(unsigned v, unsigned tag) { return (u64(tag) << 32) | v; }
 
+// LDS triples as one 96-bit access.
+typedef float v3f __attribute__((ext_vector_type(3), aligned(4)));
+__device__ __forceinline__ f3 lds_ld(const f3* p) {
+    const v3f v = *reinterpret_cast<const v3f*>(p);
+    return {v.x, v.y, v.z};
+}
+__device__ __forceinline__ void lds_st(f3* p, f3 v) {
+    v3f w;
+    w.x = v.x;
+    w.y = v.y;
+    w.z = v.z;
+    *reinterpret_cast<v3f*>(p) = w;
+}
+// Keeps a value that the loop does not change from being re-derived ahead of
+// the loop (addresses and masks of every block would not fit the registers).
+__device__ __forceinline__ unsigned opaque(unsigned v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 struct ResLds {
-    f3 prod[kHeld * CHX_RES_PART_MAX];             // transposed products, by target row
+    // transposed products by target row, then one unread slot per lane for
+    // blocks without a target
+    f3 prod[kHeld * CHX_RES_PART_MAX + kWave];
     f3 p[CHX_RES_PART_MAX + CHX_RES_HALO_MAX];     // source vector: own rows, halo rows
     float diag[6][CHX_RES_PART_MAX];
     f3 x[CHX_RES_PART_MAX];
+    float ghost[9][CHX_RES_GHOST_MAX];
     double leaf[kLeaves][kSums];
     double tot[8];
-    int bad_sums, bad_halo;  // a wait gave up (two words: each read before the other's next write)
+    int bad;         // a wait gave up
     unsigned mail;   // mailbox word of the workgroup
 };
 
@@ -103,32 +129,30 @@ struct Watch {
     }
 };
 
-// N tagged words from p on; false: the wait was given up.
+// N tagged words from p on, read until every tag is the awaited one; false:
+// the wait was given up.
 template <int N>
 __device__ __forceinline__ bool await(const u64* p, unsigned tag, unsigned (&v)[N], const Barrier& bar) {
     u64 w[N];
-    bool ok = true;
+    auto read = [&] {
+        bool ok = true;
 #pragma unroll
-    for (int k = 0; k < N; ++k) w[k] = ld64(p + k);
+        for (int k = 0; k < N; ++k) w[k] = ld64(p + k);
 #pragma unroll
-    for (int k = 0; k < N; ++k) ok = ok && unsigned(w[k] >> 32) == tag;
-    if (!ok) {
+        for (int k = 0; k < N; ++k) ok = ok && unsigned(w[k] >> 32) == tag;
+        return ok;
+    };
+    if (!read()) {
         Watch watch(bar);
         unsigned seen = 0;
         do {
             if (!watch.again(nullptr, seen)) return false;
-#pragma unroll
-            for (int k = 0; k < N; ++k) w[k] = ld64(p + k);
-            ok = true;
-#pragma unroll
-            for (int k = 0; k < N; ++k) ok = ok && unsigned(w[k] >> 32) == tag;
-        } while (!ok);
+        } while (!read());
     }
 #pragma unroll
     for (int k = 0; k < N; ++k) v[k] = unsigned(w[k]);
     return true;
 }
-
 __device__ __forceinline__ f3 mv9t(const float (&m)[9], f3 v) {
     const float b[9] = {m[0], m[3], m[6], m[1], m[4], m[7], m[2], m[5], m[8]};
     return mv9(b, v);
@@ -149,6 +173,58 @@ __device__ __forceinline__ void ld6u(gp<const float> m, unsigned i, float (&u)[6
 }
 __device__ __forceinline__ f3 axpy(float a, f3 x, f3 y) { return mk(fmaf(a, x.x, y.x), fmaf(a, x.y, y.y), fmaf(a, x.z, y.z)); }
 
+// The wave's two leaf sums of kSums values into S.leaf.  Halving butterfly:
+// each step adds lane pairs and packs two values into the two halves of the
+// pairs, so five values of two leaves take 14 FP64 adds instead of 60.
+template <int CTRL>
+__device__ __forceinline__ double dpp64(double v) {
+    const u64 b = u64(__double_as_longlong(v));
+    const unsigned lo = unsigned(__builtin_amdgcn_mov_dpp(int(unsigned(b)), CTRL, 0xf, 0xf, true));
+    const unsigned hi = unsigned(__builtin_amdgcn_mov_dpp(int(unsigned(b >> 32)), CTRL, 0xf, 0xf, true));
+    return __longlong_as_double((long long)((u64(hi) << 32) | lo));
+}
+constexpr int kRor8 = 0x128, kHalfMirror = 0x141, kXor2 = 0x4e, kXor1 = 0xb1;  // DPP controls
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+// lanes of half 0: a summed over the pairs; of half 1: b
+__device__ __forceinline__ double fold32(double a, double b) {
+    const u64 x = u64(__double_as_longlong(a)), y = u64(__double_as_longlong(b));
+    const v2u lo = __builtin_amdgcn_permlane32_swap(unsigned(x), unsigned(y), false, false);
+    const v2u hi = __builtin_amdgcn_permlane32_swap(unsigned(x >> 32), unsigned(y >> 32), false, false);
+    return __longlong_as_double((long long)((u64(hi.x) << 32) | lo.x)) +
+           __longlong_as_double((long long)((u64(hi.y) << 32) | lo.y));
+}
+__device__ __forceinline__ double fold16(double a, double b) {
+    const u64 x = u64(__double_as_longlong(a)), y = u64(__double_as_longlong(b));
+    const v2u lo = __builtin_amdgcn_permlane16_swap(unsigned(x), unsigned(y), false, false);
+    const v2u hi = __builtin_amdgcn_permlane16_swap(unsigned(x >> 32), unsigned(y >> 32), false, false);
+    return __longlong_as_double((long long)((u64(hi.x) << 32) | lo.x)) +
+           __longlong_as_double((long long)((u64(hi.y) << 32) | lo.y));
+}
+__device__ __forceinline__ double fold8(double a, double b, unsigned lane) {
+    const bool up = (lane & 8u) != 0u;
+    return (up ? b : a) + dpp64<kRor8>(up ? a : b);
+}
+__device__ __forceinline__ void leaf_sums(const double (&a)[kSums], const double (&b)[kSums], ResLds& S, unsigned wave,
+                                          unsigned lane) {
+    double v[kSums];
+#pragma unroll
+    for (int k = 0; k < kSums; ++k) v[k] = fold32(a[k], b[k]);  // half h: leaf of slot h
+    // rows (16 lanes) 2h, 2h + 1 of half h: values 0 | 1, 2 | 3, 4 | 4
+    const double x = fold16(v[0], v[1]), y = fold16(v[2], v[3]), z = fold16(v[4], v[4]);
+    double w0 = fold8(x, y, lane);             // half-rows: values 0 2 | 1 3
+    double w1 = z + dpp64<kRor8>(z);           // value 4 everywhere
+    w0 += dpp64<kHalfMirror>(w0);
+    w1 += dpp64<kHalfMirror>(w1);
+    w0 += dpp64<kXor2>(w0);
+    w1 += dpp64<kXor2>(w1);
+    w0 += dpp64<kXor1>(w0);
+    w1 += dpp64<kXor1>(w1);
+    double(&out)[kSums] = S.leaf[(lane >> 5) * kWaves + wave];
+    const unsigned place = lane & 31u;
+    if ((place & 7u) == 0u) out[(place >> 4) + ((place & 8u) >> 2)] = w0;
+    if (place == 1u) out[4] = w1;
+}
+
 // Solves instance `inst` together with the workgroups that hold its other
 // parts; this one holds part `part`.  False: aborted.
 __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst& I, int inst, int part, unsigned epoch, ResLds& S,
@@ -161,12 +237,18 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     const unsigned n_own = hdr[0], n_halo = hdr[1], halo_at = hdr[2], n_ghost = hdr[3], ghost_at = hdr[4];
     const unsigned pos0 = unsigned(part) * unsigned(I.res_part_rows);
     const unsigned rows_at = 8u * parts, meta_at = rows_at + n, exp_at = meta_at + n, held_at = exp_at + n;
-    // exchange areas: [2][parts] lines of 16 words, then [2][exports] rows of 3
+    // exchange areas: [2][kSums][parts] pairs of words, then [2][exports] rows of 3
     u64* const xsum = B.xbuf + I.res_xbase;
-    u64* const xrow = xsum + 32ull * parts;
+    u64* const xgroup = xsum + 4u * kSums * parts;  // [2][kCopies][kSums][kFan] pairs
+    u64* const xrow = xgroup + (parts > unsigned(kWave) ? 4u * kCopies * kSums * kFan : 0u);
     const unsigned exports = unsigned(I.res_exports);
     auto tag_of = [&](int t) { return (epoch << 8) | (unsigned(t) & 255u); };
-    auto sum_line = [&](int t, unsigned q) { return xsum + 16ull * ((unsigned(t) & 1u) * parts + q); };
+    auto sum_words = [&](int t, unsigned v, unsigned q) {
+        return xsum + 2u * (((unsigned(t) & 1u) * kSums + v) * parts + q);
+    };
+    auto group_words = [&](int t, unsigned copy, unsigned v, unsigned g) {
+        return xgroup + 2u * ((((unsigned(t) & 1u) * kCopies + copy) * kSums + v) * kFan + g);
+    };
     auto row_words = [&](int t, unsigned e) { return xrow + 3ull * ((unsigned(t) & 1u) * exports + e); };
 
     auto send_row = [&](int t, unsigned e, f3 v) {
@@ -177,7 +259,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     };
 
     // ---- load: own rows, ghost block, halo row ----
-    unsigned lp[kSlots], row[kSlots], ns[kSlots], nh[kSlots], ex[kSlots], word[kSlots][kHeld];
+    unsigned lp[kSlots], ex[kSlots], word[kSlots][kHeld];
     bool live[kSlots], on[kSlots];  // this lane's row exists; this wave has a row
     float V[kSlots][kHeld][9], M[kSlots][6];
     f3 r[kSlots], p[kSlots], q[kSlots];
@@ -187,55 +269,65 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         on[s] = (unsigned(s) * kWaves + wave) * kWave < n_own;
         live[s] = lp[s] < n_own;
         const unsigned K = pos0 + (live[s] ? lp[s] : 0u);
-        row[s] = 0u;
-        ns[s] = nh[s] = 0u;
         ex[s] = CHX_RES_NONE;
+        r[s] = p[s] = q[s] = mk(0.f, 0.f, 0.f);
         if (on[s]) {
-            row[s] = ldx(plan, rows_at + K);
+            unsigned ns = 0u, nh = 0u;
+            const unsigned row = ldx(plan, rows_at + K);
             const unsigned meta = ldx(plan, meta_at + K);
             if (live[s]) {
-                ns[s] = meta & 15u;
-                nh[s] = meta >> 4;
+                ns = meta & 15u;
+                nh = meta >> 4;
                 ex[s] = ldx(plan, exp_at + K);
             }
-            const unsigned vs = unsigned(ldx(I.upper_offsets, row[s] / CHX_SLICE_ROWS)) + row[s] % CHX_SLICE_ROWS;
+            const unsigned vs = unsigned(ldx(I.upper_offsets, row / CHX_SLICE_ROWS)) + row % CHX_SLICE_ROWS;
 #pragma unroll
             for (int u = 0; u < kHeld; ++u) {
-                const bool has = unsigned(u) < nh[s];
-                word[s][u] = has ? ldx(plan, held_at + unsigned(u) * n + K) : (kNoSlot << 16);
+                // a block that is not there is zero, of the row itself, and
+                // its product slot stays zero: both are added like the others
+                const bool has = unsigned(u) < nh;
+                unsigned w = has ? ldx(plan, held_at + unsigned(u) * n + K) : (kNoSlot << 16) | lp[s];
+                if ((w >> 16) == kNoSlot) w = (w & 0xffffu) | ((kHeld * kPart + lane) << 16);
+                word[s][u] = w;
+                if (unsigned(u) >= ns) S.prod[unsigned(u) * kPart + lp[s]] = mk(0.f, 0.f, 0.f);
 #pragma unroll
                 for (int c = 0; c < 9; ++c) V[s][u][c] = 0.0f;
                 if (has) ld9p(gp<const float>(I.values), vs + unsigned(u) * CHX_SLICE_ROWS, V[s][u]);
             }
             float d[6], full[9];
-            ld6u(gp<const float>(I.diag), row[s], d);
+            ld6u(gp<const float>(I.diag), row, d);
 #pragma unroll
             for (int c = 0; c < 6; ++c) S.diag[c][lp[s]] = d[c];
             inverse_sym(d, M[s], full);
-            p[s] = ld3g(I.x, row[s]);
+            if (live[s]) p[s] = ld3g(I.x, row);
             S.x[lp[s]] = p[s];
             S.p[lp[s]] = p[s];
         }
     }
-    float Gv[9];
+    // ghost blocks and halo rows from the last thread down: in a small part
+    // the first waves have the rows
+    const unsigned rtid = unsigned(kThreads - 1) - tid;
     unsigned gword = 0;
-    if (tid < n_ghost) {
-        const unsigned vs = ldx(plan, ghost_at + 2u * tid);
-        gword = ldx(plan, ghost_at + 2u * tid + 1u);
-        ld9p(gp<const float>(I.values), vs, Gv);
+    if (rtid < n_ghost) {
+        const unsigned vs = ldx(plan, ghost_at + 2u * rtid);
+        gword = ldx(plan, ghost_at + 2u * rtid + 1u);
+        float g[9];
+        ld9p(gp<const float>(I.values), vs, g);
+#pragma unroll
+        for (int c = 0; c < 9; ++c) S.ghost[c][rtid] = g[c];
     }
     float hM[6];
     f3 hr = mk(0.f, 0.f, 0.f);
     unsigned hex = 0;
-    if (tid < n_halo) {
-        const unsigned hrow = ldx(plan, halo_at + 2u * tid);
-        hex = ldx(plan, halo_at + 2u * tid + 1u);
+    if (rtid < n_halo) {
+        const unsigned hrow = ldx(plan, halo_at + 2u * rtid);
+        hex = ldx(plan, halo_at + 2u * rtid + 1u);
         float d[6], full[9];
         ld6u(gp<const float>(I.diag), hrow, d);
         inverse_sym(d, hM, full);
-        S.p[kPart + tid] = ld3g(I.x, hrow);
+        S.p[kPart + rtid] = ld3g(I.x, hrow);
     }
-    if (tid == 0) S.bad_sums = S.bad_halo = 0;
+    if (tid == 0) S.bad = 0;
     if (tid < kLeaves * kSums) S.leaf[tid / kSums][tid % kSums] = 0.0;
 
     // A times the vector in S.p (own rows also in v); S.p and
@@ -245,45 +337,38 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         for (int s = 0; s < kSlots; ++s)
             if (on[s]) {
 #pragma unroll
-                for (int u = 0; u < kHeld; ++u) {
-                    const unsigned t = word[s][u] >> 16;
-                    if (t != kNoSlot) S.prod[t] = mv9t(V[s][u], v[s]);
-                }
+                for (int u = 0; u < kHeld; ++u) lds_st(&S.prod[opaque(word[s][u]) >> 16], mv9t(V[s][u], v[s]));
             }
         __syncthreads();
-        if (tid < n_ghost) S.prod[gword >> 16] = mv9t(Gv, S.p[gword & 0xffffu]);
+        if (rtid < n_ghost) {
+            float g[9];
+#pragma unroll
+            for (int c = 0; c < 9; ++c) g[c] = S.ghost[c][rtid];
+            lds_st(&S.prod[gword >> 16], mv9t(g, lds_ld(&S.p[gword & 0xffffu])));
+        }
         __syncthreads();
 #pragma unroll
         for (int s = 0; s < kSlots; ++s)
             if (on[s]) {
                 float d[6];
+                f3 low[kHeld], src[kHeld];
+#pragma unroll
+                for (int u = 0; u < kHeld; ++u) src[u] = lds_ld(&S.p[opaque(word[s][u]) & 0xffffu]);
 #pragma unroll
                 for (int c = 0; c < 6; ++c) d[c] = S.diag[c][lp[s]];
+#pragma unroll
+                for (int l = 0; l < kHeld; ++l) low[l] = lds_ld(&S.prod[unsigned(l) * kPart + lp[s]]);
                 f3 sum = mv_sym(d, v[s]);
 #pragma unroll
-                for (int l = 0; l < kHeld; ++l) {
-                    const f3 t = S.prod[unsigned(l) * kPart + lp[s]];
-                    if (unsigned(l) < ns[s]) sum = add(sum, t);
-                }
+                for (int l = 0; l < kHeld; ++l) sum = add(sum, low[l]);
 #pragma unroll
-                for (int u = 0; u < kHeld; ++u) {
-                    const f3 t = mv9(V[s][u], S.p[word[s][u] & 0xffffu]);
-                    if (unsigned(u) < nh[s]) sum = add(sum, t);
-                }
+                for (int u = 0; u < kHeld; ++u) sum = add(sum, mv9(V[s][u], src[u]));
                 out[s] = sum;
             }
     };
     // Sums of phase t: per leaf, then over the part's leaves, sent to the gang.
     auto send_sums = [&](int t, double (&acc)[kSlots][kSums]) {
-#pragma unroll
-        for (int s = 0; s < kSlots; ++s)
-            if (on[s]) {
-#pragma unroll
-                for (int v = 0; v < kSums; ++v) {
-                    const double w = wave_sum(acc[s][v]);
-                    if (lane == 0) S.leaf[unsigned(s) * kWaves + wave][v] = w;
-                }
-            }
+        leaf_sums(acc[0], acc[1], S, wave, lane);
         __syncthreads();
         if (tid < 8 * kSums) {
             const unsigned v = tid >> 3, i = tid & 7u;
@@ -296,37 +381,54 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                     S.tot[v] = w;
                 } else {
                     const u64 b = u64(__double_as_longlong(w));
-                    u64* const line = sum_line(t, unsigned(part)) + 2 * v;
-                    st64(line, tagged(unsigned(b), tag_of(t)));
-                    st64(line + 1, tagged(unsigned(b >> 32), tag_of(t)));
+                    u64* const w2 = sum_words(t, v, unsigned(part));
+                    st64(w2, tagged(unsigned(b), tag_of(t)));
+                    st64(w2 + 1, tagged(unsigned(b >> 32), tag_of(t)));
                 }
             }
         }
     };
-    // The instance's sums of phase t into S.tot (tree over the parts).
+    // The instance's sums of phase t into S.tot: a tree over the parts, read
+    // by everyone up to 64 parts; above, the first part of every 16 sums them
+    // up and sends the result to kCopies places, each read by some of the
+    // parts (256 readers of 256 parts' words took 20 us a phase).
     auto take_sums = [&](int t) -> bool {
         if (parts > 1 && wave < kSums) {
-            double w = 0.0;
+            auto fetch = [&](const u64* at, bool mine, double& w) {
+                unsigned b[2];
+                w = 0.0;
+                if (!mine) return true;
+                if (!await<2>(at, tag_of(t), b, bar)) return false;
+                w = __longlong_as_double((long long)((u64(b[1]) << 32) | b[0]));
+                return true;
+            };
+            double w;
             bool ok = true;
-            const unsigned per = parts > unsigned(kWave) ? 4u : 1u;
-            double part_sum[4] = {0.0, 0.0, 0.0, 0.0};
+            if (parts <= unsigned(kWave)) {
+                ok = fetch(sum_words(t, wave, lane), lane < parts, w);
 #pragma unroll
-            for (unsigned k = 0; k < 4; ++k) {
-                const unsigned j = per * lane + k;
-                if (k < per && j < parts) {
-                    unsigned b[2];
-                    ok = ok && await<2>(sum_line(t, j) + 2 * wave, tag_of(t), b, bar);
-                    if (ok) part_sum[k] = __longlong_as_double((long long)((u64(b[1]) << 32) | b[0]));
+                for (int m = 1; m < kWave; m <<= 1) w += __shfl_xor(w, m);
+            } else {
+                if ((unsigned(part) % kFan) == 0u) {
+                    ok = fetch(sum_words(t, wave, unsigned(part) + lane), lane < kFan && unsigned(part) + lane < parts, w);
+#pragma unroll
+                    for (unsigned m = 1; m < kFan; m <<= 1) w += __shfl_xor(w, int(m));
+                    w = __shfl(w, 0);
+                    const u64 b = u64(__double_as_longlong(w));
+                    if (ok && lane < 2u * kCopies)
+                        st64(group_words(t, lane >> 1, wave, unsigned(part) / kFan) + (lane & 1u),
+                             tagged((lane & 1u) != 0u ? unsigned(b >> 32) : unsigned(b), tag_of(t)));
                 }
-            }
-            w = per == 4 ? (part_sum[0] + part_sum[1]) + (part_sum[2] + part_sum[3]) : part_sum[0];
+                ok = __ballot(!ok) == 0ull &&
+                     fetch(group_words(t, unsigned(part) % kCopies, wave, lane), lane < (parts + kFan - 1u) / kFan, w);
 #pragma unroll
-            for (int m = 1; m < kWave; m <<= 1) w += __shfl_xor(w, m);
+                for (unsigned m = 1; m < kFan; m <<= 1) w += __shfl_xor(w, int(m));
+            }
             if (lane == 0) S.tot[wave] = w;
-            if (!ok) S.bad_sums = 1;
+            if (!ok) S.bad = 1;
         }
         __syncthreads();
-        return S.bad_sums == 0;
+        return S.bad == 0;
     };
 
     // ---- set-up: r_0 = b - A x, z_0 = p_0 = M^-1 r_0 ----
@@ -338,7 +440,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
 #pragma unroll
         for (int v = 0; v < kSums; ++v) acc[s][v] = 0.0;
         if (on[s] && live[s]) {
-            const f3 b = ld3g(I.rhs, row[s]);
+            const f3 b = ld3g(I.rhs, ldx(plan, rows_at + pos0 + lp[s]));
             r[s] = sub(b, q[s]);
             p[s] = mv_sym(M[s], r[s]);
             if (ex[s] != CHX_RES_NONE) send_row(0, ex[s], r[s]);
@@ -351,6 +453,17 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     }
     double bb = 0.0;
     for (int k = 0;; ++k) {
+        const bool last = k > 0 && k >= I.max_iter;  // at the cap: the last update only
+        // The halo rows' q_{k-1} (set-up: r_0), sent before the sums: waiting
+        // for them first hides their way behind the sums'.
+        f3 h = mk(0.f, 0.f, 0.f);
+        if (rtid < n_halo && !last) {
+            unsigned w[3];
+            if (await<3>(row_words(k, hex), tag_of(k), w, bar))
+                h = mk(__uint_as_float(w[0]), __uint_as_float(w[1]), __uint_as_float(w[2]));
+            else
+                S.bad = 1;
+        }
         if (!take_sums(k)) return false;
         const double rho = S.tot[0], sig = S.tot[1], del = S.tot[2], gam = S.tot[3], rr = S.tot[4];
         if (k == 0) bb = sig;
@@ -373,21 +486,14 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             (void)__hip_atomic_fetch_add(&B.xbuf[RES_PROGRESS], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         float alpha = 0.0f, beta = 0.0f;
         if (k > 0) merged_scalars(rho, sig, del, gam, alpha, beta);
-        const bool last = k >= I.max_iter;  // at the cap: the last update only
         // halo rows: r_k, z_k, p_k as their owners form them
-        if (tid < n_halo && !last) {
-            unsigned w[3];
-            if (await<3>(row_words(k, hex), tag_of(k), w, bar)) {
-                const f3 h = mk(__uint_as_float(w[0]), __uint_as_float(w[1]), __uint_as_float(w[2]));
-                if (k == 0) {
-                    hr = h;
-                    S.p[kPart + tid] = mv_sym(hM, hr);
-                } else {
-                    hr = axpy(-alpha, h, hr);
-                    S.p[kPart + tid] = axpy(beta, S.p[kPart + tid], mv_sym(hM, hr));
-                }
+        if (rtid < n_halo && !last) {
+            if (k == 0) {
+                hr = h;
+                lds_st(&S.p[kPart + rtid], mv_sym(hM, hr));
             } else {
-                S.bad_halo = 1;
+                hr = axpy(-alpha, h, hr);
+                lds_st(&S.p[kPart + rtid], axpy(beta, lds_ld(&S.p[kPart + rtid]), mv_sym(hM, hr)));
             }
         }
 #pragma unroll
@@ -400,10 +506,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                 }
                 S.p[lp[s]] = p[s];
             }
-        if (!last) {
-            apply(p, q);
-            if (S.bad_halo != 0) return false;
-        }
+        if (!last) apply(p, q);
         double acc[kSlots][kSums];
 #pragma unroll
         for (int s = 0; s < kSlots; ++s) {
@@ -425,7 +528,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     }
 #pragma unroll
     for (int s = 0; s < kSlots; ++s)
-        if (on[s] && live[s]) st3g(I.x, row[s], S.x[lp[s]]);
+        if (live[s]) st3g(I.x, ldx(plan, rows_at + pos0 + lp[s]), S.x[lp[s]]);
     return true;
 }
 
@@ -584,6 +687,13 @@ int resident_grid_limit() {
 }
 
 void launch_resident(const chx_cloth_batch& B, int finalize, hipStream_t stream) {
+    if (B.res_grid == 1) {
+        // nothing waits for another workgroup: an ordinary launch, without the
+        // ~11 us before and after that a cooperative one takes
+        resident_kernel<<<1, kThreads, 0, stream>>>(B, finalize);
+        hip_check(hipGetLastError(), "resident_kernel launch");
+        return;
+    }
     chx_cloth_batch arg = B;
     int fin = finalize;
     void* args[] = {&arg, &fin};
