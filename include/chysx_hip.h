@@ -164,15 +164,31 @@ typedef struct chx_unit {
  * and ghost blocks (blocks of halo rows whose column is in the part).
  *
  * res_plan (32-bit words): 8 words per part {rows, halo rows, word offset of
- * its halo list, ghost blocks, word offset of its ghost list, 0, 0, 0}; then
- * over the n_rows positions: the row, (lower blocks | upper blocks << 4),
- * the row's export index (CHX_RES_NONE: no other part reads it), and
- * CHX_RES_HELD planes of (local index of the upper block's column) |
- * (product slot << 16); then the halo lists {row, export index} and ghost
- * lists {value slot, local index of the source row | product slot << 16}.
- * Local indices: position in the part, or CHX_RES_PART_MAX + halo index.
- * A product slot is (place among the target row's lower blocks) *
- * CHX_RES_PART_MAX + (target's position in the part); 0xffff: none. */
+ * its halo list, ghost blocks, word offset of its ghost list, widest row, 0,
+ * 0}; then over the n_rows positions: the row, (blocks the row gets through
+ * product slots | blocks its thread holds << 8), the row's export index
+ * (CHX_RES_NONE: no other part reads it), planes of held blocks, and the
+ * lists: halo {row, export index}, ghost {value slot, local index of the
+ * source row | product slot << 16}.  Local indices: position in the part, or
+ * part capacity + halo index.
+ *
+ * Sheet form (res_general 0; every row at most CHX_RES_HELD lower and upper
+ * blocks): CHX_RES_HELD planes, word = local index of upper block u's column
+ * | product slot << 16.  A product slot is (place among the target row's
+ * lower blocks) * CHX_RES_PART_MAX + (target's position); 0xffff: none.
+ *
+ * General form (res_general 1; at most CHX_RES_GEN_WIDTH blocks a row, parts
+ * of at most CHX_RES_GEN_PART rows): every pair's block is held by one of
+ * its rows, at most CHX_RES_GEN_HELD a row: CHX_RES_GEN_HELD planes of words
+ * local index of the other row | product slot << 10 | place in the row's own
+ * column order << 24, then as many planes of value slots (bit 31: the
+ * row needs the transpose).  Product slots are (place in the target row's
+ * column order) * CHX_RES_GEN_PART + (target's position); 0x3fff: none.  The
+ * ghost lists' value slots carry bit 31 when the target row needs the block
+ * as stored. */
+#define CHX_RES_GEN_PART 512
+#define CHX_RES_GEN_HELD 8
+#define CHX_RES_GEN_WIDTH 16
 #define CHX_RES_LEAF 64
 #define CHX_RES_PART_MAX 1024
 #define CHX_RES_HELD 6
@@ -272,7 +288,9 @@ typedef struct chx_instance {
     int res_part_rows;               /* rows per part                                        */
     int res_parts;                   /* ceil(n_rows / res_part_rows)                         */
     int res_exports;                 /* exported rows                                        */
+    int res_general;                 /* the plan's form                                      */
     unsigned res_xbase;              /* first word of the instance's exchange area in xbuf   */
+    int res_pad;
 } chx_instance;
 
 /* A batch of instances advanced together.  Work lists are device int4
@@ -347,7 +365,7 @@ typedef struct chx_cloth_batch {
                                      /* workgroups: solved in list order by the ranks     */
                                      /* from their first rank on                          */
     int res_groups;
-    int res_pad;
+    int res_general;                 /* form of all the instances' plans                  */
     unsigned long long res_xwords;   /* 64-bit words of xbuf                              */
 } chx_cloth_batch;
 

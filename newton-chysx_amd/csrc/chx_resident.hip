@@ -41,18 +41,36 @@ namespace {
 
 constexpr int kThreads = 512;  // two waves per SIMD with 256 VGPRs each
 constexpr int kWaves = kThreads / kWave;
-constexpr int kSlots = CHX_RES_PART_MAX / kThreads;  // own rows per thread
-constexpr int kHeld = CHX_RES_HELD;
-constexpr unsigned kPart = CHX_RES_PART_MAX;
 constexpr int kLeaves = CHX_RES_PART_MAX / CHX_RES_LEAF;
+// The two forms of a plan (chysx_hip.h).  Sheet: a row's lower blocks come
+// through product slots and are summed before the upper ones that its thread
+// holds, which is column order.  General: all of a row's products go through
+// its slots, in column order; twice the slots and wider rows, so half the
+// rows.
+template <bool GEN>
+struct Form {
+    static constexpr unsigned kRows = GEN ? CHX_RES_GEN_PART : CHX_RES_PART_MAX;
+    static constexpr int kSlots = kRows / kThreads;  // own rows per thread
+    static constexpr int kHeld = GEN ? CHX_RES_GEN_HELD : CHX_RES_HELD;
+    static constexpr unsigned kPlaces = GEN ? CHX_RES_GEN_WIDTH : CHX_RES_HELD;  // product slots per row
+    static constexpr unsigned kNoSlot = GEN ? 0x3fffu : 0xffffu;
+    static constexpr unsigned kSpare = kPlaces * kRows;  // first of the unread product slots
+    // fields of a held block's word
+    static __device__ __forceinline__ unsigned src(unsigned w) { return w & (GEN ? 0x3ffu : 0xffffu); }
+    static __device__ __forceinline__ unsigned slot(unsigned w) { return GEN ? (w >> 10) & 0x3fffu : w >> 16; }
+    static __device__ __forceinline__ unsigned word(unsigned s, unsigned t) { return s | (t << (GEN ? 10 : 16)); }
+};
+static_assert(Form<true>::kSpare + kWave <= Form<true>::kNoSlot && Form<false>::kSpare + kWave <= Form<false>::kNoSlot &&
+                  Form<true>::kRows + CHX_RES_HALO_MAX <= 1024,
+              "word fields");
 constexpr int kSums = 5;  // rho, sigma, delta, gamma, ||r||^2 (set-up: ||b||^2 in place of sigma)
 constexpr int kMaxParts = 256;
 constexpr unsigned kFan = 16;    // parts per group and groups, above 64 parts
 constexpr unsigned kCopies = 16;  // copies of the groups' sums
 static_assert(kFan * kFan >= kMaxParts && 2 * kCopies <= 64, "two levels");
-constexpr unsigned kNoSlot = 0xffffu;
 constexpr unsigned kExit = 0xffffffu;  // mailbox item: nothing left
-static_assert(CHX_RES_LEAF == kWave && kSlots == 2 && kLeaves == 16, "a leaf per wave and slot");
+static_assert(CHX_RES_LEAF == kWave && Form<false>::kSlots == 2 && Form<true>::kSlots == 1 && kLeaves == 2 * kWaves,
+              "a leaf per wave and slot");
 static_assert(CHX_RES_HALO_MAX <= kThreads && CHX_RES_GHOST_MAX <= kThreads, "one halo row and ghost block a thread");
 
 typedef unsigned long long u64;
@@ -85,13 +103,14 @@ __device__ __forceinline__ unsigned opaque(unsigned v) {
     return v;
 }
 
+template <bool GEN>
 struct ResLds {
-    // transposed products by target row, then one unread slot per lane for
-    // blocks without a target
-    f3 prod[kHeld * CHX_RES_PART_MAX + kWave];
-    f3 p[CHX_RES_PART_MAX + CHX_RES_HALO_MAX];     // source vector: own rows, halo rows
-    float diag[6][CHX_RES_PART_MAX];
-    f3 x[CHX_RES_PART_MAX];
+    // products by target row, then one unread slot per lane for blocks
+    // without a target
+    f3 prod[Form<GEN>::kSpare + kWave];
+    f3 p[Form<GEN>::kRows + CHX_RES_HALO_MAX];     // source vector: own rows, halo rows
+    float diag[6][Form<GEN>::kRows];
+    f3 x[Form<GEN>::kRows];
     float ghost[9][CHX_RES_GHOST_MAX];
     double leaf[kLeaves][kSums];
     double tot[8];
@@ -153,6 +172,15 @@ __device__ __forceinline__ bool await(const u64* p, unsigned tag, unsigned (&v)[
     for (int k = 0; k < N; ++k) v[k] = unsigned(w[k]);
     return true;
 }
+__device__ __forceinline__ void transpose9(float (&m)[9]) {
+    const float a = m[1], b = m[2], c = m[5];
+    m[1] = m[3];
+    m[2] = m[6];
+    m[5] = m[7];
+    m[3] = a;
+    m[6] = b;
+    m[7] = c;
+}
 __device__ __forceinline__ f3 mv9t(const float (&m)[9], f3 v) {
     const float b[9] = {m[0], m[3], m[6], m[1], m[4], m[7], m[2], m[5], m[8]};
     return mv9(b, v);
@@ -204,8 +232,8 @@ __device__ __forceinline__ double fold8(double a, double b, unsigned lane) {
     const bool up = (lane & 8u) != 0u;
     return (up ? b : a) + dpp64<kRor8>(up ? a : b);
 }
-__device__ __forceinline__ void leaf_sums(const double (&a)[kSums], const double (&b)[kSums], ResLds& S, unsigned wave,
-                                          unsigned lane) {
+__device__ __forceinline__ void leaf_sums(const double (&a)[kSums], const double (&b)[kSums],
+                                          double (&leaf)[kLeaves][kSums], unsigned wave, unsigned lane) {
     double v[kSums];
 #pragma unroll
     for (int k = 0; k < kSums; ++k) v[k] = fold32(a[k], b[k]);  // half h: leaf of slot h
@@ -219,7 +247,7 @@ __device__ __forceinline__ void leaf_sums(const double (&a)[kSums], const double
     w1 += dpp64<kXor2>(w1);
     w0 += dpp64<kXor1>(w0);
     w1 += dpp64<kXor1>(w1);
-    double(&out)[kSums] = S.leaf[(lane >> 5) * kWaves + wave];
+    double(&out)[kSums] = leaf[(lane >> 5) * kWaves + wave];
     const unsigned place = lane & 31u;
     if ((place & 7u) == 0u) out[(place >> 4) + ((place & 8u) >> 2)] = w0;
     if (place == 1u) out[4] = w1;
@@ -227,14 +255,18 @@ __device__ __forceinline__ void leaf_sums(const double (&a)[kSums], const double
 
 // Solves instance `inst` together with the workgroups that hold its other
 // parts; this one holds part `part`.  False: aborted.
-__device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst& I, int inst, int part, unsigned epoch, ResLds& S,
-                           const Barrier& bar, int& trace_e) {
+template <bool GEN>
+__device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst& I, int inst, int part, unsigned epoch,
+                                           ResLds<GEN>& S, const Barrier& bar, int& trace_e) {
+    using F = Form<GEN>;
+    constexpr int kSlots = F::kSlots, kHeld = F::kHeld;
+    constexpr unsigned kPart = F::kRows;
     const unsigned tid = threadIdx.x, lane = tid & (kWave - 1);
     const unsigned wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const gp<const unsigned> plan = I.res_plan;
     const unsigned n = unsigned(I.n_rows), parts = unsigned(I.res_parts);
     const gp<const unsigned> hdr = plan + 8 * part;
-    const unsigned n_own = hdr[0], n_halo = hdr[1], halo_at = hdr[2], n_ghost = hdr[3], ghost_at = hdr[4];
+    const unsigned n_own = hdr[0], n_halo = hdr[1], halo_at = hdr[2], n_ghost = hdr[3], ghost_at = hdr[4], widest = hdr[5];
     const unsigned pos0 = unsigned(part) * unsigned(I.res_part_rows);
     const unsigned rows_at = 8u * parts, meta_at = rows_at + n, exp_at = meta_at + n, held_at = exp_at + n;
     // exchange areas: [2][kSums][parts] pairs of words, then [2][exports] rows of 3
@@ -259,7 +291,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     };
 
     // ---- load: own rows, ghost block, halo row ----
-    unsigned lp[kSlots], ex[kSlots], word[kSlots][kHeld];
+    unsigned lp[kSlots], ex[kSlots], holds[kSlots], word[kSlots][kHeld];
     bool live[kSlots], on[kSlots];  // this lane's row exists; this wave has a row
     float V[kSlots][kHeld][9], M[kSlots][6];
     f3 r[kSlots], p[kSlots], q[kSlots];
@@ -270,30 +302,40 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         live[s] = lp[s] < n_own;
         const unsigned K = pos0 + (live[s] ? lp[s] : 0u);
         ex[s] = CHX_RES_NONE;
+        holds[s] = 0u;
         r[s] = p[s] = q[s] = mk(0.f, 0.f, 0.f);
         if (on[s]) {
             unsigned ns = 0u, nh = 0u;
             const unsigned row = ldx(plan, rows_at + K);
             const unsigned meta = ldx(plan, meta_at + K);
             if (live[s]) {
-                ns = meta & 15u;
-                nh = meta >> 4;
+                ns = meta & 255u;
+                nh = meta >> 8;
                 ex[s] = ldx(plan, exp_at + K);
             }
+            holds[s] = nh;
             const unsigned vs = unsigned(ldx(I.upper_offsets, row / CHX_SLICE_ROWS)) + row % CHX_SLICE_ROWS;
 #pragma unroll
             for (int u = 0; u < kHeld; ++u) {
-                // a block that is not there is zero, of the row itself, and
-                // its product slot stays zero: both are added like the others
+                // a block that is not there is zero, of the row itself
                 const bool has = unsigned(u) < nh;
-                unsigned w = has ? ldx(plan, held_at + unsigned(u) * n + K) : (kNoSlot << 16) | lp[s];
-                if ((w >> 16) == kNoSlot) w = (w & 0xffffu) | ((kHeld * kPart + lane) << 16);
+                unsigned w = has ? ldx(plan, held_at + unsigned(u) * n + K) : F::word(lp[s], F::kNoSlot);
+                if (F::slot(w) == F::kNoSlot) w = (w & ~F::word(0u, F::kNoSlot)) | F::word(0u, F::kSpare + lane);
                 word[s][u] = w;
-                if (unsigned(u) >= ns) S.prod[unsigned(u) * kPart + lp[s]] = mk(0.f, 0.f, 0.f);
 #pragma unroll
                 for (int c = 0; c < 9; ++c) V[s][u][c] = 0.0f;
-                if (has) ld9p(gp<const float>(I.values), vs + unsigned(u) * CHX_SLICE_ROWS, V[s][u]);
+                if (has) {
+                    unsigned v = vs + unsigned(u) * CHX_SLICE_ROWS;
+                    if (GEN) v = ldx(plan, held_at + unsigned(kHeld + u) * n + K);
+                    ld9p(gp<const float>(I.values), v & 0x7fffffffu, V[s][u]);
+                    if (GEN && (v >> 31) != 0u) transpose9(V[s][u]);
+                }
             }
+            // product slots that no block fills stay zero and are added like
+            // the others
+#pragma unroll
+            for (unsigned u = 0; u < F::kPlaces; ++u)
+                if (u >= ns) S.prod[u * kPart + lp[s]] = mk(0.f, 0.f, 0.f);
             float d[6], full[9];
             ld6u(gp<const float>(I.diag), row, d);
 #pragma unroll
@@ -312,7 +354,8 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         const unsigned vs = ldx(plan, ghost_at + 2u * rtid);
         gword = ldx(plan, ghost_at + 2u * rtid + 1u);
         float g[9];
-        ld9p(gp<const float>(I.values), vs, g);
+        ld9p(gp<const float>(I.values), vs & 0x7fffffffu, g);
+        if (GEN && (vs >> 31) != 0u) transpose9(g);
 #pragma unroll
         for (int c = 0; c < 9; ++c) S.ghost[c][rtid] = g[c];
     }
@@ -337,7 +380,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         for (int s = 0; s < kSlots; ++s)
             if (on[s]) {
 #pragma unroll
-                for (int u = 0; u < kHeld; ++u) lds_st(&S.prod[opaque(word[s][u]) >> 16], mv9t(V[s][u], v[s]));
+                for (int u = 0; u < kHeld; ++u) lds_st(&S.prod[F::slot(opaque(word[s][u]))], mv9t(V[s][u], v[s]));
             }
         __syncthreads();
         if (rtid < n_ghost) {
@@ -346,29 +389,54 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             for (int c = 0; c < 9; ++c) g[c] = S.ghost[c][rtid];
             lds_st(&S.prod[gword >> 16], mv9t(g, lds_ld(&S.p[gword & 0xffffu])));
         }
+        if (GEN && on[0]) {
+            f3 src[kHeld];
+#pragma unroll
+            for (int u = 0; u < kHeld; ++u) src[u] = lds_ld(&S.p[F::src(opaque(word[0][u]))]);
+#pragma unroll
+            for (int u = 0; u < kHeld; ++u)
+                if (unsigned(u) < opaque(holds[0]))
+                    lds_st(&S.prod[(opaque(word[0][u]) >> 24) * kPart + lp[0]], mv9(V[0][u], src[u]));
+        }
         __syncthreads();
 #pragma unroll
         for (int s = 0; s < kSlots; ++s)
             if (on[s]) {
                 float d[6];
-                f3 low[kHeld], src[kHeld];
-#pragma unroll
-                for (int u = 0; u < kHeld; ++u) src[u] = lds_ld(&S.p[opaque(word[s][u]) & 0xffffu]);
 #pragma unroll
                 for (int c = 0; c < 6; ++c) d[c] = S.diag[c][lp[s]];
+                if (GEN) {
+                    f3 sum = mv_sym(d, v[s]);
 #pragma unroll
-                for (int l = 0; l < kHeld; ++l) low[l] = lds_ld(&S.prod[unsigned(l) * kPart + lp[s]]);
-                f3 sum = mv_sym(d, v[s]);
+                    for (unsigned t = 0; t < F::kPlaces; t += 4)
+                        if (t < widest) {
+                            f3 y[4];
 #pragma unroll
-                for (int l = 0; l < kHeld; ++l) sum = add(sum, low[l]);
+                            for (unsigned u = 0; u < 4; ++u) y[u] = lds_ld(&S.prod[(t + u) * kPart + lp[s]]);
 #pragma unroll
-                for (int u = 0; u < kHeld; ++u) sum = add(sum, mv9(V[s][u], src[u]));
-                out[s] = sum;
+                            for (unsigned u = 0; u < 4; ++u) sum = add(sum, y[u]);
+                        }
+                    out[s] = sum;
+                } else {
+                    f3 low[kHeld], src[kHeld];
+#pragma unroll
+                    for (int u = 0; u < kHeld; ++u) src[u] = lds_ld(&S.p[F::src(opaque(word[s][u]))]);
+#pragma unroll
+                    for (int l = 0; l < kHeld; ++l) low[l] = lds_ld(&S.prod[unsigned(l) * kPart + lp[s]]);
+                    f3 sum = mv_sym(d, v[s]);
+#pragma unroll
+                    for (int l = 0; l < kHeld; ++l) sum = add(sum, low[l]);
+#pragma unroll
+                    for (int u = 0; u < kHeld; ++u) sum = add(sum, mv9(V[s][u], src[u]));
+                    out[s] = sum;
+                }
             }
     };
     // Sums of phase t: per leaf, then over the part's leaves, sent to the gang.
     auto send_sums = [&](int t, double (&acc)[kSlots][kSums]) {
-        leaf_sums(acc[0], acc[1], S, wave, lane);
+        const double none[kSums] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        if constexpr (kSlots == 2) leaf_sums(acc[0], acc[1], S.leaf, wave, lane);
+        else leaf_sums(acc[0], none, S.leaf, wave, lane);
         __syncthreads();
         if (tid < 8 * kSums) {
             const unsigned v = tid >> 3, i = tid & 7u;
@@ -538,8 +606,8 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
 // finished gang frees always holds the next one; with no gang left running
 // every workgroup of the group is idle and any item of the list fits.
 __device__ unsigned next_item(const chx_cloth_batch& B, unsigned group, unsigned first, unsigned stride, unsigned idx,
-                              unsigned epoch, unsigned had, ResLds& S, const Barrier& bar) {
-    __syncthreads();  // readers of S.mail are done
+                              unsigned epoch, unsigned had, unsigned& out, const Barrier& bar) {
+    __syncthreads();  // its readers are done
     if (threadIdx.x == 0) {
         u64* const idle = &B.xbuf[RES_IDLE + 16 * group];
         u64* const next = &B.xbuf[RES_NEXT];
@@ -600,14 +668,15 @@ __device__ unsigned next_item(const chx_cloth_batch& B, unsigned group, unsigned
             }
             backoff(level);
         }
-        S.mail = got;
+        out = got;
     }
     __syncthreads();
-    return S.mail;
+    return out;
 }
 
+template <bool GEN>
 __global__ __launch_bounds__(kThreads, 2) void resident_kernel(chx_cloth_batch B, int finalize) {
-    __shared__ ResLds S;
+    __shared__ ResLds<GEN> S;
     const int G = int(gridDim.x);
     const Barrier bar = make_barrier(B);
     unsigned* const progress = reinterpret_cast<unsigned*>(&B.xbuf[RES_PROGRESS]);
@@ -646,7 +715,7 @@ __global__ __launch_bounds__(kThreads, 2) void resident_kernel(chx_cloth_batch B
             __syncthreads();  // the previous solve's readers of S are done
         } else {
             if (B.res_n_items == B.res_n_big) break;
-            had = next_item(B, group, group, groups, idx, epoch, had, S, bar);
+            had = next_item(B, group, group, groups, idx, epoch, had, S.mail, bar);
             if ((had >> 8) == kExit) {
                 ok = (had & 255u) == 0u;
                 break;
@@ -655,7 +724,7 @@ __global__ __launch_bounds__(kThreads, 2) void resident_kernel(chx_cloth_batch B
             part = int(__builtin_amdgcn_readfirstlane(had & 255u));
         }
         const Inst I = inst_at(B, inst);
-        ok = solve_part(B, I, inst, part, epoch, S, bar, trace_e);
+        ok = solve_part<GEN>(B, I, inst, part, epoch, S, bar, trace_e);
         if (!ok) break;
     }
     // pos and vel change only when every instance was solved
@@ -663,6 +732,9 @@ __global__ __launch_bounds__(kThreads, 2) void resident_kernel(chx_cloth_batch B
     if (G > 1 && !grid_sync(bar, unsigned(G), -1, nullptr, progress)) return;
     if (finalize) finalize_tiles(B, G);
 }
+
+using ResFn = void (*)(chx_cloth_batch, int);
+ResFn resident_fn(bool general) { return general ? resident_kernel<true> : resident_kernel<false>; }
 
 std::mutex g_mu;
 int g_limit[16] = {0};
@@ -677,11 +749,15 @@ int resident_grid_limit() {
     if (l == 0) {
         hipDeviceProp_t prop;
         hip_check(hipGetDeviceProperties(&prop, dev), "hipGetDeviceProperties");
-        int per_cu = 0;
-        hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(resident_kernel),
-                                                               kThreads, 0),
-                  "hipOccupancyMaxActiveBlocksPerMultiprocessor");
-        l = per_cu < 1 ? -1 : std::min(kMaxParts, prop.multiProcessorCount);
+        bool fits = true;
+        for (bool general : {false, true}) {
+            int per_cu = 0;
+            hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                          &per_cu, reinterpret_cast<const void*>(resident_fn(general)), kThreads, 0),
+                      "hipOccupancyMaxActiveBlocksPerMultiprocessor");
+            fits = fits && per_cu >= 1;
+        }
+        l = fits ? std::min(kMaxParts, prop.multiProcessorCount) : -1;
     }
     return std::max(l, 0);
 }
@@ -690,15 +766,15 @@ void launch_resident(const chx_cloth_batch& B, int finalize, hipStream_t stream)
     if (B.res_grid == 1) {
         // nothing waits for another workgroup: an ordinary launch, without the
         // ~11 us before and after that a cooperative one takes
-        resident_kernel<<<1, kThreads, 0, stream>>>(B, finalize);
+        resident_fn(B.res_general != 0)<<<1, kThreads, 0, stream>>>(B, finalize);
         hip_check(hipGetLastError(), "resident_kernel launch");
         return;
     }
     chx_cloth_batch arg = B;
     int fin = finalize;
     void* args[] = {&arg, &fin};
-    hip_check(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(resident_kernel), dim3(B.res_grid),
-                                         dim3(kThreads), args, 0, stream),
+    hip_check(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(resident_fn(B.res_general != 0)),
+                                         dim3(B.res_grid), dim3(kThreads), args, 0, stream),
               "hipLaunchCooperativeKernel(resident pcg)");
 }
 

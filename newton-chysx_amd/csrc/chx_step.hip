@@ -1878,6 +1878,8 @@ void validate_batch(const chx_cloth_batch* b) {
                          (I.res_part_rows == 256 || I.res_part_rows == 512 || I.res_part_rows == CHX_RES_PART_MAX) &&
                          I.res_parts == (I.n_rows + I.res_part_rows - 1) / I.res_part_rows &&
                          I.res_parts <= b->res_grid && I.res_exports >= 0 &&
+                         (I.res_general != 0) == (b->res_general != 0) &&
+                         (b->res_general == 0 || I.res_part_rows <= CHX_RES_GEN_PART) &&
                          I.res_xbase + CHX_RES_XWORDS(I.res_parts, I.res_exports) <= b->res_xwords),
                     "chysx: resident plan does not match its instance");
         } else {

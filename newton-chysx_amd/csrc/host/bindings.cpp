@@ -513,7 +513,8 @@ PYBIND11_MODULE(_chysx_native, m) {
         py::arg("n"), py::arg("rows"), py::arg("cols"));
     topo.def(
         "resident_plan",
-        [](int n, IArr row_offsets, IArr col_indices, IArr block_slots, int part_rows) -> py::object {
+        [](int n, IArr row_offsets, IArr col_indices, IArr block_slots, int part_rows,
+           bool general) -> py::object {
             // Canonical row order and part image of the resident solve, or
             // None when the pattern does not fit it.
             chysx::topology::Pattern p;
@@ -522,7 +523,8 @@ PYBIND11_MODULE(_chysx_native, m) {
             p.col_indices.assign(col_indices.data(), col_indices.data() + col_indices.size());
             const std::vector<int> bs(block_slots.data(), block_slots.data() + block_slots.size());
             const std::vector<int> order = chysx::engine::resident_order(p);
-            const auto r = chysx::engine::resident_plan(p, bs, order, part_rows);
+            const auto r = general ? chysx::engine::resident_plan_general(p, bs, order, part_rows)
+                                   : chysx::engine::resident_plan(p, bs, order, part_rows);
             if (r.blob.empty()) return py::none();
             py::dict d;
             d["order"] = to_array(order);
@@ -533,7 +535,8 @@ PYBIND11_MODULE(_chysx_native, m) {
             d["blob"] = b;
             return d;
         },
-        py::arg("n"), py::arg("row_offsets"), py::arg("col_indices"), py::arg("block_slots"), py::arg("part_rows"));
+        py::arg("n"), py::arg("row_offsets"), py::arg("col_indices"), py::arg("block_slots"), py::arg("part_rows"),
+        py::arg("general") = false);
     topo.def(
         "cloth_system",
         [](int n, IArr tris, IArr pins, bool stretch, bool shear, bool bending) {

@@ -31,14 +31,21 @@ void ClothBatch::clear() noexcept {
 std::vector<chx_instance> ClothBatch::descriptors(float dt, std::uintptr_t cuda_stream) {
     std::vector<int> rows;
     for (ClothSimulator* s : sims_) rows.push_back(s->buffers().particle_count());
-    const int part_rows = engine::resident_part_rows(rows);
     std::vector<chx_instance> ds;
-    ds.reserve(sims_.size());
-    for (ClothSimulator* s : sims_) {
-        ds.push_back(s->prepare_instance(dt, cuda_stream, part_rows));
-        if (bf16_ && ds.back().n_rows > 0 && ds.back().diag_c == nullptr)
-            throw std::invalid_argument(
-                "ClothBatch: BF16 mode needs every instance switched with set_bf16_blocks(true)");
+    // the resident solve wants all plans in one form: sheets, or else general
+    for (bool general : {false, true}) {
+        const int part_rows = engine::resident_part_rows(rows, general);
+        ds.clear();
+        ds.reserve(sims_.size());
+        bool all = true;
+        for (ClothSimulator* s : sims_) {
+            ds.push_back(s->prepare_instance(dt, cuda_stream, part_rows, general));
+            if (bf16_ && ds.back().n_rows > 0 && ds.back().diag_c == nullptr)
+                throw std::invalid_argument(
+                    "ClothBatch: BF16 mode needs every instance switched with set_bf16_blocks(true)");
+            all = all && ds.back().res_plan != nullptr;
+        }
+        if (all || bf16_) break;
     }
     return ds;
 }

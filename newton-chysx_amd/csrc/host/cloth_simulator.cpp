@@ -352,11 +352,14 @@ void ClothSimulator::step(float dt, std::uintptr_t cuda_stream) {
 // The descriptor of the simulator's own (single-instance) launches.
 chx_instance ClothSimulator::single_descriptor(const engine::InstanceSource& s, std::uintptr_t stream) {
     chx_instance d = inst_.descriptor(s);
-    if (!bf16_) inst_.attach_plan(d, pattern_, engine::resident_part_rows({s.n}), stream);
+    for (bool general : {false, true})
+        if (!bf16_ && d.res_plan == nullptr)
+            inst_.attach_plan(d, pattern_, engine::resident_part_rows({s.n}, general), general, stream);
     return d;
 }
 
-chx_instance ClothSimulator::prepare_instance(float dt, std::uintptr_t cuda_stream, int part_rows) {
+chx_instance ClothSimulator::prepare_instance(float dt, std::uintptr_t cuda_stream, int part_rows,
+                                             bool general) {
     const int n = buffers_.particle_count();
     if (n <= 0) throw std::runtime_error("ClothSimulator::prepare_instance: no particles bound");
     if (buffers_.pos.data() == nullptr || buffers_.vel.data() == nullptr)
@@ -368,7 +371,7 @@ chx_instance ClothSimulator::prepare_instance(float dt, std::uintptr_t cuda_stre
     engine::InstanceSource s = source();
     s.dt = dt;
     chx_instance d = inst_.descriptor(s);
-    if (!bf16_) inst_.attach_plan(d, pattern_, part_rows, cuda_stream);
+    if (!bf16_) inst_.attach_plan(d, pattern_, part_rows, general, cuda_stream);
     return d;
 }
 

@@ -684,16 +684,20 @@ chx_instance InstanceData::descriptor(const InstanceSource& s) const {
     return I;
 }
 
-void InstanceData::attach_plan(chx_instance& d, const topology::Pattern& p, int part_rows, std::uintptr_t stream) {
+void InstanceData::attach_plan(chx_instance& d, const topology::Pattern& p, int part_rows, bool general,
+                               std::uintptr_t stream) {
+    d.res_plan = nullptr;
     if (part_rows == 0 || n_ == 0) return;
     // what one workgroup holds needs no exchange: 32x32 rows take 3.3 us an
     // iteration in one part, 3.3-3.9 in four or two
-    if (n_ <= CHX_RES_PART_MAX) part_rows = CHX_RES_PART_MAX;
-    Plan& pl = plans_[part_rows == 256 ? 0 : (part_rows == 512 ? 1 : 2)];
+    const int most = general ? CHX_RES_GEN_PART : CHX_RES_PART_MAX;
+    if (n_ <= most) part_rows = most;
+    Plan& pl = plans_[(general ? 3 : 0) + (part_rows == 256 ? 0 : (part_rows == 512 ? 1 : 2))];
     if (!pl.tried) {
         pl.tried = true;
         if (order_.empty()) order_ = resident_order(p);
-        ResidentPlan r = resident_plan(p, block_slots_.host(), order_, part_rows);
+        ResidentPlan r = general ? resident_plan_general(p, block_slots_.host(), order_, part_rows)
+                                 : resident_plan(p, block_slots_.host(), order_, part_rows);
         if (!r.blob.empty()) {
             pl.parts = r.parts;
             pl.exports = r.exports;
@@ -708,19 +712,21 @@ void InstanceData::attach_plan(chx_instance& d, const topology::Pattern& p, int 
     d.res_part_rows = part_rows;
     d.res_parts = pl.parts;
     d.res_exports = pl.exports;
+    d.res_general = general ? 1 : 0;
 }
 
-int resident_part_rows(const std::vector<int>& rows) {
+int resident_part_rows(const std::vector<int>& rows, bool general) {
     constexpr long kWorkgroups = 256;
-    for (int pr : {256, 512, CHX_RES_PART_MAX}) {
+    const int largest = general ? CHX_RES_GEN_PART : CHX_RES_PART_MAX;
+    for (int pr = 256; pr <= largest; pr *= 2) {
         long parts = 0, most = 0;
         for (int n : rows) {
-            const long q = n <= CHX_RES_PART_MAX ? 1 : (n + pr - 1) / pr;
+            const long q = n <= largest ? 1 : (n + pr - 1) / pr;
             parts += q;
             most = std::max(most, q);
         }
         if (parts <= kWorkgroups) return pr;
-        if (pr == CHX_RES_PART_MAX && most <= kWorkgroups) return pr;
+        if (pr == largest && most <= kWorkgroups) return pr;
     }
     return 0;
 }
@@ -735,7 +741,7 @@ void BatchRunner::layout_resident(std::vector<chx_instance>& ds, std::uintptr_t 
     int total = 0, most = 0;
     for (const chx_instance& d : ds) {
         if (d.n_rows == 0) continue;
-        if (d.res_plan == nullptr) return;
+        if (d.res_plan == nullptr || d.res_general != ds[0].res_general) return;
         total += d.res_parts;
         most = std::max(most, d.res_parts);
     }
@@ -804,6 +810,7 @@ void BatchRunner::layout_resident(std::vector<chx_instance>& ds, std::uintptr_t 
     desc_.xbuf = xbuf_.gpu_data();
     desc_.res_xwords = xbuf_.gpu_size();
     desc_.res_groups = groups;
+    desc_.res_general = ds[0].res_general;
     desc_.res_grid = grid;
 }
 

@@ -74,7 +74,8 @@ public:
     // Adds the resident-solve plan for parts of `part_rows` rows to a
     // descriptor (none when the pattern does not fit it, or part_rows is 0).
     // Plans are built on first use and kept until the next build().
-    void attach_plan(chx_instance& d, const topology::Pattern& p, int part_rows, std::uintptr_t stream);
+    // `general`: the general form (parts of at most CHX_RES_GEN_PART rows).
+    void attach_plan(chx_instance& d, const topology::Pattern& p, int part_rows, bool general, std::uintptr_t stream);
     bool built() const noexcept { return built_; }
     int n_rows() const noexcept { return n_; }
     int nnz() const noexcept { return nnz_; }
@@ -126,7 +127,7 @@ private:
         int parts = 0, exports = 0;
         DeviceArray<std::uint32_t> blob;
     };
-    Plan plans_[3];           // parts of 256, 512 and 1024 rows
+    Plan plans_[5];           // sheet form with parts of 256, 512 and 1024 rows, general form with 256 and 512
     std::vector<int> order_;  // canonical row order of the plans
     DeviceArray<chx_plane> planes_;
     DeviceArray<chx_box> boxes_;
@@ -135,7 +136,7 @@ private:
 // Rows per part of the resident solve of cloths with `rows` vertices each:
 // the smallest part size whose parts all run at once on 256 workgroups, else
 // the largest; 0 when some cloth alone has more parts than that.
-int resident_part_rows(const std::vector<int>& rows);
+int resident_part_rows(const std::vector<int>& rows, bool general);
 
 class BatchRunner {
 public:

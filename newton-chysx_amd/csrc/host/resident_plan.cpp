@@ -119,16 +119,121 @@ std::vector<int> resident_order(const topology::Pattern& p) {
     return order;
 }
 
+namespace {
+
+// Halo rows, ghost blocks and exports of both forms.  Planes: words per
+// position behind the first three (row, meta, export).  For every part,
+// row(k, i) writes position k's planes and meta, and may add ghost blocks.
+struct Builder {
+    const topology::Pattern& p;
+    const std::vector<int>& order;
+    int part_rows, capacity, planes;
+    std::vector<int> pos, local;
+    std::vector<std::uint32_t> blob, halos, ghosts;
+    std::size_t N, rows_at, meta_at, exp_at, held_at;
+    int parts, exports = 0;
+    int a = 0, b = 0, widest = 0;  // the part at hand
+
+    Builder(const topology::Pattern& pat, const std::vector<int>& ord, int rows, int cap, int n_planes)
+        : p(pat), order(ord), part_rows(rows), capacity(cap), planes(n_planes), N(static_cast<std::size_t>(pat.n)) {
+        parts = (p.n + rows - 1) / rows;
+        pos.resize(N);
+        local.assign(N, 0);
+        for (int k = 0; k < p.n; ++k) pos[order[k]] = k;
+        rows_at = 8u * static_cast<std::size_t>(parts);
+        meta_at = rows_at + N;
+        exp_at = meta_at + N;
+        held_at = exp_at + N;
+        blob.assign(held_at + static_cast<std::size_t>(planes) * N, 0u);
+    }
+    bool own(int j) const { return pos[j] >= a && pos[j] < b; }
+    std::uint32_t local_of(int j) const { return static_cast<std::uint32_t>(own(j) ? pos[j] - a : local[j]); }
+    std::uint32_t& plane(int u, int k) {
+        return blob[held_at + static_cast<std::size_t>(u) * N + static_cast<std::size_t>(k)];
+    }
+    void ghost(std::uint32_t value, std::uint32_t word) {
+        ghosts.push_back(value);
+        ghosts.push_back(word);
+    }
+    template <class Row>
+    bool build(Row row) {
+        const auto& ro = p.row_offsets;
+        const auto& ci = p.col_indices;
+        // exported rows, numbered part by part in canonical order
+        std::vector<std::uint32_t> exp(N, CHX_RES_NONE);
+        for (int k = 0; k < p.n; ++k) {
+            const int i = order[k], q = k / part_rows;
+            for (int c = ro[i]; c < ro[i + 1] && exp[i] == CHX_RES_NONE; ++c)
+                if (pos[ci[c]] / part_rows != q) exp[i] = static_cast<std::uint32_t>(exports++);
+        }
+        std::vector<int> stamp(N, -1), halo;
+        for (int q = 0; q < parts; ++q) {
+            a = q * part_rows;
+            b = std::min(p.n, a + part_rows);
+            widest = 0;
+            halo.clear();
+            for (int k = a; k < b; ++k) {
+                const int i = order[k];
+                widest = std::max(widest, ro[i + 1] - ro[i]);
+                for (int c = ro[i]; c < ro[i + 1]; ++c)
+                    if (!own(ci[c]) && stamp[ci[c]] != q) {
+                        stamp[ci[c]] = q;
+                        halo.push_back(ci[c]);
+                    }
+            }
+            if (halo.size() > CHX_RES_HALO_MAX) return false;
+            std::sort(halo.begin(), halo.end(), [&](int i, int j) { return pos[i] < pos[j]; });
+            for (std::size_t h = 0; h < halo.size(); ++h) local[halo[h]] = capacity + static_cast<int>(h);
+            const std::size_t ghost0 = ghosts.size() / 2;
+            for (int k = a; k < b; ++k) {
+                const int i = order[k];
+                blob[rows_at + static_cast<std::size_t>(k)] = static_cast<std::uint32_t>(i);
+                blob[exp_at + static_cast<std::size_t>(k)] = exp[i];
+                blob[meta_at + static_cast<std::size_t>(k)] = row(k, i);
+            }
+            const std::size_t n_ghosts = ghosts.size() / 2 - ghost0;
+            if (n_ghosts > CHX_RES_GHOST_MAX) return false;
+            std::uint32_t* H = blob.data() + 8 * static_cast<std::size_t>(q);
+            H[0] = static_cast<std::uint32_t>(b - a);
+            H[1] = static_cast<std::uint32_t>(halo.size());
+            H[2] = static_cast<std::uint32_t>(halos.size());
+            H[3] = static_cast<std::uint32_t>(n_ghosts);
+            H[4] = static_cast<std::uint32_t>(2 * ghost0);
+            H[5] = static_cast<std::uint32_t>(widest);
+            for (int j : halo) {
+                halos.push_back(static_cast<std::uint32_t>(j));
+                halos.push_back(exp[j]);
+            }
+        }
+        // the lists behind the planes, at absolute word offsets
+        const std::size_t halo_at = blob.size(), ghost_at = halo_at + halos.size();
+        if (ghost_at + ghosts.size() >= (std::size_t(1) << 30)) return false;
+        for (int q = 0; q < parts; ++q) {
+            blob[8 * static_cast<std::size_t>(q) + 2] += static_cast<std::uint32_t>(halo_at);
+            blob[8 * static_cast<std::size_t>(q) + 4] += static_cast<std::uint32_t>(ghost_at);
+        }
+        blob.insert(blob.end(), halos.begin(), halos.end());
+        blob.insert(blob.end(), ghosts.begin(), ghosts.end());
+        return true;
+    }
+    ResidentPlan take() {
+        ResidentPlan out;
+        out.part_rows = part_rows;
+        out.parts = parts;
+        out.exports = exports;
+        out.blob = std::move(blob);
+        return out;
+    }
+};
+
+}  // namespace
+
 ResidentPlan resident_plan(const topology::Pattern& p, const std::vector<int>& block_slots,
                            const std::vector<int>& order, int part_rows) {
-    ResidentPlan out;
     const int n = p.n;
-    if (n <= 0) return out;
+    if (n <= 0 || part_rows > CHX_RES_PART_MAX) return {};
     const auto& ro = p.row_offsets;
     const auto& ci = p.col_indices;
-    const int parts = (n + part_rows - 1) / part_rows;
-    std::vector<int> pos(static_cast<std::size_t>(n));
-    for (int k = 0; k < n; ++k) pos[order[k]] = k;
     // lower[k]: place of upper block (i, j)'s transpose among row j's lower blocks
     std::vector<std::uint8_t> lower(ci.size(), 0), nl(static_cast<std::size_t>(n), 0);
     std::vector<int> up0(static_cast<std::size_t>(n));
@@ -136,93 +241,84 @@ ResidentPlan resident_plan(const topology::Pattern& p, const std::vector<int>& b
         int k = ro[i];
         while (k < ro[i + 1] && ci[k] < i) ++k;
         up0[i] = k;
-        if (ro[i + 1] - k > CHX_RES_HELD || k - ro[i] > CHX_RES_HELD) return out;
+        if (ro[i + 1] - k > CHX_RES_HELD || k - ro[i] > CHX_RES_HELD) return {};
         for (; k < ro[i + 1]; ++k) lower[k] = nl[ci[k]]++;
     }
-    const std::size_t N = static_cast<std::size_t>(n);
-    const std::size_t rows_at = 8u * static_cast<std::size_t>(parts), meta_at = rows_at + N, exp_at = meta_at + N,
-                      held_at = exp_at + N, lists_at = held_at + CHX_RES_HELD * N;
-    std::vector<std::uint32_t> B(lists_at, 0u);
-    std::vector<std::uint32_t> halo_all, ghost_all;
-    std::vector<int> stamp(N, -1), local(N, 0);
-    // exported rows, numbered part by part in canonical order
-    std::vector<std::uint8_t> shared(N, 0);
+    Builder B(p, order, part_rows, CHX_RES_PART_MAX, CHX_RES_HELD);
+    const bool ok = B.build([&](int k, int i) {
+        for (int c = ro[i]; c < up0[i]; ++c)  // blocks another part holds
+            if (!B.own(ci[c]))
+                B.ghost(static_cast<std::uint32_t>(-1 - block_slots[c]),
+                        B.local_of(ci[c]) |
+                            (static_cast<std::uint32_t>((c - ro[i]) * CHX_RES_PART_MAX + (k - B.a)) << 16));
+        for (int c = up0[i]; c < ro[i + 1]; ++c) {
+            const std::uint32_t lj = B.local_of(ci[c]);
+            const std::uint32_t target =
+                B.own(ci[c]) ? static_cast<std::uint32_t>(lower[c]) * CHX_RES_PART_MAX + lj : 0xffffu;
+            B.plane(c - up0[i], k) = lj | (target << 16);
+        }
+        return static_cast<std::uint32_t>((up0[i] - ro[i]) | ((ro[i + 1] - up0[i]) << 8));
+    });
+    return ok ? B.take() : ResidentPlan{};
+}
+
+ResidentPlan resident_plan_general(const topology::Pattern& p, const std::vector<int>& block_slots,
+                                   const std::vector<int>& order, int part_rows) {
+    const int n = p.n;
+    if (n <= 0 || part_rows > CHX_RES_GEN_PART) return {};
+    const auto& ro = p.row_offsets;
+    const auto& ci = p.col_indices;
+    // mirror[k]: CSR index of block k's transpose
+    std::vector<int> mirror(ci.size()), at(ro.begin(), ro.end() - 1);
+    for (int i = 0; i < n; ++i) {
+        if (ro[i + 1] - ro[i] > CHX_RES_GEN_WIDTH) return {};
+        for (int k = ro[i]; k < ro[i + 1]; ++k) mirror[k] = at[ci[k]]++;
+    }
+    // Every pair's block is held by one of its rows, half of a row's blocks
+    // (rounded up at most): walk trails over unused pairs, each held by the
+    // row the trail leaves.  Trails from rows with an odd number of pairs
+    // first: they end at such rows, and the rest close.
+    std::vector<std::uint8_t> held(ci.size(), 0), used(ci.size(), 0);
+    std::vector<int> next(ro.begin(), ro.end() - 1);
+    const auto walk = [&](int i) {
+        for (;;) {
+            int& k = next[i];
+            while (k < ro[i + 1] && used[k]) ++k;
+            if (k == ro[i + 1]) return;
+            held[k] = used[k] = used[mirror[k]] = 1;
+            i = ci[k];
+        }
+    };
     for (int i = 0; i < n; ++i)
-        for (int k = up0[i]; k < ro[i + 1]; ++k)
-            if (pos[i] / part_rows != pos[ci[k]] / part_rows) shared[i] = shared[ci[k]] = 1;
-    std::vector<std::uint32_t> exp(N, CHX_RES_NONE);
-    int exports = 0;
-    for (int k = 0; k < n; ++k)
-        if (shared[order[k]]) exp[order[k]] = static_cast<std::uint32_t>(exports++);
-    std::vector<int> halo;
-    for (int q = 0; q < parts; ++q) {
-        const int a = q * part_rows, b = std::min(n, a + part_rows);
-        halo.clear();
-        for (int k = a; k < b; ++k) {
-            const int i = order[k];
-            for (int c = ro[i]; c < ro[i + 1]; ++c) {
-                const int j = ci[c];
-                if (pos[j] >= a && pos[j] < b) continue;
-                if (stamp[j] != q) {
-                    stamp[j] = q;
-                    halo.push_back(j);
-                }
-            }
+        if ((ro[i + 1] - ro[i]) % 2 != 0) {
+            int unused = 0;
+            for (int k = ro[i]; k < ro[i + 1]; ++k) unused += used[k] ? 0 : 1;
+            if (unused % 2 != 0) walk(i);
         }
-        std::sort(halo.begin(), halo.end(), [&](int i, int j) { return pos[i] < pos[j]; });
-        if (halo.size() > CHX_RES_HALO_MAX) return out;
-        for (std::size_t h = 0; h < halo.size(); ++h) local[halo[h]] = CHX_RES_PART_MAX + static_cast<int>(h);
-        const std::size_t ghost0 = ghost_all.size() / 2;
-        for (int k = a; k < b; ++k) {
-            const int i = order[k];
-            const std::size_t K = static_cast<std::size_t>(k);
-            B[rows_at + K] = static_cast<std::uint32_t>(i);
-            B[meta_at + K] = static_cast<std::uint32_t>((up0[i] - ro[i]) | ((ro[i + 1] - up0[i]) << 4));
-            B[exp_at + K] = exp[i];
-            for (int c = ro[i]; c < up0[i]; ++c) {  // blocks another part holds
-                const int j = ci[c];
-                if (pos[j] >= a && pos[j] < b) continue;
-                ghost_all.push_back(static_cast<std::uint32_t>(-1 - block_slots[c]));
-                ghost_all.push_back(static_cast<std::uint32_t>(local[j]) |
-                                    (static_cast<std::uint32_t>((c - ro[i]) * CHX_RES_PART_MAX + (k - a)) << 16));
-            }
-            for (int c = up0[i]; c < ro[i + 1]; ++c) {
-                const int j = ci[c];
-                const bool own = pos[j] >= a && pos[j] < b;
-                const std::uint32_t lj = static_cast<std::uint32_t>(own ? pos[j] - a : local[j]);
+    for (int i = 0; i < n; ++i) walk(i);
+    static_assert(CHX_RES_GEN_HELD * 2 >= CHX_RES_GEN_WIDTH, "half of the widest row");
+    Builder B(p, order, part_rows, CHX_RES_GEN_PART, 2 * CHX_RES_GEN_HELD);
+    const bool ok = B.build([&](int k, int i) {
+        int u = 0;
+        for (int c = ro[i]; c < ro[i + 1]; ++c) {
+            const int j = ci[c];
+            const std::uint32_t value = static_cast<std::uint32_t>(block_slots[c] < 0 ? -1 - block_slots[c] : block_slots[c]);
+            const std::uint32_t place = static_cast<std::uint32_t>(c - ro[i]);
+            if (held[c]) {
+                const std::uint32_t lj = B.local_of(j);
                 const std::uint32_t target =
-                    own ? static_cast<std::uint32_t>(lower[c]) * CHX_RES_PART_MAX + lj : 0xffffu;
-                B[held_at + static_cast<std::size_t>(c - up0[i]) * N + K] = lj | (target << 16);
+                    B.own(j) ? static_cast<std::uint32_t>(mirror[c] - ro[j]) * CHX_RES_GEN_PART + lj : 0x3fffu;
+                B.plane(u, k) = lj | (target << 10) | (place << 24);
+                B.plane(CHX_RES_GEN_HELD + u, k) = value | (j < i ? 0x80000000u : 0u);
+                ++u;
+            } else if (!B.own(j)) {
+                B.ghost(value | (j > i ? 0x80000000u : 0u),
+                        B.local_of(j) | ((place * CHX_RES_GEN_PART + static_cast<std::uint32_t>(k - B.a)) << 16));
             }
         }
-        const std::size_t ghosts = ghost_all.size() / 2 - ghost0;
-        if (ghosts > CHX_RES_GHOST_MAX) return out;
-        std::uint32_t* H = B.data() + 8 * static_cast<std::size_t>(q);
-        H[0] = static_cast<std::uint32_t>(b - a);
-        H[1] = static_cast<std::uint32_t>(halo.size());
-        H[2] = static_cast<std::uint32_t>(halo_all.size() / 2);
-        H[3] = static_cast<std::uint32_t>(ghosts);
-        H[4] = static_cast<std::uint32_t>(ghost0);
-        for (int j : halo) {
-            halo_all.push_back(static_cast<std::uint32_t>(j));
-            halo_all.push_back(exp[j]);
-        }
-    }
-    // absolute word offsets of the lists
-    const std::size_t halo_at = lists_at, ghost_at = halo_at + halo_all.size();
-    if (ghost_at + ghost_all.size() >= (std::size_t(1) << 30)) return out;
-    for (int q = 0; q < parts; ++q) {
-        std::uint32_t* H = B.data() + 8 * static_cast<std::size_t>(q);
-        H[2] = static_cast<std::uint32_t>(halo_at + 2 * H[2]);
-        H[4] = static_cast<std::uint32_t>(ghost_at + 2 * H[4]);
-    }
-    B.insert(B.end(), halo_all.begin(), halo_all.end());
-    B.insert(B.end(), ghost_all.begin(), ghost_all.end());
-    out.part_rows = part_rows;
-    out.parts = parts;
-    out.exports = exports;
-    out.blob = std::move(B);
-    return out;
+        return static_cast<std::uint32_t>((ro[i + 1] - ro[i]) | (u << 8));
+    });
+    return ok ? B.take() : ResidentPlan{};
 }
 
 }  // namespace engine

@@ -18,19 +18,21 @@ namespace engine {
 std::vector<int> resident_order(const topology::Pattern& p);
 
 // The parts of `part_rows` consecutive positions each.  blob is the device
-// image (layout: include/chysx_hip.h, chx_instance::res_plan); empty when
-// the pattern does not fit the kernel's limits (a row with more than
-// CHX_RES_HELD upper or lower blocks, a part with more than
-// CHX_RES_HALO_MAX halo rows or CHX_RES_GHOST_MAX ghost blocks).
-// block_slots: value slot of CSR block k (-1 - partner's slot: lower).
+// image (layout: include/chysx_hip.h, CHX_RES_*); empty when the pattern does
+// not fit the form's limits (blocks of a row, halo rows and ghost blocks of
+// a part).  block_slots: value slot of CSR block k (-1 - partner's: lower).
 struct ResidentPlan {
     int part_rows = 0;
     int parts = 0;
     int exports = 0;  // rows that some other part reads
     std::vector<std::uint32_t> blob;
 };
+// Sheet form: the upper blocks of a row are held by the row.
 ResidentPlan resident_plan(const topology::Pattern& p, const std::vector<int>& block_slots,
                            const std::vector<int>& order, int part_rows);
+// General form: any numbering, wider rows, smaller parts.
+ResidentPlan resident_plan_general(const topology::Pattern& p, const std::vector<int>& block_slots,
+                                   const std::vector<int>& order, int part_rows);
 
 }  // namespace engine
 }  // namespace chysx

@@ -8,7 +8,8 @@ import pytest
 import chysx
 from chysx import scenes
 
-LEAF, PART, HELD, HALO, GHOST, NONE = 64, 1024, 6, 512, 512, 0xFFFFFFFF
+PART, HELD, HALO, GHOST, NONE = 1024, 6, 512, 512, 0xFFFFFFFF
+GEN_PART, GEN_HELD, GEN_WIDTH = 512, 8, 16
 
 
 def _pattern(nx, ny):
@@ -79,7 +80,7 @@ def test_plan_product_is_the_matrix_product(nx, ny, part_rows):
         for k in range(own):
             i = int(blob[rows_at + a + k])
             assert i == order[a + k]
-            nl, nh = blob[meta_at + a + k] & 15, blob[meta_at + a + k] >> 4
+            nl, nh = blob[meta_at + a + k] & 255, blob[meta_at + a + k] >> 8
             assert nl <= HELD and nh <= HELD and nl + nh == ro[i + 1] - ro[i]
             for u in range(nh):
                 w = blob[held_at + u * n + a + k]
@@ -90,7 +91,7 @@ def test_plan_product_is_the_matrix_product(nx, ny, part_rows):
                     assert col < own and (w >> 16) % PART == col
                     put(w >> 16, v * p[k])
         for k in range(own):
-            i, nl = int(order[a + k]), blob[meta_at + a + k] & 15
+            i, nl = int(order[a + k]), blob[meta_at + a + k] & 255
             at = np.arange(HELD) * PART + k
             assert filled[at[:nl]].all() and not filled[at[nl:]].any()
             got[i] += prod[at[:nl]].sum()
@@ -98,6 +99,65 @@ def test_plan_product_is_the_matrix_product(nx, ny, part_rows):
             lower = ci[ro[i]:ro[i] + nl]
             assert (prod[at[:nl]] == val[-1 - bs[ro[i]:ro[i] + nl]] * x[lower]).all()
     assert (got == want).all()
+
+
+@pytest.mark.parametrize("nx,ny,shuffle", [(2, 2, False), (16, 16, True), (33, 31, False), (33, 31, True), (65, 40, True)])
+@pytest.mark.parametrize("part_rows", [256, 512])
+def test_general_plan_product_is_the_matrix_product(nx, ny, shuffle, part_rows):
+    """Any numbering: every pair's block is held once (or is a ghost of the
+    other part), every product lands at its place in the column order of its
+    row, with the transpose marked where the stored block is the other
+    row's."""
+    n = nx * ny
+    _, tris = scenes.cloth_grid(nx, ny)
+    if shuffle:
+        tris = np.random.default_rng(n).permutation(n).astype(np.int32)[tris]
+    d = chysx.topology.cloth_system(n, tris, np.zeros(0, np.int32))
+    ro, ci = d["row_offsets"], d["col_indices"]
+    bs, n_values = _slots(n, ro, ci)
+    plan = chysx.topology.resident_plan(n, ro, ci, bs, part_rows, general=True)
+    order, blob, parts = plan["order"], plan["blob"].astype(np.int64), plan["parts"]
+    assert sorted(order) == list(range(n)) and parts == -(-n // part_rows)
+    rows_at, meta_at, exp_at, held_at = 8 * parts, 8 * parts + n, 8 * parts + 2 * n, 8 * parts + 3 * n
+    export_row = {int(blob[exp_at + k]): int(order[k]) for k in range(n) if blob[exp_at + k] != NONE}
+    assert sorted(export_row) == list(range(plan["exports"]))
+    for q in range(parts):
+        own, halo, halo_at, ghost, ghost_at, widest = blob[8 * q:8 * q + 6]
+        a = q * part_rows
+        assert own == min(part_rows, n - a) and halo <= HALO and ghost <= GHOST
+        halo_rows = blob[halo_at:halo_at + 2 * halo].reshape(-1, 2)
+        assert all(export_row[int(e)] == r for r, e in halo_rows)
+        row_of = {k: int(order[a + k]) for k in range(own)}
+        row_of.update({GEN_PART + h: int(halo_rows[h, 0]) for h in range(halo)})
+        got = {}  # product slot -> (row, column, value slot, as stored)
+
+        def put(slot, *what):
+            assert slot not in got and slot < GEN_WIDTH * GEN_PART
+            got[slot] = what
+
+        for value, w in blob[ghost_at:ghost_at + 2 * ghost].reshape(-1, 2):
+            i, j = row_of[(w >> 16) % GEN_PART], row_of[w & 0xFFFF]
+            # the kernel transposes a ghost block unless its mark is set
+            put(w >> 16, i, j, value & 0x7FFFFFFF, bool(value >> 31))
+        for k in range(own):
+            i, meta = row_of[k], blob[meta_at + a + k]
+            assert blob[rows_at + a + k] == i and meta & 255 == ro[i + 1] - ro[i] <= widest and meta >> 8 <= GEN_HELD
+            for u in range(meta >> 8):
+                w, value = blob[held_at + u * n + a + k], blob[held_at + (GEN_HELD + u) * n + a + k]
+                j, flip = row_of[w & 0x3FF], bool(value >> 31)
+                put((w >> 24) * GEN_PART + k, i, j, value & 0x7FFFFFFF, not flip)
+                t = (w >> 10) & 0x3FFF
+                assert (t == 0x3FFF) == ((w & 0x3FF) >= GEN_PART)
+                if t != 0x3FFF:
+                    assert t % GEN_PART == w & 0x3FF
+                    put(t, j, i, value & 0x7FFFFFFF, flip)
+        want = {}
+        for k in range(own):
+            i = row_of[k]
+            for t, c in enumerate(range(ro[i], ro[i + 1])):
+                j = int(ci[c])
+                want[t * GEN_PART + k] = (i, j, bs[c] if j > i else -1 - bs[c], j > i)
+        assert got == want
 
 
 def test_pattern_outside_the_limits_has_no_plan():
@@ -108,3 +168,4 @@ def test_pattern_outside_the_limits_has_no_plan():
     ro, ci = chysx.topology.build_pattern(n, rows, cols)
     bs, _ = _slots(n, ro, ci)
     assert chysx.topology.resident_plan(n, ro, ci, bs, 256) is None
+    assert chysx.topology.resident_plan(n, ro, ci, bs, 256, general=True) is None
