@@ -172,12 +172,12 @@ typedef struct chx_unit {
  * source row | product slot << 16}.  Local indices: position in the part, or
  * part capacity + halo index.
  *
- * Sheet form (res_general 0; every row at most CHX_RES_HELD lower and upper
+ * Sheet form (res_form 0; every row at most CHX_RES_HELD lower and upper
  * blocks): CHX_RES_HELD planes, word = local index of upper block u's column
  * | product slot << 16.  A product slot is (place among the target row's
  * lower blocks) * CHX_RES_PART_MAX + (target's position); 0xffff: none.
  *
- * General form (res_general 1; at most CHX_RES_GEN_WIDTH blocks a row, parts
+ * General form (res_form 1; at most CHX_RES_GEN_WIDTH blocks a row, parts
  * of at most CHX_RES_GEN_PART rows): every pair's block is held by one of
  * its rows, at most CHX_RES_GEN_HELD a row: CHX_RES_GEN_HELD planes of words
  * local index of the other row | product slot << 10 | place in the row's own
@@ -185,7 +185,13 @@ typedef struct chx_unit {
  * row needs the transpose).  Product slots are (place in the target row's
  * column order) * CHX_RES_GEN_PART + (target's position); 0x3fff: none.  The
  * ghost lists' value slots carry bit 31 when the target row needs the block
- * as stored. */
+ * as stored.
+ *
+ * Rows form (res_form 2; a caller's row-major CSR matrix, at most
+ * CHX_RES_ROW_WIDTH blocks a row, parts of at most CHX_RES_GEN_PART rows):
+ * every row holds all of its blocks, in CSR order: CHX_RES_ROW_WIDTH planes
+ * of local column indices; no product slots, no ghost blocks. */
+#define CHX_RES_ROW_WIDTH 12
 #define CHX_RES_GEN_PART 512
 #define CHX_RES_GEN_HELD 8
 #define CHX_RES_GEN_WIDTH 16
@@ -288,10 +294,21 @@ typedef struct chx_instance {
     int res_part_rows;               /* rows per part                                        */
     int res_parts;                   /* ceil(n_rows / res_part_rows)                         */
     int res_exports;                 /* exported rows                                        */
-    int res_general;                 /* the plan's form                                      */
+    int res_form;                    /* the plan's form                                      */
     unsigned res_xbase;              /* first word of the instance's exchange area in xbuf   */
     int res_pad;
 } chx_instance;
+
+/* Plan of a caller's matrix for the resident standalone solve (rows form). */
+typedef struct chx_rows_plan {
+    const unsigned* plan;            /* device image (chx_instance::res_plan)                */
+    int part_rows, parts, exports;
+    int pad;
+    unsigned long long* xbuf;        /* exchange area, zero before its first solve; solves   */
+                                     /* that overlap must not share it                       */
+    unsigned long long xwords;       /* its 64-bit words: at least CHX_RES_CONTROL_WORDS +   */
+                                     /* CHX_RES_XWORDS(parts, exports)                       */
+} chx_rows_plan;
 
 /* A batch of instances advanced together.  Work lists are device int4
  * arrays: row tiles {instance, row_begin, row_end, 0} (local rows, row_begin
@@ -365,7 +382,7 @@ typedef struct chx_cloth_batch {
                                      /* workgroups: solved in list order by the ranks     */
                                      /* from their first rank on                          */
     int res_groups;
-    int res_general;                 /* form of all the instances' plans                  */
+    int res_form;                    /* form of all the instances' plans                  */
     unsigned long long res_xwords;   /* 64-bit words of xbuf                              */
 } chx_cloth_batch;
 
@@ -383,6 +400,9 @@ int chx_device_info(int* cu_count, int* max_pcg_blocks, int* occupancy_blocks_pe
 int chx_pcg_grid_limit(int lanes_per_row, int bf16_blocks, int no_lds_staging, int* max_blocks);
 /* The same for the resident PCG kernel (one workgroup per compute unit). */
 int chx_resident_grid_limit(int* max_blocks);
+/* Workgroups and groups of a resident launch of one instance with `parts`
+ * parts, at most `limit` workgroups (parts <= limit). */
+int chx_resident_grid(int parts, int limit, int* grid, int* groups);
 
 /* Device memory: replaces CudaArray<T> (ChysX/src/memory/cuda_array.h:64-284,
  * cuda_array.cu:41-90). */
@@ -506,6 +526,14 @@ int chx_contact_bake_diag(int n_rows, float* diag, const chx_contact_op* op, flo
 /* y += alpha * cross-slot contact terms * x (AoS float3 [n_rows*3]). */
 int chx_contact_spmv(int n_rows, const chx_contact_op* op, const float* x, float* y, float alpha, void* workspace,
                      size_t workspace_bytes, uintptr_t stream);
+/* chx_pcg_solve_bsr3 with a resident plan of the matrix's pattern: at 8 lanes
+ * per row the solve keeps the matrix on chip (the same operations; only the
+ * order of the FP64 inner products differs).  plan NULL, or its plan NULL:
+ * chx_pcg_solve_bsr3. */
+int chx_pcg_solve_bsr3_plan(int n_rows, const float* diag, const int* row_offsets, const int* col_indices,
+                            const float* values, const float* b, float* x, int max_iterations, double tol,
+                            int lanes_per_row, void* workspace, size_t workspace_bytes, const chx_rows_plan* plan,
+                            int* iterations, double* rr, double* bb, uintptr_t stream);
 /* chx_pcg_solve_bsr3 on (A + C_off): the contact cross-slot terms join the
  * residual and every SpMV (the caller bakes the same-slot terms into diag). */
 int chx_pcg_solve_bsr3_contact(int n_rows, const float* diag, const int* row_offsets, const int* col_indices,

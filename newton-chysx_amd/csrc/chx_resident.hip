@@ -1,8 +1,8 @@
-// Resident block-Jacobi PCG of the FP32 cloth instances: a workgroup keeps
-// its part of an instance's matrix in registers and its vectors in registers
-// and LDS from the first product to the last, so an iteration reads no
-// matrix from memory.  What crosses workgroups in an iteration is the halo
-// rows of q = A p and five partial sums, in one hop.
+// Resident block-Jacobi PCG: a workgroup keeps its part of a matrix in
+// registers and its vectors in registers and LDS from the first product to
+// the last, so an iteration reads no matrix from memory.  What crosses
+// workgroups in an iteration is the halo rows of q = A p and a few partial
+// sums.
 //
 // Why: streaming the matrix every iteration cost 20.5 ms per solve of the
 // 512-cloth batch (2.08 M rows, 66 iterations on average), set by the
@@ -12,24 +12,27 @@
 // 262,144 rows, and the instances of a batch are independent: they are
 // solved one after another by gangs of ceil(rows / 1024) workgroups.
 //
-// Arithmetic: the single-barrier recurrence of pcg1_kernel (chx_step.hip),
-// operation for operation; every row sums its diagonal product, its lower
-// blocks and its upper blocks in column order.  A row's upper blocks are in
-// its thread's registers: it forms A_ij p_j for itself and A_ij^T p_i for
-// row j, which it leaves in row j's product slot in LDS.  Blocks between
-// parts are held by both (the second copy is a "ghost block").  Halo rows'
-// r, z and p are kept by every part that reads them, updated from the
-// published q with the same operations as by their owner.
+// Two solvers, operation for operation those of chx_step.hip: the merged
+// recurrence of pcg1_kernel (one exchange an iteration: halo rows of q and
+// five sums), and the two-reduction one of pcg_kernel (BF16 mode and caller's
+// row-major systems: halo rows of q and sigma, then rho and ||r||^2).  Every
+// row sums its products in the order of those kernels.
+//
+// Products: a thread's held block serves its own row (A_ij p_j) and, through
+// a product slot in LDS, the row of its transpose (A_ij^T p_i).  Blocks
+// between parts are held by both (the second copy is a "ghost block").
+// Halo rows' r, z and p are kept by every part that reads them, updated from
+// the sent q with the same operations as by their owner.
 //
 // Inner products: FP64, one sum per 64-row leaf (a wavefront), combined over
 // the leaves of the instance by a fixed binary tree that does not depend on
 // how many leaves a part has: the same bits for every part size and gang.
 //
-// Exchange: 64-bit words {value, tag}, the tag naming launch and phase, so a
-// reader needs no ordering between words and no cache maintenance: it reads
+// Exchange: 64-bit words {value, tag}, the tag naming launch and exchange, so
+// a reader needs no ordering between words and no cache maintenance: it reads
 // a word until its tag is the awaited one.  Words alternate between two
-// slots; slot t is rewritten in phase t + 2, which its writer enters only
-// after every part's sums of phase t + 1, sent after their reads of phase t.
+// slots; slot t is rewritten in exchange t + 2, which its writer enters only
+// after every part's sums of exchange t + 1, sent after their reads of t.
 #include <algorithm>
 #include <mutex>
 
@@ -42,34 +45,48 @@ namespace {
 constexpr int kThreads = 512;  // two waves per SIMD with 256 VGPRs each
 constexpr int kWaves = kThreads / kWave;
 constexpr int kLeaves = CHX_RES_PART_MAX / CHX_RES_LEAF;
-// The two forms of a plan (chysx_hip.h).  Sheet: a row's lower blocks come
+// The forms of a plan (chysx_hip.h).  Sheet: a row's lower blocks come
 // through product slots and are summed before the upper ones that its thread
 // holds, which is column order.  General: all of a row's products go through
 // its slots, in column order; twice the slots and wider rows, so half the
-// rows.
-template <bool GEN>
+// rows.  Rows: a caller's matrix, every row holding all of its own blocks.
+enum { SHEET = 0, GENERAL = 1, ROWS = 2 };
+template <int FORM>
 struct Form {
-    static constexpr unsigned kRows = GEN ? CHX_RES_GEN_PART : CHX_RES_PART_MAX;
+    static constexpr unsigned kRows = FORM == SHEET ? CHX_RES_PART_MAX : CHX_RES_GEN_PART;
     static constexpr int kSlots = kRows / kThreads;  // own rows per thread
-    static constexpr int kHeld = GEN ? CHX_RES_GEN_HELD : CHX_RES_HELD;
-    static constexpr unsigned kPlaces = GEN ? CHX_RES_GEN_WIDTH : CHX_RES_HELD;  // product slots per row
-    static constexpr unsigned kNoSlot = GEN ? 0x3fffu : 0xffffu;
+    static constexpr int kHeld = FORM == SHEET ? CHX_RES_HELD : (FORM == GENERAL ? CHX_RES_GEN_HELD : CHX_RES_ROW_WIDTH);
+    // product slots per row
+    static constexpr unsigned kPlaces = FORM == SHEET ? CHX_RES_HELD : (FORM == GENERAL ? CHX_RES_GEN_WIDTH : 0);
     static constexpr unsigned kSpare = kPlaces * kRows;  // first of the unread product slots
-    // fields of a held block's word
-    static __device__ __forceinline__ unsigned src(unsigned w) { return w & (GEN ? 0x3ffu : 0xffffu); }
-    static __device__ __forceinline__ unsigned slot(unsigned w) { return GEN ? (w >> 10) & 0x3fffu : w >> 16; }
-    static __device__ __forceinline__ unsigned word(unsigned s, unsigned t) { return s | (t << (GEN ? 10 : 16)); }
+    // A held block's word in the plan, and here: the LDS word index of its
+    // source vector entry, of its product slot and its place in the row.
+    static __device__ __forceinline__ unsigned unpack(unsigned w, unsigned lane) {
+        if (FORM == ROWS) return 3u * w;
+        const unsigned src = FORM == SHEET ? w & 0xffffu : w & 0x3ffu;
+        unsigned slot = FORM == SHEET ? w >> 16 : (w >> 10) & 0x3fffu;
+        if (slot == (FORM == SHEET ? 0xffffu : 0x3fffu)) slot = kSpare + lane;
+        return FORM == SHEET ? 3u * src | (3u * slot) << 16 : 3u * src | (3u * slot) << 12 | (w >> 24) << 27;
+    }
+    static __device__ __forceinline__ unsigned src(unsigned w) {
+        return FORM == ROWS ? w : w & (FORM == SHEET ? 0xffffu : 0xfffu);
+    }
+    static __device__ __forceinline__ unsigned slot(unsigned w) { return FORM == SHEET ? w >> 16 : (w >> 12) & 0x7fffu; }
+    static __device__ __forceinline__ unsigned place(unsigned w) { return w >> 27; }
 };
-static_assert(Form<true>::kSpare + kWave <= Form<true>::kNoSlot && Form<false>::kSpare + kWave <= Form<false>::kNoSlot &&
-                  Form<true>::kRows + CHX_RES_HALO_MAX <= 1024,
+static_assert(3 * (Form<SHEET>::kSpare + kWave) < (1u << 16) && 3 * (Form<GENERAL>::kSpare + kWave) < (1u << 15) &&
+                  3 * (Form<GENERAL>::kRows + CHX_RES_HALO_MAX) <= (1u << 12) && CHX_RES_GEN_WIDTH <= 16,
               "word fields");
-constexpr int kSums = 5;  // rho, sigma, delta, gamma, ||r||^2 (set-up: ||b||^2 in place of sigma)
+// Sums of an exchange: merged solver rho, sigma, delta, gamma, ||r||^2
+// (set-up: ||b||^2 in place of sigma); two-reduction solver sigma, or rho and
+// ||r||^2 (set-up: and ||b||^2).
+constexpr int kSums = 5;
 constexpr int kMaxParts = 256;
 constexpr unsigned kFan = 16;    // parts per group and groups, above 64 parts
 constexpr unsigned kCopies = 16;  // copies of the groups' sums
 static_assert(kFan * kFan >= kMaxParts && 2 * kCopies <= 64, "two levels");
 constexpr unsigned kExit = 0xffffffu;  // mailbox item: nothing left
-static_assert(CHX_RES_LEAF == kWave && Form<false>::kSlots == 2 && Form<true>::kSlots == 1 && kLeaves == 2 * kWaves,
+static_assert(CHX_RES_LEAF == kWave && Form<SHEET>::kSlots == 2 && Form<GENERAL>::kSlots == 1 && kLeaves == 2 * kWaves,
               "a leaf per wave and slot");
 static_assert(CHX_RES_HALO_MAX <= kThreads && CHX_RES_GHOST_MAX <= kThreads, "one halo row and ghost block a thread");
 
@@ -83,18 +100,12 @@ __device__ __forceinline__ void st64(u64* p, u64 v) {
 }
 __device__ __forceinline__ u64 tagged(unsigned v, unsigned tag) { return (u64(tag) << 32) | v; }
 
-// LDS triples as one 96-bit access.
-typedef float v3f __attribute__((ext_vector_type(3), aligned(4)));
-__device__ __forceinline__ f3 lds_ld(const f3* p) {
-    const v3f v = *reinterpret_cast<const v3f*>(p);
-    return {v.x, v.y, v.z};
-}
-__device__ __forceinline__ void lds_st(f3* p, f3 v) {
-    v3f w;
-    w.x = v.x;
-    w.y = v.y;
-    w.z = v.z;
-    *reinterpret_cast<v3f*>(p) = w;
+// Triples in LDS, by the index of their first word.
+__device__ __forceinline__ f3 lds_ld(const float* m, unsigned i) { return {m[i], m[i + 1u], m[i + 2u]}; }
+__device__ __forceinline__ void lds_st(float* m, unsigned i, f3 v) {
+    m[i] = v.x;
+    m[i + 1u] = v.y;
+    m[i + 2u] = v.z;
 }
 // Keeps a value that the loop does not change from being re-derived ahead of
 // the loop (addresses and masks of every block would not fit the registers).
@@ -103,15 +114,15 @@ __device__ __forceinline__ unsigned opaque(unsigned v) {
     return v;
 }
 
-template <bool GEN>
+template <int FORM, bool FULL>
 struct ResLds {
     // products by target row, then one unread slot per lane for blocks
     // without a target
-    f3 prod[Form<GEN>::kSpare + kWave];
-    f3 p[Form<GEN>::kRows + CHX_RES_HALO_MAX];     // source vector: own rows, halo rows
-    float diag[6][Form<GEN>::kRows];
-    f3 x[Form<GEN>::kRows];
-    float ghost[9][CHX_RES_GHOST_MAX];
+    float prod[3 * (Form<FORM>::kSpare + kWave)];
+    float p[3 * (Form<FORM>::kRows + CHX_RES_HALO_MAX)];  // source vector: own rows, halo rows
+    float diag[FULL ? 9 : 6][Form<FORM>::kRows];
+    float x[3 * Form<FORM>::kRows];
+    float ghost[FORM == ROWS ? 1 : 9][CHX_RES_GHOST_MAX];
     double leaf[kLeaves][kSums];
     double tot[8];
     int bad;         // a wait gave up
@@ -201,9 +212,6 @@ __device__ __forceinline__ void ld6u(gp<const float> m, unsigned i, float (&u)[6
 }
 __device__ __forceinline__ f3 axpy(float a, f3 x, f3 y) { return mk(fmaf(a, x.x, y.x), fmaf(a, x.y, y.y), fmaf(a, x.z, y.z)); }
 
-// The wave's two leaf sums of kSums values into S.leaf.  Halving butterfly:
-// each step adds lane pairs and packs two values into the two halves of the
-// pairs, so five values of two leaves take 14 FP64 adds instead of 60.
 template <int CTRL>
 __device__ __forceinline__ double dpp64(double v) {
     const u64 b = u64(__double_as_longlong(v));
@@ -232,11 +240,14 @@ __device__ __forceinline__ double fold8(double a, double b, unsigned lane) {
     const bool up = (lane & 8u) != 0u;
     return (up ? b : a) + dpp64<kRor8>(up ? a : b);
 }
-__device__ __forceinline__ void leaf_sums(const double (&a)[kSums], const double (&b)[kSums],
-                                          double (&leaf)[kLeaves][kSums], unsigned wave, unsigned lane) {
-    double v[kSums];
+// The wave's two leaf sums of five values into `leaf`.  Halving butterfly:
+// each step adds lane pairs and packs two values into the two halves of the
+// pairs, so five values of two leaves take 14 FP64 adds instead of 60.
+__device__ __forceinline__ void leaf_sums(const double (&a)[5], const double (&b)[5], double (&leaf)[kLeaves][kSums],
+                                          unsigned wave, unsigned lane) {
+    double v[5];
 #pragma unroll
-    for (int k = 0; k < kSums; ++k) v[k] = fold32(a[k], b[k]);  // half h: leaf of slot h
+    for (int k = 0; k < 5; ++k) v[k] = fold32(a[k], b[k]);  // half h: leaf of slot h
     // rows (16 lanes) 2h, 2h + 1 of half h: values 0 | 1, 2 | 3, 4 | 4
     const double x = fold16(v[0], v[1]), y = fold16(v[2], v[3]), z = fold16(v[4], v[4]);
     double w0 = fold8(x, y, lane);             // half-rows: values 0 2 | 1 3
@@ -252,15 +263,39 @@ __device__ __forceinline__ void leaf_sums(const double (&a)[kSums], const double
     if ((place & 7u) == 0u) out[(place >> 4) + ((place & 8u) >> 2)] = w0;
     if (place == 1u) out[4] = w1;
 }
+// The same for up to three values (the second and third in one row each).
+template <int N>
+__device__ __forceinline__ void leaf_sums(const double (&a)[N], const double (&b)[N], double (&leaf)[kLeaves][kSums],
+                                          unsigned wave, unsigned lane) {
+    static_assert(N >= 1 && N <= 3, "values");
+    double w = fold16(fold32(a[0], b[0]), N > 1 ? fold32(a[N > 1 ? 1 : 0], b[N > 1 ? 1 : 0]) : 0.0);
+    double y = 0.0;
+    if constexpr (N == 3) {
+        y = fold32(a[2], b[2]);
+        y = fold16(y, y);
+    }
+    w = fold8(w, y, lane);
+    w += dpp64<kHalfMirror>(w);
+    w += dpp64<kXor2>(w);
+    w += dpp64<kXor1>(w);
+    double(&out)[kSums] = leaf[(lane >> 5) * kWaves + wave];
+    const unsigned place = lane & 31u;
+    if (place == 0u) out[0] = w;
+    if (N > 1 && place == 16u) out[1] = w;
+    if (N > 2 && place == 8u) out[2] = w;
+}
 
 // Solves instance `inst` together with the workgroups that hold its other
-// parts; this one holds part `part`.  False: aborted.
-template <bool GEN>
+// parts; this one holds part `part`.  TWO: the two-reduction solver (with
+// B.bf16_blocks on the BF16 matrix).  False: aborted.
+template <int FORM, bool TWO>
 __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst& I, int inst, int part, unsigned epoch,
-                                           ResLds<GEN>& S, const Barrier& bar, int& trace_e) {
-    using F = Form<GEN>;
+                                           ResLds<FORM, TWO>& S, const Barrier& bar, int& trace_e) {
+    using F = Form<FORM>;
     constexpr int kSlots = F::kSlots, kHeld = F::kHeld;
     constexpr unsigned kPart = F::kRows;
+    constexpr int kDiag = TWO ? 9 : 6;       // words of a diagonal block in LDS
+    constexpr int kMinv = FORM == ROWS ? 9 : 6;  // words of an inverse
     const unsigned tid = threadIdx.x, lane = tid & (kWave - 1);
     const unsigned wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const gp<const unsigned> plan = I.res_plan;
@@ -269,9 +304,10 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     const unsigned n_own = hdr[0], n_halo = hdr[1], halo_at = hdr[2], n_ghost = hdr[3], ghost_at = hdr[4], widest = hdr[5];
     const unsigned pos0 = unsigned(part) * unsigned(I.res_part_rows);
     const unsigned rows_at = 8u * parts, meta_at = rows_at + n, exp_at = meta_at + n, held_at = exp_at + n;
-    // exchange areas: [2][kSums][parts] pairs of words, then [2][exports] rows of 3
+    // exchange areas: [2][kSums][parts] pairs of words, above 64 parts
+    // [2][kCopies][kSums][kFan] pairs, then [2][exports] rows of 3
     u64* const xsum = B.xbuf + I.res_xbase;
-    u64* const xgroup = xsum + 4u * kSums * parts;  // [2][kCopies][kSums][kFan] pairs
+    u64* const xgroup = xsum + 4u * kSums * parts;
     u64* const xrow = xgroup + (parts > unsigned(kWave) ? 4u * kCopies * kSums * kFan : 0u);
     const unsigned exports = unsigned(I.res_exports);
     auto tag_of = [&](int t) { return (epoch << 8) | (unsigned(t) & 255u); };
@@ -282,7 +318,6 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         return xgroup + 2u * ((((unsigned(t) & 1u) * kCopies + copy) * kSums + v) * kFan + g);
     };
     auto row_words = [&](int t, unsigned e) { return xrow + 3ull * ((unsigned(t) & 1u) * exports + e); };
-
     auto send_row = [&](int t, unsigned e, f3 v) {
         u64* const w = row_words(t, e);
         st64(w, tagged(__float_as_uint(v.x), tag_of(t)));
@@ -293,8 +328,80 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     // ---- load: own rows, ghost block, halo row ----
     unsigned lp[kSlots], ex[kSlots], holds[kSlots], word[kSlots][kHeld];
     bool live[kSlots], on[kSlots];  // this lane's row exists; this wave has a row
-    float V[kSlots][kHeld][9], M[kSlots][6];
+    float V[kSlots][kHeld][9], M[kSlots][kMinv];
     f3 r[kSlots], p[kSlots], q[kSlots];
+    // ghost blocks and halo rows from the last thread down: in a small part
+    // the first waves have the rows
+    const unsigned rtid = unsigned(kThreads - 1) - tid;
+    // the matrix blocks: FP32, or the BF16 copies and compensated diagonal
+    auto load_blocks = [&](bool half) {
+        auto block = [&](unsigned v, float (&m)[9]) {
+            if (FORM == ROWS) {
+                const gp<const float> b = rec_at(gp<const float>(I.values), v, 9u);
+#pragma unroll
+                for (int c = 0; c < 9; ++c) m[c] = b[c];
+            } else if (TWO && half) {
+                ld9p(gp<const uint16_t>(I.values16), v & 0x7fffffffu, m);
+            } else {
+                ld9p(gp<const float>(I.values), v & 0x7fffffffu, m);
+            }
+            if (FORM == GENERAL && (v >> 31) != 0u) transpose9(m);
+        };
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s)
+            if (on[s]) {
+                const unsigned K = pos0 + (live[s] ? lp[s] : 0u);
+                const unsigned row = ldx(plan, rows_at + K);
+                const unsigned first = FORM == ROWS ? unsigned(ldx(I.row_offsets, row))
+                                                    : unsigned(ldx(I.upper_offsets, row / CHX_SLICE_ROWS)) +
+                                                          row % CHX_SLICE_ROWS;
+#pragma unroll
+                for (int u = 0; u < kHeld; ++u) {
+#pragma unroll
+                    for (int c = 0; c < 9; ++c) V[s][u][c] = 0.0f;
+                    if (unsigned(u) < holds[s]) {
+                        unsigned v = first + unsigned(u) * (FORM == ROWS ? 1u : unsigned(CHX_SLICE_ROWS));
+                        if (FORM == GENERAL) v = ldx(plan, held_at + unsigned(kHeld + u) * n + K);
+                        block(v, V[s][u]);
+                    }
+                }
+                float d[9];
+                if (FORM == ROWS) {
+                    const gp<const float> b = rec_at(gp<const float>(I.diag), row, 9u);
+#pragma unroll
+                    for (int c = 0; c < 9; ++c) d[c] = b[c];
+                } else if (TWO && half) {
+                    ld9p(gp<const float>(I.diag_c), row, d);
+                } else {
+                    ld6p(gp<const float>(I.diag), row, d);
+                }
+#pragma unroll
+                for (unsigned c = 0; c < unsigned(kDiag); ++c) S.diag[c][lp[s]] = d[kDiag == 9 ? c : sym6_pos(c)];
+            }
+        if (FORM != ROWS && rtid < n_ghost) {
+            float g[9];
+            block(ldx(plan, ghost_at + 2u * rtid), g);
+#pragma unroll
+            for (int c = 0; c < 9; ++c) S.ghost[c][rtid] = g[c];
+        }
+    };
+    auto apply_minv = [&](const float (&m)[kMinv], f3 v) {
+        if constexpr (FORM == ROWS) return mv9(m, v);
+        else return mv_sym(m, v);
+    };
+    auto invert = [&](unsigned row, float (&m)[kMinv]) {
+        float d[9], full[9];
+        if (FORM == ROWS) {
+            const gp<const float> b = rec_at(gp<const float>(I.diag), row, 9u);
+#pragma unroll
+            for (int c = 0; c < 9; ++c) d[c] = b[c];
+        } else {
+            ld6p(gp<const float>(I.diag), row, d);
+        }
+        inverse9(d, full);
+#pragma unroll
+        for (unsigned c = 0; c < unsigned(kMinv); ++c) m[c] = full[kMinv == 9 ? c : sym6_pos(c)];
+    };
 #pragma unroll
     for (int s = 0; s < kSlots; ++s) {
         lp[s] = (unsigned(s) * kWaves + wave) * kWave + lane;
@@ -305,145 +412,153 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         holds[s] = 0u;
         r[s] = p[s] = q[s] = mk(0.f, 0.f, 0.f);
         if (on[s]) {
-            unsigned ns = 0u, nh = 0u;
+            unsigned ns = 0u;
             const unsigned row = ldx(plan, rows_at + K);
             const unsigned meta = ldx(plan, meta_at + K);
             if (live[s]) {
                 ns = meta & 255u;
-                nh = meta >> 8;
+                holds[s] = meta >> 8;
                 ex[s] = ldx(plan, exp_at + K);
             }
-            holds[s] = nh;
-            const unsigned vs = unsigned(ldx(I.upper_offsets, row / CHX_SLICE_ROWS)) + row % CHX_SLICE_ROWS;
 #pragma unroll
             for (int u = 0; u < kHeld; ++u) {
                 // a block that is not there is zero, of the row itself
-                const bool has = unsigned(u) < nh;
-                unsigned w = has ? ldx(plan, held_at + unsigned(u) * n + K) : F::word(lp[s], F::kNoSlot);
-                if (F::slot(w) == F::kNoSlot) w = (w & ~F::word(0u, F::kNoSlot)) | F::word(0u, F::kSpare + lane);
-                word[s][u] = w;
-#pragma unroll
-                for (int c = 0; c < 9; ++c) V[s][u][c] = 0.0f;
-                if (has) {
-                    unsigned v = vs + unsigned(u) * CHX_SLICE_ROWS;
-                    if (GEN) v = ldx(plan, held_at + unsigned(kHeld + u) * n + K);
-                    ld9p(gp<const float>(I.values), v & 0x7fffffffu, V[s][u]);
-                    if (GEN && (v >> 31) != 0u) transpose9(V[s][u]);
-                }
+                unsigned w = FORM == SHEET ? (0xffffu << 16) | lp[s] : (FORM == GENERAL ? (0x3fffu << 10) | lp[s] : lp[s]);
+                if (unsigned(u) < holds[s]) w = ldx(plan, held_at + unsigned(u) * n + K);
+                word[s][u] = F::unpack(w, lane);
             }
             // product slots that no block fills stay zero and are added like
             // the others
 #pragma unroll
             for (unsigned u = 0; u < F::kPlaces; ++u)
-                if (u >= ns) S.prod[u * kPart + lp[s]] = mk(0.f, 0.f, 0.f);
-            float d[6], full[9];
-            ld6u(gp<const float>(I.diag), row, d);
-#pragma unroll
-            for (int c = 0; c < 6; ++c) S.diag[c][lp[s]] = d[c];
-            inverse_sym(d, M[s], full);
+                if (u >= ns) lds_st(S.prod, 3u * (u * kPart + lp[s]), mk(0.f, 0.f, 0.f));
+            invert(row, M[s]);
             if (live[s]) p[s] = ld3g(I.x, row);
-            S.x[lp[s]] = p[s];
-            S.p[lp[s]] = p[s];
+            lds_st(S.x, 3u * lp[s], p[s]);
+            lds_st(S.p, 3u * lp[s], p[s]);
         }
     }
-    // ghost blocks and halo rows from the last thread down: in a small part
-    // the first waves have the rows
-    const unsigned rtid = unsigned(kThreads - 1) - tid;
-    unsigned gword = 0;
-    if (rtid < n_ghost) {
-        const unsigned vs = ldx(plan, ghost_at + 2u * rtid);
-        gword = ldx(plan, ghost_at + 2u * rtid + 1u);
-        float g[9];
-        ld9p(gp<const float>(I.values), vs & 0x7fffffffu, g);
-        if (GEN && (vs >> 31) != 0u) transpose9(g);
-#pragma unroll
-        for (int c = 0; c < 9; ++c) S.ghost[c][rtid] = g[c];
+    if constexpr (!TWO) load_blocks(false);
+    unsigned gsrc = 0, gslot = 0;
+    if (FORM != ROWS && rtid < n_ghost) {
+        const unsigned g = ldx(plan, ghost_at + 2u * rtid + 1u);
+        gsrc = 3u * (g & 0xffffu);
+        gslot = 3u * (g >> 16);
     }
-    float hM[6];
+    float hM[kMinv];
     f3 hr = mk(0.f, 0.f, 0.f);
     unsigned hex = 0;
+    const unsigned hslot = 3u * (kPart + rtid);
     if (rtid < n_halo) {
         const unsigned hrow = ldx(plan, halo_at + 2u * rtid);
         hex = ldx(plan, halo_at + 2u * rtid + 1u);
-        float d[6], full[9];
-        ld6u(gp<const float>(I.diag), hrow, d);
-        inverse_sym(d, hM, full);
-        S.p[kPart + rtid] = ld3g(I.x, hrow);
+        invert(hrow, hM);
+        lds_st(S.p, hslot, ld3g(I.x, hrow));
     }
     if (tid == 0) S.bad = 0;
     if (tid < kLeaves * kSums) S.leaf[tid / kSums][tid % kSums] = 0.0;
 
-    // A times the vector in S.p (own rows also in v); S.p and
-    // S.prod are read until the next workgroup barrier.
+    // A times the vector in S.p (own rows also in v); S.p and S.prod are read
+    // until the next workgroup barrier.
     auto apply = [&](const f3 (&v)[kSlots], f3 (&out)[kSlots]) {
+        if constexpr (FORM != ROWS) {
 #pragma unroll
-        for (int s = 0; s < kSlots; ++s)
-            if (on[s]) {
+            for (int s = 0; s < kSlots; ++s)
+                if (on[s]) {
 #pragma unroll
-                for (int u = 0; u < kHeld; ++u) lds_st(&S.prod[F::slot(opaque(word[s][u]))], mv9t(V[s][u], v[s]));
+                    for (int u = 0; u < kHeld; ++u) lds_st(S.prod, F::slot(opaque(word[s][u])), mv9t(V[s][u], v[s]));
+                }
+        }
+        __syncthreads();
+        if constexpr (FORM != ROWS) {
+            if (rtid < n_ghost) {
+                float g[9];
+#pragma unroll
+                for (int c = 0; c < 9; ++c) g[c] = S.ghost[c][rtid];
+                lds_st(S.prod, gslot, mv9t(g, lds_ld(S.p, gsrc)));
             }
-        __syncthreads();
-        if (rtid < n_ghost) {
-            float g[9];
-#pragma unroll
-            for (int c = 0; c < 9; ++c) g[c] = S.ghost[c][rtid];
-            lds_st(&S.prod[gword >> 16], mv9t(g, lds_ld(&S.p[gword & 0xffffu])));
         }
-        if (GEN && on[0]) {
-            f3 src[kHeld];
+        if constexpr (FORM == GENERAL) {
+            if (on[0]) {
+                f3 src[kHeld];
 #pragma unroll
-            for (int u = 0; u < kHeld; ++u) src[u] = lds_ld(&S.p[F::src(opaque(word[0][u]))]);
+                for (int u = 0; u < kHeld; ++u) src[u] = lds_ld(S.p, F::src(opaque(word[0][u])));
 #pragma unroll
-            for (int u = 0; u < kHeld; ++u)
-                if (unsigned(u) < opaque(holds[0]))
-                    lds_st(&S.prod[(opaque(word[0][u]) >> 24) * kPart + lp[0]], mv9(V[0][u], src[u]));
+                for (int u = 0; u < kHeld; ++u)
+                    if (unsigned(u) < opaque(holds[0]))
+                        lds_st(S.prod, 3u * (F::place(opaque(word[0][u])) * kPart + lp[0]), mv9(V[0][u], src[u]));
+            }
         }
-        __syncthreads();
+        if constexpr (FORM != ROWS) __syncthreads();
 #pragma unroll
         for (int s = 0; s < kSlots; ++s)
             if (on[s]) {
-                float d[6];
+                f3 src[kHeld], low[kHeld];
+                float d[9];
+                if constexpr (FORM != GENERAL) {
 #pragma unroll
-                for (int c = 0; c < 6; ++c) d[c] = S.diag[c][lp[s]];
-                if (GEN) {
-                    f3 sum = mv_sym(d, v[s]);
+                    for (int u = 0; u < kHeld; ++u) src[u] = lds_ld(S.p, F::src(opaque(word[s][u])));
+                }
+#pragma unroll
+                for (int c = 0; c < kDiag; ++c) d[kDiag == 9 ? unsigned(c) : sym6_pos(unsigned(c))] = S.diag[c][lp[s]];
+                if constexpr (kDiag == 6) {
+                    d[3] = d[1];
+                    d[6] = d[2];
+                    d[7] = d[5];
+                }
+                f3 sum;
+                if constexpr (FORM == SHEET) {
+#pragma unroll
+                    for (int l = 0; l < kHeld; ++l) low[l] = lds_ld(S.prod, 3u * (unsigned(l) * kPart + lp[s]));
+                    sum = mv9(d, v[s]);
+#pragma unroll
+                    for (int l = 0; l < kHeld; ++l) sum = add(sum, low[l]);
+#pragma unroll
+                    for (int u = 0; u < kHeld; ++u) sum = add(sum, mv9(V[s][u], src[u]));
+                } else if constexpr (FORM == GENERAL) {
+                    sum = mv9(d, v[s]);
 #pragma unroll
                     for (unsigned t = 0; t < F::kPlaces; t += 4)
                         if (t < widest) {
                             f3 y[4];
 #pragma unroll
-                            for (unsigned u = 0; u < 4; ++u) y[u] = lds_ld(&S.prod[(t + u) * kPart + lp[s]]);
+                            for (unsigned u = 0; u < 4; ++u) y[u] = lds_ld(S.prod, 3u * ((t + u) * kPart + lp[s]));
 #pragma unroll
                             for (unsigned u = 0; u < 4; ++u) sum = add(sum, y[u]);
                         }
-                    out[s] = sum;
                 } else {
-                    f3 low[kHeld], src[kHeld];
+                    // the order of spmv_core<8>: lane l's diag (l = 0) and
+                    // blocks l, l + 8, then the lanes' butterfly
+                    static_assert(kHeld > 8 && kHeld <= 16, "two rounds of eight");
+                    f3 w[8];
 #pragma unroll
-                    for (int u = 0; u < kHeld; ++u) src[u] = lds_ld(&S.p[F::src(opaque(word[s][u]))]);
+                    for (int l = 0; l < 8; ++l) {
+                        w[l] = mv9(V[s][l], src[l]);
+                        if (l == 0) w[0] = add(mv9(d, v[s]), w[0]);
+                        if (l + 8 < kHeld) w[l] = add(w[l], mv9(V[s][l + 8 < kHeld ? l + 8 : l], src[l + 8 < kHeld ? l + 8 : l]));
+                    }
 #pragma unroll
-                    for (int l = 0; l < kHeld; ++l) low[l] = lds_ld(&S.prod[unsigned(l) * kPart + lp[s]]);
-                    f3 sum = mv_sym(d, v[s]);
+                    for (int m = 4; m > 0; m >>= 1)
 #pragma unroll
-                    for (int l = 0; l < kHeld; ++l) sum = add(sum, low[l]);
-#pragma unroll
-                    for (int u = 0; u < kHeld; ++u) sum = add(sum, mv9(V[s][u], src[u]));
-                    out[s] = sum;
+                        for (int l = 0; l < m; ++l) w[l] = add(w[l], w[l + m]);
+                    sum = w[0];
                 }
+                out[s] = sum;
             }
     };
-    // Sums of phase t: per leaf, then over the part's leaves, sent to the gang.
-    auto send_sums = [&](int t, double (&acc)[kSlots][kSums]) {
-        const double none[kSums] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        if constexpr (kSlots == 2) leaf_sums(acc[0], acc[1], S.leaf, wave, lane);
-        else leaf_sums(acc[0], none, S.leaf, wave, lane);
+    // The sums of exchange t: per leaf, then over the part's leaves, sent to
+    // the gang.
+    auto send_sums = [&](int t, auto& acc) {
+        constexpr int N = int(sizeof(acc[0]) / sizeof(double));
+        double none[N] = {};
+        leaf_sums(acc[0], kSlots == 2 ? acc[kSlots - 1] : none, S.leaf, wave, lane);
         __syncthreads();
-        if (tid < 8 * kSums) {
+        if (tid < 8u * N) {
             const unsigned v = tid >> 3, i = tid & 7u;
             double w = S.leaf[2 * i][v] + S.leaf[2 * i + 1][v];
-            w += __shfl_xor(w, 1);
-            w += __shfl_xor(w, 2);
-            w += __shfl_xor(w, 4);
+            w += dpp64<kXor1>(w);
+            w += dpp64<kXor2>(w);
+            w += dpp64<kHalfMirror>(w);
             if (i == 0) {
                 if (parts == 1) {
                     S.tot[v] = w;
@@ -456,12 +571,12 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             }
         }
     };
-    // The instance's sums of phase t into S.tot: a tree over the parts, read
-    // by everyone up to 64 parts; above, the first part of every 16 sums them
-    // up and sends the result to kCopies places, each read by some of the
-    // parts (256 readers of 256 parts' words took 20 us a phase).
-    auto take_sums = [&](int t) -> bool {
-        if (parts > 1 && wave < kSums) {
+    // The instance's N sums of exchange t into S.tot: a tree over the parts,
+    // read by everyone up to 64 parts; above, the first part of every 16 sums
+    // them up and sends the result to kCopies places, each read by some of
+    // the parts (256 readers of 256 parts' words took 20 us an exchange).
+    auto take_sums = [&](int t, unsigned N) -> bool {
+        if (parts > 1 && wave < N) {
             auto fetch = [&](const u64* at, bool mine, double& w) {
                 unsigned b[2];
                 w = 0.0;
@@ -470,18 +585,25 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                 w = __longlong_as_double((long long)((u64(b[1]) << 32) | b[0]));
                 return true;
             };
+            auto tree16 = [](double w) {
+                w += dpp64<kXor1>(w);
+                w += dpp64<kXor2>(w);
+                w += dpp64<kHalfMirror>(w);
+                return w + dpp64<kRor8>(w);
+            };
             double w;
             bool ok = true;
             if (parts <= unsigned(kWave)) {
                 ok = fetch(sum_words(t, wave, lane), lane < parts, w);
-#pragma unroll
-                for (int m = 1; m < kWave; m <<= 1) w += __shfl_xor(w, m);
+                w = tree16(w);
+                if (parts > 16u) {
+                    w = fold16(w, w);
+                    w = fold32(w, w);
+                }
             } else {
                 if ((unsigned(part) % kFan) == 0u) {
                     ok = fetch(sum_words(t, wave, unsigned(part) + lane), lane < kFan && unsigned(part) + lane < parts, w);
-#pragma unroll
-                    for (unsigned m = 1; m < kFan; m <<= 1) w += __shfl_xor(w, int(m));
-                    w = __shfl(w, 0);
+                    w = __shfl(tree16(w), 0);
                     const u64 b = u64(__double_as_longlong(w));
                     if (ok && lane < 2u * kCopies)
                         st64(group_words(t, lane >> 1, wave, unsigned(part) / kFan) + (lane & 1u),
@@ -489,8 +611,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                 }
                 ok = __ballot(!ok) == 0ull &&
                      fetch(group_words(t, unsigned(part) % kCopies, wave, lane), lane < (parts + kFan - 1u) / kFan, w);
-#pragma unroll
-                for (unsigned m = 1; m < kFan; m <<= 1) w += __shfl_xor(w, int(m));
+                w = tree16(w);
             }
             if (lane == 0) S.tot[wave] = w;
             if (!ok) S.bad = 1;
@@ -498,105 +619,242 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         __syncthreads();
         return S.bad == 0;
     };
-
-    // ---- set-up: r_0 = b - A x, z_0 = p_0 = M^-1 r_0 ----
-    apply(p, q);
-    {
-    double acc[kSlots][kSums];
-#pragma unroll
-    for (int s = 0; s < kSlots; ++s) {
-#pragma unroll
-        for (int v = 0; v < kSums; ++v) acc[s][v] = 0.0;
-        if (on[s] && live[s]) {
-            const f3 b = ld3g(I.rhs, ldx(plan, rows_at + pos0 + lp[s]));
-            r[s] = sub(b, q[s]);
-            p[s] = mv_sym(M[s], r[s]);
-            if (ex[s] != CHX_RES_NONE) send_row(0, ex[s], r[s]);
-            acc[s][0] = dot64(r[s], p[s]);
-            acc[s][1] = dot64(b, b);
-            acc[s][4] = dot64(r[s], r[s]);
-        }
-    }
-    send_sums(0, acc);
-    }
-    double bb = 0.0;
-    for (int k = 0;; ++k) {
-        const bool last = k > 0 && k >= I.max_iter;  // at the cap: the last update only
-        // The halo rows' q_{k-1} (set-up: r_0), sent before the sums: waiting
-        // for them first hides their way behind the sums'.
+    // The halo row's triple of exchange t (sent before its sums: waiting for
+    // it first hides its way behind the sums').
+    auto take_halo = [&](int t) {
         f3 h = mk(0.f, 0.f, 0.f);
-        if (rtid < n_halo && !last) {
+        if (rtid < n_halo) {
             unsigned w[3];
-            if (await<3>(row_words(k, hex), tag_of(k), w, bar))
+            if (await<3>(row_words(t, hex), tag_of(t), w, bar))
                 h = mk(__uint_as_float(w[0]), __uint_as_float(w[1]), __uint_as_float(w[2]));
             else
                 S.bad = 1;
         }
-        if (!take_sums(k)) return false;
-        const double rho = S.tot[0], sig = S.tot[1], del = S.tot[2], gam = S.tot[3], rr = S.tot[4];
-        if (k == 0) bb = sig;
+        return h;
+    };
+    auto mark_trace = [&] {
         if (B.trace != nullptr) {
             trace_point(B, trace_e, unsigned(B.n_instances) - unsigned(ld64(&B.xbuf[RES_DONE])));
             ++trace_e;
         }
-        const int its = k > 0 ? k - 1 : 0;  // updates of x so far
-        if (its >= I.max_iter || (I.tol > 0.0 && rr <= I.tol * I.tol * bb)) {
-            if (part == 0 && tid == 0) {
-                B.inst_iters[inst] = its;
-                B.inst_rr[inst] = rr;
-                B.inst_bb[inst] = bb;
-                if (B.inst_rho != nullptr) B.inst_rho[inst] = rho;
-                (void)__hip_atomic_fetch_add(&B.xbuf[RES_DONE], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            break;
+    };
+    auto stop = [&](int its, double rr, double bb, double rho) {
+        if (part == 0 && tid == 0) {
+            B.inst_iters[inst] = its;
+            B.inst_rr[inst] = rr;
+            B.inst_bb[inst] = bb;
+            if (B.inst_rho != nullptr) B.inst_rho[inst] = rho;
+            (void)__hip_atomic_fetch_add(&B.xbuf[RES_DONE], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
+    };
+    auto alive = [&](int k) {
         if (part == 0 && tid == 0 && (k & 7) == 0)
             (void)__hip_atomic_fetch_add(&B.xbuf[RES_PROGRESS], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        float alpha = 0.0f, beta = 0.0f;
-        if (k > 0) merged_scalars(rho, sig, del, gam, alpha, beta);
-        // halo rows: r_k, z_k, p_k as their owners form them
-        if (rtid < n_halo && !last) {
-            if (k == 0) {
-                hr = h;
-                lds_st(&S.p[kPart + rtid], mv_sym(hM, hr));
-            } else {
-                hr = axpy(-alpha, h, hr);
-                lds_st(&S.p[kPart + rtid], axpy(beta, lds_ld(&S.p[kPart + rtid]), mv_sym(hM, hr)));
-            }
-        }
-#pragma unroll
-        for (int s = 0; s < kSlots; ++s)
-            if (on[s]) {
-                if (k > 0) {
-                    r[s] = axpy(-alpha, q[s], r[s]);
-                    S.x[lp[s]] = axpy(alpha, p[s], S.x[lp[s]]);
-                    p[s] = axpy(beta, p[s], mv_sym(M[s], r[s]));
-                }
-                S.p[lp[s]] = p[s];
-            }
-        if (!last) apply(p, q);
-        double acc[kSlots][kSums];
+    };
+    // r = b - A x (A x in q) and its sums; the exported rows of r are sent.
+    auto residual = [&](int t) {
+        double acc[kSlots][3];  // rho, ||b||^2, ||r||^2
 #pragma unroll
         for (int s = 0; s < kSlots; ++s) {
-#pragma unroll
-            for (int v = 0; v < kSums; ++v) acc[s][v] = 0.0;
+            acc[s][0] = acc[s][1] = acc[s][2] = 0.0;
             if (on[s] && live[s]) {
-                if (!last && ex[s] != CHX_RES_NONE) send_row(k + 1, ex[s], q[s]);
-                const f3 z = mv_sym(M[s], r[s]);
-                acc[s][0] = dot64(r[s], z);
-                acc[s][4] = dot64(r[s], r[s]);
-                if (!last) {
-                    acc[s][1] = dot64(p[s], q[s]);
-                    acc[s][2] = dot64(q[s], z);
-                    acc[s][3] = dot64(q[s], mv_sym(M[s], q[s]));
-                }
+                const f3 b = ld3g(I.rhs, ldx(plan, rows_at + pos0 + lp[s]));
+                r[s] = sub(b, q[s]);
+                if (ex[s] != CHX_RES_NONE) send_row(t, ex[s], r[s]);
+                acc[s][0] = dot64(r[s], apply_minv(M[s], r[s]));
+                acc[s][1] = dot64(b, b);
+                acc[s][2] = dot64(r[s], r[s]);
             }
         }
-        send_sums(k + 1, acc);
+        send_sums(t, acc);
+    };
+
+    if constexpr (!TWO) {
+        // ---- set-up: r_0 = b - A x, z_0 = p_0 = M^-1 r_0 ----
+        apply(p, q);
+        residual(0);
+        hr = take_halo(0);
+        if (!take_sums(0, 3)) return false;
+        double rho = S.tot[0], rr = S.tot[2];
+        const double bb = S.tot[1];
+        mark_trace();
+        double sig = 0.0, del = 0.0, gam = 0.0;
+        for (int k = 0;; ++k) {
+            const bool last = k > 0 && k >= I.max_iter;  // at the cap: the last update only
+            f3 h = mk(0.f, 0.f, 0.f);
+            if (k > 0) {
+                if (!last) h = take_halo(k);
+                if (!take_sums(k, 5)) return false;
+                rho = S.tot[0];
+                sig = S.tot[1];
+                del = S.tot[2];
+                gam = S.tot[3];
+                rr = S.tot[4];
+                mark_trace();
+            }
+            const int its = k > 0 ? k - 1 : 0;  // updates of x so far
+            if (its >= I.max_iter || (I.tol > 0.0 && rr <= I.tol * I.tol * bb)) {
+                stop(its, rr, bb, rho);
+                break;
+            }
+            alive(k);
+            float alpha = 0.0f, beta = 0.0f;
+            if (k > 0) merged_scalars(rho, sig, del, gam, alpha, beta);
+            // halo rows: r_k, z_k, p_k as their owners form them
+            if (rtid < n_halo && !last) {
+                if (k > 0) {
+                    hr = axpy(-alpha, h, hr);
+                    lds_st(S.p, hslot, axpy(beta, lds_ld(S.p, hslot), apply_minv(hM, hr)));
+                } else {
+                    lds_st(S.p, hslot, apply_minv(hM, hr));
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < kSlots; ++s)
+                if (on[s]) {
+                    if (k > 0) {
+                        r[s] = axpy(-alpha, q[s], r[s]);
+                        lds_st(S.x, 3u * lp[s], axpy(alpha, p[s], lds_ld(S.x, 3u * lp[s])));
+                        p[s] = axpy(beta, p[s], apply_minv(M[s], r[s]));
+                    } else {
+                        p[s] = apply_minv(M[s], r[s]);
+                    }
+                    lds_st(S.p, 3u * lp[s], p[s]);
+                }
+            if (!last) apply(p, q);
+            double acc[kSlots][5];
+#pragma unroll
+            for (int s = 0; s < kSlots; ++s) {
+#pragma unroll
+                for (int v = 0; v < 5; ++v) acc[s][v] = 0.0;
+                if (on[s] && live[s]) {
+                    if (!last && ex[s] != CHX_RES_NONE) send_row(k + 1, ex[s], q[s]);
+                    const f3 z = apply_minv(M[s], r[s]);
+                    acc[s][0] = dot64(r[s], z);
+                    acc[s][4] = dot64(r[s], r[s]);
+                    if (!last) {
+                        acc[s][1] = dot64(p[s], q[s]);
+                        acc[s][2] = dot64(q[s], z);
+                        acc[s][3] = dot64(q[s], apply_minv(M[s], q[s]));
+                    }
+                }
+            }
+            send_sums(k + 1, acc);
+        }
+    } else {
+        // With B.bf16_blocks the inner iterations run on the BF16 matrix and
+        // test the recursive residual; when it meets the tolerance one slot
+        // computes the true residual with the FP32 blocks: the solve stops on
+        // that, or CG restarts from it (pcg_kernel, instance_slot).
+        const bool half = FORM != ROWS && B.bf16_blocks != 0;
+        constexpr int kMaxRefine = 1;
+        double rho = 0.0, rr = 0.0, bb = 0.0;
+        float beta = 0.0f;
+        bool residual_step = true;        // set-up, then refinement: r = b - A x, x in p and S.p
+        bool exact = true, fresh = true;  // rr is of b - A x; p starts from z
+        int k = 0, refines = -1, t = -1;  // t: the last exchange
+        int blocks = -1;                  // which matrix V holds
+        for (;;) {
+            if (!residual_step) {
+                const bool met = I.tol > 0.0 && rr <= I.tol * I.tol * bb;
+                if (k >= I.max_iter || (met && (!half || exact || refines >= kMaxRefine))) {
+                    stop(k, rr, bb, rho);
+                    break;
+                }
+                alive(k);
+                if (met) {
+                    // this slot computes the true residual: halo rows of x first
+                    residual_step = true;
+                    ++k;
+                    ++t;
+                    double zero[kSlots][1] = {};
+#pragma unroll
+                    for (int s = 0; s < kSlots; ++s)
+                        if (on[s]) {
+                            p[s] = lds_ld(S.x, 3u * lp[s]);
+                            if (live[s] && ex[s] != CHX_RES_NONE) send_row(t, ex[s], p[s]);
+                        }
+                    send_sums(t, zero);
+                    const f3 hx = take_halo(t);
+                    if (!take_sums(t, 1)) return false;
+                    if (rtid < n_halo) lds_st(S.p, hslot, hx);
+                } else {
+                    if (rtid < n_halo) {
+                        const f3 z = apply_minv(hM, hr);
+                        lds_st(S.p, hslot, fresh ? z : axpy(beta, lds_ld(S.p, hslot), z));
+                    }
+#pragma unroll
+                    for (int s = 0; s < kSlots; ++s)
+                        if (on[s]) {
+                            const f3 z = apply_minv(M[s], r[s]);
+                            p[s] = fresh ? z : axpy(beta, p[s], z);
+                        }
+                }
+#pragma unroll
+                for (int s = 0; s < kSlots; ++s)
+                    if (on[s]) lds_st(S.p, 3u * lp[s], p[s]);
+            }
+            const int want = half && !residual_step ? 1 : 0;
+            if (want != blocks) {
+                load_blocks(want != 0);
+                blocks = want;
+            }
+            apply(p, q);
+            if (residual_step) {
+                ++t;
+                residual(t);
+                hr = take_halo(t);
+                if (!take_sums(t, 3)) return false;
+                rho = S.tot[0];
+                bb = S.tot[1];
+                rr = S.tot[2];
+                residual_step = false;
+                exact = fresh = true;
+                ++refines;
+                mark_trace();
+                continue;
+            }
+            ++t;
+            double sum[kSlots][1];
+#pragma unroll
+            for (int s = 0; s < kSlots; ++s) {
+                sum[s][0] = 0.0;
+                if (on[s] && live[s]) {
+                    if (ex[s] != CHX_RES_NONE) send_row(t, ex[s], q[s]);
+                    sum[s][0] = dot64(p[s], q[s]);
+                }
+            }
+            send_sums(t, sum);
+            const f3 h = take_halo(t);
+            if (!take_sums(t, 1)) return false;
+            const float alpha = guarded_div(rho, S.tot[0]);
+            mark_trace();
+            if (rtid < n_halo) hr = axpy(-alpha, h, hr);
+            ++t;
+            double acc[kSlots][2];
+#pragma unroll
+            for (int s = 0; s < kSlots; ++s) {
+                acc[s][0] = acc[s][1] = 0.0;
+                if (on[s] && live[s]) {
+                    lds_st(S.x, 3u * lp[s], axpy(alpha, p[s], lds_ld(S.x, 3u * lp[s])));
+                    r[s] = axpy(-alpha, q[s], r[s]);
+                    acc[s][0] = dot64(r[s], apply_minv(M[s], r[s]));
+                    acc[s][1] = dot64(r[s], r[s]);
+                }
+            }
+            send_sums(t, acc);
+            if (!take_sums(t, 2)) return false;
+            beta = guarded_div(S.tot[0], rho);
+            rho = S.tot[0];
+            rr = S.tot[1];
+            exact = fresh = false;
+            mark_trace();
+            ++k;
+        }
     }
 #pragma unroll
     for (int s = 0; s < kSlots; ++s)
-        if (live[s]) st3g(I.x, ldx(plan, rows_at + pos0 + lp[s]), S.x[lp[s]]);
+        if (live[s]) st3g(I.x, ldx(plan, rows_at + pos0 + lp[s]), lds_ld(S.x, 3u * lp[s]));
     return true;
 }
 
@@ -674,9 +932,9 @@ __device__ unsigned next_item(const chx_cloth_batch& B, unsigned group, unsigned
     return out;
 }
 
-template <bool GEN>
+template <int FORM, bool TWO>
 __global__ __launch_bounds__(kThreads, 2) void resident_kernel(chx_cloth_batch B, int finalize) {
-    __shared__ ResLds<GEN> S;
+    __shared__ ResLds<FORM, TWO> S;
     const int G = int(gridDim.x);
     const Barrier bar = make_barrier(B);
     unsigned* const progress = reinterpret_cast<unsigned*>(&B.xbuf[RES_PROGRESS]);
@@ -724,7 +982,7 @@ __global__ __launch_bounds__(kThreads, 2) void resident_kernel(chx_cloth_batch B
             part = int(__builtin_amdgcn_readfirstlane(had & 255u));
         }
         const Inst I = inst_at(B, inst);
-        ok = solve_part<GEN>(B, I, inst, part, epoch, S, bar, trace_e);
+        ok = solve_part<FORM, TWO>(B, I, inst, part, epoch, S, bar, trace_e);
         if (!ok) break;
     }
     // pos and vel change only when every instance was solved
@@ -734,7 +992,15 @@ __global__ __launch_bounds__(kThreads, 2) void resident_kernel(chx_cloth_batch B
 }
 
 using ResFn = void (*)(chx_cloth_batch, int);
-ResFn resident_fn(bool general) { return general ? resident_kernel<true> : resident_kernel<false>; }
+// form: a plan's; two: the two-reduction solver (always for a caller's rows)
+ResFn resident_fn(int form, bool two) {
+    if (form == ROWS) return resident_kernel<ROWS, true>;
+    // the BF16 mode's plans are general ones: at 1024 rows its kernel would
+    // spill 430 registers
+    if (form == GENERAL) return two ? resident_kernel<GENERAL, true> : resident_kernel<GENERAL, false>;
+    return resident_kernel<SHEET, false>;
+}
+ResFn resident_fn(const chx_cloth_batch& B) { return resident_fn(B.res_form, B.bf16_blocks != 0); }
 
 std::mutex g_mu;
 int g_limit[16] = {0};
@@ -750,13 +1016,14 @@ int resident_grid_limit() {
         hipDeviceProp_t prop;
         hip_check(hipGetDeviceProperties(&prop, dev), "hipGetDeviceProperties");
         bool fits = true;
-        for (bool general : {false, true}) {
-            int per_cu = 0;
-            hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                          &per_cu, reinterpret_cast<const void*>(resident_fn(general)), kThreads, 0),
-                      "hipOccupancyMaxActiveBlocksPerMultiprocessor");
-            fits = fits && per_cu >= 1;
-        }
+        for (int form : {SHEET, GENERAL, ROWS})
+            for (bool two : {false, true}) {
+                int per_cu = 0;
+                hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                              &per_cu, reinterpret_cast<const void*>(resident_fn(form, two)), kThreads, 0),
+                          "hipOccupancyMaxActiveBlocksPerMultiprocessor");
+                fits = fits && per_cu >= 1;
+            }
         l = fits ? std::min(kMaxParts, prop.multiProcessorCount) : -1;
     }
     return std::max(l, 0);
@@ -766,14 +1033,14 @@ void launch_resident(const chx_cloth_batch& B, int finalize, hipStream_t stream)
     if (B.res_grid == 1) {
         // nothing waits for another workgroup: an ordinary launch, without the
         // ~11 us before and after that a cooperative one takes
-        resident_fn(B.res_general != 0)<<<1, kThreads, 0, stream>>>(B, finalize);
+        resident_fn(B)<<<1, kThreads, 0, stream>>>(B, finalize);
         hip_check(hipGetLastError(), "resident_kernel launch");
         return;
     }
     chx_cloth_batch arg = B;
     int fin = finalize;
     void* args[] = {&arg, &fin};
-    hip_check(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(resident_fn(B.res_general != 0)),
+    hip_check(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(resident_fn(B)),
                                          dim3(B.res_grid), dim3(kThreads), args, 0, stream),
               "hipLaunchCooperativeKernel(resident pcg)");
 }

@@ -1800,10 +1800,14 @@ int pcg_variant(const chx_cloth_batch& B, bool row_major) {
     return (B.bf16_blocks != 0 ? 2 : 1) + (B.entries16 != 0 ? 2 : 0);
 }
 
-// Whether the resident kernel takes the launch: FP32 cloth instances that
-// all have a plan, in the default solver form.
+// Whether the resident kernel takes the launch: instances that all have a
+// plan, in the default solver form (BF16 mode: general plans), or a caller's
+// rows with one.
 bool resident(const chx_cloth_batch& B, bool row_major) {
-    return !row_major && B.res_grid > 0 && B.bf16_blocks == 0 && B.pcg_form == 0 && B.no_lds_staging == 0;
+    if (B.res_grid <= 0) return false;
+    if (row_major) return B.res_form == 2;
+    if (B.bf16_blocks != 0) return B.res_form == 1 && B.no_lds_staging == 0;
+    return B.res_form <= 1 && B.pcg_form == 0 && B.no_lds_staging == 0;
 }
 
 void launch_pcg(const chx_cloth_batch& B, int finalize, hipStream_t stream, bool row_major = false) {
@@ -1878,8 +1882,8 @@ void validate_batch(const chx_cloth_batch* b) {
                          (I.res_part_rows == 256 || I.res_part_rows == 512 || I.res_part_rows == CHX_RES_PART_MAX) &&
                          I.res_parts == (I.n_rows + I.res_part_rows - 1) / I.res_part_rows &&
                          I.res_parts <= b->res_grid && I.res_exports >= 0 &&
-                         (I.res_general != 0) == (b->res_general != 0) &&
-                         (b->res_general == 0 || I.res_part_rows <= CHX_RES_GEN_PART) &&
+                         (I.res_form != 0) == (b->res_form != 0) &&
+                         (b->res_form == 0 || I.res_part_rows <= CHX_RES_GEN_PART) &&
                          I.res_xbase + CHX_RES_XWORDS(I.res_parts, I.res_exports) <= b->res_xwords),
                     "chysx: resident plan does not match its instance");
         } else {
@@ -2079,7 +2083,8 @@ void* scratch_address() {
 void solve_bsr3(int n_rows, const float* diag, const int* row_offsets, const int* col_indices, const float* values,
                 const float* b, float* x, int max_iterations, double tol, int lanes_per_row, void* workspace,
                 size_t workspace_bytes, const chx_contact_op* op, void* contact_workspace,
-                size_t contact_workspace_bytes, int* iterations, double* rr, double* bb, uintptr_t stream) {
+                size_t contact_workspace_bytes, int* iterations, double* rr, double* bb, uintptr_t stream,
+                const chx_rows_plan* plan = nullptr) {
     {
         require(n_rows >= 0, "pcg: negative row count");
         require(max_iterations >= 0, "pcg: negative iteration cap");
@@ -2115,10 +2120,30 @@ void solve_bsr3(int n_rows, const float* diag, const int* row_offsets, const int
             B.contact_rows = ix.rows;
             B.contact_entries = ix.entries;
         }
+        // the resident solve sums a row in the order of eight lanes
+        if (plan != nullptr && plan->plan != nullptr && lanes_per_row == 8 && B.contact_rows == nullptr) {
+            const int limit = resident_grid_limit();
+            require((plan->part_rows == 256 || plan->part_rows == CHX_RES_GEN_PART) &&
+                        plan->parts == (n_rows + plan->part_rows - 1) / plan->part_rows && plan->exports >= 0 &&
+                        plan->xbuf != nullptr &&
+                        plan->xwords >= CHX_RES_CONTROL_WORDS + CHX_RES_XWORDS(plan->parts, plan->exports),
+                    "pcg: resident plan does not match the matrix");
+            if (plan->parts <= limit) {
+                B.single.res_plan = plan->plan;
+                B.single.res_part_rows = plan->part_rows;
+                B.single.res_parts = plan->parts;
+                B.single.res_exports = plan->exports;
+                B.single.res_form = B.res_form = 2;
+                B.single.res_xbase = CHX_RES_CONTROL_WORDS;
+                B.xbuf = plan->xbuf;
+                B.res_xwords = plan->xwords;
+                B.res_grid = single_grid(plan->parts, limit, &B.res_groups);
+            }
+        }
         // The workspace needs no initialisation: every control word is
         // cleared, status included (an earlier solve's abort is reported by
         // its own synchronous read or chx_pcg_last_stats before this call).
-        reset_sync_kernel<<<1, kBlock, 0, s>>>(B.sync, 1, nullptr);
+        reset_sync_kernel<<<1, kBlock, 0, s>>>(B.sync, 1, B.xbuf);
         hip_check(hipGetLastError(), "reset_sync_kernel launch");
         launch_pcg(B, 0, s, true);
         if (iterations || rr || bb) read_workspace_stats(B, iterations, rr, bb, nullptr, s);
@@ -2152,6 +2177,23 @@ int chx_pcg_solve_bsr3(int n_rows, const float* diag, const int* row_offsets, co
     return guarded([&] {
         solve_bsr3(n_rows, diag, row_offsets, col_indices, values, b, x, max_iterations, tol, lanes_per_row,
                    workspace, workspace_bytes, nullptr, nullptr, 0, iterations, rr, bb, stream);
+    });
+}
+
+int chx_pcg_solve_bsr3_plan(int n_rows, const float* diag, const int* row_offsets, const int* col_indices,
+                            const float* values, const float* b, float* x, int max_iterations, double tol,
+                            int lanes_per_row, void* workspace, size_t workspace_bytes, const chx_rows_plan* plan,
+                            int* iterations, double* rr, double* bb, uintptr_t stream) {
+    return guarded([&] {
+        solve_bsr3(n_rows, diag, row_offsets, col_indices, values, b, x, max_iterations, tol, lanes_per_row,
+                   workspace, workspace_bytes, nullptr, nullptr, 0, iterations, rr, bb, stream, plan);
+    });
+}
+
+int chx_resident_grid(int parts, int limit, int* grid, int* groups) {
+    return guarded([&] {
+        require(grid != nullptr && groups != nullptr && parts > 0, "chx_resident_grid: bad argument");
+        *grid = single_grid(parts, limit, groups);
     });
 }
 

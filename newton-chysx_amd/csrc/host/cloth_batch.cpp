@@ -33,8 +33,10 @@ std::vector<chx_instance> ClothBatch::descriptors(float dt, std::uintptr_t cuda_
     for (ClothSimulator* s : sims_) rows.push_back(s->buffers().particle_count());
     std::vector<chx_instance> ds;
     // the resident solve wants all plans in one form: sheets, or else general
+    // (the BF16 solve: general)
     for (bool general : {false, true}) {
-        const int part_rows = engine::resident_part_rows(rows, general);
+        if (bf16_ && !general) continue;
+        const int part_rows = engine::resident_part_rows(rows, general ? CHX_RES_GEN_PART : CHX_RES_PART_MAX);
         ds.clear();
         ds.reserve(sims_.size());
         bool all = true;
@@ -45,7 +47,7 @@ std::vector<chx_instance> ClothBatch::descriptors(float dt, std::uintptr_t cuda_
                     "ClothBatch: BF16 mode needs every instance switched with set_bf16_blocks(true)");
             all = all && ds.back().res_plan != nullptr;
         }
-        if (all || bf16_) break;
+        if (all) break;
     }
     return ds;
 }

@@ -352,9 +352,13 @@ void ClothSimulator::step(float dt, std::uintptr_t cuda_stream) {
 // The descriptor of the simulator's own (single-instance) launches.
 chx_instance ClothSimulator::single_descriptor(const engine::InstanceSource& s, std::uintptr_t stream) {
     chx_instance d = inst_.descriptor(s);
+    // the BF16 solve takes general plans only
     for (bool general : {false, true})
-        if (!bf16_ && d.res_plan == nullptr)
-            inst_.attach_plan(d, pattern_, engine::resident_part_rows({s.n}, general), general, stream);
+        if (general || !bf16_) {
+            const int most = general ? CHX_RES_GEN_PART : CHX_RES_PART_MAX;
+            inst_.attach_plan(d, pattern_, engine::resident_part_rows({s.n}, most), general, stream);
+            if (d.res_plan != nullptr) break;
+        }
     return d;
 }
 
@@ -371,7 +375,7 @@ chx_instance ClothSimulator::prepare_instance(float dt, std::uintptr_t cuda_stre
     engine::InstanceSource s = source();
     s.dt = dt;
     chx_instance d = inst_.descriptor(s);
-    if (!bf16_) inst_.attach_plan(d, pattern_, part_rows, general, cuda_stream);
+    inst_.attach_plan(d, pattern_, part_rows, general, cuda_stream);
     return d;
 }
 

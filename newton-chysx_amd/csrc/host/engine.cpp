@@ -688,8 +688,7 @@ void InstanceData::attach_plan(chx_instance& d, const topology::Pattern& p, int 
                                std::uintptr_t stream) {
     d.res_plan = nullptr;
     if (part_rows == 0 || n_ == 0) return;
-    // what one workgroup holds needs no exchange: 32x32 rows take 3.3 us an
-    // iteration in one part, 3.3-3.9 in four or two
+    // what one workgroup holds needs no exchange (resident_part_rows)
     const int most = general ? CHX_RES_GEN_PART : CHX_RES_PART_MAX;
     if (n_ <= most) part_rows = most;
     Plan& pl = plans_[(general ? 3 : 0) + (part_rows == 256 ? 0 : (part_rows == 512 ? 1 : 2))];
@@ -712,23 +711,7 @@ void InstanceData::attach_plan(chx_instance& d, const topology::Pattern& p, int 
     d.res_part_rows = part_rows;
     d.res_parts = pl.parts;
     d.res_exports = pl.exports;
-    d.res_general = general ? 1 : 0;
-}
-
-int resident_part_rows(const std::vector<int>& rows, bool general) {
-    constexpr long kWorkgroups = 256;
-    const int largest = general ? CHX_RES_GEN_PART : CHX_RES_PART_MAX;
-    for (int pr = 256; pr <= largest; pr *= 2) {
-        long parts = 0, most = 0;
-        for (int n : rows) {
-            const long q = n <= largest ? 1 : (n + pr - 1) / pr;
-            parts += q;
-            most = std::max(most, q);
-        }
-        if (parts <= kWorkgroups) return pr;
-        if (pr == largest && most <= kWorkgroups) return pr;
-    }
-    return 0;
+    d.res_form = general ? 1 : 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -741,7 +724,7 @@ void BatchRunner::layout_resident(std::vector<chx_instance>& ds, std::uintptr_t 
     int total = 0, most = 0;
     for (const chx_instance& d : ds) {
         if (d.n_rows == 0) continue;
-        if (d.res_plan == nullptr || d.res_general != ds[0].res_general) return;
+        if (d.res_plan == nullptr || d.res_form != ds[0].res_form) return;
         total += d.res_parts;
         most = std::max(most, d.res_parts);
     }
@@ -753,9 +736,7 @@ void BatchRunner::layout_resident(std::vector<chx_instance>& ds, std::uintptr_t 
     // to a group stay in one.
     int grid = 0, groups = 1, per = 0;
     if (ds.size() == 1) {
-        grid = most <= 32 ? most : (most + 7) / 8 * 8;
-        if (grid > cap) grid = most;
-        groups = grid > 32 && grid % 8 == 0 ? 8 : 1;
+        check(chx_resident_grid(most, cap, &grid, &groups), "engine", "resident grid");
     } else if (cap >= 8) {
         per = std::min({cap / 8, 32, std::max((total + 7) / 8, std::min(most, 32))});
         groups = 8;
@@ -810,7 +791,7 @@ void BatchRunner::layout_resident(std::vector<chx_instance>& ds, std::uintptr_t 
     desc_.xbuf = xbuf_.gpu_data();
     desc_.res_xwords = xbuf_.gpu_size();
     desc_.res_groups = groups;
-    desc_.res_general = ds[0].res_general;
+    desc_.res_form = ds[0].res_form;
     desc_.res_grid = grid;
 }
 

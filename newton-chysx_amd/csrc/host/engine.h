@@ -133,11 +133,6 @@ private:
     DeviceArray<chx_box> boxes_;
 };
 
-// Rows per part of the resident solve of cloths with `rows` vertices each:
-// the smallest part size whose parts all run at once on 256 workgroups, else
-// the largest; 0 when some cloth alone has more parts than that.
-int resident_part_rows(const std::vector<int>& rows, bool general);
-
 class BatchRunner {
 public:
     BatchRunner() = default;

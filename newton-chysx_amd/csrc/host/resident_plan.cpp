@@ -161,11 +161,11 @@ struct Builder {
         const auto& ci = p.col_indices;
         // exported rows, numbered part by part in canonical order
         std::vector<std::uint32_t> exp(N, CHX_RES_NONE);
-        for (int k = 0; k < p.n; ++k) {
-            const int i = order[k], q = k / part_rows;
-            for (int c = ro[i]; c < ro[i + 1] && exp[i] == CHX_RES_NONE; ++c)
-                if (pos[ci[c]] / part_rows != q) exp[i] = static_cast<std::uint32_t>(exports++);
-        }
+        for (int k = 0; k < p.n; ++k)
+            for (int c = ro[order[k]]; c < ro[order[k] + 1]; ++c)
+                if (pos[ci[c]] / part_rows != k / part_rows) exp[ci[c]] = 0u;
+        for (int k = 0; k < p.n; ++k)
+            if (exp[order[k]] == 0u) exp[order[k]] = static_cast<std::uint32_t>(exports++);
         std::vector<int> stamp(N, -1), halo;
         for (int q = 0; q < parts; ++q) {
             a = q * part_rows;
@@ -319,6 +319,34 @@ ResidentPlan resident_plan_general(const topology::Pattern& p, const std::vector
         return static_cast<std::uint32_t>((ro[i + 1] - ro[i]) | (u << 8));
     });
     return ok ? B.take() : ResidentPlan{};
+}
+
+ResidentPlan resident_plan_rows(const topology::Pattern& p, const std::vector<int>& order, int part_rows) {
+    if (p.n <= 0 || part_rows > CHX_RES_GEN_PART) return {};
+    const auto& ro = p.row_offsets;
+    for (int i = 0; i < p.n; ++i)
+        if (ro[i + 1] - ro[i] > CHX_RES_ROW_WIDTH) return {};
+    Builder B(p, order, part_rows, CHX_RES_GEN_PART, CHX_RES_ROW_WIDTH);
+    const bool ok = B.build([&](int k, int i) {
+        for (int c = ro[i]; c < ro[i + 1]; ++c) B.plane(c - ro[i], k) = B.local_of(p.col_indices[c]);
+        return static_cast<std::uint32_t>((ro[i + 1] - ro[i]) << 8);
+    });
+    return ok ? B.take() : ResidentPlan{};
+}
+
+int resident_part_rows(const std::vector<int>& rows, int largest) {
+    constexpr long kWorkgroups = 256;
+    for (int pr = 256; pr <= largest; pr *= 2) {
+        long parts = 0, most = 0;
+        for (int n : rows) {
+            const long q = n <= largest ? 1 : (n + pr - 1) / pr;
+            parts += q;
+            most = std::max(most, q);
+        }
+        if (parts <= kWorkgroups) return rows.size() == 1 && rows[0] <= largest ? largest : pr;
+        if (pr == largest && most <= kWorkgroups) return pr;
+    }
+    return 0;
 }
 
 }  // namespace engine

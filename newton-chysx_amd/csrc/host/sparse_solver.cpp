@@ -27,6 +27,16 @@ void BlockCSR3::build_topology(int num_block_rows, const int* host_rows, const i
     diag.ensure_device(num_block_rows);
     values.ensure_device(pattern_.col_indices.size());
     set_zero();
+    plan_ = engine::ResidentPlan{};
+    plan_image_.release();
+    const int part_rows = engine::resident_part_rows({num_block_rows}, CHX_RES_GEN_PART);
+    if (num_block_rows > 0 && part_rows > 0) {
+        plan_ = engine::resident_plan_rows(pattern_, engine::resident_order(pattern_), part_rows);
+        if (!plan_.blob.empty()) {
+            plan_image_.host() = std::move(plan_.blob);
+            plan_image_.copy_to_device();
+        }
+    }
     check(chx_device_synchronize(), "sparse::BlockCSR3", "build_topology");
 }
 
@@ -161,6 +171,16 @@ void PCGSolver::initialize(int num_block_rows) {
     std::size_t bytes = 0;
     check(chx_pcg_workspace_size(num_block_rows, &bytes), "solver::PCGSolver", "workspace size");
     workspace_.ensure_device(bytes);
+    // exchange area for any pattern of that many rows the resident solve takes
+    if (engine::resident_part_rows({num_block_rows}, CHX_RES_GEN_PART) > 0) {
+        const std::size_t n = static_cast<std::size_t>(num_block_rows);
+        const std::size_t words = CHX_RES_CONTROL_WORDS + CHX_RES_XWORDS((n + 255) / 256, n);
+        if (xbuf_.gpu_size() < words) {
+            xbuf_.ensure_device(words);
+            xbuf_.zero_device();
+            check(chx_device_synchronize(), "solver::PCGSolver", "exchange area");
+        }
+    }
     n_ = num_block_rows;
 }
 
@@ -199,11 +219,21 @@ int PCGSolver::solve(const sparse::BlockCSR3& A, DeviceSpan<math::Vec3f> b, Devi
                   cbytes, itp, nullptr, nullptr, cuda_stream),
               "solver::PCGSolver", "solve");
     } else {
-        check(chx_pcg_solve_bsr3(n, reinterpret_cast<const float*>(A.diag.gpu_data()), A.row_offsets.gpu_data(),
-                                 A.col_indices.gpu_data(), reinterpret_cast<const float*>(A.values.gpu_data()),
-                                 reinterpret_cast<const float*>(b.data()), reinterpret_cast<float*>(x.data()),
-                                 params.max_iterations, params.tolerance, params.lanes_per_row, workspace_.gpu_data(),
-                                 workspace_.gpu_size(), itp, nullptr, nullptr, cuda_stream),
+        chx_rows_plan plan{};
+        if (A.plan().parts > 0 && xbuf_.gpu_size() > 0) {
+            plan.plan = A.plan_image().gpu_data();
+            plan.part_rows = A.plan().part_rows;
+            plan.parts = A.plan().parts;
+            plan.exports = A.plan().exports;
+            plan.xbuf = xbuf_.gpu_data();
+            plan.xwords = xbuf_.gpu_size();
+        }
+        check(chx_pcg_solve_bsr3_plan(n, reinterpret_cast<const float*>(A.diag.gpu_data()), A.row_offsets.gpu_data(),
+                                      A.col_indices.gpu_data(), reinterpret_cast<const float*>(A.values.gpu_data()),
+                                      reinterpret_cast<const float*>(b.data()), reinterpret_cast<float*>(x.data()),
+                                      params.max_iterations, params.tolerance, params.lanes_per_row,
+                                      workspace_.gpu_data(), workspace_.gpu_size(), &plan, itp, nullptr, nullptr,
+                                      cuda_stream),
               "solver::PCGSolver", "solve");
     }
     return wait ? it : params.max_iterations;

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "chysx_common.h"
+#include "resident_plan.h"
 #include "topology.h"
 
 namespace chysx {
@@ -37,9 +38,14 @@ public:
         topology::resolve_slots(pattern_, host_rows, host_cols, out_slots, num_pairs);
     }
     const topology::Pattern& pattern() const noexcept { return pattern_; }
+    // Resident-solve plan of the pattern (no parts: none) and its device image.
+    const engine::ResidentPlan& plan() const noexcept { return plan_; }
+    const DeviceArray<std::uint32_t>& plan_image() const noexcept { return plan_image_; }
 
 private:
     topology::Pattern pattern_;
+    engine::ResidentPlan plan_;
+    DeviceArray<std::uint32_t> plan_image_;
 };
 
 // y = alpha * A * x + beta * y (beta == 0: y not read).
@@ -136,6 +142,7 @@ private:
     int n_ = 0;
     DeviceArray<unsigned char> workspace_;
     DeviceArray<unsigned char> contact_workspace_;
+    DeviceArray<unsigned long long> xbuf_;  // exchange area of the resident solve
     std::uintptr_t last_stream_ = 0;
 };
 
