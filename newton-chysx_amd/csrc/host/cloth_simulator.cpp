@@ -345,7 +345,7 @@ void ClothSimulator::step(float dt, std::uintptr_t cuda_stream) {
     }
     engine::InstanceSource s = source();
     s.dt = dt;
-    runner_.update_single(single_descriptor(s, cuda_stream));
+    runner_.update_single(single_descriptor(s, cuda_stream), cuda_stream);
     runner_.step(cuda_stream);
 }
 
@@ -520,7 +520,7 @@ double ClothSimulator::compute_energy(int kind_mask) {
     resize_work_buffers(n);
     if (topology_dirty_ || H_num_block_rows_ != n) ensure_hessian_topology();
     else check_elements_current();
-    runner_.update_single(single_descriptor(source(), 0));
+    runner_.update_single(single_descriptor(source(), 0), 0);
     return runner_.energy(kind_mask, 0);
 }
 

@@ -1037,28 +1037,45 @@ void BatchRunner::bind_many(const std::vector<chx_instance>& ds, std::uintptr_t 
     sync_stream(stream, "bind");
 }
 
+bool BatchRunner::take(chx_instance& was, chx_instance d) {
+    const bool other = (d.res_plan == nullptr) != (was.res_plan == nullptr) || d.res_parts != was.res_parts ||
+                       d.res_part_rows != was.res_part_rows || d.res_exports != was.res_exports ||
+                       d.res_form != was.res_form;
+    d.tile_begin = was.tile_begin;
+    d.tile_end = was.tile_end;
+    d.res_xbase = was.res_xbase;
+    was = d;
+    return other;
+}
+
+void BatchRunner::update_single(const chx_instance& d, std::uintptr_t stream) {
+    desc_.entries16 = (d.n_rows > 0 && d.slice_entries16 == nullptr) ? 0 : 1;
+    if (!take(desc_.single, d)) return;
+    // queued launches may still use the old layout
+    check(chx_stream_synchronize(stream), "engine", "instance update");
+    std::vector<chx_instance> one{desc_.single};
+    layout_resident(one, stream);
+    desc_.single = one[0];
+}
+
 void BatchRunner::update_many(const std::vector<chx_instance>& ds, std::uintptr_t stream) {
     if (ds.size() != table_host_.size()) throw std::invalid_argument("chysx::engine: instance count changed");
     if (desc_.inst == nullptr) {
-        update_single(ds[0]);
+        update_single(ds[0], stream);
         table_host_[0] = desc_.single;
         return;
     }
-    bool changed = false;
+    bool changed = false, relayout = false;
     for (std::size_t i = 0; i < ds.size(); ++i) {
-        chx_instance d = ds[i];
-        d.tile_begin = table_host_[i].tile_begin;
-        d.tile_end = table_host_[i].tile_end;
-        d.res_xbase = table_host_[i].res_xbase;
-        if (std::memcmp(&d, &table_host_[i], sizeof(chx_instance)) != 0) {
-            table_host_[i] = d;
-            changed = true;
-        }
+        const chx_instance was = table_host_[i];
+        relayout = take(table_host_[i], ds[i]) || relayout;
+        changed = changed || std::memcmp(&was, &table_host_[i], sizeof(chx_instance)) != 0;
     }
     desc_.entries16 = entries16_all(table_host_);
     if (changed) {
         // The previous table may still be read by queued launches.
         check(chx_stream_synchronize(stream), "engine", "instance table update");
+        if (relayout) layout_resident(table_host_, stream);
         table_.host() = table_host_;
         table_.copy_to_device(stream);
         desc_.inst = table_.gpu_data();

@@ -147,15 +147,7 @@ public:
     // Many instances: builds the work lists and uploads the table.
     void bind_many(const std::vector<chx_instance>& ds, std::uintptr_t stream = 0);
     // Per-step scalars / external pointers of the bound instances.
-    void update_single(const chx_instance& d) {
-        const int tb = desc_.single.tile_begin, te = desc_.single.tile_end;
-        const unsigned xb = desc_.single.res_xbase;
-        desc_.entries16 = (d.n_rows > 0 && d.slice_entries16 == nullptr) ? 0 : 1;
-        desc_.single = d;
-        desc_.single.tile_begin = tb;
-        desc_.single.tile_end = te;
-        desc_.single.res_xbase = xb;
-    }
+    void update_single(const chx_instance& d, std::uintptr_t stream);
     void update_many(const std::vector<chx_instance>& ds, std::uintptr_t stream);
 
     // Launches one substep.  Raises (after synchronising) when an earlier
@@ -231,6 +223,10 @@ private:
     // instances; leaves the launch to the streaming kernels when one of them
     // has no plan or the grid does not hold its parts.
     void layout_resident(std::vector<chx_instance>& ds, std::uintptr_t stream = 0);
+    // Takes `d` over the bound descriptor `was`, keeping what the bind laid
+    // out; true when its resident plan is another one (a cloth whose pattern
+    // was rebuilt after the bind), so that the layout has to be made again.
+    static bool take(chx_instance& was, chx_instance d);
 
     chx_cloth_batch desc_{};
     void* graph_ = nullptr;           // hipGraphExec_t of one substep
