@@ -113,6 +113,11 @@ __device__ __forceinline__ unsigned opaque(unsigned v) {
     asm volatile("" : "+v"(v));
     return v;
 }
+// The thread index for addresses and masks of one use.  What the loop derives
+// from it is derived again: kept over the loop those values went to scratch,
+// and a reload waits for every store in flight, the halo rows just sent among
+// them (32 spilled registers: 6.8 us an iteration of a 256x256 cloth, 5.8 without).
+__device__ __forceinline__ unsigned tid_here() { return opaque(threadIdx.x); }
 
 template <int FORM, bool FULL>
 struct ResLds {
@@ -140,13 +145,11 @@ struct Watch {
         unsigned* sync = bar.sync;
         if ((++polls & 15u) == 0u && ld_relaxed(&sync[SYNC_ABORT]) != 0u) return false;
         if (__builtin_amdgcn_s_memrealtime() - t0 <= bar.ticks) return true;
-        if (progress != nullptr) {
-            const unsigned now = unsigned(ld64(progress));
-            if (now != seen) {
-                seen = now;
-                t0 = __builtin_amdgcn_s_memrealtime();
-                return true;
-            }
+        const unsigned now = unsigned(ld64(progress));
+        if (now != seen) {
+            seen = now;
+            t0 = __builtin_amdgcn_s_memrealtime();
+            return true;
         }
         st_relaxed(&sync[SYNC_SEEN], 0u);
         st_relaxed(&sync[SYNC_WAITING], 1u);
@@ -160,9 +163,10 @@ struct Watch {
 };
 
 // N tagged words from p on, read until every tag is the awaited one; false:
-// the wait was given up.
+// the wait was given up.  A peer may still be busy with an earlier large item
+// of the list, so the wait goes on as long as any gang iterates.
 template <int N>
-__device__ __forceinline__ bool await(const u64* p, unsigned tag, unsigned (&v)[N], const Barrier& bar) {
+__device__ __forceinline__ bool await(const u64* p, unsigned tag, unsigned (&v)[N], u64* progress, const Barrier& bar) {
     u64 w[N];
     auto read = [&] {
         bool ok = true;
@@ -176,7 +180,7 @@ __device__ __forceinline__ bool await(const u64* p, unsigned tag, unsigned (&v)[
         Watch watch(bar);
         unsigned seen = 0;
         do {
-            if (!watch.again(nullptr, seen)) return false;
+            if (!watch.again(progress, seen)) return false;
         } while (!read());
     }
 #pragma unroll
@@ -244,7 +248,8 @@ __device__ __forceinline__ double fold8(double a, double b, unsigned lane) {
 // each step adds lane pairs and packs two values into the two halves of the
 // pairs, so five values of two leaves take 14 FP64 adds instead of 60.
 __device__ __forceinline__ void leaf_sums(const double (&a)[5], const double (&b)[5], double (&leaf)[kLeaves][kSums],
-                                          unsigned wave, unsigned lane) {
+                                          unsigned wave) {
+    const unsigned lane = tid_here() & unsigned(kWave - 1);
     double v[5];
 #pragma unroll
     for (int k = 0; k < 5; ++k) v[k] = fold32(a[k], b[k]);  // half h: leaf of slot h
@@ -266,8 +271,9 @@ __device__ __forceinline__ void leaf_sums(const double (&a)[5], const double (&b
 // The same for up to three values (the second and third in one row each).
 template <int N>
 __device__ __forceinline__ void leaf_sums(const double (&a)[N], const double (&b)[N], double (&leaf)[kLeaves][kSums],
-                                          unsigned wave, unsigned lane) {
+                                          unsigned wave) {
     static_assert(N >= 1 && N <= 3, "values");
+    const unsigned lane = tid_here() & unsigned(kWave - 1);
     double w = fold16(fold32(a[0], b[0]), N > 1 ? fold32(a[N > 1 ? 1 : 0], b[N > 1 ? 1 : 0]) : 0.0);
     double y = 0.0;
     if constexpr (N == 3) {
@@ -326,13 +332,15 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     };
 
     // ---- load: own rows, ghost block, halo row ----
-    unsigned lp[kSlots], ex[kSlots], holds[kSlots], word[kSlots][kHeld];
-    bool live[kSlots], on[kSlots];  // this lane's row exists; this wave has a row
+    unsigned ex[kSlots], holds[kSlots], word[kSlots][kHeld];
+    bool on[kSlots];  // this wave has a row
+    auto row_at = [&](int s) { return unsigned(s) * kThreads + tid_here(); };  // this lane's row of slot s
+    auto live = [&](int s) { return row_at(s) < n_own; };
     float V[kSlots][kHeld][9], M[kSlots][kMinv];
     f3 r[kSlots], p[kSlots], q[kSlots];
     // ghost blocks and halo rows from the last thread down: in a small part
     // the first waves have the rows
-    const unsigned rtid = unsigned(kThreads - 1) - tid;
+    auto rtid_here = [] { return unsigned(kThreads - 1) - tid_here(); };
     // the matrix blocks: FP32, or the BF16 copies and compensated diagonal
     auto load_blocks = [&](bool half) {
         auto block = [&](unsigned v, float (&m)[9]) {
@@ -350,7 +358,8 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
 #pragma unroll
         for (int s = 0; s < kSlots; ++s)
             if (on[s]) {
-                const unsigned K = pos0 + (live[s] ? lp[s] : 0u);
+                const unsigned lp = row_at(s);
+                const unsigned K = pos0 + (lp < n_own ? lp : 0u);
                 const unsigned row = ldx(plan, rows_at + K);
                 const unsigned first = FORM == ROWS ? unsigned(ldx(I.row_offsets, row))
                                                     : unsigned(ldx(I.upper_offsets, row / CHX_SLICE_ROWS)) +
@@ -376,8 +385,9 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                     ld6p(gp<const float>(I.diag), row, d);
                 }
 #pragma unroll
-                for (unsigned c = 0; c < unsigned(kDiag); ++c) S.diag[c][lp[s]] = d[kDiag == 9 ? c : sym6_pos(c)];
+                for (unsigned c = 0; c < unsigned(kDiag); ++c) S.diag[c][lp] = d[kDiag == 9 ? c : sym6_pos(c)];
             }
+        const unsigned rtid = rtid_here();
         if (FORM != ROWS && rtid < n_ghost) {
             float g[9];
             block(ldx(plan, ghost_at + 2u * rtid), g);
@@ -404,10 +414,9 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     };
 #pragma unroll
     for (int s = 0; s < kSlots; ++s) {
-        lp[s] = (unsigned(s) * kWaves + wave) * kWave + lane;
+        const unsigned lp = row_at(s);
         on[s] = (unsigned(s) * kWaves + wave) * kWave < n_own;
-        live[s] = lp[s] < n_own;
-        const unsigned K = pos0 + (live[s] ? lp[s] : 0u);
+        const unsigned K = pos0 + (lp < n_own ? lp : 0u);
         ex[s] = CHX_RES_NONE;
         holds[s] = 0u;
         r[s] = p[s] = q[s] = mk(0.f, 0.f, 0.f);
@@ -415,7 +424,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             unsigned ns = 0u;
             const unsigned row = ldx(plan, rows_at + K);
             const unsigned meta = ldx(plan, meta_at + K);
-            if (live[s]) {
+            if (lp < n_own) {
                 ns = meta & 255u;
                 holds[s] = meta >> 8;
                 ex[s] = ldx(plan, exp_at + K);
@@ -423,7 +432,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
 #pragma unroll
             for (int u = 0; u < kHeld; ++u) {
                 // a block that is not there is zero, of the row itself
-                unsigned w = FORM == SHEET ? (0xffffu << 16) | lp[s] : (FORM == GENERAL ? (0x3fffu << 10) | lp[s] : lp[s]);
+                unsigned w = FORM == SHEET ? (0xffffu << 16) | lp : (FORM == GENERAL ? (0x3fffu << 10) | lp : lp);
                 if (unsigned(u) < holds[s]) w = ldx(plan, held_at + unsigned(u) * n + K);
                 word[s][u] = F::unpack(w, lane);
             }
@@ -431,29 +440,27 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             // the others
 #pragma unroll
             for (unsigned u = 0; u < F::kPlaces; ++u)
-                if (u >= ns) lds_st(S.prod, 3u * (u * kPart + lp[s]), mk(0.f, 0.f, 0.f));
+                if (u >= ns) lds_st(S.prod, 3u * (u * kPart + lp), mk(0.f, 0.f, 0.f));
             invert(row, M[s]);
-            if (live[s]) p[s] = ld3g(I.x, row);
-            lds_st(S.x, 3u * lp[s], p[s]);
-            lds_st(S.p, 3u * lp[s], p[s]);
+            if (lp < n_own) p[s] = ld3g(I.x, row);
+            lds_st(S.x, 3u * lp, p[s]);
+            lds_st(S.p, 3u * lp, p[s]);
         }
     }
     if constexpr (!TWO) load_blocks(false);
-    unsigned gsrc = 0, gslot = 0;
-    if (FORM != ROWS && rtid < n_ghost) {
-        const unsigned g = ldx(plan, ghost_at + 2u * rtid + 1u);
-        gsrc = 3u * (g & 0xffffu);
-        gslot = 3u * (g >> 16);
-    }
+    unsigned gword = 0;  // the ghost block's source and product slot
+    if (FORM != ROWS && rtid_here() < n_ghost) gword = ldx(plan, ghost_at + 2u * rtid_here() + 1u);
     float hM[kMinv];
     f3 hr = mk(0.f, 0.f, 0.f);
     unsigned hex = 0;
-    const unsigned hslot = 3u * (kPart + rtid);
-    if (rtid < n_halo) {
+    auto halo_slot = [&] { return 3u * (kPart + rtid_here()); };
+    auto is_halo = [&] { return rtid_here() < n_halo; };
+    if (is_halo()) {
+        const unsigned rtid = rtid_here();
         const unsigned hrow = ldx(plan, halo_at + 2u * rtid);
         hex = ldx(plan, halo_at + 2u * rtid + 1u);
         invert(hrow, hM);
-        lds_st(S.p, hslot, ld3g(I.x, hrow));
+        lds_st(S.p, halo_slot(), ld3g(I.x, hrow));
     }
     if (tid == 0) S.bad = 0;
     if (tid < kLeaves * kSums) S.leaf[tid / kSums][tid % kSums] = 0.0;
@@ -471,28 +478,32 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         }
         __syncthreads();
         if constexpr (FORM != ROWS) {
+            const unsigned rtid = rtid_here();
             if (rtid < n_ghost) {
                 float g[9];
 #pragma unroll
                 for (int c = 0; c < 9; ++c) g[c] = S.ghost[c][rtid];
-                lds_st(S.prod, gslot, mv9t(g, lds_ld(S.p, gsrc)));
+                const unsigned w = opaque(gword);
+                lds_st(S.prod, 3u * (w >> 16), mv9t(g, lds_ld(S.p, 3u * (w & 0xffffu))));
             }
         }
         if constexpr (FORM == GENERAL) {
             if (on[0]) {
+                const unsigned lp = row_at(0);
                 f3 src[kHeld];
 #pragma unroll
                 for (int u = 0; u < kHeld; ++u) src[u] = lds_ld(S.p, F::src(opaque(word[0][u])));
 #pragma unroll
                 for (int u = 0; u < kHeld; ++u)
                     if (unsigned(u) < opaque(holds[0]))
-                        lds_st(S.prod, 3u * (F::place(opaque(word[0][u])) * kPart + lp[0]), mv9(V[0][u], src[u]));
+                        lds_st(S.prod, 3u * (F::place(opaque(word[0][u])) * kPart + lp), mv9(V[0][u], src[u]));
             }
         }
         if constexpr (FORM != ROWS) __syncthreads();
 #pragma unroll
         for (int s = 0; s < kSlots; ++s)
             if (on[s]) {
+                const unsigned lp = row_at(s);
                 f3 src[kHeld], low[kHeld];
                 float d[9];
                 if constexpr (FORM != GENERAL) {
@@ -500,7 +511,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                     for (int u = 0; u < kHeld; ++u) src[u] = lds_ld(S.p, F::src(opaque(word[s][u])));
                 }
 #pragma unroll
-                for (int c = 0; c < kDiag; ++c) d[kDiag == 9 ? unsigned(c) : sym6_pos(unsigned(c))] = S.diag[c][lp[s]];
+                for (int c = 0; c < kDiag; ++c) d[kDiag == 9 ? unsigned(c) : sym6_pos(unsigned(c))] = S.diag[c][lp];
                 if constexpr (kDiag == 6) {
                     d[3] = d[1];
                     d[6] = d[2];
@@ -509,7 +520,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                 f3 sum;
                 if constexpr (FORM == SHEET) {
 #pragma unroll
-                    for (int l = 0; l < kHeld; ++l) low[l] = lds_ld(S.prod, 3u * (unsigned(l) * kPart + lp[s]));
+                    for (int l = 0; l < kHeld; ++l) low[l] = lds_ld(S.prod, 3u * (unsigned(l) * kPart + lp));
                     sum = mv9(d, v[s]);
 #pragma unroll
                     for (int l = 0; l < kHeld; ++l) sum = add(sum, low[l]);
@@ -522,7 +533,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                         if (t < widest) {
                             f3 y[4];
 #pragma unroll
-                            for (unsigned u = 0; u < 4; ++u) y[u] = lds_ld(S.prod, 3u * ((t + u) * kPart + lp[s]));
+                            for (unsigned u = 0; u < 4; ++u) y[u] = lds_ld(S.prod, 3u * ((t + u) * kPart + lp));
 #pragma unroll
                             for (unsigned u = 0; u < 4; ++u) sum = add(sum, y[u]);
                         }
@@ -551,10 +562,11 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     auto send_sums = [&](int t, auto& acc) {
         constexpr int N = int(sizeof(acc[0]) / sizeof(double));
         double none[N] = {};
-        leaf_sums(acc[0], kSlots == 2 ? acc[kSlots - 1] : none, S.leaf, wave, lane);
+        leaf_sums(acc[0], kSlots == 2 ? acc[kSlots - 1] : none, S.leaf, wave);
         __syncthreads();
-        if (tid < 8u * N) {
-            const unsigned v = tid >> 3, i = tid & 7u;
+        const unsigned me = tid_here();
+        if (me < 8u * N) {
+            const unsigned v = me >> 3, i = me & 7u;
             double w = S.leaf[2 * i][v] + S.leaf[2 * i + 1][v];
             w += dpp64<kXor1>(w);
             w += dpp64<kXor2>(w);
@@ -577,11 +589,12 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     // the parts (256 readers of 256 parts' words took 20 us an exchange).
     auto take_sums = [&](int t, unsigned N) -> bool {
         if (parts > 1 && wave < N) {
+            const unsigned lane = tid_here() & unsigned(kWave - 1);
             auto fetch = [&](const u64* at, bool mine, double& w) {
                 unsigned b[2];
                 w = 0.0;
                 if (!mine) return true;
-                if (!await<2>(at, tag_of(t), b, bar)) return false;
+                if (!await<2>(at, tag_of(t), b, &B.xbuf[RES_PROGRESS], bar)) return false;
                 w = __longlong_as_double((long long)((u64(b[1]) << 32) | b[0]));
                 return true;
             };
@@ -623,9 +636,9 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     // it first hides its way behind the sums').
     auto take_halo = [&](int t) {
         f3 h = mk(0.f, 0.f, 0.f);
-        if (rtid < n_halo) {
+        if (is_halo()) {
             unsigned w[3];
-            if (await<3>(row_words(t, hex), tag_of(t), w, bar))
+            if (await<3>(row_words(t, hex), tag_of(t), w, &B.xbuf[RES_PROGRESS], bar))
                 h = mk(__uint_as_float(w[0]), __uint_as_float(w[1]), __uint_as_float(w[2]));
             else
                 S.bad = 1;
@@ -657,8 +670,8 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
 #pragma unroll
         for (int s = 0; s < kSlots; ++s) {
             acc[s][0] = acc[s][1] = acc[s][2] = 0.0;
-            if (on[s] && live[s]) {
-                const f3 b = ld3g(I.rhs, ldx(plan, rows_at + pos0 + lp[s]));
+            if (on[s] && live(s)) {
+                const f3 b = ld3g(I.rhs, ldx(plan, rows_at + pos0 + row_at(s)));
                 r[s] = sub(b, q[s]);
                 if (ex[s] != CHX_RES_NONE) send_row(t, ex[s], r[s]);
                 acc[s][0] = dot64(r[s], apply_minv(M[s], r[s]));
@@ -701,12 +714,13 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             float alpha = 0.0f, beta = 0.0f;
             if (k > 0) merged_scalars(rho, sig, del, gam, alpha, beta);
             // halo rows: r_k, z_k, p_k as their owners form them
-            if (rtid < n_halo && !last) {
+            if (is_halo() && !last) {
                 if (k > 0) {
                     hr = axpy(-alpha, h, hr);
-                    lds_st(S.p, hslot, axpy(beta, lds_ld(S.p, hslot), apply_minv(hM, hr)));
+                    const unsigned at = halo_slot();
+                    lds_st(S.p, at, axpy(beta, lds_ld(S.p, at), apply_minv(hM, hr)));
                 } else {
-                    lds_st(S.p, hslot, apply_minv(hM, hr));
+                    lds_st(S.p, halo_slot(), apply_minv(hM, hr));
                 }
             }
 #pragma unroll
@@ -714,12 +728,13 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                 if (on[s]) {
                     if (k > 0) {
                         r[s] = axpy(-alpha, q[s], r[s]);
-                        lds_st(S.x, 3u * lp[s], axpy(alpha, p[s], lds_ld(S.x, 3u * lp[s])));
+                        const unsigned at = 3u * row_at(s);
+                        lds_st(S.x, at, axpy(alpha, p[s], lds_ld(S.x, at)));
                         p[s] = axpy(beta, p[s], apply_minv(M[s], r[s]));
                     } else {
                         p[s] = apply_minv(M[s], r[s]);
                     }
-                    lds_st(S.p, 3u * lp[s], p[s]);
+                    lds_st(S.p, 3u * row_at(s), p[s]);
                 }
             if (!last) apply(p, q);
             double acc[kSlots][5];
@@ -727,7 +742,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             for (int s = 0; s < kSlots; ++s) {
 #pragma unroll
                 for (int v = 0; v < 5; ++v) acc[s][v] = 0.0;
-                if (on[s] && live[s]) {
+                if (on[s] && live(s)) {
                     if (!last && ex[s] != CHX_RES_NONE) send_row(k + 1, ex[s], q[s]);
                     const f3 z = apply_minv(M[s], r[s]);
                     acc[s][0] = dot64(r[s], z);
@@ -771,17 +786,17 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
 #pragma unroll
                     for (int s = 0; s < kSlots; ++s)
                         if (on[s]) {
-                            p[s] = lds_ld(S.x, 3u * lp[s]);
-                            if (live[s] && ex[s] != CHX_RES_NONE) send_row(t, ex[s], p[s]);
+                            p[s] = lds_ld(S.x, 3u * row_at(s));
+                            if (ex[s] != CHX_RES_NONE) send_row(t, ex[s], p[s]);
                         }
                     send_sums(t, zero);
                     const f3 hx = take_halo(t);
                     if (!take_sums(t, 1)) return false;
-                    if (rtid < n_halo) lds_st(S.p, hslot, hx);
+                    if (is_halo()) lds_st(S.p, halo_slot(), hx);
                 } else {
-                    if (rtid < n_halo) {
+                    if (is_halo()) {
                         const f3 z = apply_minv(hM, hr);
-                        lds_st(S.p, hslot, fresh ? z : axpy(beta, lds_ld(S.p, hslot), z));
+                        lds_st(S.p, halo_slot(), fresh ? z : axpy(beta, lds_ld(S.p, halo_slot()), z));
                     }
 #pragma unroll
                     for (int s = 0; s < kSlots; ++s)
@@ -792,7 +807,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                 }
 #pragma unroll
                 for (int s = 0; s < kSlots; ++s)
-                    if (on[s]) lds_st(S.p, 3u * lp[s], p[s]);
+                    if (on[s]) lds_st(S.p, 3u * row_at(s), p[s]);
             }
             const int want = half && !residual_step ? 1 : 0;
             if (want != blocks) {
@@ -819,7 +834,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
 #pragma unroll
             for (int s = 0; s < kSlots; ++s) {
                 sum[s][0] = 0.0;
-                if (on[s] && live[s]) {
+                if (on[s] && live(s)) {
                     if (ex[s] != CHX_RES_NONE) send_row(t, ex[s], q[s]);
                     sum[s][0] = dot64(p[s], q[s]);
                 }
@@ -829,14 +844,15 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             if (!take_sums(t, 1)) return false;
             const float alpha = guarded_div(rho, S.tot[0]);
             mark_trace();
-            if (rtid < n_halo) hr = axpy(-alpha, h, hr);
+            if (is_halo()) hr = axpy(-alpha, h, hr);
             ++t;
             double acc[kSlots][2];
 #pragma unroll
             for (int s = 0; s < kSlots; ++s) {
                 acc[s][0] = acc[s][1] = 0.0;
-                if (on[s] && live[s]) {
-                    lds_st(S.x, 3u * lp[s], axpy(alpha, p[s], lds_ld(S.x, 3u * lp[s])));
+                if (on[s] && live(s)) {
+                    const unsigned at = 3u * row_at(s);
+                        lds_st(S.x, at, axpy(alpha, p[s], lds_ld(S.x, at)));
                     r[s] = axpy(-alpha, q[s], r[s]);
                     acc[s][0] = dot64(r[s], apply_minv(M[s], r[s]));
                     acc[s][1] = dot64(r[s], r[s]);
@@ -854,7 +870,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     }
 #pragma unroll
     for (int s = 0; s < kSlots; ++s)
-        if (live[s]) st3g(I.x, ldx(plan, rows_at + pos0 + lp[s]), lds_ld(S.x, 3u * lp[s]));
+        if (live(s)) st3g(I.x, ldx(plan, rows_at + pos0 + row_at(s)), lds_ld(S.x, 3u * row_at(s)));
     return true;
 }
 
