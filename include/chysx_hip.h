@@ -204,8 +204,9 @@ typedef struct chx_unit {
 /* 64-bit words of `xbuf` before the instances' exchange areas, and of one
  * instance's area with `parts` parts and `exports` exported rows. */
 #define CHX_RES_CONTROL_WORDS 4352
-#define CHX_RES_XWORDS(parts, exports) \
-    (20ull * (parts) + ((parts) > 64 ? 5120ull : 0ull) + 6ull * (exports))
+#define CHX_RES_XWORDS(parts, exports) ((32ull * (parts) + 4ull * (exports) + 15ull) & ~15ull)
+/* Most words of xbuf: 32-bit byte offsets. */
+#define CHX_RES_XWORDS_MAX (1ull << 28)
 
 /* One cloth instance: every array is the instance's own device memory, with
  * indices local to the instance, so the off-diagonal pattern is exactly the

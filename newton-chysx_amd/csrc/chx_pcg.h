@@ -71,7 +71,9 @@ enum : int {
     RES_IDLE = 64,      // per group (16 words apart): its idle workgroups
     RES_MAIL = 256      // per workgroup (16 words apart): its next item and part
 };
-constexpr unsigned kResEpochs = (1u << 24) - 1u;
+// A tag's 16 bits are a launch number's 8 and an exchange's 8: the area is
+// cleared when the launch numbers start over.
+constexpr unsigned kResEpochs = 255u;
 constexpr int kResGroups = 8;
 static_assert(RES_MAIL + 16 * 256 <= CHX_RES_CONTROL_WORDS && RES_IDLE + 16 * kResGroups <= RES_MAIL, "control words");
 

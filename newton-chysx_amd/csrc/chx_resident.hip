@@ -28,11 +28,20 @@
 // the leaves of the instance by a fixed binary tree that does not depend on
 // how many leaves a part has: the same bits for every part size and gang.
 //
-// Exchange: 64-bit words {value, tag}, the tag naming launch and exchange, so
-// a reader needs no ordering between words and no cache maintenance: it reads
-// a word until its tag is the awaited one.  Words alternate between two
+// Exchange: 64-bit words of values and a tag that names launch and exchange,
+// so a reader needs no ordering between words and no cache maintenance: it
+// reads a word until its tag is the awaited one.  Words alternate between two
 // slots; slot t is rewritten in exchange t + 2, which its writer enters only
 // after every part's sums of exchange t + 1, sent after their reads of t.
+//
+// Every part has a 128-byte line for its sums, which all parts read, 16 bytes
+// a lane.  What costs is lines with several writers: with the parts' words
+// side by side an all-to-all of five sums took 1.8 us between 16 workgroups,
+// 2.1 between 32 and 2.4 between 64; with a line each 1.3, 1.3 and 1.4, and
+// 2.9 between 256.  Two levels of any group size (3.3 to 5.3 us for 64 to 256)
+// and copies per reader lose to that, and so does more than one read in
+// flight: the floor of one store and one load is 1.0 to 1.2 us.
+// A halo row is 16 bytes: three floats and the tag's 16 bits in both words.
 #include <algorithm>
 #include <mutex>
 
@@ -82,9 +91,8 @@ static_assert(3 * (Form<SHEET>::kSpare + kWave) < (1u << 16) && 3 * (Form<GENERA
 // ||r||^2 (set-up: and ||b||^2).
 constexpr int kSums = 5;
 constexpr int kMaxParts = 256;
-constexpr unsigned kFan = 16;    // parts per group and groups, above 64 parts
-constexpr unsigned kCopies = 16;  // copies of the groups' sums
-static_assert(kFan * kFan >= kMaxParts && 2 * kCopies <= 64, "two levels");
+constexpr unsigned kLine = 16;  // words of a part's line
+static_assert(2 * kSums <= kLine, "a part's sums in one line");
 constexpr unsigned kExit = 0xffffffu;  // mailbox item: nothing left
 static_assert(CHX_RES_LEAF == kWave && Form<SHEET>::kSlots == 2 && Form<GENERAL>::kSlots == 1 && kLeaves == 2 * kWaves,
               "a leaf per wave and slot");
@@ -99,6 +107,17 @@ __device__ __forceinline__ void st64(u64* p, u64 v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ u64 tagged(unsigned v, unsigned tag) { return (u64(tag) << 32) | v; }
+
+// 16-byte accesses of the exchange area at agent scope (byte offsets).  The
+// two 64-bit words of one may be of different age: both carry the tag.
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+using Area = __amdgpu_buffer_rsrc_t;
+constexpr int kAgent = 1 << 4;  // sc1
+__device__ __forceinline__ Area exchange_area(const chx_cloth_batch& B) {
+    return __builtin_amdgcn_make_buffer_rsrc(B.xbuf, 0, int(B.res_xwords * 8ull), 0x00020000);
+}
+__device__ __forceinline__ v4u ld128(Area a, unsigned at) { return __builtin_amdgcn_raw_buffer_load_b128(a, at, 0, kAgent); }
+__device__ __forceinline__ void st128(Area a, unsigned at, v4u v) { __builtin_amdgcn_raw_buffer_store_b128(v, a, at, 0, kAgent); }
 
 // Triples in LDS, by the index of their first word.
 __device__ __forceinline__ f3 lds_ld(const float* m, unsigned i) { return {m[i], m[i + 1u], m[i + 2u]}; }
@@ -128,8 +147,11 @@ struct ResLds {
     float diag[FULL ? 9 : 6][Form<FORM>::kRows];
     float x[3 * Form<FORM>::kRows];
     float ghost[FORM == ROWS ? 1 : 9][CHX_RES_GHOST_MAX];
+    float hminv[FORM == SHEET ? 6 : 1][CHX_RES_HALO_MAX];  // halo rows' inverses (other forms: registers)
+    double bb;       // ||b||^2
     double leaf[kLeaves][kSums];
     double tot[8];
+    double wsum[kWaves][8];
     int bad;         // a wait gave up
     unsigned mail;   // mailbox word of the workgroup
 };
@@ -138,11 +160,12 @@ struct ResLds {
 // solve is aborted for every workgroup (the report of grid_sync).
 struct Watch {
     const Barrier& bar;
-    u64 t0;
+    u64 t0 = 0;
     unsigned polls = 0;
-    __device__ explicit Watch(const Barrier& b) : bar(b), t0(__builtin_amdgcn_s_memrealtime()) {}
+    __device__ explicit Watch(const Barrier& b) : bar(b) {}
     __device__ bool again(u64* progress, unsigned& seen) {
         unsigned* sync = bar.sync;
+        if (polls == 0u) t0 = __builtin_amdgcn_s_memrealtime();
         if ((++polls & 15u) == 0u && ld_relaxed(&sync[SYNC_ABORT]) != 0u) return false;
         if (__builtin_amdgcn_s_memrealtime() - t0 <= bar.ticks) return true;
         const unsigned now = unsigned(ld64(progress));
@@ -162,30 +185,23 @@ struct Watch {
     }
 };
 
-// N tagged words from p on, read until every tag is the awaited one; false:
+// The 16 bytes at at(j) for j < N, read until `mine` accepts them all; false:
 // the wait was given up.  A peer may still be busy with an earlier large item
 // of the list, so the wait goes on as long as any gang iterates.
-template <int N>
-__device__ __forceinline__ bool await(const u64* p, unsigned tag, unsigned (&v)[N], u64* progress, const Barrier& bar) {
-    u64 w[N];
-    auto read = [&] {
+template <int N, class At, class Mine>
+__device__ __forceinline__ bool await(Area area, At at, Mine mine, v4u (&w)[N], u64* progress, const Barrier& bar) {
+    Watch watch(bar);
+    unsigned seen = 0;
+    for (;;) {
+        asm volatile("" ::: "memory");  // the loads read again
         bool ok = true;
 #pragma unroll
-        for (int k = 0; k < N; ++k) w[k] = ld64(p + k);
+        for (int j = 0; j < N; ++j) w[j] = ld128(area, at(j));
 #pragma unroll
-        for (int k = 0; k < N; ++k) ok = ok && unsigned(w[k] >> 32) == tag;
-        return ok;
-    };
-    if (!read()) {
-        Watch watch(bar);
-        unsigned seen = 0;
-        do {
-            if (!watch.again(progress, seen)) return false;
-        } while (!read());
+        for (int j = 0; j < N; ++j) ok = ok && mine(w[j]);
+        if (ok) return true;
+        if (!watch.again(progress, seen)) return false;
     }
-#pragma unroll
-    for (int k = 0; k < N; ++k) v[k] = unsigned(w[k]);
-    return true;
 }
 __device__ __forceinline__ void transpose9(float (&m)[9]) {
     const float a = m[1], b = m[2], c = m[5];
@@ -310,25 +326,17 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     const unsigned n_own = hdr[0], n_halo = hdr[1], halo_at = hdr[2], n_ghost = hdr[3], ghost_at = hdr[4], widest = hdr[5];
     const unsigned pos0 = unsigned(part) * unsigned(I.res_part_rows);
     const unsigned rows_at = 8u * parts, meta_at = rows_at + n, exp_at = meta_at + n, held_at = exp_at + n;
-    // exchange areas: [2][kSums][parts] pairs of words, above 64 parts
-    // [2][kCopies][kSums][kFan] pairs, then [2][exports] rows of 3
-    u64* const xsum = B.xbuf + I.res_xbase;
-    u64* const xgroup = xsum + 4u * kSums * parts;
-    u64* const xrow = xgroup + (parts > unsigned(kWave) ? 4u * kCopies * kSums * kFan : 0u);
+    // exchange area (byte offsets): [2][parts] lines, then [2][exports] rows
+    const Area area = exchange_area(B);
+    const unsigned xsum = 8u * I.res_xbase, xrow = xsum + 2u * 8u * kLine * parts;
     const unsigned exports = unsigned(I.res_exports);
     auto tag_of = [&](int t) { return (epoch << 8) | (unsigned(t) & 255u); };
-    auto sum_words = [&](int t, unsigned v, unsigned q) {
-        return xsum + 2u * (((unsigned(t) & 1u) * kSums + v) * parts + q);
-    };
-    auto group_words = [&](int t, unsigned copy, unsigned v, unsigned g) {
-        return xgroup + 2u * ((((unsigned(t) & 1u) * kCopies + copy) * kSums + v) * kFan + g);
-    };
-    auto row_words = [&](int t, unsigned e) { return xrow + 3ull * ((unsigned(t) & 1u) * exports + e); };
+    auto line = [&](int t, unsigned q) { return xsum + 8u * kLine * ((unsigned(t) & 1u) * parts + q); };
+    auto row_bytes = [&](int t, unsigned e) { return xrow + 16u * ((unsigned(t) & 1u) * exports + e); };
     auto send_row = [&](int t, unsigned e, f3 v) {
-        u64* const w = row_words(t, e);
-        st64(w, tagged(__float_as_uint(v.x), tag_of(t)));
-        st64(w + 1, tagged(__float_as_uint(v.y), tag_of(t)));
-        st64(w + 2, tagged(__float_as_uint(v.z), tag_of(t)));
+        const unsigned x = __float_as_uint(v.x), y = __float_as_uint(v.y), z = __float_as_uint(v.z);
+        const unsigned tag = tag_of(t) << 16;
+        st128(area, row_bytes(t, e), v4u{x, (y & 0xffffu) | tag, z, (y >> 16) | tag});
     };
 
     // ---- load: own rows, ghost block, halo row ----
@@ -450,6 +458,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     if constexpr (!TWO) load_blocks(false);
     unsigned gword = 0;  // the ghost block's source and product slot
     if (FORM != ROWS && rtid_here() < n_ghost) gword = ldx(plan, ghost_at + 2u * rtid_here() + 1u);
+    constexpr bool kHaloInLds = FORM == SHEET;
     float hM[kMinv];
     f3 hr = mk(0.f, 0.f, 0.f);
     unsigned hex = 0;
@@ -460,8 +469,22 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         const unsigned hrow = ldx(plan, halo_at + 2u * rtid);
         hex = ldx(plan, halo_at + 2u * rtid + 1u);
         invert(hrow, hM);
+        if constexpr (kHaloInLds) {
+#pragma unroll
+            for (int c = 0; c < kMinv; ++c) S.hminv[c][rtid] = hM[c];
+        }
         lds_st(S.p, halo_slot(), ld3g(I.x, hrow));
     }
+    auto halo_minv = [&](f3 v) {
+        if constexpr (kHaloInLds) {
+            float m[kMinv];
+#pragma unroll
+            for (int c = 0; c < kMinv; ++c) m[c] = S.hminv[c][rtid_here()];
+            return apply_minv(m, v);
+        } else {
+            return apply_minv(hM, v);
+        }
+    };
     if (tid == 0) S.bad = 0;
     if (tid < kLeaves * kSums) S.leaf[tid / kSums][tid % kSums] = 0.0;
 
@@ -559,87 +582,115 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     };
     // The sums of exchange t: per leaf, then over the part's leaves, sent to
     // the gang.
+    auto leaf_pair = [&](unsigned v, unsigned i) { return S.leaf[2 * i][v] + S.leaf[2 * i + 1][v]; };
+    auto tree8 = [](double w) {  // over eight lanes
+        w += dpp64<kXor1>(w);
+        w += dpp64<kXor2>(w);
+        return w + dpp64<kHalfMirror>(w);
+    };
     auto send_sums = [&](int t, auto& acc) {
         constexpr int N = int(sizeof(acc[0]) / sizeof(double));
         double none[N] = {};
         leaf_sums(acc[0], kSlots == 2 ? acc[kSlots - 1] : none, S.leaf, wave);
         __syncthreads();
         const unsigned me = tid_here();
-        if (me < 8u * N) {
+        if (parts > 1 && me < 8u * N) {
             const unsigned v = me >> 3, i = me & 7u;
-            double w = S.leaf[2 * i][v] + S.leaf[2 * i + 1][v];
-            w += dpp64<kXor1>(w);
-            w += dpp64<kXor2>(w);
-            w += dpp64<kHalfMirror>(w);
-            if (i == 0) {
-                if (parts == 1) {
-                    S.tot[v] = w;
-                } else {
-                    const u64 b = u64(__double_as_longlong(w));
-                    u64* const w2 = sum_words(t, v, unsigned(part));
-                    st64(w2, tagged(unsigned(b), tag_of(t)));
-                    st64(w2 + 1, tagged(unsigned(b >> 32), tag_of(t)));
-                }
-            }
+            const u64 b = u64(__double_as_longlong(tree8(leaf_pair(v, i))));
+            if (i == 0)
+                st128(area, line(t, unsigned(part)) + 16u * v, v4u{unsigned(b), tag_of(t), unsigned(b >> 32), tag_of(t)});
         }
     };
-    // The instance's N sums of exchange t into S.tot: a tree over the parts,
-    // read by everyone up to 64 parts; above, the first part of every 16 sums
-    // them up and sends the result to kCopies places, each read by some of
-    // the parts (256 readers of 256 parts' words took 20 us an exchange).
+    // The instance's N sums of exchange t into tot: a tree over the parts.
+    // Up to 64 parts a wave reads one sum of every part (1.47 us for an
+    // exchange of 64 parts in a loop of its own, 1.94 the other way).  Above,
+    // that is 1280 reads of 16 bytes for 256 parts (2.9 us): there eight lanes
+    // read a part's line together and a wave 32 lines (2.6 us), and the waves'
+    // sums meet in LDS.  Then, and for a part that is alone, every wave adds up
+    // the eight last terms by itself.
+    double tot[kSums];
     auto take_sums = [&](int t, unsigned N) -> bool {
-        if (parts > 1 && wave < N) {
-            const unsigned lane = tid_here() & unsigned(kWave - 1);
-            auto fetch = [&](const u64* at, bool mine, double& w) {
-                unsigned b[2];
-                w = 0.0;
-                if (!mine) return true;
-                if (!await<2>(at, tag_of(t), b, &B.xbuf[RES_PROGRESS], bar)) return false;
-                w = __longlong_as_double((long long)((u64(b[1]) << 32) | b[0]));
-                return true;
-            };
-            auto tree16 = [](double w) {
-                w += dpp64<kXor1>(w);
-                w += dpp64<kXor2>(w);
-                w += dpp64<kHalfMirror>(w);
-                return w + dpp64<kRor8>(w);
-            };
-            double w;
-            bool ok = true;
-            if (parts <= unsigned(kWave)) {
-                ok = fetch(sum_words(t, wave, lane), lane < parts, w);
-                w = tree16(w);
+        const unsigned lane = tid_here() & unsigned(kWave - 1), tag = tag_of(t);
+        u64* const progress = &B.xbuf[RES_PROGRESS];
+        auto mine = [&](v4u w) { return w.y == tag && w.w == tag; };
+        auto value = [](v4u w) { return __longlong_as_double((long long)((u64(w.z) << 32) | w.x)); };
+        const bool wide = parts > unsigned(kWave);
+        if (parts == 1) {
+        } else if (!wide) {
+            if (wave < N) {
+                v4u b[1];
+                const bool has = lane < parts;
+                // lanes without a part read the first one's
+                if (!await<1>(area, [&](int) { return line(t, has ? lane : 0u) + 16u * wave; }, mine, b, progress, bar))
+                    S.bad = 1;
+                double w = tree8(has ? value(b[0]) : 0.0);
+                w += dpp64<kRor8>(w);
                 if (parts > 16u) {
                     w = fold16(w, w);
                     w = fold32(w, w);
                 }
-            } else {
-                if ((unsigned(part) % kFan) == 0u) {
-                    ok = fetch(sum_words(t, wave, unsigned(part) + lane), lane < kFan && unsigned(part) + lane < parts, w);
-                    w = __shfl(tree16(w), 0);
-                    const u64 b = u64(__double_as_longlong(w));
-                    if (ok && lane < 2u * kCopies)
-                        st64(group_words(t, lane >> 1, wave, unsigned(part) / kFan) + (lane & 1u),
-                             tagged((lane & 1u) != 0u ? unsigned(b >> 32) : unsigned(b), tag_of(t)));
-                }
-                ok = __ballot(!ok) == 0ull &&
-                     fetch(group_words(t, unsigned(part) % kCopies, wave, lane), lane < (parts + kFan - 1u) / kFan, w);
-                w = tree16(w);
+                if (lane == 0) S.tot[wave] = w;
             }
-            if (lane == 0) S.tot[wave] = w;
-            if (!ok) S.bad = 1;
+        } else {
+            constexpr int kReads = kMaxParts / (8 * kWaves);
+            double sum = 0.0;
+            if (8u * kReads * wave < parts) {
+                const unsigned first = 8u * kReads * wave + (lane >> 3);
+                const unsigned word = (lane & 7u) < N ? lane & 7u : N - 1u;
+                auto has = [&](int j) { return first + 8u * unsigned(j) < parts; };
+                v4u b[kReads];
+                if (!await<kReads>(
+                        area, [&](int j) { return line(t, has(j) ? first + 8u * unsigned(j) : 0u) + 16u * word; }, mine, b,
+                        progress, bar))
+                    S.bad = 1;
+                double w[kReads];
+#pragma unroll
+                for (int j = 0; j < kReads; ++j) {
+                    w[j] = has(j) ? value(b[j]) : 0.0;
+                    w[j] += dpp64<kRor8>(w[j]);
+                    w[j] = fold16(w[j], w[j]);
+                    w[j] = fold32(w[j], w[j]);
+                }
+                static_assert(kReads == 4, "a tree over a wave's reads");
+                sum = (w[0] + w[1]) + (w[2] + w[3]);
+            }
+            if (lane < N) S.wsum[wave][lane] = sum;
         }
-        __syncthreads();
-        return S.bad == 0;
+        if (parts > 1) {
+            __syncthreads();
+            if (S.bad != 0) return false;
+        }
+        if (parts > 1 && !wide) {
+#pragma unroll
+            for (unsigned v = 0; v < unsigned(kSums); ++v)
+                if (v < N) tot[v] = S.tot[v];
+        } else {
+            double w = 0.0;
+            if (lane < 8u * N) w = wide ? S.wsum[lane & 7u][lane >> 3] : leaf_pair(lane >> 3, lane & 7u);
+            w = tree8(w);
+            const u64 b = u64(__double_as_longlong(w));
+#pragma unroll
+            for (unsigned v = 0; v < unsigned(kSums); ++v)
+                if (v < N) {
+                    const unsigned lo = __builtin_amdgcn_readlane(unsigned(b), 8 * v);
+                    const unsigned hi = __builtin_amdgcn_readlane(unsigned(b >> 32), 8 * v);
+                    tot[v] = __longlong_as_double((long long)((u64(hi) << 32) | lo));
+                }
+        }
+        return true;
     };
     // The halo row's triple of exchange t (sent before its sums: waiting for
     // it first hides its way behind the sums').
     auto take_halo = [&](int t) {
         f3 h = mk(0.f, 0.f, 0.f);
         if (is_halo()) {
-            unsigned w[3];
-            if (await<3>(row_words(t, hex), tag_of(t), w, &B.xbuf[RES_PROGRESS], bar))
-                h = mk(__uint_as_float(w[0]), __uint_as_float(w[1]), __uint_as_float(w[2]));
+            const unsigned tag = tag_of(t) & 0xffffu;
+            v4u w[1];
+            if (await<1>(
+                    area, [&](int) { return row_bytes(t, hex); },
+                    [&](v4u v) { return v.y >> 16 == tag && v.w >> 16 == tag; }, w, &B.xbuf[RES_PROGRESS], bar))
+                h = mk(__uint_as_float(w[0].x), __uint_as_float((w[0].y & 0xffffu) | w[0].w << 16),
+                       __uint_as_float(w[0].z));
             else
                 S.bad = 1;
         }
@@ -649,14 +700,16 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         if (B.trace != nullptr) {
             trace_point(B, trace_e, unsigned(B.n_instances) - unsigned(ld64(&B.xbuf[RES_DONE])));
             ++trace_e;
+            __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), so that the loop has no load pending to wait for
         }
     };
     auto stop = [&](int its, double rr, double bb, double rho) {
-        if (part == 0 && tid == 0) {
-            B.inst_iters[inst] = its;
-            B.inst_rr[inst] = rr;
-            B.inst_bb[inst] = bb;
-            if (B.inst_rho != nullptr) B.inst_rho[inst] = rho;
+        if (part == 0 && tid_here() == 0) {
+            const unsigned i = opaque(unsigned(inst));
+            stx(glb(B.inst_iters), i, its);
+            stx(glb(B.inst_rr), i, rr);
+            stx(glb(B.inst_bb), i, bb);
+            if (B.inst_rho != nullptr) stx(glb(B.inst_rho), i, rho);
             (void)__hip_atomic_fetch_add(&B.xbuf[RES_DONE], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     };
@@ -688,8 +741,8 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         residual(0);
         hr = take_halo(0);
         if (!take_sums(0, 3)) return false;
-        double rho = S.tot[0], rr = S.tot[2];
-        const double bb = S.tot[1];
+        double rho = tot[0], rr = tot[2];
+        S.bb = tot[1];  // every thread the same
         mark_trace();
         double sig = 0.0, del = 0.0, gam = 0.0;
         for (int k = 0;; ++k) {
@@ -698,14 +751,15 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             if (k > 0) {
                 if (!last) h = take_halo(k);
                 if (!take_sums(k, 5)) return false;
-                rho = S.tot[0];
-                sig = S.tot[1];
-                del = S.tot[2];
-                gam = S.tot[3];
-                rr = S.tot[4];
+                rho = tot[0];
+                sig = tot[1];
+                del = tot[2];
+                gam = tot[3];
+                rr = tot[4];
                 mark_trace();
             }
             const int its = k > 0 ? k - 1 : 0;  // updates of x so far
+            const double bb = S.bb;
             if (its >= I.max_iter || (I.tol > 0.0 && rr <= I.tol * I.tol * bb)) {
                 stop(its, rr, bb, rho);
                 break;
@@ -718,9 +772,9 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                 if (k > 0) {
                     hr = axpy(-alpha, h, hr);
                     const unsigned at = halo_slot();
-                    lds_st(S.p, at, axpy(beta, lds_ld(S.p, at), apply_minv(hM, hr)));
+                    lds_st(S.p, at, axpy(beta, lds_ld(S.p, at), halo_minv(hr)));
                 } else {
-                    lds_st(S.p, halo_slot(), apply_minv(hM, hr));
+                    lds_st(S.p, halo_slot(), halo_minv(hr));
                 }
             }
 #pragma unroll
@@ -795,7 +849,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                     if (is_halo()) lds_st(S.p, halo_slot(), hx);
                 } else {
                     if (is_halo()) {
-                        const f3 z = apply_minv(hM, hr);
+                        const f3 z = halo_minv(hr);
                         lds_st(S.p, halo_slot(), fresh ? z : axpy(beta, lds_ld(S.p, halo_slot()), z));
                     }
 #pragma unroll
@@ -820,9 +874,9 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                 residual(t);
                 hr = take_halo(t);
                 if (!take_sums(t, 3)) return false;
-                rho = S.tot[0];
-                bb = S.tot[1];
-                rr = S.tot[2];
+                rho = tot[0];
+                bb = tot[1];
+                rr = tot[2];
                 residual_step = false;
                 exact = fresh = true;
                 ++refines;
@@ -842,7 +896,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             send_sums(t, sum);
             const f3 h = take_halo(t);
             if (!take_sums(t, 1)) return false;
-            const float alpha = guarded_div(rho, S.tot[0]);
+            const float alpha = guarded_div(rho, tot[0]);
             mark_trace();
             if (is_halo()) hr = axpy(-alpha, h, hr);
             ++t;
@@ -860,9 +914,9 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             }
             send_sums(t, acc);
             if (!take_sums(t, 2)) return false;
-            beta = guarded_div(S.tot[0], rho);
-            rho = S.tot[0];
-            rr = S.tot[1];
+            beta = guarded_div(tot[0], rho);
+            rho = tot[0];
+            rr = tot[1];
             exact = fresh = false;
             mark_trace();
             ++k;

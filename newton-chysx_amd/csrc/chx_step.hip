@@ -1873,7 +1873,7 @@ void validate_batch(const chx_cloth_batch* b) {
     if (b->res_grid > 0) {
         require(b->xbuf != nullptr && b->res_grid <= resident_grid_limit() && b->res_groups > 0 &&
                     b->res_grid % b->res_groups == 0 && b->res_groups <= kResGroups &&
-                    b->res_xwords >= CHX_RES_CONTROL_WORDS,
+                    b->res_xwords >= CHX_RES_CONTROL_WORDS && b->res_xwords <= CHX_RES_XWORDS_MAX,
                 "chysx: resident solve without its exchange area, or a grid that does not fit the device");
         if (b->inst == nullptr) {
             const chx_instance& I = b->single;
@@ -1884,6 +1884,7 @@ void validate_batch(const chx_cloth_batch* b) {
                          I.res_parts <= b->res_grid && I.res_exports >= 0 &&
                          (I.res_form != 0) == (b->res_form != 0) &&
                          (b->res_form == 0 || I.res_part_rows <= CHX_RES_GEN_PART) &&
+                         I.res_xbase % 16 == 0 &&
                          I.res_xbase + CHX_RES_XWORDS(I.res_parts, I.res_exports) <= b->res_xwords),
                     "chysx: resident plan does not match its instance");
         } else {
@@ -2126,6 +2127,7 @@ void solve_bsr3(int n_rows, const float* diag, const int* row_offsets, const int
             require((plan->part_rows == 256 || plan->part_rows == CHX_RES_GEN_PART) &&
                         plan->parts == (n_rows + plan->part_rows - 1) / plan->part_rows && plan->exports >= 0 &&
                         plan->xbuf != nullptr &&
+                        plan->xwords <= CHX_RES_XWORDS_MAX &&
                         plan->xwords >= CHX_RES_CONTROL_WORDS + CHX_RES_XWORDS(plan->parts, plan->exports),
                     "pcg: resident plan does not match the matrix");
             if (plan->parts <= limit) {

@@ -748,10 +748,10 @@ void BatchRunner::layout_resident(std::vector<chx_instance>& ds, std::uintptr_t 
     std::size_t words = CHX_RES_CONTROL_WORDS;
     for (chx_instance& d : ds) {
         if (d.n_rows == 0) continue;
-        if (words > 0xffffffffu) return;
-        d.res_xbase = static_cast<unsigned>(words);
+        d.res_xbase = static_cast<unsigned>(std::min<std::size_t>(words, CHX_RES_XWORDS_MAX));
         words += CHX_RES_XWORDS(d.res_parts, d.res_exports);
     }
+    if (words > CHX_RES_XWORDS_MAX) return;
     if (xbuf_.gpu_size() < words) {
         xbuf_.ensure_device(words);
         xbuf_.zero_device(stream);

@@ -55,11 +55,8 @@ def test_resident_step_matches_the_streaming_step(gpu, nx, ny, shuffle):
         assert helpers.rel_maxnorm(a.state()[0], b.state()[0]) <= 1e-6
 
 
-@pytest.mark.parametrize("n,extra", [(8, 0), (23, 0), (64, 0), (40, 9)])
-def test_rows_plan_matches_streamed_rows(gpu, n, extra):
-    """A caller's matrix: the resident solve (eight lanes per row) against
-    four lanes per row, which streams; `extra` blocks per row widen it past
-    the plan's limit for some rows, where both stream."""
+def _rows_system(n, extra=0):
+    """A diagonally dominant block matrix over an n-by-n grid, and a right-hand side."""
     import torch
 
     import chysx
@@ -87,6 +84,19 @@ def test_rows_plan_matches_streamed_rows(gpu, n, extra):
     A.build_topology(N, rows, cols)
     A.upload(diag, vals)
     b = torch.from_numpy(rng.normal(size=(N, 3)).astype(np.float32)).cuda()
+    return A, b
+
+
+@pytest.mark.parametrize("n,extra", [(8, 0), (23, 0), (64, 0), (40, 9)])
+def test_rows_plan_matches_streamed_rows(gpu, n, extra):
+    """A caller's matrix: the resident solve (eight lanes per row) against
+    four lanes per row, which streams; `extra` blocks per row widen it past
+    the plan's limit for some rows, where both stream."""
+    import torch
+
+    import chysx
+
+    A, b = _rows_system(n, extra)
     out = []
     for lanes in (8, 4):
         x = torch.zeros_like(b)
@@ -95,6 +105,25 @@ def test_rows_plan_matches_streamed_rows(gpu, n, extra):
         out.append((x.cpu().numpy(), S.last_iterations()))
     assert abs(out[0][1] - out[1][1]) <= 1
     assert helpers.rel_maxnorm(out[0][0], out[1][0]) <= 1e-5
+
+
+def test_launch_numbers_start_over(gpu):
+    """Tags name 255 launches; then the exchange area is cleared.  The same
+    solve on three parts gives the same bits across that point."""
+    import torch
+
+    import chysx
+
+    A, b = _rows_system(23)
+    S = chysx.PCGSolver()
+    first = None
+    for k in range(520):
+        x = torch.zeros_like(b)
+        S.solve(A, b.data_ptr(), x.data_ptr(), max_iterations=3 + k % 2)
+        x = x.cpu().numpy()
+        if k < 2:
+            first = [x] if k == 0 else first + [x]
+        assert np.array_equal(x, first[k % 2]), k
 
 
 @pytest.mark.parametrize("blocks", [0, 16, 24])
