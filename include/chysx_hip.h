@@ -401,9 +401,6 @@ int chx_device_info(int* cu_count, int* max_pcg_blocks, int* occupancy_blocks_pe
 int chx_pcg_grid_limit(int lanes_per_row, int bf16_blocks, int no_lds_staging, int* max_blocks);
 /* The same for the resident PCG kernel (one workgroup per compute unit). */
 int chx_resident_grid_limit(int* max_blocks);
-/* Workgroups and groups of a resident launch of one instance with `parts`
- * parts, at most `limit` workgroups (parts <= limit). */
-int chx_resident_grid(int parts, int limit, int* grid, int* groups);
 
 /* Device memory: replaces CudaArray<T> (ChysX/src/memory/cuda_array.h:64-284,
  * cuda_array.cu:41-90). */

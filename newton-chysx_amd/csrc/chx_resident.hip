@@ -54,6 +54,31 @@ namespace {
 constexpr int kThreads = 512;  // two waves per SIMD with 256 VGPRs each
 constexpr int kWaves = kThreads / kWave;
 constexpr int kLeaves = CHX_RES_PART_MAX / CHX_RES_LEAF;
+// Keeps a value that the loop does not change from being re-derived ahead of
+// the loop (addresses and masks of every block would not fit the registers).
+__device__ __forceinline__ unsigned opaque(unsigned v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+// The thread index for addresses and masks of one use.  What the loop derives
+// from it is derived again: kept over the loop those values went to scratch,
+// and a reload waits for every store in flight, the halo rows just sent among
+// them (32 spilled registers: 6.8 us an iteration of a 256x256 cloth, 5.8 without).
+__device__ __forceinline__ unsigned tid_here() { return opaque(threadIdx.x); }
+// Four times the low (0) or high (1) half of a word, in one instruction and
+// anew at every use.
+template <int HALF>
+__device__ __forceinline__ unsigned lds_bytes(unsigned w) {
+    unsigned r;
+    if constexpr (HALF == 0)
+        asm volatile("v_lshlrev_b32_sdwa %0, %2, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0"
+                     : "=v"(r) : "v"(w), "s"(2u));
+    else
+        asm volatile("v_lshlrev_b32_sdwa %0, %2, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1"
+                     : "=v"(r) : "v"(w), "s"(2u));
+    return r;
+}
+
 // The forms of a plan (chysx_hip.h).  Sheet: a row's lower blocks come
 // through product slots and are summed before the upper ones that its thread
 // holds, which is column order.  General: all of a row's products go through
@@ -68,22 +93,26 @@ struct Form {
     // product slots per row
     static constexpr unsigned kPlaces = FORM == SHEET ? CHX_RES_HELD : (FORM == GENERAL ? CHX_RES_GEN_WIDTH : 0);
     static constexpr unsigned kSpare = kPlaces * kRows;  // first of the unread product slots
-    // A held block's word in the plan, and here: the LDS word index of its
-    // source vector entry, of its product slot and its place in the row.
+    static constexpr unsigned kSource = 3 * (kSpare + kWave);  // LDS word of the source vector, behind the products
+    // A held block's word in the plan, and here: the LDS words of its source
+    // vector entry and of its product slot, and its place in the row.
     static __device__ __forceinline__ unsigned unpack(unsigned w, unsigned lane) {
-        if (FORM == ROWS) return 3u * w;
+        if (FORM == ROWS) return kSource + 3u * w;
         const unsigned src = FORM == SHEET ? w & 0xffffu : w & 0x3ffu;
         unsigned slot = FORM == SHEET ? w >> 16 : (w >> 10) & 0x3fffu;
         if (slot == (FORM == SHEET ? 0xffffu : 0x3fffu)) slot = kSpare + lane;
-        return FORM == SHEET ? 3u * src | (3u * slot) << 16 : 3u * src | (3u * slot) << 12 | (w >> 24) << 27;
+        return FORM == SHEET ? (kSource + 3u * src) | (3u * slot) << 16 : 3u * src | (3u * slot) << 12 | (w >> 24) << 27;
     }
+    // LDS byte offsets, formed at every use
     static __device__ __forceinline__ unsigned src(unsigned w) {
-        return FORM == ROWS ? w : w & (FORM == SHEET ? 0xffffu : 0xfffu);
+        return FORM == GENERAL ? 4u * (kSource + (opaque(w) & 0xfffu)) : lds_bytes<0>(w);
     }
-    static __device__ __forceinline__ unsigned slot(unsigned w) { return FORM == SHEET ? w >> 16 : (w >> 12) & 0x7fffu; }
+    static __device__ __forceinline__ unsigned slot(unsigned w) {
+        return FORM == SHEET ? lds_bytes<1>(w) : 4u * ((opaque(w) >> 12) & 0x7fffu);
+    }
     static __device__ __forceinline__ unsigned place(unsigned w) { return w >> 27; }
 };
-static_assert(3 * (Form<SHEET>::kSpare + kWave) < (1u << 16) && 3 * (Form<GENERAL>::kSpare + kWave) < (1u << 15) &&
+static_assert(Form<SHEET>::kSource + 3 * (Form<SHEET>::kRows + CHX_RES_HALO_MAX) < (1u << 16) && 3 * (Form<GENERAL>::kSpare + kWave) < (1u << 15) &&
                   3 * (Form<GENERAL>::kRows + CHX_RES_HALO_MAX) <= (1u << 12) && CHX_RES_GEN_WIDTH <= 16,
               "word fields");
 // Sums of an exchange: merged solver rho, sigma, delta, gamma, ||r||^2
@@ -119,25 +148,26 @@ __device__ __forceinline__ Area exchange_area(const chx_cloth_batch& B) {
 __device__ __forceinline__ v4u ld128(Area a, unsigned at) { return __builtin_amdgcn_raw_buffer_load_b128(a, at, 0, kAgent); }
 __device__ __forceinline__ void st128(Area a, unsigned at, v4u v) { __builtin_amdgcn_raw_buffer_store_b128(v, a, at, 0, kAgent); }
 
-// Triples in LDS, by the index of their first word.
+// Triples in LDS, by the byte offset of their first word in the struct that
+// starts with them, or by its index.
+template <class Lds>
+__device__ __forceinline__ f3 lds_at(const Lds& S, unsigned at) {
+    const float* const m = reinterpret_cast<const float*>(reinterpret_cast<const char*>(&S) + at);
+    return {m[0], m[1], m[2]};
+}
+template <class Lds>
+__device__ __forceinline__ void lds_put(Lds& S, unsigned at, f3 v) {
+    float* const m = reinterpret_cast<float*>(reinterpret_cast<char*>(&S) + at);
+    m[0] = v.x;
+    m[1] = v.y;
+    m[2] = v.z;
+}
 __device__ __forceinline__ f3 lds_ld(const float* m, unsigned i) { return {m[i], m[i + 1u], m[i + 2u]}; }
 __device__ __forceinline__ void lds_st(float* m, unsigned i, f3 v) {
     m[i] = v.x;
     m[i + 1u] = v.y;
     m[i + 2u] = v.z;
 }
-// Keeps a value that the loop does not change from being re-derived ahead of
-// the loop (addresses and masks of every block would not fit the registers).
-__device__ __forceinline__ unsigned opaque(unsigned v) {
-    asm volatile("" : "+v"(v));
-    return v;
-}
-// The thread index for addresses and masks of one use.  What the loop derives
-// from it is derived again: kept over the loop those values went to scratch,
-// and a reload waits for every store in flight, the halo rows just sent among
-// them (32 spilled registers: 6.8 us an iteration of a 256x256 cloth, 5.8 without).
-__device__ __forceinline__ unsigned tid_here() { return opaque(threadIdx.x); }
-
 template <int FORM, bool FULL>
 struct ResLds {
     // products by target row, then one unread slot per lane for blocks
@@ -477,9 +507,10 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     }
     auto halo_minv = [&](f3 v) {
         if constexpr (kHaloInLds) {
+            const unsigned rtid = rtid_here();
             float m[kMinv];
 #pragma unroll
-            for (int c = 0; c < kMinv; ++c) m[c] = S.hminv[c][rtid_here()];
+            for (int c = 0; c < kMinv; ++c) m[c] = S.hminv[c][rtid];
             return apply_minv(m, v);
         } else {
             return apply_minv(hM, v);
@@ -496,7 +527,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             for (int s = 0; s < kSlots; ++s)
                 if (on[s]) {
 #pragma unroll
-                    for (int u = 0; u < kHeld; ++u) lds_st(S.prod, F::slot(opaque(word[s][u])), mv9t(V[s][u], v[s]));
+                    for (int u = 0; u < kHeld; ++u) lds_put(S, F::slot(word[s][u]), mv9t(V[s][u], v[s]));
                 }
         }
         __syncthreads();
@@ -515,14 +546,15 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                 const unsigned lp = row_at(0);
                 f3 src[kHeld];
 #pragma unroll
-                for (int u = 0; u < kHeld; ++u) src[u] = lds_ld(S.p, F::src(opaque(word[0][u])));
+                for (int u = 0; u < kHeld; ++u) src[u] = lds_at(S, F::src(word[0][u]));
 #pragma unroll
                 for (int u = 0; u < kHeld; ++u)
                     if (unsigned(u) < opaque(holds[0]))
                         lds_st(S.prod, 3u * (F::place(opaque(word[0][u])) * kPart + lp), mv9(V[0][u], src[u]));
             }
         }
-        if constexpr (FORM != ROWS) __syncthreads();
+        // a sheet's part without ghost blocks has all its products already
+        if (FORM == GENERAL || (FORM == SHEET && n_ghost > 0u)) __syncthreads();
 #pragma unroll
         for (int s = 0; s < kSlots; ++s)
             if (on[s]) {
@@ -531,7 +563,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                 float d[9];
                 if constexpr (FORM != GENERAL) {
 #pragma unroll
-                    for (int u = 0; u < kHeld; ++u) src[u] = lds_ld(S.p, F::src(opaque(word[s][u])));
+                    for (int u = 0; u < kHeld; ++u) src[u] = lds_at(S, F::src(word[s][u]));
                 }
 #pragma unroll
                 for (int c = 0; c < kDiag; ++c) d[kDiag == 9 ? unsigned(c) : sym6_pos(unsigned(c))] = S.diag[c][lp];
@@ -582,7 +614,6 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     };
     // The sums of exchange t: per leaf, then over the part's leaves, sent to
     // the gang.
-    auto leaf_pair = [&](unsigned v, unsigned i) { return S.leaf[2 * i][v] + S.leaf[2 * i + 1][v]; };
     auto tree8 = [](double w) {  // over eight lanes
         w += dpp64<kXor1>(w);
         w += dpp64<kXor2>(w);
@@ -594,10 +625,12 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         leaf_sums(acc[0], kSlots == 2 ? acc[kSlots - 1] : none, S.leaf, wave);
         __syncthreads();
         const unsigned me = tid_here();
-        if (parts > 1 && me < 8u * N) {
+        if (me < 8u * N) {
             const unsigned v = me >> 3, i = me & 7u;
-            const u64 b = u64(__double_as_longlong(tree8(leaf_pair(v, i))));
-            if (i == 0)
+            const double w = tree8(S.leaf[2 * i][v] + S.leaf[2 * i + 1][v]);
+            const u64 b = u64(__double_as_longlong(w));
+            if (i == 0 && parts == 1) S.tot[v] = w;
+            if (i == 0 && parts > 1)
                 st128(area, line(t, unsigned(part)) + 16u * v, v4u{unsigned(b), tag_of(t), unsigned(b >> 32), tag_of(t)});
         }
     };
@@ -606,8 +639,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     // exchange of 64 parts in a loop of its own, 1.94 the other way).  Above,
     // that is 1280 reads of 16 bytes for 256 parts (2.9 us): there eight lanes
     // read a part's line together and a wave 32 lines (2.6 us), and the waves'
-    // sums meet in LDS.  Then, and for a part that is alone, every wave adds up
-    // the eight last terms by itself.
+    // sums meet in LDS, where every wave adds them up by itself.
     double tot[kSums];
     auto take_sums = [&](int t, unsigned N) -> bool {
         const unsigned lane = tid_here() & unsigned(kWave - 1), tag = tag_of(t);
@@ -656,17 +688,15 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             }
             if (lane < N) S.wsum[wave][lane] = sum;
         }
-        if (parts > 1) {
-            __syncthreads();
-            if (S.bad != 0) return false;
-        }
-        if (parts > 1 && !wide) {
+        __syncthreads();
+        if (S.bad != 0) return false;
+        if (!wide) {
 #pragma unroll
             for (unsigned v = 0; v < unsigned(kSums); ++v)
                 if (v < N) tot[v] = S.tot[v];
         } else {
             double w = 0.0;
-            if (lane < 8u * N) w = wide ? S.wsum[lane & 7u][lane >> 3] : leaf_pair(lane >> 3, lane & 7u);
+            if (lane < 8u * N) w = S.wsum[lane & 7u][lane >> 3];
             w = tree8(w);
             const u64 b = u64(__double_as_longlong(w));
 #pragma unroll
@@ -767,28 +797,21 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             alive(k);
             float alpha = 0.0f, beta = 0.0f;
             if (k > 0) merged_scalars(rho, sig, del, gam, alpha, beta);
-            // halo rows: r_k, z_k, p_k as their owners form them
+            // r_k, z_k, p_k (k = 0: both factors are zero), halo rows as their
+            // owners form them
             if (is_halo() && !last) {
-                if (k > 0) {
-                    hr = axpy(-alpha, h, hr);
-                    const unsigned at = halo_slot();
-                    lds_st(S.p, at, axpy(beta, lds_ld(S.p, at), halo_minv(hr)));
-                } else {
-                    lds_st(S.p, halo_slot(), halo_minv(hr));
-                }
+                hr = axpy(-alpha, h, hr);
+                const unsigned at = halo_slot();
+                lds_st(S.p, at, axpy(beta, lds_ld(S.p, at), halo_minv(hr)));
             }
 #pragma unroll
             for (int s = 0; s < kSlots; ++s)
                 if (on[s]) {
-                    if (k > 0) {
-                        r[s] = axpy(-alpha, q[s], r[s]);
-                        const unsigned at = 3u * row_at(s);
-                        lds_st(S.x, at, axpy(alpha, p[s], lds_ld(S.x, at)));
-                        p[s] = axpy(beta, p[s], apply_minv(M[s], r[s]));
-                    } else {
-                        p[s] = apply_minv(M[s], r[s]);
-                    }
-                    lds_st(S.p, 3u * row_at(s), p[s]);
+                    r[s] = axpy(-alpha, q[s], r[s]);
+                    const unsigned at = 3u * row_at(s);
+                    lds_st(S.x, at, axpy(alpha, p[s], lds_ld(S.x, at)));
+                    p[s] = axpy(beta, p[s], apply_minv(M[s], r[s]));
+                    lds_st(S.p, at, p[s]);
                 }
             if (!last) apply(p, q);
             double acc[kSlots][5];
@@ -796,7 +819,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             for (int s = 0; s < kSlots; ++s) {
 #pragma unroll
                 for (int v = 0; v < 5; ++v) acc[s][v] = 0.0;
-                if (on[s] && live(s)) {
+                if (on[s]) {  // lanes without a row add zeros
                     if (!last && ex[s] != CHX_RES_NONE) send_row(k + 1, ex[s], q[s]);
                     const f3 z = apply_minv(M[s], r[s]);
                     acc[s][0] = dot64(r[s], z);
@@ -888,7 +911,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
 #pragma unroll
             for (int s = 0; s < kSlots; ++s) {
                 sum[s][0] = 0.0;
-                if (on[s] && live(s)) {
+                if (on[s]) {
                     if (ex[s] != CHX_RES_NONE) send_row(t, ex[s], q[s]);
                     sum[s][0] = dot64(p[s], q[s]);
                 }
@@ -904,7 +927,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
 #pragma unroll
             for (int s = 0; s < kSlots; ++s) {
                 acc[s][0] = acc[s][1] = 0.0;
-                if (on[s] && live(s)) {
+                if (on[s]) {
                     const unsigned at = 3u * row_at(s);
                         lds_st(S.x, at, axpy(alpha, p[s], lds_ld(S.x, at)));
                     r[s] = axpy(-alpha, q[s], r[s]);
@@ -942,30 +965,29 @@ __device__ unsigned next_item(const chx_cloth_batch& B, unsigned group, unsigned
         const gp<const int> items = glb(B.res_items);
         const unsigned n_items = unsigned(B.res_n_items - B.res_n_big);
         auto mail = [&](unsigned i) { return &B.xbuf[RES_MAIL + 16ull * (first + stride * i)]; };
-        auto add_idle = [&](unsigned m) {
-            return unsigned(__hip_atomic_fetch_or(idle, u64(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) | m;
+        auto add_idle = [&](u64 m) {
+            return u64(__hip_atomic_fetch_or(idle, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) | m;
         };
-        auto send = [&](unsigned gang, unsigned item) {
+        auto send = [&](u64 gang, unsigned item) {
             unsigned part = 0;
-            for (unsigned m = gang; m != 0u; m &= m - 1u, ++part)
-                st64(mail(unsigned(__ffs(int(m))) - 1u), tagged((item << 8) | (item == kExit ? 0u : part), epoch));
+            for (u64 m = gang; m != 0ull; m &= m - 1ull, ++part)
+                st64(mail(unsigned(__ffsll((long long)m)) - 1u), tagged((item << 8) | (item == kExit ? 0u : part), epoch));
         };
-        unsigned have = add_idle(1u << idx);
+        u64 have = add_idle(1ull << idx);
         unsigned i = unsigned(ld64(next));
         for (;;) {
             if (i >= n_items) {  // nothing left: everyone idle leaves
-                const unsigned m = unsigned(__hip_atomic_exchange(idle, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-                send(m, kExit);
+                send(__hip_atomic_exchange(idle, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), kExit);
                 break;
             }
             const unsigned need = unsigned(items[4 * (unsigned(B.res_n_big) + i) + 1]);
-            if (unsigned(__popc(have)) < need) break;
-            unsigned gang = 0, m = have;
-            for (unsigned c = 0; c < need; ++c, m &= m - 1u) gang |= m & (0u - m);
+            if (unsigned(__popcll(have)) < need) break;
+            u64 gang = 0, m = have;
+            for (unsigned c = 0; c < need; ++c, m &= m - 1ull) gang |= m & (0ull - m);
             u64 expect = have;
-            if (!__hip_atomic_compare_exchange_strong(idle, &expect, u64(have & ~gang), __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+            if (!__hip_atomic_compare_exchange_strong(idle, &expect, have & ~gang, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                       __HIP_MEMORY_SCOPE_AGENT)) {
-                have = unsigned(expect);
+                have = expect;
                 i = unsigned(ld64(next));
                 continue;
             }
@@ -973,7 +995,7 @@ __device__ unsigned next_item(const chx_cloth_batch& B, unsigned group, unsigned
             if (__hip_atomic_compare_exchange_strong(next, &at, u64(i + 1u), __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                      __HIP_MEMORY_SCOPE_AGENT)) {
                 send(gang, unsigned(B.res_n_big) + i);
-                have = unsigned(ld64(idle));
+                have = ld64(idle);
                 i = unsigned(ld64(next));
             } else {
                 have = add_idle(gang);
@@ -1018,8 +1040,8 @@ __global__ __launch_bounds__(kThreads, 2) void resident_kernel(chx_cloth_batch B
         if (!grid_sync(bar, unsigned(G))) return;
     }
     __syncthreads();
-    // groups: workgroups b = x (mod 8), which the dispatcher places on one
-    // XCD, or all of them
+    // groups: workgroups b = x (mod groups); with eight, the dispatcher places
+    // a group on one XCD
     const unsigned groups = unsigned(B.res_groups), group = blockIdx.x % groups, idx = blockIdx.x / groups;
     const unsigned rank = group * (unsigned(G) / groups) + idx;
     int trace_e = 0;

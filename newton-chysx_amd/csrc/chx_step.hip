@@ -1889,7 +1889,7 @@ void validate_batch(const chx_cloth_batch* b) {
                     "chysx: resident plan does not match its instance");
         } else {
             require(b->res_items != nullptr && b->res_n_big >= 0 && b->res_n_items >= b->res_n_big &&
-                        b->res_grid / b->res_groups <= 32,
+                        b->res_grid / b->res_groups <= 64,
                     "chysx: resident solve without its work list");
         }
     }
@@ -2139,7 +2139,8 @@ void solve_bsr3(int n_rows, const float* diag, const int* row_offsets, const int
                 B.single.res_xbase = CHX_RES_CONTROL_WORDS;
                 B.xbuf = plan->xbuf;
                 B.res_xwords = plan->xwords;
-                B.res_grid = single_grid(plan->parts, limit, &B.res_groups);
+                B.res_grid = plan->parts;
+                B.res_groups = 1;
             }
         }
         // The workspace needs no initialisation: every control word is
@@ -2189,13 +2190,6 @@ int chx_pcg_solve_bsr3_plan(int n_rows, const float* diag, const int* row_offset
     return guarded([&] {
         solve_bsr3(n_rows, diag, row_offsets, col_indices, values, b, x, max_iterations, tol, lanes_per_row,
                    workspace, workspace_bytes, nullptr, nullptr, 0, iterations, rr, bb, stream, plan);
-    });
-}
-
-int chx_resident_grid(int parts, int limit, int* grid, int* groups) {
-    return guarded([&] {
-        require(grid != nullptr && groups != nullptr && parts > 0, "chx_resident_grid: bad argument");
-        *grid = single_grid(parts, limit, groups);
     });
 }
 
