@@ -1682,25 +1682,75 @@ __global__ __launch_bounds__(kBlock) void pcg1_kernel(chx_cloth_batch B, int fin
 
 // ---------------------------------------------------------------------------
 // Standalone SpMV: y = alpha A x + beta y (block_csr.cu:54-83).
+//
+// L lanes per row, one row per lane group.  Bound by memory (142 MB for the
+// matrix of a 512x512 grid) if enough loads are in flight: a row's blocks are
+// loaded beside their column indices and the diagonal beside the row offsets,
+// so a row takes three round trips (offsets and diagonal; blocks and indices;
+// source vector), not five.  With the matrix in HBM 34.4 us before, 30.5 now
+// (4.65 TB/s, the rate of a large copy).  Two rows per group (more registers,
+// fewer waves) took 35.5 us, a workgroup order that keeps neighbouring rows on
+// one XCD 31.6.  Per lane the sum is diag (lane 0) + off[sub] + off[sub + L] +
+// ..., then a segmented butterfly.
 // ---------------------------------------------------------------------------
 template <int L>
 __global__ __launch_bounds__(kBlock) void spmv_kernel(int n, const float* __restrict__ diag, const int* __restrict__ ro,
                                                       const int* __restrict__ ci, const float* __restrict__ val,
                                                       const float* __restrict__ x, float* __restrict__ y, float alpha,
                                                       float beta) {
-    constexpr int RPB = (kBlock / kWave) * (kWave / L);  // rows per block
-    const int rb = blockIdx.x * RPB;
-    const int re = min(n, rb + RPB);
-    const gp<const float> xg = glb(x);
+    constexpr unsigned kRows = kBlock / L;            // rows of a workgroup
+    constexpr int U = (16 / L) > 1 ? (16 / L) : 1;    // blocks per lane and pass
+    const gp<const float> xg = glb(x), dg = glb(diag), vg = glb(val);
     const gp<float> yg = glb(y);
     const gp<const int> rog = glb(ro), cig = glb(ci);
-    spmv_core<L>(
-        Mat32G{glb(diag), glb(val)}, rb, re, [&](unsigned r) { return unsigned(ldx(rog, r)); },
-        [&](unsigned k) { return unsigned(ldx(cig, k)); }, [&](unsigned j) { return ld3g(xg, j); },
-        [&](unsigned row, f3 Ax, f3) {
-            if (beta == 0.0f) st3g(yg, row, mul(Ax, alpha));
-            else st3g(yg, row, add(mul(ld3g(yg, row), beta), mul(Ax, alpha)));
-        });
+    const unsigned sub = threadIdx.x % L, at = blockIdx.x * kRows + threadIdx.x / L;
+    const bool valid = at < unsigned(n);
+    const unsigned row = valid ? at : unsigned(n) - 1u;
+    unsigned k0 = unsigned(ldx(rog, row)) + sub;
+    unsigned end = unsigned(ldx(rog, row + 1u));
+    if (!valid) end = 0u;
+    float d[9];
+    f3 xr = mk(0.f, 0.f, 0.f), acc = xr;
+    if (sub == 0) {
+#pragma unroll
+        for (int c = 0; c < 9; ++c) d[c] = rec_at(dg, row, 9u)[c];
+        xr = ld3g(xg, row);
+    }
+    // one pass: blocks k0, k0 + L, ... (clamped to k0 past the end)
+    f3 part[U];
+    auto products = [&] {
+        unsigned kc[U], col[U];
+        float m[U][9];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const unsigned k = k0 + unsigned(u * L);
+            kc[u] = k < end ? k : k0;
+            col[u] = unsigned(ldx(cig, kc[u]));
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int c = 0; c < 9; ++c) m[u][c] = rec_at(vg, kc[u], 9u)[c];
+#pragma unroll
+        for (int u = 0; u < U; ++u) part[u] = mv9(m[u], ld3g(xg, col[u]));
+    };
+    auto add_up = [&] {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (k0 + unsigned(u * L) < end) acc = add(acc, part[u]);
+        k0 += unsigned(U * L);
+    };
+    if (k0 < end) products();
+    if (sub == 0) acc = mv9(d, xr);
+    while (k0 < end) {
+        add_up();
+        if (k0 < end) products();
+    }
+    const f3 sum = mk(seg_sum<L>(acc.x), seg_sum<L>(acc.y), seg_sum<L>(acc.z));
+    if (valid && sub == 0) {
+        if (beta == 0.0f) st3g(yg, row, mul(sum, alpha));
+        else st3g(yg, row, add(mul(ld3g(yg, row), beta), mul(sum, alpha)));
+    }
 }
 
 // ---------------------------------------------------------------------------
