@@ -379,8 +379,36 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     // ghost blocks and halo rows from the last thread down: in a small part
     // the first waves have the rows
     auto rtid_here = [] { return unsigned(kThreads - 1) - tid_here(); };
+    auto halo_slot = [&] { return 3u * (kPart + rtid_here()); };
+    auto is_halo = [&] { return rtid_here() < n_halo; };
+    auto is_ghost = [&] { return FORM != ROWS && rtid_here() < n_ghost; };
+    auto position = [&](int s) { return pos0 + (live(s) ? row_at(s) : 0u); };
+    // Where the blocks of a row are (one slot per block in the general form).
+    struct Where {
+        unsigned row, first, slot[FORM == GENERAL ? kHeld : 1];
+    };
+    auto locate = [&](Where (&w)[kSlots], unsigned& ghost) {
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) {
+            const unsigned K = position(s);
+            w[s].row = ldx(plan, rows_at + K);
+            if constexpr (FORM == GENERAL) {
+#pragma unroll
+                for (int u = 0; u < kHeld; ++u) w[s].slot[u] = ldx(plan, held_at + unsigned(kHeld + u) * n + K);
+            }
+        }
+        ghost = is_ghost() ? ldx(plan, ghost_at + 2u * rtid_here()) : 0u;
+    };
+    auto find_first = [&](Where (&w)[kSlots]) {
+        if constexpr (FORM != GENERAL)
+#pragma unroll
+            for (int s = 0; s < kSlots; ++s)
+                w[s].first = FORM == ROWS ? unsigned(ldx(I.row_offsets, w[s].row))
+                                          : unsigned(ldx(I.upper_offsets, w[s].row / CHX_SLICE_ROWS)) +
+                                                w[s].row % CHX_SLICE_ROWS;
+    };
     // the matrix blocks: FP32, or the BF16 copies and compensated diagonal
-    auto load_blocks = [&](bool half) {
+    auto load_blocks = [&](bool half, const Where (&w)[kSlots], unsigned ghost) {
         auto block = [&](unsigned v, float (&m)[9]) {
             if (FORM == ROWS) {
                 const gp<const float> b = rec_at(gp<const float>(I.values), v, 9u);
@@ -396,115 +424,129 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
 #pragma unroll
         for (int s = 0; s < kSlots; ++s)
             if (on[s]) {
-                const unsigned lp = row_at(s);
-                const unsigned K = pos0 + (lp < n_own ? lp : 0u);
-                const unsigned row = ldx(plan, rows_at + K);
-                const unsigned first = FORM == ROWS ? unsigned(ldx(I.row_offsets, row))
-                                                    : unsigned(ldx(I.upper_offsets, row / CHX_SLICE_ROWS)) +
-                                                          row % CHX_SLICE_ROWS;
 #pragma unroll
                 for (int u = 0; u < kHeld; ++u) {
 #pragma unroll
                     for (int c = 0; c < 9; ++c) V[s][u][c] = 0.0f;
                     if (unsigned(u) < holds[s]) {
-                        unsigned v = first + unsigned(u) * (FORM == ROWS ? 1u : unsigned(CHX_SLICE_ROWS));
-                        if (FORM == GENERAL) v = ldx(plan, held_at + unsigned(kHeld + u) * n + K);
-                        block(v, V[s][u]);
+                        if constexpr (FORM == GENERAL) block(w[s].slot[u], V[s][u]);
+                        else block(w[s].first + unsigned(u) * (FORM == ROWS ? 1u : unsigned(CHX_SLICE_ROWS)), V[s][u]);
                     }
                 }
-                float d[9];
-                if (FORM == ROWS) {
-                    const gp<const float> b = rec_at(gp<const float>(I.diag), row, 9u);
-#pragma unroll
-                    for (int c = 0; c < 9; ++c) d[c] = b[c];
-                } else if (TWO && half) {
-                    ld9p(gp<const float>(I.diag_c), row, d);
-                } else {
-                    ld6p(gp<const float>(I.diag), row, d);
-                }
-#pragma unroll
-                for (unsigned c = 0; c < unsigned(kDiag); ++c) S.diag[c][lp] = d[kDiag == 9 ? c : sym6_pos(c)];
             }
-        const unsigned rtid = rtid_here();
-        if (FORM != ROWS && rtid < n_ghost) {
+        if (is_ghost()) {
             float g[9];
-            block(ldx(plan, ghost_at + 2u * rtid), g);
+            block(ghost, g);
+            const unsigned rtid = rtid_here();
 #pragma unroll
             for (int c = 0; c < 9; ++c) S.ghost[c][rtid] = g[c];
         }
+    };
+    auto load_diag = [&](bool half, unsigned row, float (&d)[9]) {
+        if (FORM == ROWS) {
+            const gp<const float> b = rec_at(gp<const float>(I.diag), row, 9u);
+#pragma unroll
+            for (int c = 0; c < 9; ++c) d[c] = b[c];
+        } else if (TWO && half) {
+            ld9p(gp<const float>(I.diag_c), row, d);
+        } else {
+            ld6p(gp<const float>(I.diag), row, d);
+        }
+    };
+    auto keep_diag = [&](int s, const float (&d)[9]) {
+        const unsigned lp = row_at(s);
+#pragma unroll
+        for (unsigned c = 0; c < unsigned(kDiag); ++c) S.diag[c][lp] = d[kDiag == 9 ? c : sym6_pos(c)];
     };
     auto apply_minv = [&](const float (&m)[kMinv], f3 v) {
         if constexpr (FORM == ROWS) return mv9(m, v);
         else return mv_sym(m, v);
     };
-    auto invert = [&](unsigned row, float (&m)[kMinv]) {
-        float d[9], full[9];
-        if (FORM == ROWS) {
-            const gp<const float> b = rec_at(gp<const float>(I.diag), row, 9u);
-#pragma unroll
-            for (int c = 0; c < 9; ++c) d[c] = b[c];
-        } else {
-            ld6p(gp<const float>(I.diag), row, d);
-        }
+    auto invert = [&](const float (&d)[9], float (&m)[kMinv]) {
+        float full[9];
         inverse9(d, full);
 #pragma unroll
         for (unsigned c = 0; c < unsigned(kMinv); ++c) m[c] = full[kMinv == 9 ? c : sym6_pos(c)];
     };
+    // The set-up is a chain of round trips to memory, so each link's loads are
+    // issued together: the plan's words of the rows, halo rows and ghost
+    // blocks; then diagonals, vectors and block offsets; then the blocks.
+    Where where[kSlots];
+    unsigned ghost, meta[kSlots], gword = 0, hrow = 0, hex = 0;
+    locate(where, ghost);
 #pragma unroll
     for (int s = 0; s < kSlots; ++s) {
-        const unsigned lp = row_at(s);
         on[s] = (unsigned(s) * kWaves + wave) * kWave < n_own;
-        const unsigned K = pos0 + (lp < n_own ? lp : 0u);
-        ex[s] = CHX_RES_NONE;
-        holds[s] = 0u;
-        r[s] = p[s] = q[s] = mk(0.f, 0.f, 0.f);
-        if (on[s]) {
-            unsigned ns = 0u;
-            const unsigned row = ldx(plan, rows_at + K);
-            const unsigned meta = ldx(plan, meta_at + K);
-            if (lp < n_own) {
-                ns = meta & 255u;
-                holds[s] = meta >> 8;
-                ex[s] = ldx(plan, exp_at + K);
-            }
+        const unsigned K = position(s);
+        meta[s] = ldx(plan, meta_at + K);
+        ex[s] = ldx(plan, exp_at + K);
 #pragma unroll
-            for (int u = 0; u < kHeld; ++u) {
-                // a block that is not there is zero, of the row itself
-                unsigned w = FORM == SHEET ? (0xffffu << 16) | lp : (FORM == GENERAL ? (0x3fffu << 10) | lp : lp);
-                if (unsigned(u) < holds[s]) w = ldx(plan, held_at + unsigned(u) * n + K);
-                word[s][u] = F::unpack(w, lane);
-            }
-            // product slots that no block fills stay zero and are added like
-            // the others
-#pragma unroll
-            for (unsigned u = 0; u < F::kPlaces; ++u)
-                if (u >= ns) lds_st(S.prod, 3u * (u * kPart + lp), mk(0.f, 0.f, 0.f));
-            invert(row, M[s]);
-            if (lp < n_own) p[s] = ld3g(I.x, row);
-            lds_st(S.x, 3u * lp, p[s]);
-            lds_st(S.p, 3u * lp, p[s]);
-        }
+        for (int u = 0; u < kHeld; ++u) word[s][u] = ldx(plan, held_at + unsigned(u) * n + K);
     }
-    if constexpr (!TWO) load_blocks(false);
-    unsigned gword = 0;  // the ghost block's source and product slot
-    if (FORM != ROWS && rtid_here() < n_ghost) gword = ldx(plan, ghost_at + 2u * rtid_here() + 1u);
+    if (is_ghost()) gword = ldx(plan, ghost_at + 2u * rtid_here() + 1u);  // its source and product slot
+    if (is_halo()) {
+        hrow = ldx(plan, halo_at + 2u * rtid_here());
+        hex = ldx(plan, halo_at + 2u * rtid_here() + 1u);
+    }
     constexpr bool kHaloInLds = FORM == SHEET;
     float hM[kMinv];
     f3 hr = mk(0.f, 0.f, 0.f);
-    unsigned hex = 0;
-    auto halo_slot = [&] { return 3u * (kPart + rtid_here()); };
-    auto is_halo = [&] { return rtid_here() < n_halo; };
-    if (is_halo()) {
-        const unsigned rtid = rtid_here();
-        const unsigned hrow = ldx(plan, halo_at + 2u * rtid);
-        hex = ldx(plan, halo_at + 2u * rtid + 1u);
-        invert(hrow, hM);
-        if constexpr (kHaloInLds) {
+    {
+        find_first(where);
+        float d[kSlots][9], hd[9];
+        f3 hx = hr;
 #pragma unroll
-            for (int c = 0; c < kMinv; ++c) S.hminv[c][rtid] = hM[c];
+        for (int s = 0; s < kSlots; ++s) {
+            load_diag(false, where[s].row, d[s]);
+            p[s] = ld3g(I.x, where[s].row);
+            r[s] = ld3g(I.rhs, where[s].row);
         }
-        lds_st(S.p, halo_slot(), ld3g(I.x, hrow));
+        if (is_halo()) {
+            load_diag(false, hrow, hd);
+            hx = ld3g(I.x, hrow);
+        }
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) {
+            const bool has = live(s);
+            const unsigned lp = row_at(s), ns = has ? meta[s] & 255u : 0u;
+            holds[s] = has ? meta[s] >> 8 : 0u;
+            if (!has) {
+                ex[s] = CHX_RES_NONE;
+                r[s] = p[s] = mk(0.f, 0.f, 0.f);
+            }
+            q[s] = mk(0.f, 0.f, 0.f);
+#pragma unroll
+            for (int u = 0; u < kHeld; ++u) {
+                // a block that is not there is zero, of the row itself
+                const unsigned none = FORM == SHEET ? (0xffffu << 16) | lp : (FORM == GENERAL ? (0x3fffu << 10) | lp : lp);
+                word[s][u] = F::unpack(unsigned(u) < holds[s] ? word[s][u] : none, lane);
+            }
+            if (on[s]) {
+                // product slots that no block fills stay zero and are added
+                // like the others
+#pragma unroll
+                for (unsigned u = 0; u < F::kPlaces; ++u)
+                    if (u >= ns) lds_st(S.prod, 3u * (u * kPart + lp), mk(0.f, 0.f, 0.f));
+                keep_diag(s, d[s]);
+                lds_st(S.x, 3u * lp, p[s]);
+                lds_st(S.p, 3u * lp, p[s]);
+            }
+            invert(d[s], M[s]);
+        }
+        if (is_halo()) {
+            invert(hd, hM);
+            if constexpr (kHaloInLds) {
+                const unsigned rtid = rtid_here();
+#pragma unroll
+                for (int c = 0; c < kMinv; ++c) S.hminv[c][rtid] = hM[c];
+            }
+            lds_st(S.p, halo_slot(), hx);
+        }
     }
+    load_blocks(false, where, ghost);
+    // vmcnt(0): with no load pending at its entry the loop waits for none (and
+    // so for none of its stores) where it uses what was loaded here
+    __builtin_amdgcn_s_waitcnt(0x0f70);
     auto halo_minv = [&](f3 v) {
         if constexpr (kHaloInLds) {
             const unsigned rtid = rtid_here();
@@ -532,8 +574,8 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         }
         __syncthreads();
         if constexpr (FORM != ROWS) {
-            const unsigned rtid = rtid_here();
-            if (rtid < n_ghost) {
+            if (is_ghost()) {
+                const unsigned rtid = rtid_here();
                 float g[9];
 #pragma unroll
                 for (int c = 0; c < 9; ++c) g[c] = S.ghost[c][rtid];
@@ -754,7 +796,8 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         for (int s = 0; s < kSlots; ++s) {
             acc[s][0] = acc[s][1] = acc[s][2] = 0.0;
             if (on[s] && live(s)) {
-                const f3 b = ld3g(I.rhs, ldx(plan, rows_at + pos0 + row_at(s)));
+                // at the set-up r holds b
+                const f3 b = t > 0 ? ld3g(I.rhs, ldx(plan, rows_at + pos0 + row_at(s))) : r[s];
                 r[s] = sub(b, q[s]);
                 if (ex[s] != CHX_RES_NONE) send_row(t, ex[s], r[s]);
                 acc[s][0] = dot64(r[s], apply_minv(M[s], r[s]));
@@ -845,7 +888,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         bool residual_step = true;        // set-up, then refinement: r = b - A x, x in p and S.p
         bool exact = true, fresh = true;  // rr is of b - A x; p starts from z
         int k = 0, refines = -1, t = -1;  // t: the last exchange
-        int blocks = -1;                  // which matrix V holds
+        int blocks = 0;                   // which matrix V holds
         for (;;) {
             if (!residual_step) {
                 const bool met = I.tol > 0.0 && rr <= I.tol * I.tol * bb;
@@ -888,7 +931,19 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             }
             const int want = half && !residual_step ? 1 : 0;
             if (want != blocks) {
-                load_blocks(want != 0);
+                Where at[kSlots];
+                unsigned g;
+                locate(at, g);
+                find_first(at);
+                load_blocks(want != 0, at, g);
+#pragma unroll
+                for (int s = 0; s < kSlots; ++s)
+                    if (on[s]) {
+                        float d[9];
+                        load_diag(want != 0, at[s].row, d);
+                        keep_diag(s, d);
+                    }
+                __builtin_amdgcn_s_waitcnt(0x0f70);
                 blocks = want;
             }
             apply(p, q);
