@@ -177,6 +177,9 @@ typedef struct chx_unit {
  * | product slot << 16.  A product slot is (place among the target row's
  * lower blocks) * CHX_RES_PART_MAX + (target's position); 0xffff: none.
  *
+ * Half-sheet form (res_form 3, BF16 mode): the sheet form with a part capacity of
+ * CHX_RES_GEN_PART rows in local indices and product slots.
+ *
  * General form (res_form 1; at most CHX_RES_GEN_WIDTH blocks a row, parts
  * of at most CHX_RES_GEN_PART rows): every pair's block is held by one of
  * its rows, at most CHX_RES_GEN_HELD a row: CHX_RES_GEN_HELD planes of words
@@ -191,6 +194,10 @@ typedef struct chx_unit {
  * CHX_RES_ROW_WIDTH blocks a row, parts of at most CHX_RES_GEN_PART rows):
  * every row holds all of its blocks, in CSR order: CHX_RES_ROW_WIDTH planes
  * of local column indices; no product slots, no ghost blocks. */
+#define CHX_RES_FORM_SHEET 0
+#define CHX_RES_FORM_GENERAL 1
+#define CHX_RES_FORM_ROWS 2
+#define CHX_RES_FORM_HALF 3
 #define CHX_RES_ROW_WIDTH 12
 #define CHX_RES_GEN_PART 512
 #define CHX_RES_GEN_HELD 8

@@ -84,31 +84,37 @@ __device__ __forceinline__ unsigned lds_bytes(unsigned w) {
 // holds, which is column order.  General: all of a row's products go through
 // its slots, in column order; twice the slots and wider rows, so half the
 // rows.  Rows: a caller's matrix, every row holding all of its own blocks.
-enum { SHEET = 0, GENERAL = 1, ROWS = 2 };
+// Half sheet: a sheet's plan for 512 rows, one row a thread, which leaves
+// registers for the two-reduction solver (at 1024 rows it would spill 430).
+// BF16 mode, four substeps of a 128x128 cloth: 2.30 ms, on a general plan with
+// its longer rows of product slots 2.56.  For FP32 solves of small parts it is
+// no faster than the sheet kernel with half its threads' rows idle.
+enum { SHEET = CHX_RES_FORM_SHEET, GENERAL = CHX_RES_FORM_GENERAL, ROWS = CHX_RES_FORM_ROWS, HALF = CHX_RES_FORM_HALF };
 template <int FORM>
 struct Form {
+    static constexpr bool kSheet = FORM == SHEET || FORM == HALF;
     static constexpr unsigned kRows = FORM == SHEET ? CHX_RES_PART_MAX : CHX_RES_GEN_PART;
     static constexpr int kSlots = kRows / kThreads;  // own rows per thread
-    static constexpr int kHeld = FORM == SHEET ? CHX_RES_HELD : (FORM == GENERAL ? CHX_RES_GEN_HELD : CHX_RES_ROW_WIDTH);
+    static constexpr int kHeld = kSheet ? CHX_RES_HELD : (FORM == GENERAL ? CHX_RES_GEN_HELD : CHX_RES_ROW_WIDTH);
     // product slots per row
-    static constexpr unsigned kPlaces = FORM == SHEET ? CHX_RES_HELD : (FORM == GENERAL ? CHX_RES_GEN_WIDTH : 0);
+    static constexpr unsigned kPlaces = kSheet ? CHX_RES_HELD : (FORM == GENERAL ? CHX_RES_GEN_WIDTH : 0);
     static constexpr unsigned kSpare = kPlaces * kRows;  // first of the unread product slots
     static constexpr unsigned kSource = 3 * (kSpare + kWave);  // LDS word of the source vector, behind the products
     // A held block's word in the plan, and here: the LDS words of its source
     // vector entry and of its product slot, and its place in the row.
     static __device__ __forceinline__ unsigned unpack(unsigned w, unsigned lane) {
         if (FORM == ROWS) return kSource + 3u * w;
-        const unsigned src = FORM == SHEET ? w & 0xffffu : w & 0x3ffu;
-        unsigned slot = FORM == SHEET ? w >> 16 : (w >> 10) & 0x3fffu;
-        if (slot == (FORM == SHEET ? 0xffffu : 0x3fffu)) slot = kSpare + lane;
-        return FORM == SHEET ? (kSource + 3u * src) | (3u * slot) << 16 : 3u * src | (3u * slot) << 12 | (w >> 24) << 27;
+        const unsigned src = kSheet ? w & 0xffffu : w & 0x3ffu;
+        unsigned slot = kSheet ? w >> 16 : (w >> 10) & 0x3fffu;
+        if (slot == (kSheet ? 0xffffu : 0x3fffu)) slot = kSpare + lane;
+        return kSheet ? (kSource + 3u * src) | (3u * slot) << 16 : 3u * src | (3u * slot) << 12 | (w >> 24) << 27;
     }
     // LDS byte offsets, formed at every use
     static __device__ __forceinline__ unsigned src(unsigned w) {
         return FORM == GENERAL ? 4u * (kSource + (opaque(w) & 0xfffu)) : lds_bytes<0>(w);
     }
     static __device__ __forceinline__ unsigned slot(unsigned w) {
-        return FORM == SHEET ? lds_bytes<1>(w) : 4u * ((opaque(w) >> 12) & 0x7fffu);
+        return kSheet ? lds_bytes<1>(w) : 4u * ((opaque(w) >> 12) & 0x7fffu);
     }
     static __device__ __forceinline__ unsigned place(unsigned w) { return w >> 27; }
 };
@@ -518,7 +524,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
 #pragma unroll
             for (int u = 0; u < kHeld; ++u) {
                 // a block that is not there is zero, of the row itself
-                const unsigned none = FORM == SHEET ? (0xffffu << 16) | lp : (FORM == GENERAL ? (0x3fffu << 10) | lp : lp);
+                const unsigned none = F::kSheet ? (0xffffu << 16) | lp : (FORM == GENERAL ? (0x3fffu << 10) | lp : lp);
                 word[s][u] = F::unpack(unsigned(u) < holds[s] ? word[s][u] : none, lane);
             }
             if (on[s]) {
@@ -596,7 +602,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             }
         }
         // a sheet's part without ghost blocks has all its products already
-        if (FORM == GENERAL || (FORM == SHEET && n_ghost > 0u)) __syncthreads();
+        if (FORM == GENERAL || (F::kSheet && n_ghost > 0u)) __syncthreads();
 #pragma unroll
         for (int s = 0; s < kSlots; ++s)
             if (on[s]) {
@@ -615,7 +621,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                     d[7] = d[5];
                 }
                 f3 sum;
-                if constexpr (FORM == SHEET) {
+                if constexpr (F::kSheet) {
 #pragma unroll
                     for (int l = 0; l < kHeld; ++l) low[l] = lds_ld(S.prod, 3u * (unsigned(l) * kPart + lp));
                     sum = mv9(d, v[s]);
@@ -1142,8 +1148,7 @@ using ResFn = void (*)(chx_cloth_batch, int);
 // form: a plan's; two: the two-reduction solver (always for a caller's rows)
 ResFn resident_fn(int form, bool two) {
     if (form == ROWS) return resident_kernel<ROWS, true>;
-    // the BF16 mode's plans are general ones: at 1024 rows its kernel would
-    // spill 430 registers
+    if (form == HALF) return resident_kernel<HALF, true>;
     if (form == GENERAL) return two ? resident_kernel<GENERAL, true> : resident_kernel<GENERAL, false>;
     return resident_kernel<SHEET, false>;
 }
@@ -1163,7 +1168,7 @@ int resident_grid_limit() {
         hipDeviceProp_t prop;
         hip_check(hipGetDeviceProperties(&prop, dev), "hipGetDeviceProperties");
         bool fits = true;
-        for (int form : {SHEET, GENERAL, ROWS})
+        for (int form : {SHEET, HALF, GENERAL, ROWS})
             for (bool two : {false, true}) {
                 int per_cu = 0;
                 hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(

@@ -1851,13 +1851,13 @@ int pcg_variant(const chx_cloth_batch& B, bool row_major) {
 }
 
 // Whether the resident kernel takes the launch: instances that all have a
-// plan, in the default solver form (BF16 mode: general plans), or a caller's
-// rows with one.
+// plan of a form for the solver (sheets FP32, half sheets BF16, general plans
+// both), in the default solver form, or a caller's rows with one.
 bool resident(const chx_cloth_batch& B, bool row_major) {
     if (B.res_grid <= 0) return false;
-    if (row_major) return B.res_form == 2;
-    if (B.bf16_blocks != 0) return B.res_form == 1 && B.no_lds_staging == 0;
-    return B.res_form <= 1 && B.pcg_form == 0 && B.no_lds_staging == 0;
+    if (row_major || B.res_form == CHX_RES_FORM_ROWS) return row_major && B.res_form == CHX_RES_FORM_ROWS;
+    if (B.no_lds_staging != 0) return false;
+    return B.bf16_blocks != 0 ? B.res_form != CHX_RES_FORM_SHEET : B.res_form != CHX_RES_FORM_HALF && B.pcg_form == 0;
 }
 
 void launch_pcg(const chx_cloth_batch& B, int finalize, hipStream_t stream, bool row_major = false) {
@@ -1932,8 +1932,8 @@ void validate_batch(const chx_cloth_batch* b) {
                          (I.res_part_rows == 256 || I.res_part_rows == 512 || I.res_part_rows == CHX_RES_PART_MAX) &&
                          I.res_parts == (I.n_rows + I.res_part_rows - 1) / I.res_part_rows &&
                          I.res_parts <= b->res_grid && I.res_exports >= 0 &&
-                         (I.res_form != 0) == (b->res_form != 0) &&
-                         (b->res_form == 0 || I.res_part_rows <= CHX_RES_GEN_PART) &&
+                         I.res_form == b->res_form &&
+                         (b->res_form == CHX_RES_FORM_SHEET || I.res_part_rows <= CHX_RES_GEN_PART) &&
                          I.res_xbase % 16 == 0 &&
                          I.res_xbase + CHX_RES_XWORDS(I.res_parts, I.res_exports) <= b->res_xwords),
                     "chysx: resident plan does not match its instance");
@@ -2185,7 +2185,7 @@ void solve_bsr3(int n_rows, const float* diag, const int* row_offsets, const int
                 B.single.res_part_rows = plan->part_rows;
                 B.single.res_parts = plan->parts;
                 B.single.res_exports = plan->exports;
-                B.single.res_form = B.res_form = 2;
+                B.single.res_form = B.res_form = CHX_RES_FORM_ROWS;
                 B.single.res_xbase = CHX_RES_CONTROL_WORDS;
                 B.xbuf = plan->xbuf;
                 B.res_xwords = plan->xwords;

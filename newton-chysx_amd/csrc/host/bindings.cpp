@@ -513,8 +513,8 @@ PYBIND11_MODULE(_chysx_native, m) {
         py::arg("n"), py::arg("rows"), py::arg("cols"));
     topo.def(
         "resident_plan",
-        [](int n, IArr row_offsets, IArr col_indices, IArr block_slots, int part_rows,
-           bool general) -> py::object {
+        [](int n, IArr row_offsets, IArr col_indices, IArr block_slots, int part_rows, bool general,
+           int capacity) -> py::object {
             // Canonical row order and part image of the resident solve, or
             // None when the pattern does not fit it.
             chysx::topology::Pattern p;
@@ -524,7 +524,7 @@ PYBIND11_MODULE(_chysx_native, m) {
             const std::vector<int> bs(block_slots.data(), block_slots.data() + block_slots.size());
             const std::vector<int> order = chysx::engine::resident_order(p);
             const auto r = general ? chysx::engine::resident_plan_general(p, bs, order, part_rows)
-                                   : chysx::engine::resident_plan(p, bs, order, part_rows);
+                                   : chysx::engine::resident_plan(p, bs, order, part_rows, capacity);
             if (r.blob.empty()) return py::none();
             py::dict d;
             d["order"] = to_array(order);
@@ -536,7 +536,7 @@ PYBIND11_MODULE(_chysx_native, m) {
             return d;
         },
         py::arg("n"), py::arg("row_offsets"), py::arg("col_indices"), py::arg("block_slots"), py::arg("part_rows"),
-        py::arg("general") = false);
+        py::arg("general") = false, py::arg("capacity") = CHX_RES_PART_MAX);
     topo.def(
         "cloth_system",
         [](int n, IArr tris, IArr pins, bool stretch, bool shear, bool bending) {

@@ -32,16 +32,15 @@ std::vector<chx_instance> ClothBatch::descriptors(float dt, std::uintptr_t cuda_
     std::vector<int> rows;
     for (ClothSimulator* s : sims_) rows.push_back(s->buffers().particle_count());
     std::vector<chx_instance> ds;
-    // the resident solve wants all plans in one form: sheets, or else general
-    // (the BF16 solve: general)
-    for (bool general : {false, true}) {
-        if (bf16_ && !general) continue;
-        const int part_rows = engine::resident_part_rows(rows, general ? CHX_RES_GEN_PART : CHX_RES_PART_MAX);
+    // the resident solve wants all plans in one form
+    std::vector<engine::ResidentChoice> choices = engine::resident_choices(rows, bf16_);
+    if (choices.empty()) choices.push_back({0, 0});
+    for (const engine::ResidentChoice& c : choices) {
         ds.clear();
         ds.reserve(sims_.size());
         bool all = true;
         for (ClothSimulator* s : sims_) {
-            ds.push_back(s->prepare_instance(dt, cuda_stream, part_rows, general));
+            ds.push_back(s->prepare_instance(dt, cuda_stream, c));
             if (bf16_ && ds.back().n_rows > 0 && ds.back().diag_c == nullptr)
                 throw std::invalid_argument(
                     "ClothBatch: BF16 mode needs every instance switched with set_bf16_blocks(true)");

@@ -352,18 +352,14 @@ void ClothSimulator::step(float dt, std::uintptr_t cuda_stream) {
 // The descriptor of the simulator's own (single-instance) launches.
 chx_instance ClothSimulator::single_descriptor(const engine::InstanceSource& s, std::uintptr_t stream) {
     chx_instance d = inst_.descriptor(s);
-    // the BF16 solve takes general plans only
-    for (bool general : {false, true})
-        if (general || !bf16_) {
-            const int most = general ? CHX_RES_GEN_PART : CHX_RES_PART_MAX;
-            inst_.attach_plan(d, pattern_, engine::resident_part_rows({s.n}, most), general, stream);
-            if (d.res_plan != nullptr) break;
-        }
+    for (const engine::ResidentChoice& c : engine::resident_choices({s.n}, bf16_)) {
+        inst_.attach_plan(d, pattern_, c, stream);
+        if (d.res_plan != nullptr) break;
+    }
     return d;
 }
 
-chx_instance ClothSimulator::prepare_instance(float dt, std::uintptr_t cuda_stream, int part_rows,
-                                             bool general) {
+chx_instance ClothSimulator::prepare_instance(float dt, std::uintptr_t cuda_stream, engine::ResidentChoice choice) {
     const int n = buffers_.particle_count();
     if (n <= 0) throw std::runtime_error("ClothSimulator::prepare_instance: no particles bound");
     if (buffers_.pos.data() == nullptr || buffers_.vel.data() == nullptr)
@@ -375,7 +371,7 @@ chx_instance ClothSimulator::prepare_instance(float dt, std::uintptr_t cuda_stre
     engine::InstanceSource s = source();
     s.dt = dt;
     chx_instance d = inst_.descriptor(s);
-    inst_.attach_plan(d, pattern_, part_rows, general, cuda_stream);
+    inst_.attach_plan(d, pattern_, choice, cuda_stream);
     return d;
 }
 

@@ -213,8 +213,7 @@ public:
     // Builds (or refreshes) this cloth's device arrays without stepping and
     // returns the launch descriptor for substep `dt`; ClothBatch uses it to
     // advance this cloth as one instance of a batch.
-    chx_instance prepare_instance(float dt, std::uintptr_t cuda_stream = 0, int part_rows = 0,
-                                  bool general = false);
+    chx_instance prepare_instance(float dt, std::uintptr_t cuda_stream = 0, engine::ResidentChoice choice = {0, 0});
     // Builds the Hessian pattern, scatter maps and device arrays now (the
     // first step would otherwise do it), so the set-up of a cloth can run
     // ahead of its first step, e.g. on another host thread.

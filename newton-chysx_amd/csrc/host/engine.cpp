@@ -684,19 +684,21 @@ chx_instance InstanceData::descriptor(const InstanceSource& s) const {
     return I;
 }
 
-void InstanceData::attach_plan(chx_instance& d, const topology::Pattern& p, int part_rows, bool general,
-                               std::uintptr_t stream) {
+void InstanceData::attach_plan(chx_instance& d, const topology::Pattern& p, ResidentChoice c, std::uintptr_t stream) {
     d.res_plan = nullptr;
+    int part_rows = c.part_rows;
     if (part_rows == 0 || n_ == 0) return;
     // what one workgroup holds needs no exchange (resident_part_rows)
-    const int most = general ? CHX_RES_GEN_PART : CHX_RES_PART_MAX;
+    const int most = c.form == CHX_RES_FORM_SHEET ? CHX_RES_PART_MAX : CHX_RES_GEN_PART;
     if (n_ <= most) part_rows = most;
-    Plan& pl = plans_[(general ? 3 : 0) + (part_rows == 256 ? 0 : (part_rows == 512 ? 1 : 2))];
+    const int first = c.form == CHX_RES_FORM_SHEET ? 0 : (c.form == CHX_RES_FORM_HALF ? 3 : 5);
+    Plan& pl = plans_[first + (part_rows == 256 ? 0 : (part_rows == 512 ? 1 : 2))];
     if (!pl.tried) {
         pl.tried = true;
         if (order_.empty()) order_ = resident_order(p);
-        ResidentPlan r = general ? resident_plan_general(p, block_slots_.host(), order_, part_rows)
-                                 : resident_plan(p, block_slots_.host(), order_, part_rows);
+        ResidentPlan r = c.form == CHX_RES_FORM_GENERAL
+                             ? resident_plan_general(p, block_slots_.host(), order_, part_rows)
+                             : resident_plan(p, block_slots_.host(), order_, part_rows, most);
         if (!r.blob.empty()) {
             pl.parts = r.parts;
             pl.exports = r.exports;
@@ -711,7 +713,7 @@ void InstanceData::attach_plan(chx_instance& d, const topology::Pattern& p, int 
     d.res_part_rows = part_rows;
     d.res_parts = pl.parts;
     d.res_exports = pl.exports;
-    d.res_form = general ? 1 : 0;
+    d.res_form = c.form;
 }
 
 // ---------------------------------------------------------------------------

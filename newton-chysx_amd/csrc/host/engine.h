@@ -71,11 +71,10 @@ public:
     void update_shapes(const InstanceSource& s, std::uintptr_t stream = 0);
     // Descriptor for a launch: device arrays + the step scalars of `s`.
     chx_instance descriptor(const InstanceSource& s) const;
-    // Adds the resident-solve plan for parts of `part_rows` rows to a
-    // descriptor (none when the pattern does not fit it, or part_rows is 0).
+    // Adds the resident-solve plan of a form and part size to a descriptor
+    // (none when the pattern does not fit it, or the part size is 0).
     // Plans are built on first use and kept until the next build().
-    // `general`: the general form (parts of at most CHX_RES_GEN_PART rows).
-    void attach_plan(chx_instance& d, const topology::Pattern& p, int part_rows, bool general, std::uintptr_t stream);
+    void attach_plan(chx_instance& d, const topology::Pattern& p, ResidentChoice c, std::uintptr_t stream);
     bool built() const noexcept { return built_; }
     int n_rows() const noexcept { return n_; }
     int nnz() const noexcept { return nnz_; }
@@ -127,7 +126,7 @@ private:
         int parts = 0, exports = 0;
         DeviceArray<std::uint32_t> blob;
     };
-    Plan plans_[5];           // sheet form with parts of 256, 512 and 1024 rows, general form with 256 and 512
+    Plan plans_[7];           // sheets (parts of 256, 512, 1024 rows), half sheets and general form (256, 512)
     std::vector<int> order_;  // canonical row order of the plans
     DeviceArray<chx_plane> planes_;
     DeviceArray<chx_box> boxes_;

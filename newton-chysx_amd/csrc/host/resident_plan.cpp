@@ -229,9 +229,9 @@ struct Builder {
 }  // namespace
 
 ResidentPlan resident_plan(const topology::Pattern& p, const std::vector<int>& block_slots,
-                           const std::vector<int>& order, int part_rows) {
+                           const std::vector<int>& order, int part_rows, int capacity) {
     const int n = p.n;
-    if (n <= 0 || part_rows > CHX_RES_PART_MAX) return {};
+    if (n <= 0 || part_rows > capacity || capacity > CHX_RES_PART_MAX) return {};
     const auto& ro = p.row_offsets;
     const auto& ci = p.col_indices;
     // lower[k]: place of upper block (i, j)'s transpose among row j's lower blocks
@@ -244,17 +244,17 @@ ResidentPlan resident_plan(const topology::Pattern& p, const std::vector<int>& b
         if (ro[i + 1] - k > CHX_RES_HELD || k - ro[i] > CHX_RES_HELD) return {};
         for (; k < ro[i + 1]; ++k) lower[k] = nl[ci[k]]++;
     }
-    Builder B(p, order, part_rows, CHX_RES_PART_MAX, CHX_RES_HELD);
+    Builder B(p, order, part_rows, capacity, CHX_RES_HELD);
     const bool ok = B.build([&](int k, int i) {
         for (int c = ro[i]; c < up0[i]; ++c)  // blocks another part holds
             if (!B.own(ci[c]))
                 B.ghost(static_cast<std::uint32_t>(-1 - block_slots[c]),
                         B.local_of(ci[c]) |
-                            (static_cast<std::uint32_t>((c - ro[i]) * CHX_RES_PART_MAX + (k - B.a)) << 16));
+                            (static_cast<std::uint32_t>((c - ro[i]) * capacity + (k - B.a)) << 16));
         for (int c = up0[i]; c < ro[i + 1]; ++c) {
             const std::uint32_t lj = B.local_of(ci[c]);
             const std::uint32_t target =
-                B.own(ci[c]) ? static_cast<std::uint32_t>(lower[c]) * CHX_RES_PART_MAX + lj : 0xffffu;
+                B.own(ci[c]) ? static_cast<std::uint32_t>(lower[c] * capacity) + lj : 0xffffu;
             B.plane(c - up0[i], k) = lj | (target << 16);
         }
         return static_cast<std::uint32_t>((up0[i] - ro[i]) | ((ro[i + 1] - up0[i]) << 8));
@@ -347,6 +347,15 @@ int resident_part_rows(const std::vector<int>& rows, int largest) {
         if (pr == largest && most <= kWorkgroups) return pr;
     }
     return 0;
+}
+
+std::vector<ResidentChoice> resident_choices(const std::vector<int>& rows, bool bf16) {
+    std::vector<ResidentChoice> out;
+    const int half = resident_part_rows(rows, CHX_RES_GEN_PART), full = resident_part_rows(rows, CHX_RES_PART_MAX);
+    if (bf16 && half > 0) out.push_back({CHX_RES_FORM_HALF, half});
+    if (!bf16 && full > 0) out.push_back({CHX_RES_FORM_SHEET, full});
+    if (half > 0) out.push_back({CHX_RES_FORM_GENERAL, half});
+    return out;
 }
 
 }  // namespace engine

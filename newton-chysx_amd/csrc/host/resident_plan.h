@@ -27,9 +27,10 @@ struct ResidentPlan {
     int exports = 0;  // rows that some other part reads
     std::vector<std::uint32_t> blob;
 };
-// Sheet form: the upper blocks of a row are held by the row.
+// Sheet form: the upper blocks of a row are held by the row.  `capacity`:
+// rows of the largest part (CHX_RES_PART_MAX; half sheets CHX_RES_GEN_PART).
 ResidentPlan resident_plan(const topology::Pattern& p, const std::vector<int>& block_slots,
-                           const std::vector<int>& order, int part_rows);
+                           const std::vector<int>& order, int part_rows, int capacity);
 // General form: any numbering, wider rows, smaller parts.
 ResidentPlan resident_plan_general(const topology::Pattern& p, const std::vector<int>& block_slots,
                                    const std::vector<int>& order, int part_rows);
@@ -39,9 +40,13 @@ ResidentPlan resident_plan_rows(const topology::Pattern& p, const std::vector<in
 // each and at most `largest` a part: the smallest size (from 256) whose parts
 // all run at once on 256 workgroups, else the largest; 0 when one matrix
 // alone has more parts than that.  What fits one part is one part: it needs
-// no exchange (32x32 rows: 3.3 us an iteration in one part, 3.3-3.9 in four
-// or two).
+// no exchange.
 int resident_part_rows(const std::vector<int>& rows, int largest);
-
+// Forms and part sizes for cloths that are solved together, the best first;
+// the first that every cloth's pattern fits is taken.
+struct ResidentChoice {
+    int form, part_rows;
+};
+std::vector<ResidentChoice> resident_choices(const std::vector<int>& rows, bool bf16);
 }  // namespace engine
 }  // namespace chysx

@@ -55,6 +55,24 @@ def test_resident_step_matches_the_streaming_step(gpu, nx, ny, shuffle):
         assert helpers.rel_maxnorm(a.state()[0], b.state()[0]) <= 1e-6
 
 
+@pytest.mark.parametrize("nx,ny,shuffle", [(8, 8, False), (16, 32, False), (27, 19, False), (64, 64, False), (27, 19, True)])
+def test_resident_bf16_step_matches_the_streaming_step(gpu, nx, ny, shuffle):
+    """BF16 blocks: half sheets of one part (512 rows) and several, and the
+    general plan.  The BF16 matrix is the same; the residual that is reached
+    (tolerance 1e-6, or the cap) is compared, not the iterations."""
+    from chysx import scenes
+
+    a, b = (scenes.DeviceCloth(_spec(nx, ny, 100 * nx + ny, shuffle)) for _ in range(2))
+    for c in (a, b):
+        c.sim.set_bf16_blocks(True)
+    b.sim.set_lds_staging(False)
+    for step in range(2):
+        a.step()
+        b.step()
+        print(f"{nx}x{ny} step {step}: {a.sim.last_pcg_iterations()} / {b.sim.last_pcg_iterations()} iterations", flush=True)
+        assert helpers.rel_maxnorm(a.state()[0], b.state()[0]) <= 1e-5
+
+
 def _rows_system(n, extra=0):
     """A diagonally dominant block matrix over an n-by-n grid, and a right-hand side."""
     import torch

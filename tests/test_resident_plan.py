@@ -169,3 +169,32 @@ def test_pattern_outside_the_limits_has_no_plan():
     bs, _ = _slots(n, ro, ci)
     assert chysx.topology.resident_plan(n, ro, ci, bs, 256) is None
     assert chysx.topology.resident_plan(n, ro, ci, bs, 256, general=True) is None
+
+
+@pytest.mark.parametrize("nx,ny", [(2, 2), (8, 8), (23, 22), (33, 31), (65, 66)])
+@pytest.mark.parametrize("part_rows", [256, 512])
+def test_half_sheet_is_the_sheet_with_smaller_numbers(nx, ny, part_rows):
+    """At a capacity of 512 rows a plan is the one at 1024 rows with local
+    indices and product slots numbered by the smaller capacity."""
+    n, half = nx * ny, 512
+    ro, ci = _pattern(nx, ny)
+    bs, _ = _slots(n, ro, ci)
+    full = chysx.topology.resident_plan(n, ro, ci, bs, part_rows)
+    got = chysx.topology.resident_plan(n, ro, ci, bs, part_rows, capacity=half)
+    assert (got["order"] == full["order"]).all() and got["parts"] == full["parts"] and got["exports"] == full["exports"]
+    want, blob, parts = full["blob"].astype(np.int64), got["blob"].astype(np.int64), full["parts"]
+
+    def renumber(w):
+        local, slot = w & 0xFFFF, w >> 16
+        local = np.where(local >= PART, local - PART + half, local)
+        return local | np.where(slot == 0xFFFF, slot, slot // PART * half + slot % PART) << 16
+
+    # held words of the blocks that are there, and the second words of the ghost lists
+    held_at, meta = 8 * parts + 3 * n, want[8 * parts + n:8 * parts + 2 * n]
+    for u in range(HELD):
+        at = held_at + u * n + np.flatnonzero(meta >> 8 > u)
+        want[at] = renumber(want[at])
+    for q in range(parts):
+        g, at = want[8 * q + 3:8 * q + 5]
+        want[at + 1:at + 2 * g:2] = renumber(want[at + 1:at + 2 * g:2])
+    assert (blob == want).all()
