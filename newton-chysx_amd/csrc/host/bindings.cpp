@@ -198,7 +198,7 @@ PYBIND11_MODULE(_chysx_native, m) {
         .def("set_barrier_timeout_ticks", &ClothSimulator::set_barrier_timeout_ticks, py::arg("ticks"),
              "Bound of each grid-barrier wait of the solver in 100 MHz ticks (0: one second).")
         .def("set_pcg_form", &ClothSimulator::set_pcg_form, py::arg("form"),
-             "0: one grid barrier per PCG iteration (default), 1: two")
+             "0: the reductions of a PCG iteration merged (default: resident, or one grid barrier), 1: two barriers")
         .def("pcg_form", &ClothSimulator::pcg_form)
         .def(
             "debug_move_roundtrip",
@@ -328,7 +328,7 @@ PYBIND11_MODULE(_chysx_native, m) {
              py::arg("cuda_stream") = 0)
         .def("set_barrier_timeout_ticks", &chysx::cloth::ClothBatch::set_barrier_timeout_ticks, py::arg("ticks"))
         .def("set_pcg_form", &chysx::cloth::ClothBatch::set_pcg_form, py::arg("form"),
-             "0: one grid barrier per PCG iteration (default), 1: two")
+             "0: the reductions of a PCG iteration merged (default: resident, or one grid barrier), 1: two barriers")
         .def("pcg_form", &chysx::cloth::ClothBatch::pcg_form);
 
     // ---- standalone block-CSR matrix and PCG solver --------------------------

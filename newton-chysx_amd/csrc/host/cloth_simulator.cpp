@@ -359,7 +359,7 @@ chx_instance ClothSimulator::single_descriptor(const engine::InstanceSource& s, 
     return d;
 }
 
-chx_instance ClothSimulator::prepare_instance(float dt, std::uintptr_t cuda_stream, engine::ResidentChoice choice) {
+chx_instance ClothSimulator::prepare_instance(float dt, std::uintptr_t cuda_stream) {
     const int n = buffers_.particle_count();
     if (n <= 0) throw std::runtime_error("ClothSimulator::prepare_instance: no particles bound");
     if (buffers_.pos.data() == nullptr || buffers_.vel.data() == nullptr)
@@ -370,9 +370,7 @@ chx_instance ClothSimulator::prepare_instance(float dt, std::uintptr_t cuda_stre
     else check_elements_current(cuda_stream);
     engine::InstanceSource s = source();
     s.dt = dt;
-    chx_instance d = inst_.descriptor(s);
-    inst_.attach_plan(d, pattern_, choice, cuda_stream);
-    return d;
+    return inst_.descriptor(s);
 }
 
 int ClothSimulator::last_pcg_iterations(std::uintptr_t cuda_stream) {

@@ -213,7 +213,14 @@ public:
     // Builds (or refreshes) this cloth's device arrays without stepping and
     // returns the launch descriptor for substep `dt`; ClothBatch uses it to
     // advance this cloth as one instance of a batch.
-    chx_instance prepare_instance(float dt, std::uintptr_t cuda_stream = 0, engine::ResidentChoice choice = {0, 0});
+    chx_instance prepare_instance(float dt, std::uintptr_t cuda_stream = 0);
+    // The resident-solve plan of a choice, in two steps: the host part (may
+    // run on a thread per simulator), and into the descriptor.
+    bool plan_missing(engine::ResidentChoice c) { return inst_.plan_missing(c); }
+    void make_plan(engine::ResidentChoice c) { inst_.make_plan(pattern_, c); }
+    void attach_plan(chx_instance& d, engine::ResidentChoice c, std::uintptr_t stream) {
+        inst_.attach_plan(d, pattern_, c, stream);
+    }
     // Builds the Hessian pattern, scatter maps and device arrays now (the
     // first step would otherwise do it), so the set-up of a cloth can run
     // ahead of its first step, e.g. on another host thread.

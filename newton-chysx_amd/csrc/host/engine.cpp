@@ -684,33 +684,45 @@ chx_instance InstanceData::descriptor(const InstanceSource& s) const {
     return I;
 }
 
-void InstanceData::attach_plan(chx_instance& d, const topology::Pattern& p, ResidentChoice c, std::uintptr_t stream) {
-    d.res_plan = nullptr;
-    int part_rows = c.part_rows;
-    if (part_rows == 0 || n_ == 0) return;
+InstanceData::Plan& InstanceData::plan_of(ResidentChoice& c) {
     // what one workgroup holds needs no exchange (resident_part_rows)
     const int most = c.form == CHX_RES_FORM_SHEET ? CHX_RES_PART_MAX : CHX_RES_GEN_PART;
-    if (n_ <= most) part_rows = most;
+    if (n_ <= most) c.part_rows = most;
     const int first = c.form == CHX_RES_FORM_SHEET ? 0 : (c.form == CHX_RES_FORM_HALF ? 3 : 5);
-    Plan& pl = plans_[first + (part_rows == 256 ? 0 : (part_rows == 512 ? 1 : 2))];
-    if (!pl.tried) {
-        pl.tried = true;
-        if (order_.empty()) order_ = resident_order(p);
-        ResidentPlan r = c.form == CHX_RES_FORM_GENERAL
-                             ? resident_plan_general(p, block_slots_.host(), order_, part_rows)
-                             : resident_plan(p, block_slots_.host(), order_, part_rows, most);
-        if (!r.blob.empty()) {
-            pl.parts = r.parts;
-            pl.exports = r.exports;
-            pl.blob.host() = std::move(r.blob);
-            upload(pl.blob, bytes_, stream);
-            sync_stream(stream, "resident plan");
-            pl.blob.host() = {};
-        }
+    return plans_[first + (c.part_rows == 256 ? 0 : (c.part_rows == 512 ? 1 : 2))];
+}
+
+bool InstanceData::plan_missing(ResidentChoice c) { return c.part_rows > 0 && n_ > 0 && !plan_of(c).tried; }
+
+void InstanceData::make_plan(const topology::Pattern& p, ResidentChoice c) {
+    if (!plan_missing(c)) return;
+    Plan& pl = plan_of(c);
+    if (order_.empty()) order_ = resident_order(p);
+    ResidentPlan r = c.form == CHX_RES_FORM_GENERAL
+                         ? resident_plan_general(p, block_slots_.host(), order_, c.part_rows)
+                         : resident_plan(p, block_slots_.host(), order_, c.part_rows,
+                                         c.form == CHX_RES_FORM_SHEET ? CHX_RES_PART_MAX : CHX_RES_GEN_PART);
+    if (!r.blob.empty()) {
+        pl.parts = r.parts;
+        pl.exports = r.exports;
+        pl.blob.host() = std::move(r.blob);
     }
+    pl.tried = true;
+}
+
+void InstanceData::attach_plan(chx_instance& d, const topology::Pattern& p, ResidentChoice c, std::uintptr_t stream) {
+    d.res_plan = nullptr;
+    if (c.part_rows == 0 || n_ == 0) return;
+    make_plan(p, c);
+    Plan& pl = plan_of(c);
     if (pl.parts == 0) return;
+    if (!pl.blob.host().empty()) {
+        upload(pl.blob, bytes_, stream);
+        sync_stream(stream, "resident plan");
+        pl.blob.host() = {};
+    }
     d.res_plan = pl.blob.gpu_data();
-    d.res_part_rows = part_rows;
+    d.res_part_rows = c.part_rows;
     d.res_parts = pl.parts;
     d.res_exports = pl.exports;
     d.res_form = c.form;

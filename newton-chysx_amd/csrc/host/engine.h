@@ -75,6 +75,9 @@ public:
     // (none when the pattern does not fit it, or the part size is 0).
     // Plans are built on first use and kept until the next build().
     void attach_plan(chx_instance& d, const topology::Pattern& p, ResidentChoice c, std::uintptr_t stream);
+    // Host part of it, which may run on a thread per instance.
+    bool plan_missing(ResidentChoice c);
+    void make_plan(const topology::Pattern& p, ResidentChoice c);
     bool built() const noexcept { return built_; }
     int n_rows() const noexcept { return n_; }
     int nnz() const noexcept { return nnz_; }
@@ -126,6 +129,7 @@ private:
         int parts = 0, exports = 0;
         DeviceArray<std::uint32_t> blob;
     };
+    Plan& plan_of(ResidentChoice& c);  // and the part size that this instance takes of the choice
     Plan plans_[7];           // sheets (parts of 256, 512, 1024 rows), half sheets and general form (256, 512)
     std::vector<int> order_;  // canonical row order of the plans
     DeviceArray<chx_plane> planes_;
