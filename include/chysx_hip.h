@@ -376,9 +376,9 @@ typedef struct chx_cloth_batch {
     unsigned wait_ticks;             /* bound of every grid-barrier wait in 100 MHz   */
                                      /* ticks (0: 1e8, one second); past it the solve */
                                      /* aborts                                        */
-    int pcg_form;                    /* FP32 cloth instances: 0 one grid barrier per   */
-                                     /* iteration (the two reductions merged), 1 two  */
-                                     /* barriers per iteration                        */
+    int pcg_form;                    /* FP32 cloth instances: 0 the two reductions     */
+                                     /* merged (resident, or one grid barrier per     */
+                                     /* iteration), 1 two barriers per iteration      */
     int res_grid;                    /* resident PCG: workgroups of the launch (0: the      */
                                      /* streaming kernels), dealt to res_groups groups    */
     unsigned long long* xbuf;        /* control words and exchange areas of the resident  */

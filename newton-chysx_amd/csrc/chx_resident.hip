@@ -43,6 +43,7 @@
 // flight: the floor of one store and one load is 1.0 to 1.2 us.
 // A halo row is 16 bytes: three floats and the tag's 16 bits in both words.
 #include <algorithm>
+#include <cstddef>
 #include <mutex>
 
 #include "chx_pcg.h"
@@ -118,7 +119,8 @@ struct Form {
     }
     static __device__ __forceinline__ unsigned place(unsigned w) { return w >> 27; }
 };
-static_assert(Form<SHEET>::kSource + 3 * (Form<SHEET>::kRows + CHX_RES_HALO_MAX) < (1u << 16) && 3 * (Form<GENERAL>::kSpare + kWave) < (1u << 15) &&
+static_assert(Form<SHEET>::kSource + 3 * (Form<SHEET>::kRows + CHX_RES_HALO_MAX) < (1u << 16) &&
+                  3 * (Form<GENERAL>::kSpare + kWave) < (1u << 15) &&
                   3 * (Form<GENERAL>::kRows + CHX_RES_HALO_MAX) <= (1u << 12) && CHX_RES_GEN_WIDTH <= 16,
               "word fields");
 // Sums of an exchange: merged solver rho, sigma, delta, gamma, ||r||^2
@@ -191,6 +193,14 @@ struct ResLds {
     int bad;         // a wait gave up
     unsigned mail;   // mailbox word of the workgroup
 };
+
+using SheetLds = ResLds<SHEET, false>;
+using HalfLds = ResLds<HALF, true>;
+using GeneralLds = ResLds<GENERAL, false>;
+using RowsLds = ResLds<ROWS, true>;
+static_assert(offsetof(SheetLds, p) == 4 * Form<SHEET>::kSource && offsetof(HalfLds, p) == 4 * Form<HALF>::kSource &&
+                  offsetof(GeneralLds, p) == 4 * Form<GENERAL>::kSource && offsetof(RowsLds, p) == 4 * Form<ROWS>::kSource,
+              "the source vector follows the products");
 
 // Bounded wait of one lane: true while it may go on.  After the bound the
 // solve is aborted for every workgroup (the report of grid_sync).
