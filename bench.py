@@ -9,9 +9,10 @@ instance (one assembly kernel + one persistent PCG launch).
 
 value        = sum(N_i) * K / wall-seconds of K timed substeps (inputs in HBM)
 plain        = the same instances stepped one ClothSimulator at a time
-roofline     = persistent PCG kernel: algorithmic bytes per launch
-               sum_i [B_setup_i + k_i B_iter_i + 48 N_i] / mean launch time
-               (HIP events on the stream the kernel runs on)
+roofline     = PCG kernel: bytes per launch / mean launch time (HIP events on
+               the stream the kernel runs on).  The resident kernel (default)
+               reads the matrix once: sum_i [18 nnz_i + 108 N_i]; the streaming
+               ones sum_i [B_setup_i + k_i B_iter_i + 48 N_i]
 cpu_baseline = the CPU oracle (a port of the reference step) on a bounded
                sample of the same instances, all host threads
 """
@@ -406,6 +407,7 @@ def main():
         f"at the cap")
 
     # PCG kernel alone: assemble, then time the solve launch with events on `stream`.
+    resident = args.pcg_form == 0 and not args.no_lds_staging
     ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     pcg_ms, pcg_bytes = [], []
     with torch.cuda.stream(stream):
@@ -418,7 +420,9 @@ def main():
             pcg_ms.append(ev0.elapsed_time(ev1))
             k = np.array(batch.last_pcg_iterations(sh), np.int64)
             n, nnz = sizes[:, 0], sizes[:, 1]
-            pcg_bytes.append(float(np.sum(b_setup(n, nnz) + k * b_iter(n, nnz) + 48 * n)))
+            # resident: upper blocks, diagonal, right-hand side, x in and out, finalize
+            pcg_bytes.append(float(np.sum(18 * nnz + 108 * n if resident else
+                                          b_setup(n, nnz) + k * b_iter(n, nnz) + 48 * n)))
     mean_ms = float(np.mean(pcg_ms))
     achieved = float(np.mean(pcg_bytes)) / (mean_ms * 1e-3) / 1e9
     traffic = load_traffic()
@@ -429,10 +433,11 @@ def main():
     traffic_bytes = None
     if traffic and key in traffic.get("configs", {}):
         traffic_bytes = traffic["configs"][key]["bytes_per_launch"]
-    roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+    roofline = {"bound": "instruction issue and exchange latency" if resident else "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4),
-                "traffic": traffic_bytes,
-                "kernel": "%s<%s, %s sliced entries> (persistent block-Jacobi PCG + finalize, %s)"
+                "traffic": None if resident else traffic_bytes,
+                "kernel": "resident_kernel (block-Jacobi PCG with the matrix on chip + finalize)" if resident else
+                          "%s<%s, %s sliced entries> (persistent block-Jacobi PCG + finalize, %s)"
                           % ("pcg1_kernel" if args.pcg_form == 0 else "pcg_kernel",
                              "global SpMV" if args.no_lds_staging else "LDS-staged SpMV",
                              "16-bit" if entries16 else "32-bit",
@@ -447,12 +452,15 @@ def main():
     # whole iteration per phase, algorithmic bytes B_iter.  Two-barrier form:
     # the SpMV phase (q = A p with the folded p update), B_spmv + 36N.
     spmv_phase = iteration_phase = None
-    batch.set_trace(1024)
-    with torch.cuda.stream(stream):
-        batch.assemble(dt, sh)
-        batch.solve(sh)
-        tr = np.array(batch.last_trace(sh)).astype(np.int64)
-    batch.set_trace(0)
+    # The resident solve has no common phases: its gangs iterate by themselves.
+    tr = np.zeros((0, 2), np.int64)
+    if not resident:
+        batch.set_trace(1024)
+        with torch.cuda.stream(stream):
+            batch.assemble(dt, sh)
+            batch.solve(sh)
+            tr = np.array(batch.last_trace(sh)).astype(np.int64)
+        batch.set_trace(0)
     n_all, nnz_all = int(sizes[:, 0].sum()), int(sizes[:, 1].sum())
     if args.pcg_form == 0:
         full = [k for k in range(1, len(tr) - 1) if tr[k + 1, 1] == len(specs)]
