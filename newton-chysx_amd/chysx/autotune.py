@@ -49,7 +49,8 @@ def tune_batch(batch, dt: float, stream=None, lanes=(4,), blocks_per_cu=(1, 2, 3
 
     sig = _signature(batch)
     dev = _device_name()
-    key = f"{dev}|{sig}"
+    # settings cached before the resident solve could hold its streaming forms
+    key = f"{dev}|{sig}|resident"
     if cache_path and os.path.exists(cache_path):
         try:
             with open(cache_path) as f:
