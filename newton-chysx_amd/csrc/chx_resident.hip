@@ -1019,6 +1019,10 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
 #pragma unroll
     for (int s = 0; s < kSlots; ++s)
         if (live(s)) st3g(I.x, ldx(plan, rows_at + pos0 + row_at(s)), lds_ld(S.x, 3u * row_at(s)));
+    // x is stored in the plan's row order and the finalize reads it in row
+    // order: rows of other waves, with no grid barrier in between when the
+    // launch has one workgroup
+    __syncthreads();
     return true;
 }
 
