@@ -1,0 +1,26 @@
+// Numbers, slots and tags of what the resident PCG's workgroups exchange.
+// Plain C++ for the kernel and for the host's tests.
+#pragma once
+
+namespace chx {
+
+// A word's tag: the launch number (8 bits, never 0) and the low 8 bits of
+// the exchange's number.
+constexpr unsigned exchange_tag(unsigned launch, unsigned number) { return launch << 8 | (number & 255u); }
+constexpr unsigned exchange_slot(unsigned number) { return number & 1u; }
+
+// A solve's exchanges.  Every one has sums; not every one has halo rows (the
+// two-reduction solver sends none with rho).  Each kind is numbered by
+// itself, so the word that a reader waits for last held the one of two
+// numbers before, whose tag is another one.  (With one number for both, the
+// two-reduction solver's iterations leave the rows of even numbers alone, and
+// a refinement 256 numbers after the set-up would find its tag already there.)
+struct Exchange {
+    unsigned sums = ~0u, rows = ~0u;  // numbers of the last ones
+    constexpr void next(bool with_rows) {
+        ++sums;
+        if (with_rows) ++rows;
+    }
+};
+
+}  // namespace chx

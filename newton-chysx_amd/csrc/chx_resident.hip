@@ -31,8 +31,11 @@
 // Exchange: 64-bit words of values and a tag that names launch and exchange,
 // so a reader needs no ordering between words and no cache maintenance: it
 // reads a word until its tag is the awaited one.  Words alternate between two
-// slots; slot t is rewritten in exchange t + 2, which its writer enters only
-// after every part's sums of exchange t + 1, sent after their reads of t.
+// slots; a slot is rewritten two exchanges later at the earliest, which its
+// writer enters only after every part's sums of the exchange between, sent
+// after their reads of the slot.  Sums and rows are numbered apart
+// (chx_exchange.h): iterations of the two-reduction solver send rows in every
+// second exchange.
 //
 // Every part has a 128-byte line for its sums, which all parts read, 16 bytes
 // a lane.  What costs is lines with several writers: with the parts' words
@@ -46,6 +49,7 @@
 #include <cstddef>
 #include <mutex>
 
+#include "chx_exchange.h"
 #include "chx_pcg.h"
 #include "chx_resident.h"
 
@@ -376,13 +380,14 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     const Area area = exchange_area(B);
     const unsigned xsum = 8u * I.res_xbase, xrow = xsum + 2u * 8u * kLine * parts;
     const unsigned exports = unsigned(I.res_exports);
-    auto tag_of = [&](int t) { return (epoch << 8) | (unsigned(t) & 255u); };
-    auto line = [&](int t, unsigned q) { return xsum + 8u * kLine * ((unsigned(t) & 1u) * parts + q); };
-    auto row_bytes = [&](int t, unsigned e) { return xrow + 16u * ((unsigned(t) & 1u) * exports + e); };
-    auto send_row = [&](int t, unsigned e, f3 v) {
+    // numbers of exchanges: t of the sums, u of the rows
+    auto tag_of = [&](unsigned number) { return exchange_tag(epoch, number); };
+    auto line = [&](unsigned t, unsigned q) { return xsum + 8u * kLine * (exchange_slot(t) * parts + q); };
+    auto row_bytes = [&](unsigned u, unsigned e) { return xrow + 16u * (exchange_slot(u) * exports + e); };
+    auto send_row = [&](unsigned u, unsigned e, f3 v) {
         const unsigned x = __float_as_uint(v.x), y = __float_as_uint(v.y), z = __float_as_uint(v.z);
-        const unsigned tag = tag_of(t) << 16;
-        st128(area, row_bytes(t, e), v4u{x, (y & 0xffffu) | tag, z, (y >> 16) | tag});
+        const unsigned tag = tag_of(u) << 16;
+        st128(area, row_bytes(u, e), v4u{x, (y & 0xffffu) | tag, z, (y >> 16) | tag});
     };
 
     // ---- load: own rows, ghost block, halo row ----
@@ -677,7 +682,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         w += dpp64<kXor2>(w);
         return w + dpp64<kHalfMirror>(w);
     };
-    auto send_sums = [&](int t, auto& acc) {
+    auto send_sums = [&](unsigned t, auto& acc) {
         constexpr int N = int(sizeof(acc[0]) / sizeof(double));
         double none[N] = {};
         leaf_sums(acc[0], kSlots == 2 ? acc[kSlots - 1] : none, S.leaf, wave);
@@ -699,7 +704,7 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     // read a part's line together and a wave 32 lines (2.6 us), and the waves'
     // sums meet in LDS, where every wave adds them up by itself.
     double tot[kSums];
-    auto take_sums = [&](int t, unsigned N) -> bool {
+    auto take_sums = [&](unsigned t, unsigned N) -> bool {
         const unsigned lane = tid_here() & unsigned(kWave - 1), tag = tag_of(t);
         u64* const progress = &B.xbuf[RES_PROGRESS];
         auto mine = [&](v4u w) { return w.y == tag && w.w == tag; };
@@ -767,15 +772,15 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         }
         return true;
     };
-    // The halo row's triple of exchange t (sent before its sums: waiting for
-    // it first hides its way behind the sums').
-    auto take_halo = [&](int t) {
+    // The halo row's triple of number u (sent before its exchange's sums:
+    // waiting for it first hides its way behind the sums').
+    auto take_halo = [&](unsigned u) {
         f3 h = mk(0.f, 0.f, 0.f);
         if (is_halo()) {
-            const unsigned tag = tag_of(t) & 0xffffu;
+            const unsigned tag = tag_of(u) & 0xffffu;
             v4u w[1];
             if (await<1>(
-                    area, [&](int) { return row_bytes(t, hex); },
+                    area, [&](int) { return row_bytes(u, hex); },
                     [&](v4u v) { return v.y >> 16 == tag && v.w >> 16 == tag; }, w, &B.xbuf[RES_PROGRESS], bar))
                 h = mk(__uint_as_float(w[0].x), __uint_as_float((w[0].y & 0xffffu) | w[0].w << 16),
                        __uint_as_float(w[0].z));
@@ -806,16 +811,16 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             (void)__hip_atomic_fetch_add(&B.xbuf[RES_PROGRESS], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
     // r = b - A x (A x in q) and its sums; the exported rows of r are sent.
-    auto residual = [&](int t) {
+    auto residual = [&](unsigned t, unsigned u) {
         double acc[kSlots][3];  // rho, ||b||^2, ||r||^2
 #pragma unroll
         for (int s = 0; s < kSlots; ++s) {
             acc[s][0] = acc[s][1] = acc[s][2] = 0.0;
             if (on[s] && live(s)) {
                 // at the set-up r holds b
-                const f3 b = t > 0 ? ld3g(I.rhs, ldx(plan, rows_at + pos0 + row_at(s))) : r[s];
+                const f3 b = t > 0u ? ld3g(I.rhs, ldx(plan, rows_at + pos0 + row_at(s))) : r[s];
                 r[s] = sub(b, q[s]);
-                if (ex[s] != CHX_RES_NONE) send_row(t, ex[s], r[s]);
+                if (ex[s] != CHX_RES_NONE) send_row(u, ex[s], r[s]);
                 acc[s][0] = dot64(r[s], apply_minv(M[s], r[s]));
                 acc[s][1] = dot64(b, b);
                 acc[s][2] = dot64(r[s], r[s]);
@@ -827,9 +832,9 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
     if constexpr (!TWO) {
         // ---- set-up: r_0 = b - A x, z_0 = p_0 = M^-1 r_0 ----
         apply(p, q);
-        residual(0);
-        hr = take_halo(0);
-        if (!take_sums(0, 3)) return false;
+        residual(0u, 0u);  // every exchange has rows: one number for both
+        hr = take_halo(0u);
+        if (!take_sums(0u, 3)) return false;
         double rho = tot[0], rr = tot[2];
         S.bb = tot[1];  // every thread the same
         mark_trace();
@@ -903,7 +908,8 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
         float beta = 0.0f;
         bool residual_step = true;        // set-up, then refinement: r = b - A x, x in p and S.p
         bool exact = true, fresh = true;  // rr is of b - A x; p starts from z
-        int k = 0, refines = -1, t = -1;  // t: the last exchange
+        int k = 0, refines = -1;
+        Exchange at;                      // the last exchange
         int blocks = 0;                   // which matrix V holds
         for (;;) {
             if (!residual_step) {
@@ -917,17 +923,17 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                     // this slot computes the true residual: halo rows of x first
                     residual_step = true;
                     ++k;
-                    ++t;
+                    at.next(true);
                     double zero[kSlots][1] = {};
 #pragma unroll
                     for (int s = 0; s < kSlots; ++s)
                         if (on[s]) {
                             p[s] = lds_ld(S.x, 3u * row_at(s));
-                            if (ex[s] != CHX_RES_NONE) send_row(t, ex[s], p[s]);
+                            if (ex[s] != CHX_RES_NONE) send_row(at.rows, ex[s], p[s]);
                         }
-                    send_sums(t, zero);
-                    const f3 hx = take_halo(t);
-                    if (!take_sums(t, 1)) return false;
+                    send_sums(at.sums, zero);
+                    const f3 hx = take_halo(at.rows);
+                    if (!take_sums(at.sums, 1)) return false;
                     if (is_halo()) lds_st(S.p, halo_slot(), hx);
                 } else {
                     if (is_halo()) {
@@ -947,16 +953,16 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             }
             const int want = half && !residual_step ? 1 : 0;
             if (want != blocks) {
-                Where at[kSlots];
+                Where w[kSlots];
                 unsigned g;
-                locate(at, g);
-                find_first(at);
-                load_blocks(want != 0, at, g);
+                locate(w, g);
+                find_first(w);
+                load_blocks(want != 0, w, g);
 #pragma unroll
                 for (int s = 0; s < kSlots; ++s)
                     if (on[s]) {
                         float d[9];
-                        load_diag(want != 0, at[s].row, d);
+                        load_diag(want != 0, w[s].row, d);
                         keep_diag(s, d);
                     }
                 __builtin_amdgcn_s_waitcnt(0x0f70);
@@ -964,10 +970,10 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
             }
             apply(p, q);
             if (residual_step) {
-                ++t;
-                residual(t);
-                hr = take_halo(t);
-                if (!take_sums(t, 3)) return false;
+                at.next(true);
+                residual(at.sums, at.rows);
+                hr = take_halo(at.rows);
+                if (!take_sums(at.sums, 3)) return false;
                 rho = tot[0];
                 bb = tot[1];
                 rr = tot[2];
@@ -977,37 +983,37 @@ __device__ __forceinline__ bool solve_part(const chx_cloth_batch& B, const Inst&
                 mark_trace();
                 continue;
             }
-            ++t;
+            at.next(true);
             double sum[kSlots][1];
 #pragma unroll
             for (int s = 0; s < kSlots; ++s) {
                 sum[s][0] = 0.0;
                 if (on[s]) {
-                    if (ex[s] != CHX_RES_NONE) send_row(t, ex[s], q[s]);
+                    if (ex[s] != CHX_RES_NONE) send_row(at.rows, ex[s], q[s]);
                     sum[s][0] = dot64(p[s], q[s]);
                 }
             }
-            send_sums(t, sum);
-            const f3 h = take_halo(t);
-            if (!take_sums(t, 1)) return false;
+            send_sums(at.sums, sum);
+            const f3 h = take_halo(at.rows);
+            if (!take_sums(at.sums, 1)) return false;
             const float alpha = guarded_div(rho, tot[0]);
             mark_trace();
             if (is_halo()) hr = axpy(-alpha, h, hr);
-            ++t;
+            at.next(false);
             double acc[kSlots][2];
 #pragma unroll
             for (int s = 0; s < kSlots; ++s) {
                 acc[s][0] = acc[s][1] = 0.0;
                 if (on[s]) {
-                    const unsigned at = 3u * row_at(s);
-                        lds_st(S.x, at, axpy(alpha, p[s], lds_ld(S.x, at)));
+                    const unsigned xi = 3u * row_at(s);
+                    lds_st(S.x, xi, axpy(alpha, p[s], lds_ld(S.x, xi)));
                     r[s] = axpy(-alpha, q[s], r[s]);
                     acc[s][0] = dot64(r[s], apply_minv(M[s], r[s]));
                     acc[s][1] = dot64(r[s], r[s]);
                 }
             }
-            send_sums(t, acc);
-            if (!take_sums(t, 2)) return false;
+            send_sums(at.sums, acc);
+            if (!take_sums(at.sums, 2)) return false;
             beta = guarded_div(tot[0], rho);
             rho = tot[0];
             rr = tot[1];

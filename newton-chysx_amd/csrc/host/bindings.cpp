@@ -9,6 +9,7 @@
 
 #include <stdexcept>
 
+#include "../chx_exchange.h"
 #include "cloth_batch.h"
 #include "mesh_io.h"
 #include "resident_plan.h"
@@ -537,6 +538,23 @@ PYBIND11_MODULE(_chysx_native, m) {
         },
         py::arg("n"), py::arg("row_offsets"), py::arg("col_indices"), py::arg("block_slots"), py::arg("part_rows"),
         py::arg("general") = false, py::arg("capacity") = CHX_RES_PART_MAX);
+    topo.def(
+        "resident_exchanges",
+        [](unsigned launch, const std::vector<bool>& with_rows) {
+            // Per exchange of a resident solve: slot and tag of its sums, and of
+            // its rows (None: it has none).
+            py::list out;
+            chx::Exchange at;
+            for (const bool rows : with_rows) {
+                at.next(rows);
+                const auto place = [&](unsigned n) {
+                    return py::make_tuple(chx::exchange_slot(n), chx::exchange_tag(launch, n));
+                };
+                out.append(py::make_tuple(place(at.sums), rows ? py::object(place(at.rows)) : py::object(py::none())));
+            }
+            return out;
+        },
+        py::arg("launch"), py::arg("with_rows"));
     topo.def(
         "cloth_system",
         [](int n, IArr tris, IArr pins, bool stretch, bool shear, bool bending) {

@@ -26,3 +26,96 @@ def test_finalize_takes_every_row_of_the_solution(gpu, nx, ny, shuffle, bf16):
         pos, vel = (a.astype(np.float32) for a in cloth.state())
         dx = cloth.sim.debug_dump_last_solve()[5]
         assert np.array_equal(pos, before + dx) and np.array_equal(vel, dx * inv_dt), step
+
+
+def _true_residual(cloth):
+    """||b - A dx|| / ||b|| of the last solve, in FP64."""
+    diag, ro, ci, val, rhs, dx = (np.asarray(a, np.float64) for a in cloth.sim.debug_dump_last_solve())
+    ro, ci = ro.astype(np.int64), ci.astype(np.int64)
+    rows = np.repeat(np.arange(len(diag)), np.diff(ro))
+    Ax = np.einsum("nij,nj->ni", diag, dx)
+    np.add.at(Ax, rows, np.einsum("nij,nj->ni", val, dx[ci]))
+    return np.linalg.norm(rhs - Ax) / np.linalg.norm(rhs)
+
+
+def _solve_from_rest(cloth, start, warm, cap, tol, dt=1.0 / 60.0):
+    """One substep from `start` at rest, the solve from `warm`; its iterations."""
+    cloth.pos.copy_(start)
+    cloth.vel.zero_()
+    cloth.sim.debug_set_warm_start(warm)
+    cloth.sim.set_pcg_iterations(cap)
+    cloth.sim.set_pcg_tolerance(tol)
+    cloth.step(dt)
+    return cloth.sim.last_pcg_iterations()
+
+
+@pytest.mark.parametrize("inner", [127, 255])
+def test_bf16_refinement_at_a_multiple_of_256_exchanges(gpu, inner):
+    """After 127 inner iterations the refinement's rows are sent 256 exchanges
+    after the set-up's, after 255 512.  The warm start is one for which the
+    recursive residual has a new minimum at that iteration, and the tolerance
+    lies between it and the last minimum, so that the refinement comes right
+    there.  The solve does the streaming one's operations, so its true residual
+    is that one's but for the rounding of alpha and beta: by a factor of two at
+    most, more than an iteration changes it by."""
+    from chysx import scenes
+
+    a, b = (scenes.DeviceCloth(_spec(64, 61, 0)) for _ in range(2))
+    for c in (a, b):
+        c.sim.set_bf16_blocks(True)
+    b.sim.set_lds_staging(False)  # the streaming solve
+    start = a.pos.clone()
+    for seed in range(32):
+        warm = np.random.default_rng(seed).normal(0.0, 0.01, (a.spec.n, 3)).astype(np.float32)
+        history = []
+        for cap in (inner, *range(inner - 1, inner - 40, -1)):
+            assert _solve_from_rest(a, start, warm, cap, 0.0) == cap
+            history.append(a.sim.last_relative_residual())
+            if cap < inner and history[0] > 0.98 * history[-1]:
+                break
+        else:
+            break
+    else:
+        pytest.fail("no warm start with a new minimum there")
+    tol = (history[0] * min(history[1:])) ** 0.5
+    its = [_solve_from_rest(c, start, warm, inner + 200, tol) for c in (a, b)]
+    res = [_true_residual(c) for c in (a, b)]
+    print(f"seed {seed}, tolerance {tol:.2e}: {its} iterations, true residuals {res}", flush=True)
+    assert inner < its[0] <= inner + 200 and a.sim.last_relative_residual() <= tol
+    assert res[0] <= 2.0 * res[1]
+
+
+@pytest.mark.parametrize("nx,ny,shuffle", [(32, 32, False), (64, 61, False), (40, 39, True)])
+def test_more_iterations_than_a_tag_counts(gpu, nx, ny, shuffle):
+    """600 FP32 iterations: the tags' exchange numbers go round twice.  With a
+    step of a second the solve is far from converged then, so a wrong halo row
+    would show in its residual."""
+    from chysx import scenes
+
+    a, b = (scenes.DeviceCloth(_spec(nx, ny, nx, shuffle)) for _ in range(2))
+    b.sim.set_lds_staging(False)
+    start = a.pos.clone()
+    for cap in (255, 256, 257, 600):
+        for c in (a, b):
+            assert _solve_from_rest(c, start, np.zeros((nx * ny, 3), np.float32), cap, 0.0, dt=1.0) == cap
+        res = [_true_residual(c) for c in (a, b)]
+        print(f"{nx}x{ny}, {cap} iterations: true residuals {res}", flush=True)
+        assert res[0] <= 2.0 * res[1]
+
+
+def test_rows_solve_with_more_iterations_than_a_tag_counts(gpu):
+    import torch
+
+    import chysx
+    from test_gpu_resident import _rows_system
+
+    A, b = _rows_system(40)
+    out = []
+    for lanes in (8, 4):  # four lanes per row: the streaming solve
+        x = torch.zeros_like(b)
+        S = chysx.PCGSolver()
+        S.solve(A, b.data_ptr(), x.data_ptr(), max_iterations=300, lanes_per_row=lanes)
+        assert S.last_iterations() == 300
+        out.append(x.cpu().numpy())
+    # both at the FP32 floor of this diagonally dominant system
+    assert np.abs(out[0] - out[1]).max() <= 1e-5 * np.abs(out[1]).max()

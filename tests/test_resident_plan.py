@@ -198,3 +198,21 @@ def test_half_sheet_is_the_sheet_with_smaller_numbers(nx, ny, part_rows):
         g, at = want[8 * q + 3:8 * q + 5]
         want[at + 1:at + 2 * g:2] = renumber(want[at + 1:at + 2 * g:2])
     assert (blob == want).all()
+
+
+def test_an_awaited_tag_is_never_the_old_one():
+    """Slots keep what was last written: until a word of an exchange arrives,
+    its reader finds an older one there, whose tag has to differ.  The
+    two-reduction solver sends halo rows with the set-up's residual, with
+    every iteration's sigma (not with its rho) and, after `inner` iterations,
+    with the refinement's x and residual; tags repeat after 256 numbers."""
+    for inner in [*range(520), 5118, 5119, 5120]:
+        with_rows = [True] + [True, False] * inner + [True, True] + [True, False] * 3
+        words = {}
+        for exchange in chysx.topology.resident_exchanges(9, with_rows):
+            for kind, word in zip(("sums", "rows"), exchange):
+                if word is not None:
+                    slot, tag = word
+                    assert slot in (0, 1) and tag >> 8 == 9
+                    assert words.get((kind, slot)) != tag, (inner, kind)
+                    words[kind, slot] = tag
