@@ -23,4 +23,16 @@ struct Exchange {
     }
 };
 
+// The number of the next launch, 1 .. kResEpochs, and whether old tags have to
+// be cleared before it: numbers start over, so no word may keep one.  Not
+// every launch that counts runs the resident kernel (an assembly by itself,
+// the streaming kernels), so the flag stays until that kernel has cleared.
+constexpr unsigned kResEpochs = 255u;
+struct Launch {
+    unsigned long long number, clear;
+};
+constexpr Launch next_launch(Launch last) {
+    return last.number >= kResEpochs ? Launch{1ull, 1ull} : Launch{last.number + 1ull, last.clear};
+}
+
 }  // namespace chx

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "chx_device.h"
+#include "chx_exchange.h"
 
 namespace chx {
 
@@ -64,16 +65,13 @@ __device__ __forceinline__ void merged_scalars(double rho, double sig, double de
 // ---- control words of the resident PCG (first words of chx_cloth_batch::xbuf)
 enum : int {
     RES_EPOCH = 0,      // launch number, 1 .. kResEpochs: the tag of everything exchanged
-    RES_CLEAR = 1,      // the numbers wrapped around: old tags in xbuf are cleared first
+    RES_CLEAR = 1,      // the numbers started over: the next resident launch clears old tags first
     RES_NEXT = 16,      // next item of the list
     RES_PROGRESS = 32,  // changes while any gang iterates (idle workgroups wait as long as it does)
     RES_DONE = 48,      // instances finished
     RES_IDLE = 64,      // per group (16 words apart): its idle workgroups
     RES_MAIL = 256      // per workgroup (16 words apart): its next item and part
 };
-// A tag's 16 bits are a launch number's 8 and an exchange's 8: the area is
-// cleared when the launch numbers start over.
-constexpr unsigned kResEpochs = 255u;
 constexpr int kResGroups = 8;
 static_assert(RES_MAIL + 16 * 256 <= CHX_RES_CONTROL_WORDS && RES_IDLE + 16 * kResGroups <= RES_MAIL, "control words");
 
@@ -85,9 +83,9 @@ __device__ __forceinline__ void reset_resident(unsigned long long* xbuf) {
     if (threadIdx.x == 0) {
         xbuf[RES_NEXT] = 0ull;
         xbuf[RES_DONE] = 0ull;
-        const unsigned long long e = xbuf[RES_EPOCH];
-        xbuf[RES_CLEAR] = e >= kResEpochs ? 1ull : 0ull;
-        xbuf[RES_EPOCH] = e >= kResEpochs ? 1ull : e + 1ull;
+        const Launch next = next_launch({xbuf[RES_EPOCH], xbuf[RES_CLEAR]});
+        xbuf[RES_EPOCH] = next.number;
+        xbuf[RES_CLEAR] = next.clear;
     }
 }
 

@@ -556,6 +556,21 @@ PYBIND11_MODULE(_chysx_native, m) {
         },
         py::arg("launch"), py::arg("with_rows"));
     topo.def(
+        "resident_launches",
+        [](const std::vector<bool>& runs) {
+            // Launch number of every reset of a solver's control words and, where
+            // the resident kernel runs after it, whether it clears old tags.
+            py::list out;
+            chx::Launch at{0, 0};
+            for (const bool resident : runs) {
+                at = chx::next_launch(at);
+                out.append(py::make_tuple(at.number, resident && at.clear != 0));
+                if (resident) at.clear = 0;
+            }
+            return out;
+        },
+        py::arg("runs"));
+    topo.def(
         "cloth_system",
         [](int n, IArr tris, IArr pins, bool stretch, bool shear, bool bending) {
             // Pattern + slot tables of a cloth with the given element sets, as

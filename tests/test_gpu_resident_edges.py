@@ -119,3 +119,55 @@ def test_rows_solve_with_more_iterations_than_a_tag_counts(gpu):
         out.append(x.cpu().numpy())
     # both at the FP32 floor of this diagonally dominant system
     assert np.abs(out[0] - out[1]).max() <= 1e-5 * np.abs(out[1]).max()
+
+
+@pytest.mark.parametrize("calls", ["assemble and solve", "streaming steps between"])
+def test_launch_numbers_start_over_at_any_reset(gpu, calls):
+    """An assembly by itself and a streaming solve count as launches too, so
+    the numbers start over at calls after which the resident kernel does not
+    run; the next one that does clears the old tags.  Solves of two states in
+    turn give each its first bits; what carries the same number from before
+    they started over is of the other state."""
+    import torch
+
+    import chysx
+    from chysx import scenes
+
+    cloths = [scenes.DeviceCloth(_spec(n, n + 1, n)) for n in (40, 33)]
+    batch = chysx.ClothBatch()
+    for c in cloths:
+        c.sim.set_pcg_iterations(4)
+        c.sim.set_pcg_tolerance(0.0)
+        batch.add_instance(c.sim)
+    dt = cloths[0].spec.dt
+    starts = [[c.pos + k * 1.0e-2 * torch.sin(9.0 * c.pos) for c in cloths] for k in range(2)]
+    first = {}
+
+    def solve(k):
+        for c, start in zip(cloths, starts[k % 2]):
+            c.pos.copy_(start)
+            c.vel.zero_()
+            c.sim.debug_set_warm_start(np.zeros((c.spec.n, 3), np.float32))
+        torch.cuda.synchronize()
+        if calls == "assemble and solve":
+            batch.assemble(dt)
+            batch.assemble(dt)  # three launches a solve: number 3 comes again after 255
+            batch.solve()
+        else:
+            batch.step(dt)
+        got = [c.state()[0] for c in cloths]
+        want = first.setdefault(k % 2, got)
+        assert all(np.array_equal(g, w) for g, w in zip(got, want)), k
+
+    if calls == "assemble and solve":
+        for k in range(300):
+            solve(k)
+    else:
+        for k in range(16):
+            solve(k)
+            if k < 9:
+                continue
+            batch.set_lds_staging(False)
+            for _ in range(254):
+                batch.step(dt)
+            batch.set_lds_staging(True)

@@ -216,3 +216,30 @@ def test_an_awaited_tag_is_never_the_old_one():
                     assert slot in (0, 1) and tag >> 8 == 9
                     assert words.get((kind, slot)) != tag, (inner, kind)
                     words[kind, slot] = tag
+
+
+def _resets(case, rng):
+    """Whether the resident kernel runs after each reset of the control words."""
+    if case == "steps":
+        return [True] * 1200
+    if case == "assemble and solve":
+        return [False, True] * 600 + [False, False, True] * 400
+    if case == "streaming steps between":
+        return [True] * 10 + ([False] * 254 + [True]) * 5 + ([False] * 600 + [True]) * 3
+    return [bool(x) for x in rng.random(5000) < rng.choice([0.01, 0.3, 0.9])]
+
+
+@pytest.mark.parametrize("case", ["steps", "assemble and solve", "streaming steps between", *range(12)])
+def test_a_launch_number_comes_again_only_after_a_clear(case):
+    """No launch of the resident kernel finds words of an earlier one under
+    its own number, in whatever order assemblies, streaming solves and
+    resident solves reset the control words."""
+    runs = _resets(case, np.random.default_rng(0 if isinstance(case, str) else case))
+    used = set()
+    for resident, (number, clears) in zip(runs, chysx.topology.resident_launches(runs)):
+        assert 1 <= number <= 255
+        if resident:
+            if clears:
+                used.clear()
+            assert number not in used
+            used.add(number)
