@@ -1,13 +1,10 @@
 #include "cloth_batch.h"
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
-#include <exception>
-#include <mutex>
 #include <stdexcept>
-#include <system_error>
-#include <thread>
+
+#include "threads.h"
 
 namespace chysx {
 namespace cloth {
@@ -41,27 +38,7 @@ void make_plans(const std::vector<ClothSimulator*>& sims, engine::ResidentChoice
     for (ClothSimulator* s : sims)
         if (s->plan_missing(c)) todo.push_back(s);
     if (todo.size() < 2) return;  // attach_plan makes it
-    const std::size_t threads = std::min<std::size_t>({8, todo.size(), std::max(1u, std::thread::hardware_concurrency())});
-    std::atomic<std::size_t> next{0};
-    std::exception_ptr failed;
-    std::mutex mu;
-    const auto work = [&]() noexcept {
-        try {
-            for (std::size_t i; (i = next.fetch_add(1)) < todo.size();) todo[i]->make_plan(c);
-        } catch (...) {
-            std::lock_guard<std::mutex> lk(mu);
-            failed = std::current_exception();
-        }
-    };
-    std::vector<std::thread> pool;
-    try {
-        while (pool.size() + 1 < threads) pool.emplace_back(work);
-    } catch (const std::system_error&) {
-        // no more threads: those that run share the work
-    }
-    work();
-    for (std::thread& t : pool) t.join();
-    if (failed) std::rethrow_exception(failed);
+    for_each_on_threads(todo.size(), 8, [&](std::size_t i) { todo[i]->make_plan(c); });
 }
 }  // namespace
 
