@@ -407,7 +407,7 @@ def main():
         f"at the cap")
 
     # PCG kernel alone: assemble, then time the solve launch with events on `stream`.
-    resident = args.pcg_form == 0 and not args.no_lds_staging
+    resident = batch.resident()
     ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     pcg_ms, pcg_bytes = [], []
     with torch.cuda.stream(stream):

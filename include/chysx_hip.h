@@ -408,6 +408,10 @@ int chx_device_info(int* cu_count, int* max_pcg_blocks, int* occupancy_blocks_pe
 int chx_pcg_grid_limit(int lanes_per_row, int bf16_blocks, int no_lds_staging, int* max_blocks);
 /* The same for the resident PCG kernel (one workgroup per compute unit). */
 int chx_resident_grid_limit(int* max_blocks);
+/* Which PCG a batch's launches run as it stands: 1 the resident kernel, 0 a
+ * streaming one (no plans, a grid cap below a cloth's parts, or a setting
+ * that asks for a streaming form). */
+int chx_batch_is_resident(const chx_cloth_batch* batch, int* resident);
 
 /* Device memory: replaces CudaArray<T> (ChysX/src/memory/cuda_array.h:64-284,
  * cuda_array.cu:41-90). */

@@ -27,6 +27,7 @@ _SIGS = {
     "chx_device_info": (_I, [_P, _P, _P]),
     "chx_pcg_grid_limit": (_I, [_I, _I, _I, _P]),
     "chx_resident_grid_limit": (_I, [_P]),
+    "chx_batch_is_resident": (_I, [_P, _P]),
     "chx_pcg_solve_bsr3_plan": (_I, [_I, _P, _P, _P, _P, _P, _P, _I, _D, _I, _P, _S, _P, _P, _P, _P, _U]),
     "chx_malloc": (_I, [_P, _S]),
     "chx_free": (_I, [_P]),

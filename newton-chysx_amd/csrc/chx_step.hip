@@ -1996,6 +1996,13 @@ int chx_pcg_grid_limit(int lanes_per_row, int bf16_blocks, int no_lds_staging, i
     });
 }
 
+int chx_batch_is_resident(const chx_cloth_batch* batch, int* is_resident) {
+    return guarded([&] {
+        require(batch != nullptr && is_resident != nullptr, "chx_batch_is_resident: null argument");
+        *is_resident = batch->n_tiles > 0 && resident(*batch, false) ? 1 : 0;
+    });
+}
+
 int chx_device_info(int* cu_count, int* max_pcg_blocks, int* occupancy_blocks_per_cu) {
     return guarded([&] {
         const int mb = max_coresident(8);

@@ -201,6 +201,8 @@ PYBIND11_MODULE(_chysx_native, m) {
         .def("set_pcg_form", &ClothSimulator::set_pcg_form, py::arg("form"),
              "0: the reductions of a PCG iteration merged (default: resident, or one grid barrier), 1: two barriers")
         .def("pcg_form", &ClothSimulator::pcg_form)
+        .def("resident", &ClothSimulator::resident,
+             "Whether the cloth's own steps run the resident solve (after prepare() or the first step).")
         .def(
             "debug_move_roundtrip",
             [](ClothSimulator& s) {
@@ -330,7 +332,8 @@ PYBIND11_MODULE(_chysx_native, m) {
         .def("set_barrier_timeout_ticks", &chysx::cloth::ClothBatch::set_barrier_timeout_ticks, py::arg("ticks"))
         .def("set_pcg_form", &chysx::cloth::ClothBatch::set_pcg_form, py::arg("form"),
              "0: the reductions of a PCG iteration merged (default: resident, or one grid barrier), 1: two barriers")
-        .def("pcg_form", &chysx::cloth::ClothBatch::pcg_form);
+        .def("pcg_form", &chysx::cloth::ClothBatch::pcg_form)
+        .def("resident", &chysx::cloth::ClothBatch::resident, "Whether the bound batch runs the resident solve.");
 
     // ---- standalone block-CSR matrix and PCG solver --------------------------
     // (ChysX/src/sparse/block_csr.h:59-135, ChysX/src/solver/pcg_solver.h:79-167)

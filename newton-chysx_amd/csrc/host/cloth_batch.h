@@ -84,6 +84,8 @@ public:
     // Persistent PCG form of the FP32 solve (ClothSimulator::set_pcg_form).
     void set_pcg_form(int form) { runner_.set_pcg_form(form); }
     int pcg_form() const noexcept { return runner_.pcg_form(); }
+    // Whether the bound batch is solved by the resident kernel.
+    bool resident() const { return runner_.resident(); }
     std::vector<double> last_relative_residuals(std::uintptr_t cuda_stream = 0);
 
 private:

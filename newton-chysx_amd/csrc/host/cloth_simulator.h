@@ -189,6 +189,9 @@ public:
     // uses the two-barrier form.
     void set_pcg_form(int form) { runner_.set_pcg_form(form); }
     int pcg_form() const noexcept { return runner_.pcg_form(); }
+    // Whether this cloth, stepped by itself, is solved by the resident kernel
+    // (known after prepare() or the first step).
+    bool resident() const { return runner_.resident(); }
     double last_relative_residual(std::uintptr_t cuda_stream = 0);
 
     // ---- diagnostics -----------------------------------------------------------------

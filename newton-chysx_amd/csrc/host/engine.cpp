@@ -815,6 +815,12 @@ void BatchRunner::layout_resident(std::vector<chx_instance>& ds, std::uintptr_t 
     desc_.res_grid = grid;
 }
 
+bool BatchRunner::resident() const {
+    int r = 0;
+    check(chx_batch_is_resident(&desc_, &r), "engine", "solver form");
+    return r != 0;
+}
+
 void BatchRunner::set_grid_blocks(int g) {
     g = g < 0 ? 0 : g;
     if (g == grid_) return;

@@ -211,6 +211,9 @@ public:
         desc_.pcg_form = form;
     }
     int pcg_form() const noexcept { return desc_.pcg_form; }
+    // Whether the bound instances are solved by the resident kernel (else by
+    // a streaming one).
+    bool resident() const;
 
 private:
     void size_outputs(int n_instances, int n_tiles, std::uintptr_t stream = 0);

@@ -171,3 +171,61 @@ def test_launch_numbers_start_over_at_any_reset(gpu, calls):
             for _ in range(254):
                 batch.step(dt)
             batch.set_lds_staging(True)
+
+
+def _disk(valence, rings, seed=0):
+    """A round cloth: a centre with `valence` neighbours (2 * valence blocks in
+    its row, with the opposite vertices of its bending elements) and rings."""
+    from chysx import scenes
+
+    a = 2.0 * np.pi * np.arange(valence) / valence
+    ring = np.stack([np.cos(a), np.zeros(valence), np.sin(a)], 1)
+    pos = np.concatenate([np.zeros((1, 3))] + [ring * (r + 1.0) / rings for r in range(rings)])
+    pos = (0.5 * pos + [0.0, 1.0, 0.0] + np.random.default_rng(seed).normal(0.0, 1.0e-4, pos.shape)).astype(np.float32)
+    at = lambda r, k: 1 + r * valence + k % valence
+    tris = [(0, at(0, k + 1), at(0, k)) for k in range(valence)]
+    for r in range(rings - 1):
+        for k in range(valence):
+            tris += [(at(r, k), at(r, k + 1), at(r + 1, k)), (at(r, k + 1), at(r + 1, k + 1), at(r + 1, k))]
+    start = pos.copy()
+    start[:, 1] += 0.02 * np.sin(7.0 * pos[:, 0] + 4.0 * pos[:, 2])
+    return scenes.ClothSpec(pos=pos, tris=np.array(tris, np.int32), pins=np.array([at(rings - 1, 0)], np.int32),
+                            k_stretch=100.0, k_shear=100.0, k_bend=1.0e-4, k_pin=1.0e6, density=0.2, dt=1.0 / 600.0,
+                            max_iter=60, tol=1.0e-6, pos_start=start)
+
+
+def test_a_batch_reports_the_solve_that_it_runs(gpu):
+    """Settings and cloths that leave the resident solve, and those that do not."""
+    import chysx
+    from chysx import scenes
+
+    cloths = [scenes.DeviceCloth(_spec(n, n + 1, n)) for n in (40, 33)]
+    wide, narrow = (scenes.DeviceCloth(_disk(v, 40)) for v in (9, 8))
+    batch = chysx.ClothBatch()
+    assert not batch.resident()
+    for c in cloths + [narrow]:
+        batch.add_instance(c.sim)
+    dt = cloths[0].spec.dt
+
+    def runs():
+        batch.step(dt)
+        return batch.resident()
+
+    assert runs()
+    batch.set_lds_staging(False)
+    assert not runs()
+    batch.set_lds_staging(True)
+    batch.set_pcg_form(1)
+    assert not runs()
+    batch.set_pcg_form(0)
+    batch.set_grid_blocks(4)  # the 40x41 cloth has 7 parts
+    assert not runs()
+    batch.set_grid_blocks(0)
+    assert runs()
+    batch.add_instance(wide.sim)  # one row of 18 blocks: no plan
+    assert not runs()
+    batch.remove_instance(wide.sim)
+    assert runs()
+    wide.step()
+    narrow.step()
+    assert narrow.sim.resident() and not wide.sim.resident()
