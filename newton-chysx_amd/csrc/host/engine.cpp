@@ -733,6 +733,9 @@ void InstanceData::attach_plan(chx_instance& d, const topology::Pattern& p, Resi
 // ---------------------------------------------------------------------------
 
 void BatchRunner::layout_resident(std::vector<chx_instance>& ds, std::uintptr_t stream) {
+    // no resident solve until all of it is there, also when an allocation
+    // throws: launches without it must not touch an area that is gone
+    desc_.xbuf = nullptr;
     desc_.res_grid = 0;
     desc_.res_n_items = desc_.res_n_big = 0;
     int total = 0, most = 0;
@@ -919,6 +922,8 @@ BatchRunner& BatchRunner::operator=(BatchRunner&& o) noexcept {
     inst_done_ = std::move(o.inst_done_);
     sync_ = std::move(o.sync_);
     trace_ = std::move(o.trace_);
+    relayout_ = o.relayout_;
+    table_stale_ = o.table_stale_;
     xbuf_ = std::move(o.xbuf_);
     res_items_ = std::move(o.res_items_);
     status_host_ = o.status_host_;
@@ -1016,6 +1021,7 @@ void BatchRunner::bind_single(const chx_instance& d, std::uintptr_t stream) {
     desc_.unit_items = nullptr;
     size_outputs(1, desc_.n_tiles, stream);
     sync_stream(stream, "bind");
+    relayout_ = table_stale_ = false;
 }
 
 void BatchRunner::bind_many(const std::vector<chx_instance>& ds, std::uintptr_t stream) {
@@ -1061,6 +1067,7 @@ void BatchRunner::bind_many(const std::vector<chx_instance>& ds, std::uintptr_t 
     desc_.unit_items = unit_items_.gpu_data();
     size_outputs(desc_.n_instances, desc_.n_tiles, stream);
     sync_stream(stream, "bind");
+    relayout_ = table_stale_ = false;
 }
 
 bool BatchRunner::take(chx_instance& was, chx_instance d) {
@@ -1076,12 +1083,14 @@ bool BatchRunner::take(chx_instance& was, chx_instance d) {
 
 void BatchRunner::update_single(const chx_instance& d, std::uintptr_t stream) {
     desc_.entries16 = (d.n_rows > 0 && d.slice_entries16 == nullptr) ? 0 : 1;
-    if (!take(desc_.single, d)) return;
+    relayout_ = take(desc_.single, d) || relayout_;
+    if (!relayout_) return;
     // queued launches may still use the old layout
     check(chx_stream_synchronize(stream), "engine", "instance update");
     std::vector<chx_instance> one{desc_.single};
     layout_resident(one, stream);
     desc_.single = one[0];
+    relayout_ = false;
 }
 
 void BatchRunner::update_many(const std::vector<chx_instance>& ds, std::uintptr_t stream) {
@@ -1091,20 +1100,20 @@ void BatchRunner::update_many(const std::vector<chx_instance>& ds, std::uintptr_
         table_host_[0] = desc_.single;
         return;
     }
-    bool changed = false, relayout = false;
     for (std::size_t i = 0; i < ds.size(); ++i) {
         const chx_instance was = table_host_[i];
-        relayout = take(table_host_[i], ds[i]) || relayout;
-        changed = changed || std::memcmp(&was, &table_host_[i], sizeof(chx_instance)) != 0;
+        relayout_ = take(table_host_[i], ds[i]) || relayout_;
+        table_stale_ = table_stale_ || std::memcmp(&was, &table_host_[i], sizeof(chx_instance)) != 0;
     }
     desc_.entries16 = entries16_all(table_host_);
-    if (changed) {
+    if (table_stale_ || relayout_) {
         // The previous table may still be read by queued launches.
         check(chx_stream_synchronize(stream), "engine", "instance table update");
-        if (relayout) layout_resident(table_host_, stream);
+        if (relayout_) layout_resident(table_host_, stream);
         table_.host() = table_host_;
         table_.copy_to_device(stream);
         desc_.inst = table_.gpu_data();
+        table_stale_ = relayout_ = false;
     }
 }
 

@@ -242,6 +242,8 @@ private:
     int grid_ = 0;
     int tile_rows_ = CHX_TILE_ROWS;
     bool bf16_ = false;
+    // What an update has still to do; kept when it throws.
+    bool relayout_ = false, table_stale_ = false;
     std::vector<chx_instance> table_host_;
     DeviceArray<chx_instance> table_;
     DeviceArray<int> tiles_, elem_items_, unit_items_;
