@@ -732,7 +732,12 @@ void InstanceData::attach_plan(chx_instance& d, const topology::Pattern& p, Resi
 // BatchRunner
 // ---------------------------------------------------------------------------
 
-void BatchRunner::layout_resident(std::vector<chx_instance>& ds, std::uintptr_t stream) {
+bool BatchRunner::layout_resident(std::vector<chx_instance>& ds, std::uintptr_t stream, bool queued) {
+    bool wrote = false;
+    const auto will_write = [&] {
+        if (queued && !wrote) check(chx_device_synchronize(), "engine", "work list rebuild");
+        wrote = true;
+    };
     // no resident solve until all of it is there, also when an allocation
     // throws: launches without it must not touch an area that is gone
     desc_.xbuf = nullptr;
@@ -741,11 +746,11 @@ void BatchRunner::layout_resident(std::vector<chx_instance>& ds, std::uintptr_t 
     int total = 0, most = 0;
     for (const chx_instance& d : ds) {
         if (d.n_rows == 0) continue;
-        if (d.res_plan == nullptr || d.res_form != ds[0].res_form) return;
+        if (d.res_plan == nullptr || d.res_form != ds[0].res_form) return wrote;
         total += d.res_parts;
         most = std::max(most, d.res_parts);
     }
-    if (most == 0) return;
+    if (most == 0) return wrote;
     int limit = 0;
     check(chx_resident_grid_limit(&limit), "engine", "resident grid limit");
     const int cap = grid_ > 0 ? std::min(limit, grid_) : limit;
@@ -767,21 +772,21 @@ void BatchRunner::layout_resident(std::vector<chx_instance>& ds, std::uintptr_t 
     } else {
         grid = per = cap;
     }
-    if (grid > cap || most > grid) return;
+    if (grid > cap || most > grid) return wrote;
     std::size_t words = CHX_RES_CONTROL_WORDS;
     for (chx_instance& d : ds) {
         if (d.n_rows == 0) continue;
         d.res_xbase = static_cast<unsigned>(std::min<std::size_t>(words, CHX_RES_XWORDS_MAX));
         words += CHX_RES_XWORDS(d.res_parts, d.res_exports);
     }
-    if (words > CHX_RES_XWORDS_MAX) return;
+    if (words > CHX_RES_XWORDS_MAX) return wrote;
     if (xbuf_.gpu_size() < words) {
+        will_write();
         xbuf_.ensure_device(words);
         xbuf_.zero_device(stream);
     }
-    auto& it = res_items_.host();
-    it.clear();
     if (ds.size() > 1) {
+        std::vector<int> it;
         std::vector<int> by(ds.size());
         for (std::size_t i = 0; i < by.size(); ++i) by[i] = static_cast<int>(i);
         by.erase(std::remove_if(by.begin(), by.end(), [&](int i) { return ds[i].n_rows == 0; }), by.end());
@@ -807,7 +812,13 @@ void BatchRunner::layout_resident(std::vector<chx_instance>& ds, std::uintptr_t 
             }
             it.insert(it.end(), {i, parts, base, 0});
         }
-        res_items_.copy_to_device(stream);
+        if (!items_on_device_ || it != res_items_.host()) {
+            will_write();
+            items_on_device_ = false;
+            res_items_.host() = std::move(it);
+            res_items_.copy_to_device(stream);
+            items_on_device_ = true;
+        }
         desc_.res_items = res_items_.gpu_data();
         desc_.res_n_items = static_cast<int>(by.size());
     }
@@ -816,6 +827,7 @@ void BatchRunner::layout_resident(std::vector<chx_instance>& ds, std::uintptr_t 
     desc_.res_groups = groups;
     desc_.res_form = ds[0].res_form;
     desc_.res_grid = grid;
+    return wrote;
 }
 
 bool BatchRunner::resident() const {
@@ -830,19 +842,26 @@ void BatchRunner::set_grid_blocks(int g) {
     grid_ = g;
     desc_.grid_blocks = g;
     if (!bound()) return;
-    // Queued launches may still read the old lists.
-    check(chx_device_synchronize(), "engine", "work list rebuild");
+    // What queued launches may still read is waited for only where it changes:
+    // most limits leave a batch's lists as they are, and one cloth has none.
+    bool wrote = false;
     if (desc_.inst == nullptr) {
         std::vector<chx_instance> one{desc_.single};
-        layout_resident(one);
+        wrote = layout_resident(one, 0, true);
         desc_.single = one[0];
     } else {
-        layout_resident(table_host_);
-        table_.host() = table_host_;
-        table_.copy_to_device();
-        desc_.inst = table_.gpu_data();
+        const std::vector<chx_instance> was = table_host_;
+        wrote = layout_resident(table_host_, 0, true);
+        if (std::memcmp(was.data(), table_host_.data(), was.size() * sizeof(chx_instance)) != 0) {
+            if (!wrote) check(chx_device_synchronize(), "engine", "work list rebuild");
+            wrote = table_stale_ = true;
+            table_.host() = table_host_;
+            table_.copy_to_device();
+            desc_.inst = table_.gpu_data();
+            table_stale_ = false;
+        }
     }
-    check(chx_device_synchronize(), "engine", "work list rebuild");
+    if (wrote) check(chx_device_synchronize(), "engine", "work list rebuild");
 }
 
 void BatchRunner::set_lanes_per_row(int L) {
@@ -923,6 +942,7 @@ BatchRunner& BatchRunner::operator=(BatchRunner&& o) noexcept {
     sync_ = std::move(o.sync_);
     trace_ = std::move(o.trace_);
     relayout_ = o.relayout_;
+    items_on_device_ = o.items_on_device_;
     table_stale_ = o.table_stale_;
     xbuf_ = std::move(o.xbuf_);
     res_items_ = std::move(o.res_items_);

@@ -227,8 +227,10 @@ private:
 
     // Work lists and exchange area of the resident solve of the bound
     // instances; leaves the launch to the streaming kernels when one of them
-    // has no plan or the grid does not hold its parts.
-    void layout_resident(std::vector<chx_instance>& ds, std::uintptr_t stream = 0);
+    // has no plan or the grid does not hold its parts.  With `queued` launches
+    // of the last layout may be running: it waits for them before it writes
+    // what they read.  True when it wrote device memory.
+    bool layout_resident(std::vector<chx_instance>& ds, std::uintptr_t stream = 0, bool queued = false);
     // Takes `d` over the bound descriptor `was`, keeping what the bind laid
     // out; true when its resident plan is another one (a cloth whose pattern
     // was rebuilt after the bind), so that the layout has to be made again.
@@ -254,6 +256,7 @@ private:
     DeviceArray<unsigned long long> trace_;
     DeviceArray<unsigned long long> xbuf_;
     DeviceArray<int> res_items_;
+    bool items_on_device_ = false;  // the device has res_items_' host list
 };
 
 }  // namespace engine

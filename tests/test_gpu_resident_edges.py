@@ -229,3 +229,30 @@ def test_a_batch_reports_the_solve_that_it_runs(gpu):
     wide.step()
     narrow.step()
     assert narrow.sim.resident() and not wide.sim.resident()
+
+
+def test_a_grid_limit_set_while_a_stream_is_captured(gpu):
+    """The limit is host state of the next launch: a graph captured with one
+    replays the streaming solve, without one the resident one."""
+    import torch
+
+    from chysx import scenes
+
+    cloth, eager = (scenes.DeviceCloth(_spec(40, 41, 3)) for _ in range(2))
+    dt = cloth.spec.dt
+    s = torch.cuda.Stream()
+    cloth.step(dt, s.cuda_stream)
+    eager.step(dt)
+    torch.cuda.synchronize()
+    for limit in (3, 0):
+        eager.sim.set_grid_blocks(limit)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            cloth.sim.set_grid_blocks(limit)
+            cloth.step(dt, torch.cuda.current_stream().cuda_stream)
+        assert cloth.sim.resident() == (limit == 0)
+        for _ in range(3):
+            g.replay()
+            torch.cuda.synchronize()
+            eager.step(dt)
+            assert np.array_equal(cloth.state()[0], eager.state()[0])

@@ -104,6 +104,27 @@ CASES = {
         REQUIRE(syncs == 0 && copies == 0);
     }
 """,
+    # a grid limit is a number unless the work list changes with it
+    "grid limit": r"""
+    for (int many = 0; many < 2; ++many) {
+        BatchRunner r;
+        std::vector<chx_instance> ds(many ? 3 : 1, cloth(2000, 100));
+        r.bind_many(ds);
+        syncs = copies = 0;
+        for (int limit : {256, 64, 4, 200, 0}) {
+            r.set_grid_blocks(limit);
+            REQUIRE(r.resident() == (limit != 4) && r.desc().grid_blocks == limit);
+            REQUIRE(!r.resident() || (r.desc().res_grid >= 8 && (limit == 0 || r.desc().res_grid <= limit)));
+            REQUIRE(syncs == 0 && copies == 0);
+        }
+        if (!many) continue;
+        r.set_grid_blocks(16);  // two workgroups a group: each cloth is a large item
+        REQUIRE(r.resident() && r.desc().res_n_big == 3 && syncs >= 2 && copies >= 1);
+        REQUIRE(r.desc().res_items[2] == 0 && r.desc().res_items[6] == 8);
+        r.set_grid_blocks(0);
+        REQUIRE(r.resident() && r.desc().res_n_big == 0 && r.desc().res_items[6] == 0);
+    }
+""",
 }
 
 
