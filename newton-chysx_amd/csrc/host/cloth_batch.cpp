@@ -37,7 +37,6 @@ void make_plans(const std::vector<ClothSimulator*>& sims, engine::ResidentChoice
     std::vector<ClothSimulator*> todo;
     for (ClothSimulator* s : sims)
         if (s->plan_missing(c)) todo.push_back(s);
-    if (todo.size() < 2) return;  // attach_plan makes it
     for_each_on_threads(todo.size(), 8, [&](std::size_t i) { todo[i]->make_plan(c); });
 }
 }  // namespace
@@ -54,15 +53,13 @@ std::vector<chx_instance> ClothBatch::descriptors(float dt, std::uintptr_t cuda_
             throw std::invalid_argument(
                 "ClothBatch: BF16 mode needs every instance switched with set_bf16_blocks(true)");
     }
-    // the resident solve wants all plans in one form
+    // the resident solve wants all plans in one form: they go to the device
+    // only when every cloth has one
     for (const engine::ResidentChoice& c : engine::resident_choices(rows, bf16_)) {
         make_plans(sims_, c);
-        bool all = true;
-        for (std::size_t i = 0; i < sims_.size(); ++i) {
-            sims_[i]->attach_plan(ds[i], c, cuda_stream);
-            all = all && ds[i].res_plan != nullptr;
-        }
-        if (all) break;
+        if (!std::all_of(sims_.begin(), sims_.end(), [&](ClothSimulator* s) { return s->plan_fits(c); })) continue;
+        for (std::size_t i = 0; i < sims_.size(); ++i) sims_[i]->attach_plan(ds[i], c, cuda_stream);
+        break;
     }
     return ds;
 }

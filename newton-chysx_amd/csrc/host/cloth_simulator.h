@@ -221,6 +221,7 @@ public:
     // run on a thread per simulator), and into the descriptor.
     bool plan_missing(engine::ResidentChoice c) { return inst_.plan_missing(c); }
     void make_plan(engine::ResidentChoice c) { inst_.make_plan(pattern_, c); }
+    bool plan_fits(engine::ResidentChoice c) { return inst_.plan_fits(c); }
     void attach_plan(chx_instance& d, engine::ResidentChoice c, std::uintptr_t stream) {
         inst_.attach_plan(d, pattern_, c, stream);
     }

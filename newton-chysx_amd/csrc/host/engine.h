@@ -78,6 +78,8 @@ public:
     // Host part of it, which may run on a thread per instance.
     bool plan_missing(ResidentChoice c);
     void make_plan(const topology::Pattern& p, ResidentChoice c);
+    // Whether a made plan exists (a cloth without rows needs none).
+    bool plan_fits(ResidentChoice c) { return n_ == 0 || (c.part_rows > 0 && plan_of(c).parts > 0); }
     bool built() const noexcept { return built_; }
     int n_rows() const noexcept { return n_; }
     int nnz() const noexcept { return nnz_; }

@@ -256,3 +256,24 @@ def test_a_grid_limit_set_while_a_stream_is_captured(gpu):
             torch.cuda.synchronize()
             eager.step(dt)
             assert np.array_equal(cloth.state()[0], eager.state()[0])
+
+
+def test_a_batch_that_streams_keeps_no_plans_for_its_other_cloths(gpu):
+    """One cloth without a plan: the others get none of the batch's part size
+    on the device, only the one of their own steps."""
+    import chysx
+    from chysx import scenes
+
+    batch = chysx.ClothBatch()
+    cloths = [scenes.DeviceCloth(_spec(64, 61, k)) for k in range(20)]  # 320 parts of 256 rows
+    for c in cloths:
+        c.step()  # a plan of its own, 16 parts
+    before = [c.sim.device_bytes() for c in cloths]
+    wide = scenes.DeviceCloth(_disk(9, 40))
+    for c in cloths + [wide]:
+        batch.add_instance(c.sim)
+    batch.step(cloths[0].spec.dt)
+    assert not batch.resident() and [c.sim.device_bytes() for c in cloths] == before
+    batch.remove_instance(wide.sim)
+    batch.step(cloths[0].spec.dt)
+    assert batch.resident() and all(c.sim.device_bytes() > b for c, b in zip(cloths, before))
