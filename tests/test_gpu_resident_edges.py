@@ -277,3 +277,115 @@ def test_a_batch_that_streams_keeps_no_plans_for_its_other_cloths(gpu):
     batch.remove_instance(wide.sim)
     batch.step(cloths[0].spec.dt)
     assert batch.resident() and all(c.sim.device_bytes() > b for c, b in zip(cloths, before))
+
+
+@pytest.mark.parametrize("shuffle", [False, True])
+@pytest.mark.parametrize("tile_rows", [256, 512, 1024])
+def test_streaming_solve_below_a_grid_limit(gpu, tile_rows, shuffle):
+    """A grid limit below the cloth's parts leaves its solve to the staged
+    single-barrier kernel: 16-bit and 32-bit entries, tiles of several sizes,
+    against the resident solve of the same cloth (the tolerances of
+    test_gpu_resident.py, for its reasons)."""
+    import helpers
+    from chysx import scenes
+
+    a, b = (scenes.DeviceCloth(_spec(52, 51, 5, shuffle)) for _ in range(2))  # 11 parts of 256 rows; 6 of 512
+    b.sim.set_tile_rows(tile_rows)
+    b.sim.set_grid_blocks(3)
+    for _ in range(3):
+        a.step()
+        b.step()
+        assert a.sim.resident() and not b.sim.resident() and b.sim.debug_entries16() != shuffle
+        assert abs(a.sim.last_pcg_iterations() - b.sim.last_pcg_iterations()) <= 1
+        assert helpers.rel_maxnorm(a.state()[0], b.state()[0]) <= 1e-6
+
+
+def test_a_cloth_without_a_plan_against_the_oracle(gpu):
+    """Valence 9: a row of 18 blocks, wider than a plan's."""
+    import helpers
+    from chysx import scenes
+
+    spec = _disk(9, 40)
+    cloth, oracle = scenes.DeviceCloth(spec), helpers.oracle_from_spec(spec)
+    for _ in range(3):
+        cloth.step()
+        oracle.step(spec.dt)
+    assert not cloth.sim.resident()
+    assert helpers.rel_maxnorm(cloth.state()[0], oracle.state()[0]) <= 1e-5
+
+
+def test_a_batch_with_a_cloth_without_a_plan(gpu):
+    """The whole batch streams then: every cloth as alone but for the order of
+    FP64 sums (the tolerances of test_gpu_resident.py); the one that streams
+    alone too, bit for bit."""
+    import chysx
+    import helpers
+    from chysx import scenes
+
+    specs = [_spec(40, 41, 1), _disk(9, 40), _spec(12, 13, 2), _spec(27, 19, 3, True)]
+    alone, mixed = ([scenes.DeviceCloth(s) for s in specs] for _ in range(2))
+    batch = chysx.ClothBatch()
+    for c in mixed:
+        batch.add_instance(c.sim)
+    for _ in range(3):
+        batch.step(specs[0].dt)
+        for c in alone:
+            c.step()
+        assert not batch.resident()
+        for k, (a, i) in enumerate(zip(alone, batch.last_pcg_iterations())):
+            assert abs(a.sim.last_pcg_iterations() - i) <= 1, k
+    for k, (a, m) in enumerate(zip(alone, mixed)):
+        assert helpers.rel_maxnorm(m.state()[0], a.state()[0]) <= 1e-6, k
+    assert np.array_equal(alone[1].state()[0], mixed[1].state()[0])
+
+
+@pytest.mark.parametrize("nx,ny,shuffle", [(16, 32, False), (27, 19, False), (64, 64, False), (27, 19, True)])
+def test_bf16_velocities_and_residuals_are_the_streaming_solves(gpu, nx, ny, shuffle):
+    """Velocities are the solution over the time step, so they show what
+    positions of a metre hide.  Same operations but for the rounding of alpha
+    and beta (6e-8 each, over at most 60 iterations of a preconditioned system
+    whose condition is well below 1e4): 1e-3 of the largest velocity; the
+    residual by less than an iteration changes it."""
+    import helpers
+    from chysx import scenes
+
+    a, b = (scenes.DeviceCloth(_spec(nx, ny, 100 * nx + ny, shuffle)) for _ in range(2))
+    for c in (a, b):
+        c.sim.set_bf16_blocks(True)
+    b.sim.set_lds_staging(False)  # the streaming solve
+    for _ in range(4):
+        a.step()
+        b.step()
+        assert a.sim.resident() and not b.sim.resident()
+        assert helpers.rel_maxnorm(a.state()[1], b.state()[1]) <= 1e-3
+        ra, rb = a.sim.last_relative_residual(), b.sim.last_relative_residual()
+        assert ra <= 2.0 * rb and (a.sim.last_pcg_iterations() == 60 or ra <= 1e-6)
+
+
+@pytest.mark.parametrize("grid", [0, 16, 13])
+@pytest.mark.parametrize("count", [6, 1030])
+def test_streaming_batches_are_their_cloths_alone(gpu, grid, count):
+    """A batch that a wide cloth leaves to the staged streaming kernel: every
+    cloth bit for bit as streamed alone (global gathers, the same sums in the
+    same order).  1030 instances are more than the compacted tile list holds."""
+    import chysx
+    from chysx import scenes
+
+    specs = scenes.batched(seed=15, count=count, lo=4, hi=48 if count < 1000 else 7)
+    dt = specs[0].dt
+    specs.append(_disk(9, 40))
+    alone, mixed = ([scenes.DeviceCloth(s) for s in specs] for _ in range(2))
+    batch = chysx.ClothBatch()
+    for c in mixed:
+        batch.add_instance(c.sim)
+    batch.set_grid_blocks(grid)
+    for c in alone:
+        c.sim.set_lds_staging(False)
+    for _ in range(2):
+        batch.step(dt)
+        for c in alone:
+            c.step(dt)
+        assert not batch.resident()
+        assert batch.last_pcg_iterations() == [c.sim.last_pcg_iterations() for c in alone]
+    for a, m in zip(alone, mixed):
+        assert all(np.array_equal(p, q) for p, q in zip(a.state(), m.state()))
