@@ -26,13 +26,16 @@ struct Exchange {
 // The number of the next launch, 1 .. kResEpochs, and whether old tags have to
 // be cleared before it: numbers start over, so no word may keep one.  Not
 // every launch that counts runs the resident kernel (an assembly by itself,
-// the streaming kernels), so the flag stays until that kernel has cleared.
+// the streaming kernels), so the flag stays until that kernel has run, and so
+// cleared: `solved`, the instances that it finished since the last number, is
+// not zero then.  (The kernel taking the flag back itself cost 2 us a solve.)
 constexpr unsigned kResEpochs = 255u;
 struct Launch {
     unsigned long long number, clear;
 };
-constexpr Launch next_launch(Launch last) {
-    return last.number >= kResEpochs ? Launch{1ull, 1ull} : Launch{last.number + 1ull, last.clear};
+constexpr Launch next_launch(Launch last, unsigned long long solved) {
+    return last.number >= kResEpochs ? Launch{1ull, 1ull}
+                                     : Launch{last.number + 1ull, solved != 0ull ? 0ull : last.clear};
 }
 
 }  // namespace chx

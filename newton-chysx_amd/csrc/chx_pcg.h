@@ -81,9 +81,9 @@ __device__ __forceinline__ void reset_resident(unsigned long long* xbuf) {
     if (xbuf == nullptr) return;
     if (threadIdx.x < kResGroups) xbuf[RES_IDLE + 16 * threadIdx.x] = 0ull;
     if (threadIdx.x == 0) {
+        const Launch next = next_launch({xbuf[RES_EPOCH], xbuf[RES_CLEAR]}, xbuf[RES_DONE]);
         xbuf[RES_NEXT] = 0ull;
         xbuf[RES_DONE] = 0ull;
-        const Launch next = next_launch({xbuf[RES_EPOCH], xbuf[RES_CLEAR]});
         xbuf[RES_EPOCH] = next.number;
         xbuf[RES_CLEAR] = next.clear;
     }

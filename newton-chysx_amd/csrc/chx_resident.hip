@@ -1118,7 +1118,6 @@ __global__ __launch_bounds__(kThreads, 2) void resident_kernel(chx_cloth_batch B
         for (u64 k = RES_MAIL + u64(blockIdx.x) * kThreads + threadIdx.x; k < B.res_xwords; k += u64(G) * kThreads)
             st64(&B.xbuf[k], 0ull);
         if (!grid_sync(bar, unsigned(G))) return;
-        if (blockIdx.x == 0 && threadIdx.x == 0) st64(&B.xbuf[RES_CLEAR], 0ull);  // every workgroup has read it
     }
     __syncthreads();
     // groups: workgroups b = x (mod groups); with eight, the dispatcher places

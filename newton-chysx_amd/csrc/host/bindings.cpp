@@ -565,10 +565,11 @@ PYBIND11_MODULE(_chysx_native, m) {
             // the resident kernel runs after it, whether it clears old tags.
             py::list out;
             chx::Launch at{0, 0};
+            bool ran = false;
             for (const bool resident : runs) {
-                at = chx::next_launch(at);
+                at = chx::next_launch(at, ran ? 1 : 0);
                 out.append(py::make_tuple(at.number, resident && at.clear != 0));
-                if (resident) at.clear = 0;
+                ran = resident;
             }
             return out;
         },
