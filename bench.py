@@ -107,8 +107,8 @@ def kernel_breakdown(cloth, dt, stream, lanes, reps=5, pcg_form=0, tuned=None):
         "vertices": N, "off_diag_blocks": nnz, "triangles": T, "dihedrals": D, "pins": P, "pcg_iterations": k,
         "assembly": {"ms": round(e_ms, 4), "bytes": e_b, "GB_per_s": rate(e_b, e_ms)},
         "pcg_launch": {"ms": round(s_ms, 4), "bytes": s_b, "GB_per_s": rate(s_b, s_ms)},
-        "pcg_form": pcg_form,
-        "note": "algorithmic bytes (reference counts); phase times from the solver's per-barrier trace, barrier "
+        "pcg_form": pcg_form, "resident": b.resident(),
+        "note": "algorithmic bytes (reference counts; the resident solve reads the matrix once); phase times from the solver's per-barrier trace, barrier "
                 "waits included; a 256x256 working set fits the 256 MB Infinity Cache",
     }
     if pcg_form == 0:

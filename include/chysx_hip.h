@@ -327,7 +327,18 @@ typedef struct chx_rows_plan {
  * the kernel arguments); its element and unit lists are implied by the
  * counts, and so is its tile list when `tiles` is NULL (tile_rows rows per
  * tile, CHX_TILE_ROWS when tile_rows is 0; n_tiles = ceil(n_rows / that)),
- * which saves the PCG a load of the tile record per tile and phase. */
+ * which saves the PCG a load of the tile record per tile and phase.
+ *
+ * The library checks a single instance's resident plan against xbuf; device
+ * tables it cannot read.  Of an instance table the caller guarantees: every
+ * instance with rows has a plan of the batch's res_form, its res_parts match
+ * its rows and part size, and its exchange area (CHX_RES_XWORDS words from
+ * res_xbase, a multiple of 16, at or above CHX_RES_CONTROL_WORDS) lies in
+ * xbuf and overlaps no other; res_items names every such instance once, with
+ * its parts; a leading item's ranks, first rank + parts, fit res_grid, and
+ * the others' parts fit a group (res_grid / res_groups workgroups).  Accesses
+ * outside xbuf are dropped by the hardware and waits are bounded, so a wrong
+ * exchange area ends in a reported time-out; a wrong plan does not. */
 typedef struct chx_cloth_batch {
     int n_instances;
     int n_tiles;
@@ -371,7 +382,9 @@ typedef struct chx_cloth_batch {
                                      /* barrier e (0: after set-up; two-barrier form:  */
                                      /* 2k+1 / 2k+2 after phase A / B of iteration k;  */
                                      /* single-barrier form: k+1 after phase k),       */
-                                     /* written by workgroup 0                         */
+                                     /* written by workgroup 0; resident PCG: one      */
+                                     /* entry per exchange of the solves that          */
+                                     /* workgroup 0 takes part in, in its order        */
     int trace_entries;               /* capacity of `trace` in entries (2 words each) */
     unsigned wait_ticks;             /* bound of every grid-barrier wait in 100 MHz   */
                                      /* ticks (0: 1e8, one second); past it the solve */

@@ -1,9 +1,12 @@
 """Autotuner of the batched cloth substep.
 
-Sweeps the SpMV form (LDS-staged stages or global gathers), the persistent
-PCG grid size (workgroups per compute unit, up to what the form
-keeps co-resident) and the rows per PCG tile (256, 512, 1024) on the actual
-batch (lanes per block row only shape the CSR SpMV of caller-provided
+The default is the resident solve, which has no settings: every trial whose
+grid holds the batch's cloths runs it, and the sweep keeps it unless a
+streaming trial is faster.  What is swept shapes the streaming kernels, for
+batches with a cloth that the resident solve cannot take: the SpMV form
+(LDS-staged stages or global gathers), the persistent PCG grid size
+(workgroups per compute unit, up to what the form keeps co-resident) and the
+rows per PCG tile (256, 512, 1024) on the actual batch (lanes per block row only shape the CSR SpMV of caller-provided
 row-major matrices; the cloth instances' sliced SpMV runs one lane per row,
 so `lanes` defaults to a single value), timing whole substeps with HIP events on the
 caller's stream, and keeps the fastest.  Results are cached in a JSON file

@@ -22,8 +22,11 @@ A job moves through four states:
 
 So requests that arrive while others run join as soon as memory and their
 set-up allow, and their substeps overlap on the device with everyone
-else's.  Each job's result is identical alone and in any mix (the batch runs
-the same kernels on the job's own arrays with per-instance reductions).
+else's.  Each job's result is identical alone and in any mix of jobs that take
+the resident solve (per-instance operations and reductions that do not depend
+on the batch); one that cannot (a vertex of valence 9 or more, more than
+262,144 vertices) leaves the batch it is in to the streaming solve, whose FP64
+sums have another order.
 
 Reported: throughput (vertex-substeps/s), p50/p99 request latency (arrival
 to the end of the substep that finishes the job) over the completed jobs and,

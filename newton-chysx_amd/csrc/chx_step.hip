@@ -1691,8 +1691,8 @@ __global__ __launch_bounds__(kBlock) void pcg1_kernel(chx_cloth_batch B, int fin
 // matrix of a 512x512 grid) if enough loads are in flight: a row's blocks are
 // loaded beside their column indices and the diagonal beside the row offsets,
 // so a row takes three round trips (offsets and diagonal; blocks and indices;
-// source vector), not five.  With the matrix in HBM 34.4 us before, 30.5 now
-// (4.65 TB/s, the rate of a large copy).  Two rows per group (more registers,
+// source vector), not five.  With the matrix in HBM 33.9 us before, 29.4 now
+// (4.84 TB/s, the rate of a large copy).  Two rows per group (more registers,
 // fewer waves) took 35.5 us, a workgroup order that keeps neighbouring rows on
 // one XCD 31.6.  Per lane the sum is diag (lane 0) + off[sub] + off[sub + L] +
 // ..., then a segmented butterfly.

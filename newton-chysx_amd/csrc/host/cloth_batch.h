@@ -6,9 +6,14 @@
 // Each instance is a fully set-up ClothSimulator (buffers, mesh, element
 // sets, pins, material, PCG knobs) whose device arrays stay where they are;
 // the batch only holds a table of their descriptors and the work lists.
-// Per-instance results are identical to stepping each simulator alone: the
-// same kernels run on the same arrays and every reduction is per instance,
-// over the same tiles, in the same order.  Instances can be added and
+// Per-instance results are identical to stepping each simulator alone while
+// both run the same solver: the same operations on the same arrays, and every
+// reduction is per instance, over a tree that does not depend on the batch.
+// A batch runs one solver: when one of its cloths cannot take the resident
+// solve (no plan fits: rows of more than 16 blocks, too many rows), or a grid
+// limit is below a cloth's parts, all of them stream, and one that is resident
+// alone then differs by the order of FP64 sums (resident() tells).  Instances
+// can be added and
 // removed between substeps (continuous batching) at the cost of rebuilding
 // the table.
 #pragma once
@@ -53,7 +58,9 @@ public:
     void set_lanes_per_row(int lanes) { runner_.set_lanes_per_row(lanes); }
     int lanes_per_row() const noexcept { return runner_.lanes_per_row(); }
     void set_grid_blocks(int blocks) { runner_.set_grid_blocks(blocks); }
-    // Rows per PCG tile: a multiple of CHX_STAGE_ROWS (256).
+    // Rows per PCG tile: a multiple of CHX_STAGE_ROWS (256).  Shapes the
+    // streaming kernels, like the lanes and the SpMV form; a grid limit below
+    // a cloth's parts asks for them.
     void set_tile_rows(int rows) { runner_.set_tile_rows(rows); }
     // SpMV form of the PCG launch: LDS-staged (default) or global gathers.
     // Substeps replayed from a hipGraph of the element pass, gather pass and
@@ -65,9 +72,10 @@ public:
     void set_lds_staging(bool on) { runner_.set_lds_staging(on); }
     bool lds_staging() const noexcept { return runner_.lds_staging(); }
     bool entries16() const noexcept { return runner_.entries16(); }
-    // Solver trace of the persistent PCG launch: capacity in barrier entries
-    // (0: off); last_trace() returns {stamp in 100 MHz ticks, active
-    // instances} per barrier of the last solve.
+    // Solver trace of the persistent PCG launch: capacity in entries (0:
+    // off); last_trace() returns {stamp in 100 MHz ticks, active instances}
+    // per barrier of the last solve, or per exchange of the resident solve's
+    // first workgroup.
     void set_trace(int entries) { runner_.set_trace(entries); }
     std::vector<unsigned long long> last_trace(std::uintptr_t cuda_stream = 0) { return runner_.read_trace(cuda_stream); }
     int tile_rows() const noexcept { return runner_.tile_rows(); }

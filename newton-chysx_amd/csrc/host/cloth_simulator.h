@@ -156,8 +156,8 @@ public:
     void set_tile_rows(int rows) { runner_.set_tile_rows(rows); }
     // SpMV form of the PCG launch: LDS-staged (default) or global gathers.
     void set_lds_staging(bool on) { runner_.set_lds_staging(on); }
-    // Solver trace of the persistent PCG launch: capacity in barrier entries
-    // (0: off); last_trace() returns {stamp in 100 MHz ticks, active
+    // Solver trace of the persistent PCG launch: capacity in entries, one per
+    // barrier or exchange (0: off); last_trace() returns {stamp in 100 MHz ticks, active
     // instances} per barrier of the last solve.
     void set_trace(int entries) { runner_.set_trace(entries); }
     std::vector<unsigned long long> last_trace(std::uintptr_t cuda_stream = 0) { return runner_.read_trace(cuda_stream); }

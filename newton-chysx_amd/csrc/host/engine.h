@@ -195,8 +195,8 @@ public:
 
     // Solver trace: capacity in barrier entries (0 switches it off).
     void set_trace(int entries);
-    // {stamp (100 MHz ticks), active instances} per barrier of the last
-    // solve, up to the last one written.
+    // {stamp (100 MHz ticks), active instances} per barrier (resident: per
+    // exchange of workgroup 0) of the last solve, up to the last one written.
     std::vector<unsigned long long> read_trace(std::uintptr_t stream);
 
     // Synchronous read-backs.
