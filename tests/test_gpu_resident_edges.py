@@ -389,3 +389,39 @@ def test_streaming_batches_are_their_cloths_alone(gpu, grid, count):
         assert batch.last_pcg_iterations() == [c.sim.last_pcg_iterations() for c in alone]
     for a, m in zip(alone, mixed):
         assert all(np.array_equal(p, q) for p, q in zip(a.state(), m.state()))
+
+
+def test_a_batch_whose_waits_are_given_up(gpu):
+    """A wait bound of one tick, set by the host: every workgroup of the
+    resident solve leaves normally, pos and vel stay, the next step reports it,
+    and the steps after that are those of a batch that never gave up."""
+    import torch
+
+    import chysx
+    from chysx import scenes
+
+    specs = [_spec(n, n + 1, n) for n in (40, 33, 64, 12)]
+    sets = [[scenes.DeviceCloth(s) for s in specs] for _ in range(2)]
+    batches = [chysx.ClothBatch() for _ in sets]
+    for batch, cloths in zip(batches, sets):
+        for c in cloths:
+            batch.add_instance(c.sim)
+        batch.step(specs[0].dt)
+        assert batch.resident()
+    before = [c.state() for c in sets[0]]
+    batches[0].set_barrier_timeout_ticks(1)
+    batches[0].step(specs[0].dt)
+    torch.cuda.synchronize()
+    batches[0].set_barrier_timeout_ticks(0)
+    with pytest.raises(RuntimeError, match="timed out"):
+        batches[0].step(specs[0].dt)
+    for c, (pos, vel) in zip(sets[0], before):
+        assert np.array_equal(c.state()[0], pos) and np.array_equal(c.state()[1], vel)
+    for cloths in sets:
+        for c in cloths:
+            c.sim.debug_set_warm_start(np.zeros((c.spec.n, 3), np.float32))
+    for _ in range(3):
+        for batch in batches:
+            batch.step(specs[0].dt)
+    for a, b in zip(*sets):
+        assert np.array_equal(a.state()[0], b.state()[0]) and np.array_equal(a.state()[1], b.state()[1])
