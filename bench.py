@@ -450,19 +450,26 @@ def main():
     # The phases of iterations in which every instance is solving, from the
     # solver's per-barrier trace of one more solve.  Single-barrier form: a
     # whole iteration per phase, algorithmic bytes B_iter.  Two-barrier form:
-    # the SpMV phase (q = A p with the folded p update), B_spmv + 36N.
+    # the SpMV phase (q = A p with the folded p update), B_spmv + 36N.  The
+    # resident solve has no common phases (its gangs iterate by themselves):
+    # the time between the exchanges of workgroup 0, one an iteration.
     spmv_phase = iteration_phase = None
-    # The resident solve has no common phases: its gangs iterate by themselves.
-    tr = np.zeros((0, 2), np.int64)
-    if not resident:
-        batch.set_trace(1024)
-        with torch.cuda.stream(stream):
-            batch.assemble(dt, sh)
-            batch.solve(sh)
-            tr = np.array(batch.last_trace(sh)).astype(np.int64)
-        batch.set_trace(0)
+    batch.set_trace(1024)
+    with torch.cuda.stream(stream):
+        batch.assemble(dt, sh)
+        batch.solve(sh)
+        tr = np.array(batch.last_trace(sh)).astype(np.int64)
+    batch.set_trace(0)
     n_all, nnz_all = int(sizes[:, 0].sum()), int(sizes[:, 1].sum())
-    if args.pcg_form == 0:
+    if resident:
+        full = []
+        if len(tr) > 1:
+            us = np.diff(tr[:, 0]) / 100.0
+            iteration_phase = {"iterations": len(us), "us_per_iteration": round(float(np.median(us)), 2),
+                               "note": "median time between two exchanges of workgroup 0, over the cloths it takes "
+                                       "part in (one exchange per iteration)"}
+            log(f"iteration of workgroup 0's cloths: {iteration_phase['us_per_iteration']} us (median)")
+    elif args.pcg_form == 0:
         full = [k for k in range(1, len(tr) - 1) if tr[k + 1, 1] == len(specs)]
         if full:
             us = np.array([(tr[k + 1, 0] - tr[k, 0]) / 100.0 for k in full])
