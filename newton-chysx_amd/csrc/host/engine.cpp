@@ -845,6 +845,7 @@ void BatchRunner::set_grid_blocks(int g) {
     // What queued launches may still read is waited for only where it changes:
     // most limits leave a batch's lists as they are, and one cloth has none.
     bool wrote = false;
+    relayout_ = true;  // for the next update, should this throw
     if (desc_.inst == nullptr) {
         std::vector<chx_instance> one{desc_.single};
         wrote = layout_resident(one, 0, true);
@@ -854,13 +855,13 @@ void BatchRunner::set_grid_blocks(int g) {
         wrote = layout_resident(table_host_, 0, true);
         if (std::memcmp(was.data(), table_host_.data(), was.size() * sizeof(chx_instance)) != 0) {
             if (!wrote) check(chx_device_synchronize(), "engine", "work list rebuild");
-            wrote = table_stale_ = true;
+            wrote = true;
             table_.host() = table_host_;
             table_.copy_to_device();
             desc_.inst = table_.gpu_data();
-            table_stale_ = false;
         }
     }
+    relayout_ = false;
     if (wrote) check(chx_device_synchronize(), "engine", "work list rebuild");
 }
 

@@ -104,6 +104,25 @@ CASES = {
         REQUIRE(syncs == 0 && copies == 0);
     }
 """,
+    # the same when a grid limit asks for the area
+    "refused area of a grid limit": r"""
+    for (int many = 0; many < 2; ++many) {
+        BatchRunner r;
+        r.set_grid_blocks(4);
+        std::vector<chx_instance> ds(many ? 3 : 1, cloth(2000, 100));
+        r.bind_many(ds);
+        REQUIRE(!r.resident() && r.desc().xbuf == nullptr);
+        refuse = 0;
+        bool thrown = false;
+        try { r.set_grid_blocks(0); } catch (const std::exception&) { thrown = true; }
+        refuse = -1;
+        REQUIRE(thrown && !r.resident() && r.desc().xbuf == nullptr);
+        r.update_many(ds, 0);
+        REQUIRE(r.resident() && live.count(r.desc().xbuf));
+        const chx_instance& d = many ? r.desc().inst[0] : r.desc().single;
+        REQUIRE(d.res_xbase == CHX_RES_CONTROL_WORDS);
+    }
+""",
     # a grid limit is a number unless the work list changes with it
     "grid limit": r"""
     for (int many = 0; many < 2; ++many) {
